@@ -106,8 +106,8 @@ def compile_order(ref=REF):
 
 
 def build(force=False, verbose=False):
-    if not os.path.isdir(REF):
-        print(f"build_ref: {REF} absent, nothing built")
+    if not all(os.path.isfile(os.path.join(REF, s)) for s in ROOT_SOURCES):
+        print(f"build_ref: sources absent under {REF}, nothing built")
         return None
     fc = _flang()
     if fc is None:
