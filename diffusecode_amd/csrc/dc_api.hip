@@ -11,6 +11,7 @@
 #include <cstring>
 #include <string>
 #include <functional>
+#include <map>
 #include <vector>
 
 #include "../../include/diffuse_turbo.h"
@@ -144,11 +145,147 @@ static int kchunk_atoms(long long wgs, long long natoms, int prec) {
 //   them for natoms atoms.  Small problems fill the device with few work
 //   items, so the rounds term favours smaller tiles there; large problems
 //   reduce to padded work x eff.  natoms <= 0: padded work x eff.
-Plan plan_gemm(Grid &g, int forced, int only_mapping, int prec, long long natoms) {
+// Fold tiles (mirrored pairs, dc_fold.h) apply where a side is one uniform
+// run of points and fold_mask allows it; forced >= 0 naming one where none
+// applies is ignored.
+int gemm_items(const GemmGeom &gg, int tile) {
+    const TileInfo ti = gemm_tile_info(tile);
+    if (!ti.fold) return ((gg.R + ti.rt - 1) / ti.rt) * ((gg.C + ti.ct - 1) / ti.ct);
+    const int na = gg.fold == FOLD_ROWS ? gg.C : gg.R, nb = gg.fold == FOLD_ROWS ? gg.R : gg.C;
+    return ((na + ti.rt - 1) / ti.rt) * (((nb + 1) / 2 + ti.ct / 2 - 1) / (ti.ct / 2));
+}
+
+int fold_side(const GemmGeom &gg, int fold_mask, int tile) {
+    if (!gemm_tile_info(tile).fold) return 0;
+    GemmGeom a = gg, b = gg;
+    a.fold = (fold_mask & FOLD_COLS) && gg.C0 >= gg.C ? FOLD_COLS : 0;
+    b.fold = (fold_mask & FOLD_ROWS) && gg.R0 >= gg.R ? FOLD_ROWS : 0;
+    if (!a.fold || !b.fold) return a.fold | b.fold;
+    return gemm_items(b, tile) < gemm_items(a, tile) ? b.fold : a.fold;
+}
+
+// Time model of a launch with a fold tile, in microseconds on one MI355X: a
+// stage of 32 atoms costs its MFMAs on a SIMD's two waves (measured at the
+// sustained clock: 0.091 per 16 x 16 block for the three products, 0.49 for
+// FP32) plus the operand generation that does not overlap with
+// them, and an item its set-up and epilogue.
+static double fold_stage_us(const TileInfo &ti, int prec) {
+    const double wr = ti.rt / 128.0, wc = ti.ct / 16.0;
+    const double m = prec == DC_PREC_FP32 ? 0.49 : 0.091;
+    return m * wr * wc + 0.45 + 0.55 * wr + 0.02 * wc;
+}
+static double fold_item_us(const TileInfo &ti, int prec, double atoms) {
+    return std::ceil(atoms / 32.0) * fold_stage_us(ti, prec) + 7.0;
+}
+// ... and of the FP64 reduction of its planes: the traffic of the planes, or
+// the chain of dependent batches of 4 planes that each pixel's thread walks.
+static double reduce_us(double planes, double plane_elems) {
+    return std::max(planes * plane_elems * 8.0 / 4.0e6, planes * 0.18);
+}
+
+// Shortest and longest slice of the fold tiles.  The FP32 accumulators of the
+// split schemes lose a little of every term once their sum is large, so the
+// error at the Bragg peaks grows with the slice (256,000 atoms, FP16X3, I:
+// 2,150 / 4,300 / 8,600 / 17,200 atoms 0.6 / 2.7 / 4.9 / 6.8e-7, and 6.8e-7 to
+// 1.2e-6 for 17,067 atoms in dc_gemm.hip; 8,704 costs 1% more planes and items
+// than twice that).  Launches that fill the device with shorter slices cap
+// them at the length that gives 1,024 items of 256 x 176 outputs, as
+// kchunk_atoms does (lots of 4,000 atoms: error of the cross-lot variance
+// 3.2e-7 with slices of 700 atoms in dc_gemm.hip, 7.3e-7 with 2,000 here).
+// FP32 sums are FP64: its slices are bounded by the one rounding of a plane.
+constexpr int KCHUNK_FOLD_MIN = 64, KCHUNK_FOLD_MAX = 8704, KCHUNK_FOLD_FP32 = 2048;
+static int fold_cap(const GemmGeom &gg, long long natoms, int prec) {
+    if (prec == DC_PREC_FP32) return KCHUNK_FOLD_FP32;
+    const long long k = (long long)((double)natoms * gg.R * gg.C / (256.0 * 176.0 * 1024.0));
+    return (int)std::min<long long>(std::max<long long>(k, 1024), KCHUNK_FOLD_MAX);
+}
+
+// Makespan of counted groups of equal items, (microseconds, count) in any
+// order, on ncu machines, the longest items first.
+static double makespan(std::vector<std::pair<double, long long>> groups, int ncu) {
+    std::sort(groups.begin(), groups.end(), std::greater<std::pair<double, long long>>());
+    std::map<double, long long> load;   // machines by finishing time
+    load[0.0] = ncu;
+    for (auto &gr : groups) {
+        long long left = gr.second;
+        const long long full = left / ncu - 1;
+        if (full > 0) {   // whole rounds shift every machine alike
+            std::map<double, long long> l2;
+            for (auto &kv : load) l2[kv.first + gr.first * (double)full] += kv.second;
+            load.swap(l2);
+            left -= full * ncu;
+        }
+        while (left > 0) {
+            auto it = load.begin();
+            const double t = it->first;
+            const long long n = std::min(left, it->second);
+            it->second -= n;
+            if (it->second == 0) load.erase(it);
+            load[t + gr.first] += n;
+            left -= n;
+        }
+    }
+    return load.rbegin()->first;
+}
+
+// Best slice length of a fold tile for the (type, count) segments of a
+// launch, and its predicted time: every segment is split into ceil(n / k)
+// near-equal slices (add_segments), one item per (slice, tile).  The lengths
+// tried are those of 1, 2, 3, ... slices of the longest segment, thinned to
+// steps of about 1/8 once there are many.
+int fold_slices(const GemmGeom &gg, int tile, const std::vector<std::pair<int, int>> &segs, int prec, double &best_us) {
+    const TileInfo ti = gemm_tile_info(tile);
+    const long long wgs = gemm_items(gg, tile);
+    const int ncu = device_cu_count();
+    // segments by size: a run has few distinct ones
+    std::map<int, long long, std::greater<int>> sizes;
+    long long natoms = 0;
+    for (auto &sg : segs)
+        if (sg.second > 0) {
+            sizes[sg.second]++;
+            natoms += sg.second;
+        }
+    const int cap = fold_cap(gg, natoms, prec);
+    best_us = 1e300;
+    if (sizes.empty()) return cap;
+    const int nmax = sizes.begin()->first;
+    int best = cap, n0 = (nmax + cap - 1) / cap;
+    for (int ns = n0;; ns = std::max(ns + 1, ns + ns / 8)) {
+        const int k = std::min(cap, (nmax + ns - 1) / ns);
+        if (ns > n0 && k < KCHUNK_FOLD_MIN) break;
+        std::vector<std::pair<double, long long>> groups;
+        long long planes = 0;
+        for (auto &kv : sizes) {
+            const long long q = (kv.first + k - 1) / k;
+            const int len = (int)((kv.first + q - 1) / q);
+            groups.push_back({fold_item_us(ti, prec, len), q * kv.second * wgs});
+            planes += q * kv.second;
+        }
+        const double us = makespan(groups, ncu) + reduce_us((double)planes, (double)gg.P);
+        if (us < best_us * (1.0 - 1e-9)) {
+            best_us = us;
+            best = k;
+        }
+        if (k <= 1) break;
+    }
+    return best;
+}
+
+Plan plan_gemm(Grid &g, int forced, int only_mapping, int prec, long long natoms, int fold_mask) {
     Plan best;
     double best_cost = 1e300;
     const int nt = gemm_num_tiles();
     const int ncu = device_cu_count();
+    const bool acc64 = prec == SCHEME_FP32_ACC64;
+    // The folded side needs a mapping that leaves it unwrapped.  FP16X2, whose
+    // results are only good to their rounding, and the FP64-sum scheme keep the
+    // general tiles.
+    const bool can_fold = !acc64 && prec != DC_PREC_FP16X2 && (((fold_mask & FOLD_COLS) && (g.f[2] <= 1 || only_mapping != 0)) ||
+                                     ((fold_mask & FOLD_ROWS) && only_mapping != 1));
+    if (forced >= 0) {
+        const TileInfo ti = gemm_tile_info(forced);
+        if ((ti.fold && !can_fold) || (acc64 && !ti.acc64) || (prec == DC_PREC_FP32 && ti.no_fp32)) forced = -1;
+    }
     for (int mapping = 0; mapping < 2; ++mapping) {
         if (mapping == 1 && g.f[2] <= 1) continue;
         if (only_mapping >= 0 && mapping != only_mapping) continue;
@@ -174,25 +311,25 @@ Plan plan_gemm(Grid &g, int forced, int only_mapping, int prec, long long natoms
             ps[0] = 1; ps[1] = gg.R0; ps[2] = gg.Rs;
         }
         gg.P = (long long)gg.Rs * gg.C;
-        const bool acc64 = prec == SCHEME_FP32_ACC64;
-        // FP32 with FP64 sums is built for a few tiles only; a forced tile
-        // outside them is ignored for it
-        const bool use_forced = forced >= 0 && (!acc64 || gemm_tile_info(forced).acc64) &&
-                                !(prec == DC_PREC_FP32 && gemm_tile_info(forced).no_fp32);
         for (int t = 0; t < nt; ++t) {
-            if (use_forced && t != forced) continue;
+            if (forced >= 0 && t != forced) continue;
             TileInfo ti = gemm_tile_info(t);
-            if (!use_forced && ti.split_only && prec == DC_PREC_FP32) continue;
+            if (forced < 0 && (bool)ti.fold != can_fold) continue;
+            if (forced < 0 && ti.split_only && prec == DC_PREC_FP32) continue;
             if (acc64 && !ti.acc64) continue;
             if ((acc64 || prec == DC_PREC_FP32) && ti.no_fp32) continue;
-            const double work = (double)padded(gg.R, ti.rt) * (double)padded(gg.C, ti.ct);
+            gg.fold = fold_side(gg, fold_mask, t);
+            if (ti.fold && !gg.fold) continue;
+            const long long wgs = gemm_items(gg, t);
+            const double work = (double)wgs * ti.rt * ti.ct;
             double cost;
-            if (prec == DC_PREC_FP32 || acc64 || use_forced) {
+            if (ti.fold && forced < 0 && natoms > 0) {
+                (void)fold_slices(gg, t, {{0, (int)std::min<long long>(natoms, INT32_MAX)}}, prec, cost);
+            } else if (prec == DC_PREC_FP32 || acc64 || forced >= 0) {
                 cost = work * (1.0 + 0.5 * (16.0 / ti.rt + 16.0 / ti.ct));
             } else if (natoms <= 0) {
                 cost = work * ti.eff;
             } else {
-                const long long wgs = (long long)((gg.R + ti.rt - 1) / ti.rt) * ((gg.C + ti.ct - 1) / ti.ct);
                 const long long k = kchunk_atoms(wgs, natoms, prec);
                 const long long nsl = (natoms + k - 1) / k;
                 const long long rounds = (wgs * nsl + ncu - 1) / ncu;
@@ -212,10 +349,21 @@ Plan plan_gemm(Grid &g, int forced, int only_mapping, int prec, long long natoms
     return best;
 }
 
+int mirrored_sides(const GemmGeom &gg, const float *sq) {
+    auto mirrored = [](const float *v, int n) {
+        float top = 0.0f;
+        for (int i = 0; i < n; ++i) top = std::max(top, std::fabs(v[i]));
+        for (int i = 0; i < n / 2; ++i)
+            if (!(std::fabs(v[i] - v[n - 1 - i]) <= 4e-7f * top)) return false;
+        return true;
+    };
+    return (mirrored(sq, gg.R) ? FOLD_ROWS : 0) | (mirrored(sq + gg.R, gg.C) ? FOLD_COLS : 0);
+}
+
 int kchunk_for(const Plan &pl, long long natoms_batch, int prec) {
-    TileInfo ti = gemm_tile_info(pl.tile);
-    long long wgs = (long long)((pl.gg.R + ti.rt - 1) / ti.rt) * ((pl.gg.C + ti.ct - 1) / ti.ct);
-    return kchunk_atoms(wgs, natoms_batch, prec);
+    if (gemm_tile_info(pl.tile).fold)
+        return kchunk_for(pl, std::vector<std::pair<int, int>>{{0, (int)std::min<long long>(natoms_batch, INT32_MAX)}}, prec);
+    return kchunk_atoms(gemm_items(pl.gg, pl.tile), natoms_batch, prec);
 }
 
 // Slice length for the (type, count) segments of one
@@ -235,6 +383,10 @@ int kchunk_for(const Plan &pl, long long natoms_batch, int prec) {
 // Launches that already have 16 rounds of items or more, and
 // populations (many segments), keep the rule of kchunk_atoms.
 int kchunk_for(const Plan &pl, const std::vector<std::pair<int, int>> &segs, int prec) {
+    if (gemm_tile_info(pl.tile).fold) {
+        double us;
+        return fold_slices(pl.gg, pl.tile, segs, prec, us);
+    }
     long long natoms = 0;
     for (auto &sg : segs) natoms += std::max(sg.second, 0);
     const int k0 = kchunk_for(pl, natoms, prec);
@@ -244,8 +396,7 @@ int kchunk_for(const Plan &pl, const std::vector<std::pair<int, int>> &segs, int
     const bool capped = prec == DC_PREC_FP32;
     const int kmax = capped ? k0 : KCHUNK_SEARCH_MAX;
     const int kmin = capped ? k0 / 2 : KCHUNK_MIN;
-    const TileInfo ti = gemm_tile_info(pl.tile);
-    const long long wgs = (long long)((pl.gg.R + ti.rt - 1) / ti.rt) * ((pl.gg.C + ti.ct - 1) / ti.ct);
+    const long long wgs = gemm_items(pl.gg, pl.tile);
     const int ncu = device_cu_count();
     long long items0 = 0;
     for (auto &sg : segs)
@@ -315,11 +466,30 @@ void add_segments(SliceSet &s, const std::vector<std::pair<int, int>> &segs, int
     }
 }
 
-int run_gemm(dc_ctx *c, const Plan &pl, int nslice, float2 *partial, const float *sq) {
+int run_gemm(dc_ctx *c, const Plan &pl, const std::vector<int> &beg, float2 *partial, const float *sq) {
     GemmGeom gg = launch_geom(c, pl.gg);
     gg.pad_hash = c->rec_hash && !sq;
+    const int nslice = (int)beg.size() - 1;
     if (nslice <= 0) return 0;
     int st = 0;
+    // Slices of uneven length over more than one round of work-groups start
+    // longest first; even ones keep the XCD-chunked order of the kernels
+    // (three types of 85,100 to 85,600 atoms: 17 slices, some 1/6 longer than
+    // the others, ran four rounds for three).
+    if (nslice <= 4096 && (long long)nslice * gemm_items(gg, pl.tile) > device_cu_count()) {
+        int lo = beg[1] - beg[0], hi = lo;
+        for (int q = 1; q < nslice; ++q) {
+            lo = std::min(lo, beg[q + 1] - beg[q]);
+            hi = std::max(hi, beg[q + 1] - beg[q]);
+        }
+        if (hi - lo > hi / 50) {
+            std::vector<int> order(nslice);
+            for (int q = 0; q < nslice; ++q) order[q] = q;
+            std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return beg[x + 1] - beg[x] > beg[y + 1] - beg[y]; });
+            if ((st = upload(c, c->slice_order, order.data(), order.size()))) return st;
+            gg.order = ptr<int>(c->slice_order);
+        }
+    }
     hipEvent_t e0, e1;
     if ((st = mark(c, e0))) return st;
     // launch in chunks of slices so that the cancel flag is polled
@@ -899,7 +1069,7 @@ int gemm_segments(dc_ctx *c, const Grid &g, const Plan &pl, GatherList &gl,
     for (int v : group_seg) gsl.push_back(ss.seg_first[v]);
     if ((st = upload(c, c->lot_slice, gsl.data(), gsl.size()))) return st;
     if ((st = ensure(c, c->partial, sizeof(float2) * gg.P * std::max(nslice, 1)))) return st;
-    return run_gemm(c, pl, ngemm, ptr<float2>(c->partial));
+    return run_gemm(c, pl, ss.beg, ptr<float2>(c->partial));
 }
 
 }  // namespace

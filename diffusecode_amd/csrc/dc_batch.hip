@@ -23,6 +23,7 @@ struct BatchState {
     // key: the shape of the batch
     int nmembers = 0, nscat = 0, ncfact = 0, prec = -1, tile_forced = -2, autotune = -1, graphs = -1;
     int slice_atoms = -1, dither = -1;
+    int fold_mask = 0;                       // sides the mirrored-pair tiles may fold (dc_fold.h)
     bool want_grad = false, want_icalc = false, have_weight = false, any_b = false;
     std::vector<int64_t> atom_beg;
     std::vector<int> type;
@@ -111,8 +112,7 @@ int check_desc(dc_ctx *c, const dc_batch_desc *d) {
 
 // s^2 row / column parts for every member's metric; errors on grids that are
 // not metric-orthogonal between rows and columns when B or gradients need it.
-int member_sq(dc_ctx *c, const BatchState &b, const dc_batch_desc *d, std::vector<float> &sq, bool need_sep) {
-    const GemmGeom &gg = b.pl.gg;
+int member_sq(dc_ctx *c, const Grid &g, const GemmGeom &gg, const dc_batch_desc *d, std::vector<float> &sq, bool need_sep) {
     const int stride = gg.R + gg.C;
     sq.assign((size_t)stride * d->nmembers, 0.0f);
     const double *v1 = d->vi, *v2 = d->vi + 3, *v3 = d->vi + 6;
@@ -136,12 +136,12 @@ int member_sq(dc_ctx *c, const BatchState &b, const dc_batch_desc *d, std::vecto
         }
         for (int col = 0; col < gg.C; ++col) {
             const int j = col % gg.C0, l = col / gg.C0;
-            if (j >= b.g.f[1]) continue;
+            if (j >= g.f[1]) continue;
             double v[3];
             for (int k = 0; k < 3; ++k) v[k] = j * v2[k] + l * v3[k];
             s[gg.R + col] = (float)((dotg(v, G, v) + 2.0 * dotg(v, G, d->eck)) / 4.0);
         }
-        Grid gm = b.g;
+        Grid gm = g;
         for (int k = 0; k < 9; ++k) gm.rten[k] = G[k];
         if (max_corner_bin(gm) >= d->ncfact) return set_err(c, DC_ERR_ISTL, DC_ER_FOUR, "sin(theta)/lambda beyond table");
     }
@@ -184,6 +184,19 @@ int make_slices(dc_ctx *c, BatchState &b, int kchunk) {
     return ensure(c, b.partial, sizeof(float2) * gg.P * std::max(b.nslice, 1));
 }
 
+Grid batch_grid(const dc_batch_desc *d) {
+    Grid g{};
+    for (int k = 0; k < 3; ++k) {
+        g.n[k] = g.f[k] = d->inc[k];
+        g.xm[k] = d->eck[k];
+        g.uin[k] = d->vi[k];
+        g.vin[k] = d->vi[3 + k];
+        g.win[k] = d->vi[6 + k];
+    }
+    g.P = (long long)g.f[0] * g.f[1] * g.f[2];
+    return g;
+}
+
 int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
     b.nmembers = d->nmembers;
     b.nscat = d->nscat;
@@ -202,15 +215,8 @@ int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
     std::memcpy(b.vi, d->vi, sizeof(b.vi));
     std::memcpy(b.inc, d->inc, sizeof(b.inc));
     Grid &g = b.g;
-    for (int k = 0; k < 3; ++k) {
-        g.n[k] = g.f[k] = d->inc[k];
-        g.xm[k] = d->eck[k];
-        g.uin[k] = d->vi[k];
-        g.vin[k] = d->vi[3 + k];
-        g.win[k] = d->vi[6 + k];
-    }
-    g.P = (long long)g.f[0] * g.f[1] * g.f[2];
-    b.pl = plan_gemm(g, c->tile, 0, c->prec, d->atom_beg[d->nmembers]);
+    g = batch_grid(d);
+    b.pl = plan_gemm(g, c->tile, 0, model_scheme(c->prec), d->atom_beg[d->nmembers], b.fold_mask);
     const GemmGeom &gg = b.pl.gg;
 
     // member-major, type-sorted atom order; adjoint tiles; slices
@@ -255,7 +261,7 @@ int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
     int st;
     const size_t P = (size_t)g.P, M = (size_t)d->nmembers, T = (size_t)std::max<int64_t>(b.natoms, 1);
     if ((st = upload(c, b.idx, b.order.data(), b.order.size()))) return st;
-    if ((st = make_slices(c, b, slice_len(c, kchunk_for(b.pl, b.nsorted, b.prec))))) return st;
+    if ((st = make_slices(c, b, slice_len(c, kchunk_for(b.pl, b.segs, b.pl.scheme))))) return st;
     if ((st = upload(c, b.atiles, tiles.data(), tiles.size()))) return st;
     if ((st = ensure(c, b.pos, sizeof(double) * 3 * T))) return st;
     if ((st = ensure(c, b.occ, sizeof(double) * T))) return st;
@@ -329,6 +335,7 @@ int enqueue(dc_ctx *c, BatchState &b, int tile, int nwg, bool prep, int rest, bo
         if (b.nsorted > 0) HIPCHK(launch_prep(pa, ptr<AtomRec>(b.rec), c->st));
     }
     GemmGeom lg = launch_geom(c, gg);
+    lg.fold = fold_side(gg, b.fold_mask, tile);
     lg.order = ptr<int>(b.sorder);
     if (queue) {
         int st = ensure(c, b.wq, 256);
@@ -337,7 +344,7 @@ int enqueue(dc_ctx *c, BatchState &b, int tile, int nwg, bool prep, int rest, bo
         HIPCHK(hipGetLastError());
         lg.queue = ptr<int>(b.wq);
     }
-    HIPCHK(launch_phase_gemm(c->prec, tile, ptr<AtomRec>(b.rec), ptr<int>(b.sbeg), ptr<float2>(b.partial),
+    HIPCHK(launch_phase_gemm(b.pl.scheme, tile, ptr<AtomRec>(b.rec), ptr<int>(b.sbeg), ptr<float2>(b.partial),
                              b.any_b ? ptr<float>(b.sq) : nullptr, lg, 0, b.nslice, c->st, nwg, ptr<int>(b.ssq)));
     if (rest < 1) return 0;
     int st = reduce_planes(c, b);
@@ -398,7 +405,24 @@ int enqueue(dc_ctx *c, BatchState &b, int tile, int nwg, bool prep, int rest, bo
 // 96-member population the planned length wins).
 int autotune(dc_ctx *c, BatchState &b) {
     const bool fp32_only = b.prec == DC_PREC_FP32;    // tiles built without an FP32 variant are skipped
-    if (c->tile >= 0 && !(fp32_only && gemm_tile_info(c->tile).no_fp32)) b.pl.tile = c->tile;
+    auto built = [&](int t) {
+        const TileInfo ti = gemm_tile_info(t);
+        return !(fp32_only && ti.no_fp32) && !(ti.fold && !fold_side(b.pl.gg, b.fold_mask, t));
+    };
+    // predicted cost: microseconds of the planner's model where a side can be
+    // folded (the fold tiles alone are candidates then), else padded work
+    const bool folds = b.pl.gg.fold != 0;
+    auto candidate = [&](int t) { return built(t) && (gemm_tile_info(t).fold != 0) == folds; };
+    auto cost = [&](int t) {
+        GemmGeom gg = b.pl.gg;
+        gg.fold = fold_side(gg, b.fold_mask, t);
+        const TileInfo ti = gemm_tile_info(t);
+        double us;
+        if (!folds) return (double)gemm_items(gg, t) * ti.rt * ti.ct;
+        (void)fold_slices(gg, t, b.segs, b.pl.scheme, us);
+        return us;
+    };
+    if (c->tile >= 0 && built(c->tile)) b.pl.tile = c->tile;
     b.nwg = 0;
     if (c->tile >= 0 || !c->autotune || b.nslice == 0) return 0;
     hipDeviceProp_t prop;
@@ -423,17 +447,13 @@ int autotune(dc_ctx *c, BatchState &b) {
     int bt = b.pl.tile, bn = 0, bk = b.kchunk;
     int st = time_ms(0, 0, true, red);
     if (st) return st;
-    // candidates: tiles whose padded work is within 1.5x of the least padded one
+    // candidates: tiles whose padded work is within 1.5x of the least padded
+    // one, or whose predicted time is within 1.2x of the shortest
     double wmin = 1e300;
+    for (int t = 0; t < gemm_num_tiles(); ++t)
+        if (candidate(t)) wmin = std::min(wmin, cost(t));
     for (int t = 0; t < gemm_num_tiles(); ++t) {
-        const TileInfo ti = gemm_tile_info(t);
-        if (fp32_only && ti.no_fp32) continue;
-        wmin = std::min(wmin, (double)padded(b.pl.gg.R, ti.rt) * (double)padded(b.pl.gg.C, ti.ct));
-    }
-    for (int t = 0; t < gemm_num_tiles(); ++t) {
-        const TileInfo ti = gemm_tile_info(t);
-        if (fp32_only && ti.no_fp32) continue;
-        if ((double)padded(b.pl.gg.R, ti.rt) * (double)padded(b.pl.gg.C, ti.ct) > 1.5 * wmin) continue;
+        if (!candidate(t) || cost(t) > (folds ? 1.2 : 1.5) * wmin) continue;
         for (int nwg : {0, ncu, 2 * ncu, -ncu}) {
             float g = 0.f;
             if ((st = time_ms(t, nwg, false, g))) return st;
@@ -523,13 +543,24 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
     if (d->bdw && !dev)
         for (int64_t k = 0; k < natoms && !any_b; ++k) any_b = d->type[k] > 0 && d->bdw[k] != 0.0;
     const bool want_grad = grad != nullptr, want_icalc = icalc != nullptr, have_weight = weight != nullptr;
-    if (!same_shape(c->batch, c, d, want_grad, want_icalc, have_weight, any_b)) {
+    // s^2 of this call's metrics; with per-atom B the mirrored-pair tiles fold
+    // a side only where every member's s^2 is mirrored about its centre
+    std::vector<float> sq;
+    int fold_mask = FOLD_COLS | FOLD_ROWS;
+    {
+        Grid g = batch_grid(d);
+        const GemmGeom gg = plan_gemm(g, c->tile, 0, model_scheme(c->prec), natoms).gg;
+        if ((st = member_sq(c, g, gg, d, sq, any_b || want_grad))) return st;
+        for (int m = 0; m < d->nmembers && any_b; ++m) fold_mask &= mirrored_sides(gg, sq.data() + (size_t)m * (gg.R + gg.C));
+    }
+    if (!same_shape(c->batch, c, d, want_grad, want_icalc, have_weight, any_b) || c->batch->fold_mask != fold_mask) {
         batch_release(c);
         c->batch = new BatchState();
         c->batch->want_grad = want_grad;
         c->batch->want_icalc = want_icalc;
         c->batch->have_weight = have_weight;
         c->batch->any_b = any_b;
+        c->batch->fold_mask = fold_mask;
         if ((st = build_state(c, d, *c->batch))) {
             batch_release(c);
             return st;
@@ -537,8 +568,6 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
     }
     BatchState &b = *c->batch;
     const size_t P = (size_t)b.g.P, M = (size_t)d->nmembers;
-    std::vector<float> sq;
-    if ((st = member_sq(c, b, d, sq, any_b || want_grad))) return st;
     HIPCHK(hipEventRecord(c->ev[0], c->st));
     HIPCHK(hipMemcpyAsync(b.pos.p, d->pos, sizeof(double) * 3 * natoms, in, c->st));
     HIPCHK(hipMemcpyAsync(b.occ.p, d->occ, sizeof(double) * natoms, in, c->st));
@@ -594,7 +623,7 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
     c->stats.pairs = (double)b.nsorted * (double)P;
     c->stats.slices = b.nslice;
     c->stats.gemm_launches = 1;
-    c->stats.gemm_scheme = b.prec;
+    c->stats.gemm_scheme = b.pl.scheme;
     c->stats.gemm_ms = b.tune_best_ms;
     c->stats.adjoint_walk = want_grad ? b.walk : 0;
     return DC_OK;

@@ -28,6 +28,10 @@ struct alignas(16) AtomRec {
 };
 static_assert(sizeof(AtomRec) == 48, "AtomRec layout");
 
+// Sides of a GEMM that are one uniform run of points (no wrap), so that the
+// mirrored-pair kernels (dc_fold.h) can fold them; a mask in the planner.
+constexpr int FOLD_COLS = 1, FOLD_ROWS = 2;
+
 // GEMM problem geometry.  R rows x C cols per slice, output element
 // (r, c) stored at partial[slice * P + r + Rs * c]; the column stride Rs is R
 // rounded up to 16 rows where that adds at most 1/16 to the plane, so that
@@ -40,6 +44,7 @@ struct GemmGeom {
     const int *order;  // launch order of the slices (null: slice0, slice0 + 1, ...)
     int *queue;        // work-item counter, zero at launch (null: static assignment)
     int pad_hash;      // split schemes, undamped: AtomRec::pad holds dither_hash32 of the record (prep)
+    int fold;          // side whose points the fold tiles pair about its centre: 0 none, FOLD_COLS, FOLD_ROWS
 };
 
 // Per-atom phase rotation of the phase GEMM: a pseudo-random turn fraction
@@ -109,6 +114,35 @@ __device__ __forceinline__ void sincos_turn(uint32_t x, float &c, float &s) {
     float s1 = (q & 1) ? cs : sn;
     uint32_t negc = ((q + 1) & 2) << 30;   // q = 1, 2
     uint32_t negs = (q & 2) << 30;         // q = 2, 3
+    c = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, c1) ^ negc);
+    s = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, s1) ^ negs);
+}
+
+// The same to half a unit in the last place or so: the 30-bit reduced argument
+// is kept as a float and its remainder, which sincos_turn drops (4e-8 of an
+// eighth turn).  For the FP32 schemes, whose operand error it would dominate.
+__device__ __forceinline__ void sincos_turn_fine(uint32_t x, float &c, float &s) {
+    const uint32_t xs = x + 0x20000000u;
+    const uint32_t q = xs >> 30;
+    const int32_t r = (int32_t)(xs & 0x3FFFFFFFu) - 0x20000000;
+    const int32_t rh = r & ~63;                       // 23 bits and a sign: exact in FP32
+    const float h = (float)rh, l = (float)(r - rh);
+    const float k = 1.4629180792671596e-09f;          // 2 pi / 2^32 ...
+    const float kl = -4.0709403e-17f;                             // ... and what FP32 leaves of it
+    const float t = h * k;
+    const float e = __builtin_fmaf(h, k, -t) + __builtin_fmaf(h, kl, l * k);
+    const float u = t * t;
+    float ps = __builtin_fmaf(u, 2.716169092e-06f, -1.983906404e-04f);
+    ps = __builtin_fmaf(u, ps, 8.333328180e-03f);
+    ps = __builtin_fmaf(u, ps, -1.666666716e-01f);
+    float pc = __builtin_fmaf(u, 2.439410309e-05f, -1.388680888e-03f);
+    pc = __builtin_fmaf(u, pc, 4.166662320e-02f);
+    const float hz = 0.5f * u, w = 1.0f - hz;
+    const float sn = t + __builtin_fmaf(t * u, ps, e * w);
+    const float cs = w + (((1.0f - w) - hz) + __builtin_fmaf(u * u, pc, -e * t));
+    const float c1 = (q & 1) ? sn : cs;
+    const float s1 = (q & 1) ? cs : sn;
+    const uint32_t negc = ((q + 1) & 2) << 30, negs = (q & 2) << 30;
     c = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, c1) ^ negc);
     s = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, s1) ^ negs);
 }

@@ -63,63 +63,11 @@
 // (a slice = a contiguous atom range of one type of one lot).
 #include <type_traits>
 
-#include "dc_internal.h"
+#include "dc_fold.h"
 
 namespace dc {
 
-constexpr int SCH_FP32 = 0;
-constexpr int SCH_BF16X3 = 1;
-constexpr int SCH_FP16X2 = 2;
-constexpr int SCH_FP16X3 = 3;
-constexpr int SCH_FP32D = SCHEME_FP32_ACC64;
-// FP32 operands on v_mfma_f32_16x16x4_f32 (FP32D: partial sums kept in FP64)
-__host__ __device__ constexpr bool fp32ops(int s) { return s == SCH_FP32 || s == SCH_FP32D; }
-// three products (hi.hi, hi.lo, lo.hi) with both sides split
-__host__ __device__ constexpr bool split3(int s) { return s == SCH_BF16X3 || s == SCH_FP16X3; }
-// FP16 operands (v_mfma_f32_16x16x32_f16)
-__host__ __device__ constexpr bool f16ops(int s) { return s == SCH_FP16X2 || s == SCH_FP16X3; }
-
 constexpr int KS = 16;            // atoms per LDS stage
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-template <int SCHEME>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-    if constexpr (f16ops(SCHEME))
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2));
-    else
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
-}
-template <int SCHEME>
-__device__ __forceinline__ f32x2 unpack2(uint32_t w) {
-    if constexpr (f16ops(SCHEME))
-        return __builtin_convertvector(__builtin_bit_cast(f16x2, w), f32x2);
-    else
-        return (f32x2){__builtin_bit_cast(float, w << 16), __builtin_bit_cast(float, w & 0xFFFF0000u)};
-}
-
-// Low FP16 halves of a split: given h = (f16(x), f16(y)) packed, returns
-// (f16(x - h.x), f16(y - h.y)) packed.  x - h.x is exact in FP32, so each
-// half is one rounding, as with a conversion of the FP32 difference; the
-// mixed-precision FMAs take 2 instructions where unpacking h, subtracting
-// and packing again takes 5.
-__device__ __forceinline__ uint32_t lo_halves_f16(uint32_t h, float x, float y) {
-    uint32_t r;
-    asm("v_fma_mixlo_f16 %0, -1.0, %1, %2 op_sel_hi:[0,1,0]\n\t"
-        "v_fma_mixhi_f16 %0, -1.0, %1, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]"
-        : "=&v"(r)
-        : "v"(h), "v"(x), "v"(y));
-    return r;
-}
-
-// Round the 64-bit phase to the 32-bit turn fraction used by sincos_turn.
-__device__ __forceinline__ uint32_t phase_top(uint64_t p) { return (uint32_t)((p + 0x80000000ull) >> 32); }
 
 // Work-group layout: NWR x NWC waves, each owning a (16 WR) x (16 WC) block of
 // the (16 WR NWR) x (16 WC NWC) tile.  Every wave both builds a share of the
@@ -134,11 +82,6 @@ struct TileCfg {
     static constexpr int RH = RT / 16, CH = CT / 16;
 };
 
-// Packed planes hold one u32 (re | im << 16) per (row, atom): 16 words per
-// row, the four 16-byte atom quads of a row XOR-swizzled by bits 2..3 of the
-// row so that 16-byte accesses of the element builders (4 atom quads x 4 rows) and
-// of the MFMA operand reads (16 rows, one quad) fall on distinct banks.
-__device__ __forceinline__ int pk_off(int row, int quad) { return row * 16 + 4 * (quad ^ ((row >> 2) & 3)); }
 // FP32 planes: (row, k') with k' = 2*atom + (0 re, 1 im), 36 floats per row.
 constexpr int FST = 36;
 
@@ -190,15 +133,6 @@ struct alignas(16) Smem {
 struct Side {
     int start, a0, hi0, period;
 };
-
-__device__ __forceinline__ float2 cmul(float2 x, float2 y) {
-    return make_float2(__builtin_fmaf(x.x, y.x, -x.y * y.y), __builtin_fmaf(x.x, y.y, x.y * y.x));
-}
-__device__ __forceinline__ float2 cis(uint64_t ph) {
-    float c, s;
-    sincos_turn(phase_top(ph), c, s);
-    return make_float2(c, s);
-}
 
 // ---------------------------------------------------------------------------
 // Tables of one stage, built by all threads (pt = thread index).  Each atom
@@ -852,6 +786,7 @@ using CfgF = TileCfg<1, 4, 1, 4>;   //  16 x 256 (lines / few rows)
 using CfgG = TileCfg<2, 11, 8, 1>;  // 256 x 176 (flattened rows x one short axis, e.g. 161)
 using CfgH = TileCfg<1, 11, 8, 1>;  // 128 x 176
 using CfgI = TileCfg<2, 8, 8, 1>;   // 256 x 128 (column counts that are multiples of 128, e.g. 256^2 layers)
+constexpr int FOLD_TILE0 = 9;       // first of the mirrored-pair tiles (dc_fold.h)
 
 // split_only: tiles whose FP32 variant (two accumulator sets) spills so much
 // that it is slower than the 96x256 tile (which spills a little and is still
@@ -869,6 +804,9 @@ static const TileInfo kTiles[] = {
     {CfgE::RT, CfgE::CT, CfgE::NT, 0, 1.65f, 1, 0}, {CfgF::RT, CfgF::CT, CfgF::NT, 0, 6.30f, 1, 0},
     {CfgG::RT, CfgG::CT, CfgG::NT, 1, 1.00f, 0, 0}, {CfgH::RT, CfgH::CT, CfgH::NT, 1, 1.33f, 0, 0},
     {CfgI::RT, CfgI::CT, CfgI::NT, 1, 1.10f, 0, 1},
+#define X(i, wr, wc) {128 * wr, 16 * wc, 512, !fold_built(SCH_FP32, wr, wc), 0.5f, 0, !fold_built(SCH_FP32, wr, wc), 1},
+    DC_FOLD_TILES(X)
+#undef X
 };
 
 // FP32D keeps 2 x WR x WC x 4 FP64 sums per lane beside the FP32 chains: only
@@ -924,6 +862,31 @@ static hipError_t launch_scheme(int tile, const AtomRec *rec, const int *slice_b
     }
 }
 
+#define X(name)                                                                                                        \
+    hipError_t launch_fold_##name(int t, const AtomRec *rec, const int *slice_beg, float2 *partial, const float *sq,   \
+                                  const int *slice_sq, const GemmGeom &g, const FoldGeom &fg, int slice0, int nslice,  \
+                                  int nwg, hipStream_t st);
+X(fp32) X(bf16x3) X(fp16x3)
+#undef X
+
+// Mirrored-pair tile t on the side that g.fold names.
+static hipError_t launch_fold(int scheme, int t, const AtomRec *rec, const int *slice_beg, float2 *partial, const float *sq,
+                              const int *slice_sq, const GemmGeom &g, int slice0, int nslice, int nwg, hipStream_t st) {
+    FoldGeom fg{};
+    if (g.fold == FOLD_COLS && g.C0 >= g.C)
+        fg = {g.R, g.R0, g.C, 0, 1, g.Rs};
+    else if (g.fold == FOLD_ROWS && g.R0 >= g.R)
+        fg = {g.C, g.C0, g.R, 1, g.Rs, 1};
+    else
+        return hipErrorInvalidValue;
+    switch (scheme) {
+    case SCH_FP32: return launch_fold_fp32(t, rec, slice_beg, partial, sq, slice_sq, g, fg, slice0, nslice, nwg, st);
+    case SCH_BF16X3: return launch_fold_bf16x3(t, rec, slice_beg, partial, sq, slice_sq, g, fg, slice0, nslice, nwg, st);
+    case SCH_FP16X3: return launch_fold_fp16x3(t, rec, slice_beg, partial, sq, slice_sq, g, fg, slice0, nslice, nwg, st);
+    default: return hipErrorInvalidValue;
+    }
+}
+
 hipError_t launch_phase_gemm(int scheme, int tile, const AtomRec *rec, const int *slice_beg, float2 *partial,
                              const float *sq, const GemmGeom &g, int slice0, int nslice, hipStream_t st, int nwg,
                              const int *slice_sq) {
@@ -932,6 +895,8 @@ hipError_t launch_phase_gemm(int scheme, int tile, const AtomRec *rec, const int
     if (g.C0 < 16 && g.C0 != g.C) return hipErrorInvalidValue;
     if (nslice <= 0) return hipSuccess;
     if ((long long)((g.C + 15) / 16) * ((g.R + 15) / 16) * nslice > INT32_MAX) return hipErrorInvalidValue;
+    if (tile >= FOLD_TILE0)
+        return launch_fold(scheme, tile - FOLD_TILE0, rec, slice_beg, partial, sq, slice_sq, g, slice0, nslice, nwg, st);
     switch (scheme) {
     case SCH_FP32: return launch_scheme<SCH_FP32>(tile, rec, slice_beg, partial, sq, slice_sq, g, slice0, nslice, nwg, st);
     case SCH_BF16X3: return launch_scheme<SCH_BF16X3>(tile, rec, slice_beg, partial, sq, slice_sq, g, slice0, nslice, nwg, st);

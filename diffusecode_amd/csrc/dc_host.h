@@ -46,7 +46,7 @@ struct dc_ctx {
     std::vector<hipEvent_t> tev;
     size_t tev_used = 0;
     // device buffers of the Fourier run
-    DevBuf rec, slice_beg, slice_type, lot_slice, partial, cfact, istl, idx, oid, offs, xat, w;
+    DevBuf rec, slice_beg, slice_order, slice_type, lot_slice, partial, cfact, istl, idx, oid, offs, xat, w;
     DevBuf acsf, dsi, csf, wm, wv, lat, out_tcsf, out[5];
     // device buffers of the refinement model
     DevBuf m_pos, m_w, m_b, m_sq, m_q, m_part, m_grad, m_tiles, m_gi, m_f, m_tgt, m_qt, m_qs, m_bd, m_jw, m_jidx, m_dsl, m_di;
@@ -76,7 +76,7 @@ struct dc_ctx {
     bool rec_hash = false;
 
     std::vector<DevBuf *> buffers() {
-        return {&rec, &slice_beg, &slice_type, &lot_slice, &partial, &cfact, &istl, &idx, &oid, &offs, &xat, &w,
+        return {&rec, &slice_beg, &slice_order, &slice_type, &lot_slice, &partial, &cfact, &istl, &idx, &oid, &offs, &xat, &w,
                 &acsf, &dsi, &csf, &wm, &wv, &lat, &out_tcsf, &out[0], &out[1], &out[2], &out[3], &out[4],
                 &m_pos, &m_w, &m_b, &m_sq, &m_q, &m_part, &m_grad, &m_tiles, &m_gi, &m_f, &m_tgt, &m_qt, &m_qs, &m_bd, &m_jw, &m_jidx, &m_dsl, &m_di,
                 &pos, &iscat, &type_idx, &runs};
@@ -193,11 +193,23 @@ struct SliceSet {
 
 long long padded(long long n, long long t);
 int max_corner_bin(const Grid &g);   // largest sin(theta)/lambda bin over the grid corners
-Plan plan_gemm(Grid &g, int forced, int only_mapping = -1, int prec = 1, long long natoms = 0);
+// Work items per slice of a tile on a geometry (gg.fold names the folded
+// side of a mirrored-pair tile), and the better side a mask allows (0: none).
+int gemm_items(const GemmGeom &gg, int tile);
+int fold_side(const GemmGeom &gg, int fold_mask, int tile);
+// fold_mask: sides that the mirrored-pair tiles may fold (FOLD_COLS |
+// FOLD_ROWS); a damped launch needs s^2 mirrored about the side's centre.
+Plan plan_gemm(Grid &g, int forced, int only_mapping = -1, int prec = 1, long long natoms = 0,
+               int fold_mask = FOLD_COLS | FOLD_ROWS);
+// Slice length of a fold tile for a launch's segments, and its predicted time.
+int fold_slices(const GemmGeom &gg, int tile, const std::vector<std::pair<int, int>> &segs, int prec, double &best_us);
+// the sides whose s^2 parts (R row values, then C column values) are mirrored
+int mirrored_sides(const GemmGeom &gg, const float *sq);
 int kchunk_for(const Plan &pl, long long natoms_batch, int prec);
 int kchunk_for(const Plan &pl, const std::vector<std::pair<int, int>> &segs, int prec);
 void add_segments(SliceSet &s, const std::vector<std::pair<int, int>> &segs, int kchunk, int &atom_off);
-int run_gemm(dc_ctx *c, const Plan &pl, int nslice, float2 *partial, const float *sq = nullptr);
+// beg: the slices' atom offsets, as uploaded to c->slice_beg (nslice + 1)
+int run_gemm(dc_ctx *c, const Plan &pl, const std::vector<int> &beg, float2 *partial, const float *sq = nullptr);
 // atoms per slice: the context's forced length (dc_set_slice_atoms) or the planned one
 inline int slice_len(const dc_ctx *c, int planned) { return c->slice_atoms > 0 ? c->slice_atoms : planned; }
 // the plan's geometry with the context's dither salt
@@ -211,5 +223,9 @@ void post_release(dc_ctx *c);    // frees the FFT plans and buffers of the post-
 void nufft_release(dc_ctx *c);   // frees the NUFFT fine grid, plans and buffers
 int noalloc_attach(dc_ctx *c);   // device address of this device's dc_scratch (dc_noalloc.hip)
 PrepArgs base_prep(const Grid &g, int mapping);
+// Products of the refinement model's and the populations' forward sums: a
+// gradient amplifies the error of F, so BF16X3 runs the FP16X3 products there
+// (the same MFMA rate), as the Bragg-subtracted runs do.
+inline int model_scheme(int prec) { return prec == DC_PREC_BF16X3 ? DC_PREC_FP16X3 : prec; }
 
 }  // namespace dc

@@ -60,8 +60,7 @@ int plan_model(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
     }
     for (int k = 0; k < 9; ++k) g.rten[k] = m->rten[k];
     g.P = (long long)g.f[0] * g.f[1] * g.f[2];
-    mp.pl = plan_gemm(g, c->tile, 0, c->prec, m->natoms);
-    const GemmGeom &gg = mp.pl.gg;
+    const GemmGeom gg = plan_gemm(g, c->tile, 0, model_scheme(c->prec), m->natoms).gg;
 
     // metric orthogonality of the abscissa against the other axes
     const double *v1 = m->vi, *v2 = m->vi + 3, *v3 = m->vi + 6;
@@ -101,6 +100,10 @@ int plan_model(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
     }
     for (int t = 1; t <= m->nscat; ++t)
         if (cnt[t] > 0) mp.segs.push_back({t - 1, cnt[t]});
+    // the planes of mapping 0 are the same for every tile; with per-atom B a
+    // side is folded only where its s^2 is mirrored
+    mp.pl = plan_gemm(g, c->tile, 0, model_scheme(c->prec), m->natoms,
+                      mp.any_b ? mirrored_sides(gg, mp.sq.data()) : FOLD_COLS | FOLD_ROWS);
     if (mp.any_b && !mp.separable)
         return set_err(c, DC_ERR_ARG, DC_ER_LIB, "model: per-atom B needs vi(:,1) metric-orthogonal to vi(:,2), vi(:,3)");
     if (max_corner_bin(g) >= m->ncfact)
@@ -142,7 +145,7 @@ int model_forward(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
     const GemmGeom &gg = mp.pl.gg;
     SliceSet ss;
     int off = 0;
-    add_segments(ss, mp.segs, slice_len(c, kchunk_for(mp.pl, mp.segs, c->prec)), off);
+    add_segments(ss, mp.segs, slice_len(c, kchunk_for(mp.pl, mp.segs, mp.pl.scheme)), off);
     if (ss.beg.empty()) ss.beg.push_back(0);
     const int nslice = (int)ss.type.size();
     ss.lot = {0, nslice};
@@ -154,7 +157,7 @@ int model_forward(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
     if ((st = ensure(c, c->m_f, sizeof(double) * 2 * mp.g.P))) return st;
     if ((st = ensure(c, c->dsi, sizeof(double) * mp.g.P))) return st;
     HIPCHK(hipEventRecord(c->ev[4], c->st));
-    if ((st = run_gemm(c, mp.pl, nslice, ptr<float2>(c->partial), mp.any_b ? ptr<float>(c->m_sq) : nullptr))) return st;
+    if ((st = run_gemm(c, mp.pl, ss.beg, ptr<float2>(c->partial), mp.any_b ? ptr<float>(c->m_sq) : nullptr))) return st;
     ReduceArgs ra{};
     ra.g = mp.g;
     ra.partial = ptr<float2>(c->partial);
@@ -345,7 +348,9 @@ int dc_model_jvp(dc_ctx *c, const dc_model_desc *m, const double *fcalc, int ndi
     if (m->bdw && (st = upload(c, c->m_bd, m->bdw, (size_t)m->natoms))) return st;
     if ((st = ensure(c, c->m_di, sizeof(double) * (size_t)P * std::max(ndir, 1) * (df ? 3 : 1)))) return st;
     // directions per batch so that the slice planes fit the budget
-    const int kchunk = slice_len(c, kchunk_for(mp.pl, (long long)ns * 5, c->prec));
+    std::vector<std::pair<int, int>> all;
+    for (int k = 0; k < 5 * std::min(ndir, 64); ++k) all.insert(all.end(), mp.segs.begin(), mp.segs.end());
+    const int kchunk = slice_len(c, kchunk_for(mp.pl, all, mp.pl.scheme));
     long long slices_per_dir = 0;
     for (auto &sg : mp.segs) slices_per_dir += 5 * ((sg.second + kchunk - 1) / kchunk);
     const double dir_bytes = (double)std::max<long long>(slices_per_dir, 1) * gg.P * sizeof(float2);
@@ -393,7 +398,7 @@ int dc_model_jvp(dc_ctx *c, const dc_model_desc *m, const double *fcalc, int ndi
         pa.n = (long long)w.size();
         if (pa.n > 0) HIPCHK(launch_prep(pa, ptr<AtomRec>(c->rec), c->st));
         c->rec_hash = false;
-        if ((st = run_gemm(c, mp.pl, nslice, ptr<float2>(c->partial), mp.any_b ? ptr<float>(c->m_sq) : nullptr))) return st;
+        if ((st = run_gemm(c, mp.pl, ss.beg, ptr<float2>(c->partial), mp.any_b ? ptr<float>(c->m_sq) : nullptr))) return st;
         JvpArgs ja{};
         ja.g = mp.g;
         ja.partial = ptr<float2>(c->partial);

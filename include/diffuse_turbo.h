@@ -54,7 +54,9 @@ extern "C" {
 #define DC_PREC_FP32 0          /* plain FP32 MFMA (the drop-in)            */
 #define DC_PREC_BF16X3 1        /* split BF16 hi/lo, 3 MFMA products; runs with
                                    the <F> subtraction or the cross-lot variance
-                                   use the FP16X3 products (dc_four_run*)    */
+                                   (dc_four_run*) and the forward sums of
+                                   dc_model_* and dc_batch_* use the FP16X3
+                                   products                                  */
 #define DC_PREC_FP16X2 2        /* split FP16 hi/lo on one side, 2 products */
 #define DC_PREC_FP16X3 3        /* split FP16 hi/lo on both sides, 3 MFMA products */
 
@@ -85,10 +87,11 @@ int dc_gemm_tile_shape(int tile, int *rows, int *cols, int *threads);
  * counterpart in DISCUS (whose sum runs atom by atom in FP64); a tuning and
  * test knob, like dc_set_gemm_tile. */
 int dc_set_slice_atoms(dc_ctx *ctx, int n);
-/* Per-atom phase rotation of the phase GEMM (on by default): row operands
+/* Per-atom decorrelation of the phase GEMM (on by default): row operands
  * carry +psi_n and column operands -psi_n, psi_n a fixed pseudo-random turn
- * per atom, so the products are unchanged and each atom's operand rounding
- * differs.  Off, atoms with equal phases (Bragg peaks of a crystal) add the
+ * per atom (mirrored-pair tiles: a pseudo-random scale and its reciprocal,
+ * and turns inside each operand's tables), so the products are unchanged and
+ * each atom's operand rounding differs.  Off, atoms with equal phases (Bragg peaks of a crystal) add the
  * same rounding error once per atom.  No counterpart in DISCUS; a test knob. */
 int dc_set_phase_dither(dc_ctx *ctx, int on);
 /* Polled between kernel launches of long runs; a non-zero value aborts the
