@@ -35,7 +35,7 @@ EXPORTS = [
     "dc_create", "dc_destroy", "dc_last_error", "dc_last_error_type", "dc_set_precision",
     "dc_get_precision", "dc_set_gemm_tile", "dc_set_slice_atoms", "dc_set_phase_dither", "dc_set_adjoint_walk", "dc_gemm_num_tiles", "dc_gemm_tile_shape", "dc_set_cancel_flag", "dc_version", "dc_device_info", "dc_measure_peaks", "dc_strucf", "dc_strucf_dev_noalloc", "dc_four_stltab",
     "dc_crystal_set", "dc_four_run", "dc_four_run_dev", "dc_last_stats", "dc_synchronize",
-    "dc_model_intensity", "dc_model_vjp", "dc_model_chi2", "dc_model_jvp",
+    "dc_model_intensity", "dc_model_vjp", "dc_model_chi2", "dc_model_chi2_dev", "dc_device_index", "dc_model_jvp",
     "dc_batch_chi2", "dc_batch_chi2_dev", "dc_set_autotune", "dc_set_graphs", "dc_batch_info",
     "dc_four_post", "dc_four_post_dev", "dc_four_fill", "dc_four_fill_dev", "dc_four_accumulate_dev",
     "dc_qval", "dc_qval_dev", "dc_nufft1", "dc_nufft1_dev", "dc_four_strucf_nufft", "dc_four_strucf_nufft_dev",
@@ -149,6 +149,8 @@ def lib():
     L.dc_model_intensity.argtypes = [C.c_void_p, C.POINTER(ModelDesc), _dp, _dp]
     L.dc_model_vjp.argtypes = [C.c_void_p, C.POINTER(ModelDesc), _dp, _dp, _dp]
     L.dc_model_chi2.argtypes = [C.c_void_p, C.POINTER(ModelDesc), _dp, _dp, _dp, _dp, _dp]
+    L.dc_model_chi2_dev.argtypes = [C.c_void_p, C.POINTER(ModelDesc), C.c_void_p, C.c_void_p, _dp, C.c_void_p, C.c_void_p]
+    L.dc_device_index.argtypes = [C.c_void_p]
     L.dc_model_jvp.argtypes = [C.c_void_p, C.POINTER(ModelDesc), _dp, C.c_int, _dp, _dp, _dp]
     L.dc_batch_chi2.argtypes = [C.c_void_p, C.POINTER(BatchDesc), _dp, _dp, _dp, _dp, _dp]
     L.dc_batch_chi2_dev.argtypes = [C.c_void_p, C.POINTER(BatchDesc), C.c_void_p, C.c_void_p, _dp, C.c_void_p,
@@ -491,6 +493,24 @@ class Context:
         chi = C.c_double()
         self.check(lib().dc_model_chi2(self.h, C.byref(desc), _d(t), _d(w), C.byref(chi), _d(icalc), _d(grad)))
         return chi.value, icalc.reshape(num, order="F"), None if grad is None else grad.reshape(-1, 5)
+
+    def device_index(self):
+        return lib().dc_device_index(self.h)
+
+    def model_chi2_dev(self, desc, pos, occ, bdw, target, weight=None, icalc=None, grad=None):
+        """Device variant: pos (N, 3), occ (N), bdw (N) or None, target, weight
+        and icalc over the grid (abscissa fastest) and grad (N, 5), float64 CUDA
+        tensors or addresses on the context's device; the other fields of desc
+        are the host ones of model_desc.  Returns chi2."""
+        def p(t):
+            return None if t is None else (t if isinstance(t, int) else t.data_ptr())
+        d = ModelDesc.from_buffer_copy(desc)
+        d.pos = C.cast(C.c_void_p(p(pos)), _dp)
+        d.occ = C.cast(C.c_void_p(p(occ)), _dp)
+        d.bdw = C.cast(C.c_void_p(p(bdw)), _dp) if bdw is not None else None
+        chi = C.c_double()
+        self.check(lib().dc_model_chi2_dev(self.h, C.byref(d), p(target), p(weight), C.byref(chi), p(icalc), p(grad)))
+        return chi.value
 
     # -- population scoring ----------------------------------------------------
     def set_autotune(self, on):

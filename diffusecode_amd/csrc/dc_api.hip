@@ -11,7 +11,6 @@
 #include <cstring>
 #include <string>
 #include <functional>
-#include <map>
 #include <vector>
 
 #include "../../include/diffuse_turbo.h"
@@ -174,9 +173,7 @@ static double fold_stage_us(const TileInfo &ti, int prec) {
     const double m = prec == DC_PREC_FP32 ? 0.49 : 0.091;
     return m * wr * wc + 0.45 + 0.55 * wr + 0.02 * wc;
 }
-static double fold_item_us(const TileInfo &ti, int prec, double atoms) {
-    return std::ceil(atoms / 32.0) * fold_stage_us(ti, prec) + 7.0;
-}
+constexpr double FOLD_ITEM_US = 7.0;
 // ... and of the FP64 reduction of its planes: the traffic of the planes, or
 // the chain of dependent batches of 4 planes that each pixel's thread walks.
 static double reduce_us(double planes, double plane_elems) {
@@ -200,32 +197,37 @@ static int fold_cap(const GemmGeom &gg, long long natoms, int prec) {
     return (int)std::min<long long>(std::max<long long>(k, 1024), KCHUNK_FOLD_MAX);
 }
 
-// Makespan of counted groups of equal items, (microseconds, count) in any
-// order, on ncu machines, the longest items first.
-static double makespan(std::vector<std::pair<double, long long>> groups, int ncu) {
-    std::sort(groups.begin(), groups.end(), std::greater<std::pair<double, long long>>());
-    std::map<double, long long> load;   // machines by finishing time
-    load[0.0] = ncu;
-    for (auto &gr : groups) {
-        long long left = gr.second;
+// Makespan of n counted groups of equal items, (microseconds, count), the
+// longest items first, on ncu machines.  (Called for every candidate of every
+// plan: a few small vectors, no allocation per item.)
+struct ItemGroup {
+    double us;
+    long long count;
+};
+static double makespan(ItemGroup *gr, int n, int ncu) {
+    if (n == 1) return gr[0].us * (double)((gr[0].count + ncu - 1) / ncu);
+    std::sort(gr, gr + n, [](const ItemGroup &x, const ItemGroup &y) { return x.us > y.us; });
+    std::vector<ItemGroup> load{{0.0, ncu}};   // machines by finishing time, ascending
+    for (int q = 0; q < n; ++q) {
+        long long left = gr[q].count;
         const long long full = left / ncu - 1;
         if (full > 0) {   // whole rounds shift every machine alike
-            std::map<double, long long> l2;
-            for (auto &kv : load) l2[kv.first + gr.first * (double)full] += kv.second;
-            load.swap(l2);
+            for (auto &l : load) l.us += gr[q].us * (double)full;
             left -= full * ncu;
         }
         while (left > 0) {
-            auto it = load.begin();
-            const double t = it->first;
-            const long long n = std::min(left, it->second);
-            it->second -= n;
-            if (it->second == 0) load.erase(it);
-            load[t + gr.first] += n;
-            left -= n;
+            const ItemGroup first = load.front();
+            const long long m = std::min(left, first.count);
+            if (m == first.count) load.erase(load.begin());
+            else load.front().count -= m;
+            const double t = first.us + gr[q].us;
+            auto it = std::lower_bound(load.begin(), load.end(), t, [](const ItemGroup &x, double v) { return x.us < v; });
+            if (it != load.end() && it->us == t) it->count += m;
+            else load.insert(it, {t, m});
+            left -= m;
         }
     }
-    return load.rbegin()->first;
+    return load.back().us;
 }
 
 // Best slice length of a fold tile for the (type, count) segments of a
@@ -237,31 +239,40 @@ int fold_slices(const GemmGeom &gg, int tile, const std::vector<std::pair<int, i
     const TileInfo ti = gemm_tile_info(tile);
     const long long wgs = gemm_items(gg, tile);
     const int ncu = device_cu_count();
-    // segments by size: a run has few distinct ones
-    std::map<int, long long, std::greater<int>> sizes;
+    // segments by size, descending: a run has few distinct ones
+    std::vector<std::pair<int, long long>> sizes;
+    sizes.reserve(segs.size());
     long long natoms = 0;
     for (auto &sg : segs)
         if (sg.second > 0) {
-            sizes[sg.second]++;
+            sizes.push_back({sg.second, 1});
             natoms += sg.second;
         }
     const int cap = fold_cap(gg, natoms, prec);
     best_us = 1e300;
     if (sizes.empty()) return cap;
-    const int nmax = sizes.begin()->first;
+    std::sort(sizes.begin(), sizes.end(), std::greater<std::pair<int, long long>>());
+    // lots of nearly equal atom counts: counts within 1/32 are one size
+    size_t ns1 = 0;
+    for (size_t q = 1; q < sizes.size(); ++q) {
+        if (sizes[q].first >= sizes[ns1].first - sizes[ns1].first / 32) sizes[ns1].second += sizes[q].second;
+        else sizes[++ns1] = sizes[q];
+    }
+    sizes.resize(ns1 + 1);
+    const int nmax = sizes[0].first;
+    const double stage_us = fold_stage_us(ti, prec);
+    std::vector<ItemGroup> groups(sizes.size());
     int best = cap, n0 = (nmax + cap - 1) / cap;
     for (int ns = n0;; ns = std::max(ns + 1, ns + ns / 8)) {
         const int k = std::min(cap, (nmax + ns - 1) / ns);
         if (ns > n0 && k < KCHUNK_FOLD_MIN) break;
-        std::vector<std::pair<double, long long>> groups;
         long long planes = 0;
-        for (auto &kv : sizes) {
-            const long long q = (kv.first + k - 1) / k;
-            const int len = (int)((kv.first + q - 1) / q);
-            groups.push_back({fold_item_us(ti, prec, len), q * kv.second * wgs});
-            planes += q * kv.second;
+        for (size_t q = 0; q < sizes.size(); ++q) {
+            const long long sl = (sizes[q].first + k - 1) / k, len = (sizes[q].first + sl - 1) / sl;
+            groups[q] = {(double)((len + 31) / 32) * stage_us + FOLD_ITEM_US, sl * sizes[q].second * wgs};
+            planes += sl * sizes[q].second;
         }
-        const double us = makespan(groups, ncu) + reduce_us((double)planes, (double)gg.P);
+        const double us = makespan(groups.data(), (int)groups.size(), ncu) + reduce_us((double)planes, (double)gg.P);
         if (us < best_us * (1.0 - 1e-9)) {
             best_us = us;
             best = k;
@@ -269,6 +280,40 @@ int fold_slices(const GemmGeom &gg, int tile, const std::vector<std::pair<int, i
         if (k <= 1) break;
     }
     return best;
+}
+
+// Geometry and plane strides of a mapping.
+static void map_geom(const Grid &g, int mapping, GemmGeom &gg, long long ps[3]) {
+    if (mapping == 0) {
+        gg.R = g.f[0];
+        gg.R0 = g.f[0];
+        gg.C0 = g.f[2] > 1 ? std::max(16, g.f[1]) : g.f[1];
+        gg.C = gg.C0 * g.f[2];
+    } else {
+        gg.R0 = g.f[1] > 1 ? std::max(16, g.f[0]) : g.f[0];
+        gg.R = gg.R0 * g.f[1];
+        gg.C = g.f[2];
+        gg.C0 = g.f[2];
+    }
+    // plane column stride: whole 16-row blocks (128-byte lines) unless
+    // that grows the plane by more than 1/16 (short columns)
+    gg.Rs = (padded(gg.R, 16) - gg.R) * 16 <= gg.R ? (int)padded(gg.R, 16) : gg.R;
+    ps[0] = 1;
+    if (mapping == 0) {
+        ps[1] = gg.Rs;
+        ps[2] = (long long)gg.Rs * gg.C0;
+    } else {
+        ps[1] = gg.R0;
+        ps[2] = gg.Rs;
+    }
+    gg.P = (long long)gg.Rs * gg.C;
+}
+
+GemmGeom mapping0_geom(const Grid &g) {
+    GemmGeom gg{};
+    long long ps[3];
+    map_geom(g, 0, gg, ps);
+    return gg;
 }
 
 Plan plan_gemm(Grid &g, int forced, int only_mapping, int prec, long long natoms, int fold_mask) {
@@ -291,26 +336,7 @@ Plan plan_gemm(Grid &g, int forced, int only_mapping, int prec, long long natoms
         if (only_mapping >= 0 && mapping != only_mapping) continue;
         GemmGeom gg{};
         long long ps[3];
-        if (mapping == 0) {
-            gg.R = g.f[0];
-            gg.R0 = g.f[0];
-            gg.C0 = g.f[2] > 1 ? std::max(16, g.f[1]) : g.f[1];
-            gg.C = gg.C0 * g.f[2];
-        } else {
-            gg.R0 = g.f[1] > 1 ? std::max(16, g.f[0]) : g.f[0];
-            gg.R = gg.R0 * g.f[1];
-            gg.C = g.f[2];
-            gg.C0 = g.f[2];
-        }
-        // plane column stride: whole 16-row blocks (128-byte lines) unless
-        // that grows the plane by more than 1/16 (short columns)
-        gg.Rs = (padded(gg.R, 16) - gg.R) * 16 <= gg.R ? (int)padded(gg.R, 16) : gg.R;
-        if (mapping == 0) {
-            ps[0] = 1; ps[1] = gg.Rs; ps[2] = (long long)gg.Rs * gg.C0;
-        } else {
-            ps[0] = 1; ps[1] = gg.R0; ps[2] = gg.Rs;
-        }
-        gg.P = (long long)gg.Rs * gg.C;
+        map_geom(g, mapping, gg, ps);
         for (int t = 0; t < nt; ++t) {
             if (forced >= 0 && t != forced) continue;
             TileInfo ti = gemm_tile_info(t);
@@ -466,7 +492,7 @@ void add_segments(SliceSet &s, const std::vector<std::pair<int, int>> &segs, int
     }
 }
 
-int run_gemm(dc_ctx *c, const Plan &pl, const std::vector<int> &beg, float2 *partial, const float *sq) {
+int run_gemm(dc_ctx *c, const Plan &pl, const std::vector<int> &beg, const int *d_beg, float2 *partial, const float *sq) {
     GemmGeom gg = launch_geom(c, pl.gg);
     gg.pad_hash = c->rec_hash && !sq;
     const int nslice = (int)beg.size() - 1;
@@ -486,10 +512,12 @@ int run_gemm(dc_ctx *c, const Plan &pl, const std::vector<int> &beg, float2 *par
             std::vector<int> order(nslice);
             for (int q = 0; q < nslice; ++q) order[q] = q;
             std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return beg[x + 1] - beg[x] > beg[y + 1] - beg[y]; });
-            if ((st = upload(c, c->slice_order, order.data(), order.size()))) return st;
-            gg.order = ptr<int>(c->slice_order);
+            int *d_order;
+            if ((st = stage(c, c->slice_order, order.data(), order.size(), d_order))) return st;
+            gg.order = d_order;
         }
     }
+    if ((st = stage_flush(c))) return st;
     hipEvent_t e0, e1;
     if ((st = mark(c, e0))) return st;
     // launch in chunks of slices so that the cancel flag is polled
@@ -497,7 +525,7 @@ int run_gemm(dc_ctx *c, const Plan &pl, const std::vector<int> &beg, float2 *par
     for (int s0 = 0; s0 < nslice; s0 += per) {
         if (cancelled(c)) return set_err(c, DC_ERR_CANCEL, DC_ER_COMM, "cancelled");
         int ns = std::min(per, nslice - s0);
-        HIPCHK(launch_phase_gemm(pl.scheme, pl.tile, ptr<AtomRec>(c->rec), ptr<int>(c->slice_beg),
+        HIPCHK(launch_phase_gemm(pl.scheme, pl.tile, ptr<AtomRec>(c->rec), d_beg,
                                  partial + (long long)s0 * gg.P * planes_per_slice(pl.scheme), sq, gg, s0, ns,
                                  c->st));
         c->stats.gemm_launches++;
@@ -582,6 +610,8 @@ void dc_destroy(dc_ctx *c) {
     nufft_release(c);
     for (DevBuf *b : c->buffers())
         if (b->p) (void)hipFree(b->p);
+    for (PinBuf *b : {&c->h_arena, &c->h_out})
+        if (b->p) (void)hipHostFree(b->p);
     for (auto &e : c->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto &e : c->tev) (void)hipEventDestroy(e);
@@ -645,6 +675,8 @@ int dc_set_cancel_flag(dc_ctx *c, const volatile int *flag) {
     c->cancel = flag;
     return DC_OK;
 }
+
+int dc_device_index(const dc_ctx *c) { return c ? c->device : -1; }
 
 int dc_device_info(const dc_ctx *c, char *name, int len, int *num_cu) {
     if (!c) return DC_ERR_ARG;
@@ -721,9 +753,9 @@ int strucf_setup(dc_ctx *c, const void *xat, int64_t nxat, int64_t ld_xat, const
 int strucf_core(dc_ctx *c, const Grid &g0, long long ntot, const double *d_xat, int64_t nxat, int64_t ld_xat,
                 const double off_shift[9], const int lmn[6], const double2 *d_cfact, int64_t ncfact,
                 const int *d_istl, int lform, AtomRec *rec, int *slice_beg, float2 *partial, double plane_bytes,
-                double *d_tcsf) {
+                double *d_tcsf, int fold_mask) {
     Grid g = g0;
-    const Plan pl = plan_gemm(g, c->tile, -1, c->prec, nxat);
+    const Plan pl = plan_gemm(g, c->tile, -1, c->prec, nxat, fold_mask);
     const double one_plane = (double)sizeof(float2) * (double)pl.gg.P * planes_per_slice(pl.scheme);
     if (one_plane > plane_bytes) return set_err(c, DC_ERR_ARG, DC_ER_LIB, "dc_strucf: one slice plane exceeds the plane budget");
     PrepArgs pa = base_prep(g, pl.mapping);
@@ -734,13 +766,20 @@ int strucf_core(dc_ctx *c, const Grid &g0, long long ntot, const double *d_xat, 
     pa.src_ld = std::max<int64_t>(ld_xat, 1);
     pa.n = nxat;
     pa.hash_salt = launch_geom(c, pl.gg).dither;   // undamped launches below
-    HIPCHK(launch_prep(pa, rec, c->st));
     SliceSet ss;
     int off = 0;
     add_segments(ss, {{0, (int)nxat}}, slice_len(c, kchunk_for(pl, nxat, pl.scheme)), off);
     if (ss.beg.empty()) ss.beg.push_back(0);
     const int nslice = (int)ss.type.size();
-    HIPCHK(hipMemcpyAsync(slice_beg, ss.beg.data(), sizeof(int) * ss.beg.size(), hipMemcpyHostToDevice, c->st));
+    // staged with the call's other arrays, or (noalloc) copied into the scratch
+    if (slice_beg) {
+        HIPCHK(hipMemcpyAsync(slice_beg, ss.beg.data(), sizeof(int) * ss.beg.size(), hipMemcpyHostToDevice, c->st));
+    } else {
+        int st;
+        if ((st = stage(c, c->slice_beg, ss.beg.data(), ss.beg.size(), slice_beg))) return st;
+        if ((st = stage_flush(c))) return st;
+    }
+    HIPCHK(launch_prep(pa, rec, c->st));
     ReduceArgs ra{};
     ra.g = g;
     ra.partial = partial;
@@ -794,14 +833,34 @@ int dc_strucf(dc_ctx *c, const double *xat, int64_t nxat, int64_t ld_xat, const 
     HIPCHK(hipSetDevice(c->device));
     stats_begin(c);
     HIPCHK(hipEventRecord(c->ev[0], c->st));
-    // positions: xat(ld,3) columns packed into (n,3) Fortran layout on device
-    if ((st = ensure(c, c->xat, sizeof(double) * 3 * std::max<int64_t>(nxat, 1)))) return st;
-    for (int col = 0; col < 3 && nxat > 0; ++col)
-        HIPCHK(hipMemcpyAsync(ptr<double>(c->xat) + col * nxat, xat + col * ld_xat, sizeof(double) * nxat,
-                              hipMemcpyHostToDevice, c->st));
+    // positions (read by the record kernel in place when they fit the staging
+    // memory), form factors and bins
+    if ((st = stage_begin(c))) return st;
+    const int64_t n1 = std::max<int64_t>(nxat, 1);
+    const double *d_xat = nullptr;
+    double2 *d_cfact = nullptr;
+    int *d_istl = nullptr;
+    int rows = (int)ncfact;
     if (lform) {
-        if ((st = upload(c, c->cfact, cfact_col, 2 * (size_t)ncfact))) return st;
-        if (istl && (st = upload(c, c->istl, istl, (size_t)ntot))) return st;
+        if (!istl) rows = cfact_rows(max_corner_bin(g), rows);
+        if ((st = stage_cfact(c, cfact_col, (int)ncfact, 1, rows, d_cfact))) return st;
+        if (istl && (st = stage(c, c->istl, istl, (size_t)ntot, d_istl))) return st;
+    }
+    const size_t xbytes = (sizeof(double) * 3 * (size_t)nxat + 255) & ~(size_t)255;
+    c->arena_want += xbytes;
+    if (xbytes + 4096 <= c->h_arena.n - c->arena_n) {
+        if ((st = stage_flush(c))) return st;
+        double *h = reinterpret_cast<double *>(c->h_arena.p + c->arena_n);
+        for (int col = 0; col < 3 && nxat > 0; ++col) std::memcpy(h + col * nxat, xat + col * ld_xat, sizeof(double) * nxat);
+        d_xat = h;
+        c->arena_n = c->arena_done = c->arena_n + xbytes;
+        c->arena_busy = true;
+    } else {
+        if ((st = ensure(c, c->xat, sizeof(double) * 3 * n1))) return st;
+        for (int col = 0; col < 3 && nxat > 0; ++col)
+            HIPCHK(hipMemcpyAsync(ptr<double>(c->xat) + col * nxat, xat + col * ld_xat, sizeof(double) * nxat,
+                                  hipMemcpyHostToDevice, c->st));
+        d_xat = ptr<double>(c->xat);
     }
     // buffers for the records, the slice boundaries and the planes of all
     // slices, or of as many as PARTIAL_BUDGET holds (the GEMM then runs in
@@ -813,17 +872,25 @@ int dc_strucf(dc_ctx *c, const double *xat, int64_t nxat, int64_t ld_xat, const 
     const double plane = (double)sizeof(float2) * (double)pl.gg.P;
     const double planes = std::max(plane, std::min((double)PARTIAL_BUDGET, plane * (double)nslice));
     if ((st = ensure(c, c->rec, sizeof(AtomRec) * std::max<int64_t>(nxat, 1)))) return st;
-    if ((st = ensure(c, c->slice_beg, sizeof(int) * (size_t)(nslice + 1)))) return st;
     if ((st = ensure(c, c->partial, (size_t)planes))) return st;
-    if ((st = ensure(c, c->out_tcsf, sizeof(double) * 2 * ntot))) return st;
-    if ((st = strucf_core(c, g, ntot, ptr<double>(c->xat), nxat, std::max<int64_t>(nxat, 1), off_shift, lmn,
-                          lform ? ptr<double2>(c->cfact) : nullptr, ncfact, lform && istl ? ptr<int>(c->istl) : nullptr,
-                          lform, ptr<AtomRec>(c->rec), ptr<int>(c->slice_beg), ptr<float2>(c->partial), planes,
-                          ptr<double>(c->out_tcsf))))
+    const size_t obytes = sizeof(double) * 2 * (size_t)ntot;
+    const bool pinned = obytes <= HOST_OUT_BYTES && nslice * plane <= planes;   // one pass writes the output
+    double *d_out;
+    if (pinned) {
+        if ((st = pin_ensure(c, c->h_out, std::max<size_t>(obytes, 4096)))) return st;
+        d_out = reinterpret_cast<double *>(c->h_out.p);
+    } else {
+        if ((st = ensure(c, c->out_tcsf, obytes))) return st;
+        d_out = ptr<double>(c->out_tcsf);
+    }
+    if ((st = strucf_core(c, g, ntot, d_xat, nxat, n1, off_shift, lmn, d_cfact, rows, d_istl, lform, ptr<AtomRec>(c->rec),
+                          nullptr, ptr<float2>(c->partial), planes, d_out, FOLD_COLS | FOLD_ROWS)))
         return st;
-    HIPCHK(hipMemcpyAsync(tcsf, c->out_tcsf.p, sizeof(double) * 2 * ntot, hipMemcpyDeviceToHost, c->st));
+    if (!pinned) HIPCHK(hipMemcpyAsync(tcsf, d_out, obytes, hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipEventRecord(c->ev[1], c->st));
     HIPCHK(hipStreamSynchronize(c->st));
+    c->arena_busy = false;
+    if (pinned) std::memcpy(tcsf, d_out, obytes);
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
     c->stats.total_ms = ms;
@@ -1004,11 +1071,11 @@ long long lot_type_runs(const dc_ctx *c, const std::vector<CellRun> &cruns, int 
 // c->partial.  Positions come from the resident crystal (idx/oid/offs) or,
 // when explicit != null, from an explicit (n,3) list.  group_seg (ascending
 // segment indices, the last one = gl.segs.size()) marks groups of segments
-// (the lots of a batch): their slice boundaries go to c->lot_slice, uploaded
-// with the slice tables before the launch.
+// (the lots of a batch): their slice boundaries go to lot_slice and the slices'
+// types to slice_type, staged with the slice tables before the launch.
 int gemm_segments(dc_ctx *c, const Grid &g, const Plan &pl, GatherList &gl,
                   const double *explicit_pos, SliceSet &ss, int &nslice, bool use_type_lists,
-                  const std::vector<int> &group_seg) {
+                  const std::vector<int> &group_seg, const int *&lot_slice, const int *&slice_type) {
     const GemmGeom &gg = pl.gg;
     const int mapping = pl.mapping;
     int st = 0;
@@ -1017,35 +1084,38 @@ int gemm_segments(dc_ctx *c, const Grid &g, const Plan &pl, GatherList &gl,
     PrepArgs pa = base_prep(g, mapping);
     pa.n = n;
     if (explicit_pos) {
-        if ((st = upload(c, c->xat, explicit_pos, 3 * (size_t)std::max<long long>(n, 1)))) return st;
-        pa.src = ptr<double>(c->xat);
+        double *d = nullptr;
+        if ((st = stage(c, c->xat, explicit_pos, 3 * (size_t)n, d))) return st;
+        pa.src = d;
         pa.src_ld = 0;
     } else {
         pa.src = ptr<double>(c->pos);
         if (use_type_lists) {
             pa.idx = ptr<int>(c->type_idx);
         } else if (!gl.runs.empty()) {
-            if ((st = upload(c, c->runs, gl.runs.data(), gl.runs.size()))) return st;
-            if ((st = upload(c, c->offs, gl.offs.data(), gl.offs.size()))) return st;
+            int4 *d_runs;
+            double *d_offs;
+            if ((st = stage(c, c->runs, gl.runs.data(), gl.runs.size(), d_runs))) return st;
+            if ((st = stage(c, c->offs, gl.offs.data(), gl.offs.size(), d_offs))) return st;
             pa.idx = ptr<int>(c->type_idx);
-            pa.runs = ptr<int4>(c->runs);
+            pa.runs = d_runs;
             pa.nruns = (int)gl.runs.size();
-            pa.offs = ptr<double>(c->offs);
+            pa.offs = d_offs;
         } else {
-            if ((st = upload(c, c->idx, gl.idx.data(), gl.idx.size()))) return st;
-            pa.idx = ptr<int>(c->idx);
+            int *d_idx, *d_oid;
+            double *d_offs;
+            if ((st = stage(c, c->idx, gl.idx.data(), gl.idx.size(), d_idx))) return st;
+            pa.idx = d_idx;
             if (!gl.oid.empty()) {
-                if ((st = upload(c, c->oid, gl.oid.data(), gl.oid.size()))) return st;
-                if ((st = upload(c, c->offs, gl.offs.data(), gl.offs.size()))) return st;
-                pa.oid = ptr<int>(c->oid);
-                pa.offs = ptr<double>(c->offs);
+                if ((st = stage(c, c->oid, gl.oid.data(), gl.oid.size(), d_oid))) return st;
+                if ((st = stage(c, c->offs, gl.offs.data(), gl.offs.size(), d_offs))) return st;
+                pa.oid = d_oid;
+                pa.offs = d_offs;
             }
         }
     }
     if ((st = ensure(c, c->rec, sizeof(AtomRec) * std::max<long long>(n, 1)))) return st;
     pa.hash_salt = launch_geom(c, gg).dither;   // run_gemm below launches undamped
-    HIPCHK(launch_prep(pa, ptr<AtomRec>(c->rec), c->st));
-    c->rec_hash = true;
     int off = 0;
     ss = SliceSet();
     add_segments(ss, gl.segs, slice_len(c, kchunk_for(pl, gl.segs, pl.scheme)), off);
@@ -1062,20 +1132,26 @@ int gemm_segments(dc_ctx *c, const Grid &g, const Plan &pl, GatherList &gl,
         for (int &v : ss.seg_first) v *= pps;
     }
     nslice = ngemm * pps;
-    if ((st = upload(c, c->slice_beg, ss.beg.data(), ss.beg.size()))) return st;
-    if ((st = upload(c, c->slice_type, ss.type.data(), std::max<size_t>(ss.type.size(), 1)))) return st;
+    int *d_beg, *d_type, *d_lot;
+    if ((st = stage(c, c->slice_beg, ss.beg.data(), ss.beg.size(), d_beg))) return st;
+    if ((st = stage(c, c->slice_type, ss.type.data(), ss.type.size(), d_type))) return st;
     ss.seg_first.push_back(nslice);
     std::vector<int> gsl;
     for (int v : group_seg) gsl.push_back(ss.seg_first[v]);
-    if ((st = upload(c, c->lot_slice, gsl.data(), gsl.size()))) return st;
+    if ((st = stage(c, c->lot_slice, gsl.data(), gsl.size(), d_lot))) return st;
+    lot_slice = d_lot;
+    slice_type = d_type;
     if ((st = ensure(c, c->partial, sizeof(float2) * gg.P * std::max(nslice, 1)))) return st;
-    return run_gemm(c, pl, ss.beg, ptr<float2>(c->partial));
+    if ((st = stage_flush(c))) return st;
+    HIPCHK(launch_prep(pa, ptr<AtomRec>(c->rec), c->st));
+    c->rec_hash = true;
+    return run_gemm(c, pl, ss.beg, d_beg, ptr<float2>(c->partial));
 }
 
 }  // namespace
 
-int dc_four_run_dev(dc_ctx *c, const dc_run_desc *r, double *d_csf, double *d_acsf, double *d_dsi,
-                    double *d_fmean, double *d_dvar) {
+static int four_run(dc_ctx *c, const dc_run_desc *r, double *d_csf, double *d_acsf, double *d_dsi, double *d_fmean,
+                    double *d_dvar) {
     if (!c) return DC_ERR_ARG;
     c->err.clear();
     c->err_typ = DC_ER_NONE;
@@ -1124,7 +1200,8 @@ int dc_four_run_dev(dc_ctx *c, const dc_run_desc *r, double *d_csf, double *d_ac
     g.P = (long long)fnum[0] * fnum[1] * fnum[2];
     g.friedel = fried != 0;
     const long long ntot = (long long)g.n[0] * g.n[1] * g.n[2];
-    if (max_corner_bin(g) > std::min(CFPKT, r->ncfact - 1))
+    const int top_bin = max_corner_bin(g);
+    if (top_bin > std::min(CFPKT, r->ncfact - 1))
         return set_err(c, DC_ERR_ISTL, DC_ER_FOUR, "sin(theta)/lambda beyond the form factor table");
 
     // atoms of one GEMM launch: the crystal, or the lots of a batch
@@ -1147,7 +1224,11 @@ int dc_four_run_dev(dc_ctx *c, const dc_run_desc *r, double *d_csf, double *d_ac
                        : c->prec == DC_PREC_BF16X3 ? DC_PREC_FP16X3 : c->prec;
     const Plan pl = plan_gemm(g, c->tile, -1, scheme, natoms_launch);
     int st = 0;
-    if ((st = upload(c, c->cfact, r->cfact, 2 * (size_t)r->ncfact * c->nscat))) return st;
+    if ((st = stage_begin(c))) return st;
+    const int rows = cfact_rows(top_bin, r->ncfact);
+    double2 *d_cfact;
+    if ((st = stage_cfact(c, r->cfact, r->ncfact, c->nscat, rows, d_cfact))) return st;
+    const int *lot_slice = nullptr, *slice_type = nullptr;
 
     // compact-region state: every element is written before it is read (<F>
     // by its reduction, dsi and the moments by the first lot batch's
@@ -1194,18 +1275,18 @@ int dc_four_run_dev(dc_ctx *c, const dc_run_desc *r, double *d_csf, double *d_ac
         }
         SliceSet ss;
         int nslice = 0;
-        if ((st = gemm_segments(c, g, pl, gl, nullptr, ss, nslice, false, {0, (int)gl.segs.size()}))) return st;
+        if ((st = gemm_segments(c, g, pl, gl, nullptr, ss, nslice, false, {0, (int)gl.segs.size()}, lot_slice, slice_type))) return st;
         pairs += (double)gl.idx.size() * (double)ntot;
         nslices_total += nslice;
         ReduceArgs ra{};
         ra.g = g;
         ra.partial = ptr<float2>(c->partial);
-        ra.lot_slice = ptr<int>(c->lot_slice);
-        ra.slice_type = ptr<int>(c->slice_type);
+        ra.lot_slice = lot_slice;
+        ra.slice_type = slice_type;
         ra.nlots = 1;
         ra.lform = 1;
-        ra.cfact = ptr<double2>(c->cfact);
-        ra.ncfact = r->ncfact;
+        ra.cfact = d_cfact;
+        ra.ncfact = rows;
         HIPCHK(launch_reduce_sum(ra, ptr<double>(c->acsf), 0, c->st));
         // lattice of the lot shape over the full grid (four_getav :2440-2510)
         std::vector<double> lp;
@@ -1241,14 +1322,14 @@ int dc_four_run_dev(dc_ctx *c, const dc_run_desc *r, double *d_csf, double *d_ac
         const Plan pll = plan_gemm(gl_full, c->tile, -1, scheme, (long long)(lp.size() / 3));
         GatherList gll;
         gll.segs.push_back({0, (int)(lp.size() / 3)});
-        if ((st = gemm_segments(c, gl_full, pll, gll, lp.data(), ss, nslice, false, {0, 1}))) return st;
+        if ((st = gemm_segments(c, gl_full, pll, gll, lp.data(), ss, nslice, false, {0, 1}, lot_slice, slice_type))) return st;
         pairs += (double)(lp.size() / 3) * (double)ntot;
         nslices_total += nslice;
         if ((st = ensure(c, c->lat, sizeof(double) * 2 * ntot))) return st;
         ReduceArgs rl{};
         rl.g = gl_full;
         rl.partial = ptr<float2>(c->partial);
-        rl.lot_slice = ptr<int>(c->lot_slice);
+        rl.lot_slice = lot_slice;
         rl.nlots = 1;
         rl.lform = 0;
         HIPCHK(launch_reduce_sum(rl, ptr<double>(c->lat), 0, c->st));
@@ -1303,20 +1384,20 @@ int dc_four_run_dev(dc_ctx *c, const dc_run_desc *r, double *d_csf, double *d_ac
         lot_first_seg.push_back((int)gl.segs.size());
         SliceSet ss;
         int nslice = 0;
-        if ((st = gemm_segments(c, g, pl, gl, nullptr, ss, nslice, !lots, lot_first_seg))) return st;
+        if ((st = gemm_segments(c, g, pl, gl, nullptr, ss, nslice, !lots, lot_first_seg, lot_slice, slice_type))) return st;
         pairs += (double)n_batch * (double)ntot;
         nslices_total += nslice;
         ReduceArgs ra{};
         ra.g = g;
         ra.partial = ptr<float2>(c->partial);
         ra.slice0 = 0;
-        ra.lot_slice = ptr<int>(c->lot_slice);
-        ra.slice_type = ptr<int>(c->slice_type);
+        ra.lot_slice = lot_slice;
+        ra.slice_type = slice_type;
         ra.nlots = l1 - lot;
         ra.lot0 = lot;
         ra.lform = 1;
-        ra.cfact = ptr<double2>(c->cfact);
-        ra.ncfact = r->ncfact;
+        ra.cfact = d_cfact;
+        ra.ncfact = rows;
         ra.ntype = c->nscat;
         ra.acsf = acsf;
         ra.dsi = ptr<double>(c->dsi);
@@ -1353,6 +1434,7 @@ int dc_four_run_dev(dc_ctx *c, const dc_run_desc *r, double *d_csf, double *d_ac
     HIPCHK(launch_finalize(fa, c->st));
     HIPCHK(hipEventRecord(c->ev[1], c->st));
     HIPCHK(hipEventSynchronize(c->ev[1]));
+    c->arena_busy = false;
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
     c->stats.total_ms = ms;
@@ -1363,6 +1445,11 @@ int dc_four_run_dev(dc_ctx *c, const dc_run_desc *r, double *d_csf, double *d_ac
     return warn;
 }
 
+int dc_four_run_dev(dc_ctx *c, const dc_run_desc *r, double *d_csf, double *d_acsf, double *d_dsi,
+                    double *d_fmean, double *d_dvar) {
+    return four_run(c, r, d_csf, d_acsf, d_dsi, d_fmean, d_dvar);
+}
+
 int dc_four_run(dc_ctx *c, const dc_run_desc *r, double *csf, double *acsf, double *dsi, double *fmean,
                 double *dvar) {
     if (!c || !r) return DC_ERR_ARG;
@@ -1371,16 +1458,38 @@ int dc_four_run(dc_ctx *c, const dc_run_desc *r, double *csf, double *acsf, doub
     const int width[5] = {2, 2, 1, 2, 1};
     double *dev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     int st = 0;
+    // without the <F> subtraction acsf is zero: filled here
+    const bool zero_acsf = acsf && r->fave == 0.0;
+    size_t bytes = 0;
     for (int k = 0; k < 5; ++k)
-        if (host[k]) {
-            if ((st = ensure(c, c->out[k], sizeof(double) * width[k] * ntot))) return st;
+        if (host[k] && !(k == 1 && zero_acsf)) bytes += sizeof(double) * width[k] * ntot;
+    const bool pinned = bytes <= HOST_OUT_BYTES;
+    if (pinned && (st = pin_ensure(c, c->h_out, std::max<size_t>(bytes, 4096)))) return st;
+    size_t off = 0;
+    for (int k = 0; k < 5; ++k) {
+        if (!host[k] || (k == 1 && zero_acsf)) continue;
+        const size_t n = sizeof(double) * width[k] * ntot;
+        if (pinned) {
+            dev[k] = reinterpret_cast<double *>(c->h_out.p + off);
+            off += n;
+        } else {
+            if ((st = ensure(c, c->out[k], n))) return st;
             dev[k] = ptr<double>(c->out[k]);
         }
-    st = dc_four_run_dev(c, r, dev[0], dev[1], dev[2], dev[3], dev[4]);
+    }
+    st = four_run(c, r, dev[0], dev[1], dev[2], dev[3], dev[4]);
     if (st < 0) return st;
-    for (int k = 0; k < 5; ++k)
-        if (host[k]) HIPCHK(hipMemcpyAsync(host[k], dev[k], sizeof(double) * width[k] * ntot, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
+    for (int k = 0; k < 5; ++k) {
+        const size_t n = sizeof(double) * width[k] * ntot;
+        if (!host[k]) continue;
+        if (k == 1 && zero_acsf)
+            std::memset(host[k], 0, n);
+        else if (pinned)
+            std::memcpy(host[k], dev[k], n);
+        else
+            HIPCHK(hipMemcpyAsync(host[k], dev[k], n, hipMemcpyDeviceToHost, c->st));
+    }
+    if (!pinned) HIPCHK(hipStreamSynchronize(c->st));
     return st;
 }
 

@@ -41,6 +41,8 @@ struct BatchState {
     int walk = 1, nset = 0;              // adjoint column tiles per work-group, partial sets
     int walk_req = 0;                    // the context's adjoint walk setting at planning
     int64_t natoms = 0;
+    int rows = 0;                        // form-factor rows on the device (the bins the metrics reach, and a margin)
+    PinBuf h_cf, h_sq, h_chi;            // pinned: form-factor rows, s^2 parts, chi^2 of the members
     DevBuf pos, occ, bdw, idx, rec, sbeg, stype, ssq, msl, sorder, partial, cfact, rten, sq, target, weight, icalc,
         chi, q, qs, atiles, part, grad, wq;
     bool queue = false;                  // GEMM items from a device counter (autotuner's choice)
@@ -64,6 +66,8 @@ void batch_release(dc_ctx *c) {
     if (b->graph) (void)hipGraphDestroy(b->graph);
     for (DevBuf *d : b->buffers())
         if (d->p) (void)hipFree(d->p);
+    for (PinBuf *p : {&b->h_cf, &b->h_sq, &b->h_chi})
+        if (p->p) (void)hipHostFree(p->p);
     delete b;
     c->batch = nullptr;
 }
@@ -79,6 +83,7 @@ double dotg(const double *a, const double *g, const double *b) {
     return s;
 }
 
+// The cached state fits the call, its atom types apart (same_types).
 bool same_shape(const BatchState *b, const dc_ctx *c, const dc_batch_desc *d, bool want_grad, bool want_icalc,
                 bool have_weight, bool any_b) {
     if (!b) return false;
@@ -90,8 +95,10 @@ bool same_shape(const BatchState *b, const dc_ctx *c, const dc_batch_desc *d, bo
     if (std::memcmp(b->eck, d->eck, sizeof(b->eck)) || std::memcmp(b->vi, d->vi, sizeof(b->vi)) ||
         std::memcmp(b->inc, d->inc, sizeof(b->inc)))
         return false;
-    if (!std::equal(b->atom_beg.begin(), b->atom_beg.end(), d->atom_beg)) return false;
-    return std::equal(b->type.begin(), b->type.end(), d->type);
+    return std::equal(b->atom_beg.begin(), b->atom_beg.end(), d->atom_beg);
+}
+bool same_types(const BatchState &b, const dc_batch_desc *d) {
+    return std::memcmp(b.type.data(), d->type, sizeof(int) * b.type.size()) == 0;
 }
 
 int check_desc(dc_ctx *c, const dc_batch_desc *d) {
@@ -103,16 +110,22 @@ int check_desc(dc_ctx *c, const dc_batch_desc *d) {
         if (d->atom_beg[m + 1] < d->atom_beg[m]) return set_err(c, DC_ERR_ARG, DC_ER_LIB, "batch: atom_beg decreasing");
     const int64_t n = d->atom_beg[d->nmembers];
     if (n > INT32_MAX / 8) return set_err(c, DC_ERR_ARG, DC_ER_LIB, "batch: too many atoms");
-    for (int64_t k = 0; k < n; ++k)
-        if (d->type[k] < 0 || d->type[k] > d->nscat) return set_err(c, DC_ERR_ARG, DC_ER_LIB, "batch: type outside 0..nscat");
     for (int k = 0; k < 3; ++k)
         if (d->inc[k] < 1) return set_err(c, DC_ERR_ARG, DC_ER_LIB, "batch: bad inc");
+    return 0;
+}
+int check_types(dc_ctx *c, const dc_batch_desc *d) {
+    const int64_t n = d->atom_beg[d->nmembers];
+    for (int64_t k = 0; k < n; ++k)
+        if (d->type[k] < 0 || d->type[k] > d->nscat) return set_err(c, DC_ERR_ARG, DC_ER_LIB, "batch: type outside 0..nscat");
     return 0;
 }
 
 // s^2 row / column parts for every member's metric; errors on grids that are
 // not metric-orthogonal between rows and columns when B or gradients need it.
-int member_sq(dc_ctx *c, const Grid &g, const GemmGeom &gg, const dc_batch_desc *d, std::vector<float> &sq, bool need_sep) {
+int member_sq(dc_ctx *c, const Grid &g, const GemmGeom &gg, const dc_batch_desc *d, std::vector<float> &sq, bool need_sep,
+              int &top_bin) {
+    top_bin = 0;
     const int stride = gg.R + gg.C;
     sq.assign((size_t)stride * d->nmembers, 0.0f);
     const double *v1 = d->vi, *v2 = d->vi + 3, *v3 = d->vi + 6;
@@ -143,7 +156,8 @@ int member_sq(dc_ctx *c, const Grid &g, const GemmGeom &gg, const dc_batch_desc 
         }
         Grid gm = g;
         for (int k = 0; k < 9; ++k) gm.rten[k] = G[k];
-        if (max_corner_bin(gm) >= d->ncfact) return set_err(c, DC_ERR_ISTL, DC_ER_FOUR, "sin(theta)/lambda beyond table");
+        top_bin = std::max(top_bin, max_corner_bin(gm));
+        if (top_bin >= d->ncfact) return set_err(c, DC_ERR_ISTL, DC_ER_FOUR, "sin(theta)/lambda beyond table");
     }
     return 0;
 }
@@ -259,20 +273,17 @@ int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
     b.nblk = (int)std::min<long long>((g.P + 255) / 256, 256);
 
     int st;
-    const size_t P = (size_t)g.P, M = (size_t)d->nmembers, T = (size_t)std::max<int64_t>(b.natoms, 1);
+    const size_t M = (size_t)d->nmembers;
     if ((st = upload(c, b.idx, b.order.data(), b.order.size()))) return st;
     if ((st = make_slices(c, b, slice_len(c, kchunk_for(b.pl, b.segs, b.pl.scheme))))) return st;
     if ((st = upload(c, b.atiles, tiles.data(), tiles.size()))) return st;
-    if ((st = ensure(c, b.pos, sizeof(double) * 3 * T))) return st;
-    if ((st = ensure(c, b.occ, sizeof(double) * T))) return st;
-    if ((st = ensure(c, b.bdw, sizeof(double) * T))) return st;
     if ((st = ensure(c, b.rec, sizeof(AtomRec) * std::max(b.nsorted, 1)))) return st;
-    if ((st = ensure(c, b.cfact, sizeof(double) * 2 * (size_t)d->ncfact * d->nscat * M))) return st;
+    if ((st = ensure(c, b.cfact, sizeof(double) * 2 * (size_t)b.rows * d->nscat * M))) return st;
+    if ((st = pin_ensure(c, b.h_cf, sizeof(double) * (2 * (size_t)b.rows * d->nscat + 9) * M))) return st;
+    if ((st = pin_ensure(c, b.h_sq, sizeof(float) * (size_t)(gg.R + gg.C) * M))) return st;
+    if ((st = pin_ensure(c, b.h_chi, sizeof(double) * M))) return st;
     if ((st = ensure(c, b.rten, sizeof(double) * 9 * M))) return st;
     if ((st = ensure(c, b.sq, sizeof(float) * (size_t)(gg.R + gg.C) * M))) return st;
-    if ((st = ensure(c, b.target, sizeof(double) * P * M))) return st;
-    if (b.have_weight && (st = ensure(c, b.weight, sizeof(double) * P * M))) return st;
-    if (b.want_icalc && (st = ensure(c, b.icalc, sizeof(double) * P * M))) return st;
     if ((st = ensure(c, b.chi, sizeof(double) * (size_t)b.nblk * M))) return st;
     if (b.want_grad) {
         if ((st = ensure(c, b.q, sizeof(float2) * gg.P * d->nscat * M))) return st;
@@ -283,14 +294,39 @@ int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
             const size_t rg = (size_t)((gg.R + 15) / 16) * 4;
             if ((st = ensure(c, b.qs, sizeof(uint32_t) * 8 * rg * gg.C * d->nscat * M))) return st;
         }
-        if ((st = ensure(c, b.grad, sizeof(double) * 5 * T))) return st;
     }
     return 0;
 }
 
+// Arrays of one step: the state's own (host entry point, replayed graph) or the
+// caller's device arrays.
+struct StepIO {
+    const double *pos, *occ, *bdw, *target, *weight;
+    double *icalc, *grad;
+};
+StepIO own_io(BatchState &b) {
+    return {ptr<double>(b.pos), ptr<double>(b.occ), b.any_b ? ptr<double>(b.bdw) : nullptr, ptr<double>(b.target),
+            b.have_weight ? ptr<double>(b.weight) : nullptr, b.want_icalc ? ptr<double>(b.icalc) : nullptr,
+            b.want_grad ? ptr<double>(b.grad) : nullptr};
+}
+
+// chi^2 of every member from the reduction's block sums, into pinned memory.
+__global__ void chi_finish_kernel(const double *__restrict__ part, int nblk, double *__restrict__ out) {
+    __shared__ double red[256];
+    double s = 0.0;
+    for (int k = threadIdx.x; k < nblk; k += 256) s += part[(size_t)blockIdx.x * nblk + k];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int h = 128; h > 0; h >>= 1) {
+        if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[blockIdx.x] = red[0];
+}
+
 // The reduction of the slice planes: every member's I, its chi^2 partial sums
 // and, when gradients are wanted, the Q planes.
-int reduce_planes(dc_ctx *c, BatchState &b) {
+int reduce_planes(dc_ctx *c, BatchState &b, const StepIO &io) {
     const GemmGeom &gg = b.pl.gg;
     BatchReduceArgs ra{};
     ra.g = b.g;
@@ -302,13 +338,13 @@ int reduce_planes(dc_ctx *c, BatchState &b) {
     ra.mslice = ptr<int>(b.msl);
     ra.slice_type = ptr<int>(b.stype);
     ra.cfact = ptr<double2>(b.cfact);
-    ra.ncfact = b.ncfact;
+    ra.ncfact = b.rows;
     ra.nscat = b.nscat;
     ra.nmembers = b.nmembers;
     ra.rten = ptr<double>(b.rten);
-    ra.target = ptr<double>(b.target);
-    ra.weight = b.have_weight ? ptr<double>(b.weight) : nullptr;
-    ra.icalc = b.want_icalc ? ptr<double>(b.icalc) : nullptr;
+    ra.target = io.target;
+    ra.weight = io.weight;
+    ra.icalc = io.icalc;
     ra.chi_part = ptr<double>(b.chi);
     ra.q = b.want_grad ? ptr<float2>(b.q) : nullptr;
     HIPCHK(launch_batch_reduce(ra, b.nblk, c->st));
@@ -316,41 +352,45 @@ int reduce_planes(dc_ctx *c, BatchState &b) {
 }
 
 // Kernels of one population step, in stream order (captured into the graph).
-// rest: 0 = records (prep) and GEMM only, 1 = and the reduction (I, chi^2,
-// Q planes), 2 = and the adjoint when gradients are wanted.
+// part: STEP_GEMM = records (prep) and GEMM, STEP_REST = the reduction (I,
+// chi^2, Q planes) and the adjoint when gradients are wanted.
+constexpr int STEP_GEMM = 1, STEP_REST = 2;
 __global__ void zero_counter_kernel(int *p) {
     if (threadIdx.x == 0) *p = 0;
 }
 
-int enqueue(dc_ctx *c, BatchState &b, int tile, int nwg, bool prep, int rest, bool queue) {
+int enqueue(dc_ctx *c, BatchState &b, const StepIO &io, int tile, int nwg, bool prep, int part, bool queue) {
     const GemmGeom &gg = b.pl.gg;
+    int st;
     if (prep) {
         PrepArgs pa = base_prep(b.g, 0);
-        pa.src = ptr<double>(b.pos);
+        pa.src = io.pos;
         pa.src_ld = 0;
         pa.idx = ptr<int>(b.idx);
-        pa.occ_src = ptr<double>(b.occ);
-        pa.bdw_src = b.any_b ? ptr<double>(b.bdw) : nullptr;
+        pa.occ_src = io.occ;
+        pa.bdw_src = io.bdw;
         pa.n = b.nsorted;
         if (b.nsorted > 0) HIPCHK(launch_prep(pa, ptr<AtomRec>(b.rec), c->st));
     }
-    GemmGeom lg = launch_geom(c, gg);
-    lg.fold = fold_side(gg, b.fold_mask, tile);
-    lg.order = ptr<int>(b.sorder);
-    if (queue) {
-        int st = ensure(c, b.wq, 256);
-        if (st) return st;
-        zero_counter_kernel<<<1, 64, 0, c->st>>>(ptr<int>(b.wq));
-        HIPCHK(hipGetLastError());
-        lg.queue = ptr<int>(b.wq);
+    if (part & STEP_GEMM) {
+        GemmGeom lg = launch_geom(c, gg);
+        lg.fold = fold_side(gg, b.fold_mask, tile);
+        lg.order = ptr<int>(b.sorder);
+        if (queue) {
+            if ((st = ensure(c, b.wq, 256))) return st;
+            zero_counter_kernel<<<1, 64, 0, c->st>>>(ptr<int>(b.wq));
+            HIPCHK(hipGetLastError());
+            lg.queue = ptr<int>(b.wq);
+        }
+        HIPCHK(launch_phase_gemm(b.pl.scheme, tile, ptr<AtomRec>(b.rec), ptr<int>(b.sbeg), ptr<float2>(b.partial),
+                                 b.any_b ? ptr<float>(b.sq) : nullptr, lg, 0, b.nslice, c->st, nwg, ptr<int>(b.ssq)));
     }
-    HIPCHK(launch_phase_gemm(b.pl.scheme, tile, ptr<AtomRec>(b.rec), ptr<int>(b.sbeg), ptr<float2>(b.partial),
-                             b.any_b ? ptr<float>(b.sq) : nullptr, lg, 0, b.nslice, c->st, nwg, ptr<int>(b.ssq)));
-    if (rest < 1) return 0;
-    int st = reduce_planes(c, b);
-    if (st) return st;
-    if (rest >= 2 && b.want_grad) {
-        HIPCHK(launch_fill_zero(ptr<double>(b.grad), 5 * b.natoms, c->st));
+    if (!(part & STEP_REST)) return 0;
+    if ((st = reduce_planes(c, b, io))) return st;
+    chi_finish_kernel<<<b.nmembers, 256, 0, c->st>>>(ptr<double>(b.chi), b.nblk, reinterpret_cast<double *>(b.h_chi.p));
+    HIPCHK(hipGetLastError());
+    if (b.want_grad) {
+        HIPCHK(launch_fill_zero(io.grad, 5 * b.natoms, c->st));
         AdjArgs aa{};
         aa.rec = ptr<AtomRec>(b.rec);
         aa.tiles = ptr<int4>(b.atiles);
@@ -380,11 +420,11 @@ int enqueue(dc_ctx *c, BatchState &b, int tile, int nwg, bool prep, int rest, bo
         fa.ntile_c = b.nset;
         fa.natoms = b.nsorted;
         fa.idx = ptr<int>(b.idx);
-        fa.occ = ptr<double>(b.occ);
+        fa.occ = io.occ;
         for (int k = 0; k < 3; ++k)
             fa.hc[k] = b.eck[k] + (double)aa.rc * b.vi[k] + (double)aa.jc * b.vi[3 + k] + (double)aa.mc * b.vi[6 + k];
         for (int k = 0; k < 9; ++k) fa.v[k] = b.vi[k];
-        fa.grad = ptr<double>(b.grad);
+        fa.grad = io.grad;
         HIPCHK(launch_adjoint_finish(fa, c->st));
     }
     return 0;
@@ -403,7 +443,7 @@ int enqueue(dc_ctx *c, BatchState &b, int tile, int nwg, bool prep, int rest, bo
 // changes the FP32 summation order, so a choice made on noise would change
 // the results' last bits from one context to the next for nothing (on the
 // 96-member population the planned length wins).
-int autotune(dc_ctx *c, BatchState &b) {
+int autotune(dc_ctx *c, BatchState &b, const StepIO &io) {
     const bool fp32_only = b.prec == DC_PREC_FP32;    // tiles built without an FP32 variant are skipped
     auto built = [&](int t) {
         const TileInfo ti = gemm_tile_info(t);
@@ -432,11 +472,11 @@ int autotune(dc_ctx *c, BatchState &b) {
     auto time_ms = [&](int t, int nwg, bool reduce, float &ms) -> int {
         const bool qu = nwg < 0;
         const int n = qu ? -nwg : nwg;
-        int st = reduce ? reduce_planes(c, b) : enqueue(c, b, t, n, false, 0, qu);
+        int st = reduce ? reduce_planes(c, b, io) : enqueue(c, b, io, t, n, false, STEP_GEMM, qu);
         if (st) return st;
         HIPCHK(hipEventRecord(c->ev[2], c->st));
         for (int r = 0; r < 2; ++r)
-            if ((st = reduce ? reduce_planes(c, b) : enqueue(c, b, t, n, false, 0, qu))) return st;
+            if ((st = reduce ? reduce_planes(c, b, io) : enqueue(c, b, io, t, n, false, STEP_GEMM, qu))) return st;
         HIPCHK(hipEventRecord(c->ev[3], c->st));
         HIPCHK(hipEventSynchronize(c->ev[3]));
         HIPCHK(hipEventElapsedTime(&ms, c->ev[2], c->ev[3]));
@@ -522,9 +562,10 @@ int dc_batch_info(const dc_ctx *c, int *tile, int *nwg, int *graph, double *tune
 namespace {
 
 // One population step.  dev = false: pos/occ/bdw of d, target, weight, icalc
-// and grad are host arrays; dev = true: they are device arrays (the inputs
-// are copied on the device into the buffers the graph reads, the outputs
-// out of them), and a non-null bdw counts as per-atom B.
+// and grad are host arrays, copied to and from the buffers that the replayed
+// graph works on; dev = true: they are device arrays, which the kernels of the
+// step, launched one by one, read and write in place (96 members, 1.8M atoms:
+// the copies moved 400 MB), and a non-null bdw counts as per-atom B.
 int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const double *weight, double *chi2,
                double *icalc, double *grad, bool dev) {
     if (!c) return DC_ERR_ARG;
@@ -537,8 +578,6 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
     HIPCHK(hipSetDevice(c->device));
     stats_begin(c);
     const int64_t natoms = d->atom_beg[d->nmembers];
-    const hipMemcpyKind in = dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-    const hipMemcpyKind out = dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     bool any_b = dev && d->bdw != nullptr;
     if (d->bdw && !dev)
         for (int64_t k = 0; k < natoms && !any_b; ++k) any_b = d->type[k] > 0 && d->bdw[k] != 0.0;
@@ -546,14 +585,41 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
     // s^2 of this call's metrics; with per-atom B the mirrored-pair tiles fold
     // a side only where every member's s^2 is mirrored about its centre
     std::vector<float> sq;
-    int fold_mask = FOLD_COLS | FOLD_ROWS;
+    int fold_mask = FOLD_COLS | FOLD_ROWS, top_bin = 0;
     {
-        Grid g = batch_grid(d);
-        const GemmGeom gg = plan_gemm(g, c->tile, 0, model_scheme(c->prec), natoms).gg;
-        if ((st = member_sq(c, g, gg, d, sq, any_b || want_grad))) return st;
+        const Grid g = batch_grid(d);
+        const GemmGeom gg = mapping0_geom(g);
+        if ((st = member_sq(c, g, gg, d, sq, any_b || want_grad, top_bin))) return st;
         for (int m = 0; m < d->nmembers && any_b; ++m) fold_mask &= mirrored_sides(gg, sq.data() + (size_t)m * (gg.R + gg.C));
     }
-    if (!same_shape(c->batch, c, d, want_grad, want_icalc, have_weight, any_b) || c->batch->fold_mask != fold_mask) {
+    const bool shape = same_shape(c->batch, c, d, want_grad, want_icalc, have_weight, any_b) &&
+                       c->batch->fold_mask == fold_mask && cfact_rows(top_bin, d->ncfact) <= c->batch->rows;
+    // Device arrays and a state of this shape: the records and the GEMM start
+    // on the cached plan while the host compares the atom types with the
+    // plan's (1.8M atoms: 0.5 ms) and packs the form factors; other types
+    // discard what was started.  Everything that was started stays inside the
+    // state's buffers, whose sizes the shape fixes.
+    const bool early = dev && shape && c->batch->primed;
+    const StepIO io_dev{d->pos, d->occ, any_b ? d->bdw : nullptr, target, weight, icalc, grad};
+    auto send_sq = [&](BatchState &b) -> int {
+        std::memcpy(b.h_sq.p, sq.data(), sizeof(float) * sq.size());
+        HIPCHK(hipMemcpyAsync(b.sq.p, b.h_sq.p, sizeof(float) * sq.size(), hipMemcpyHostToDevice, c->st));
+        return 0;
+    };
+    if (early) {
+        BatchState &b = *c->batch;
+        HIPCHK(hipEventRecord(c->ev[0], c->st));
+        if ((st = send_sq(b))) return st;
+        HIPCHK(hipEventRecord(c->ev[4], c->st));
+        if ((st = enqueue(c, b, io_dev, b.pl.tile, b.nwg, true, STEP_GEMM, b.queue))) return st;
+    }
+    bool fits = shape && same_types(*c->batch, d);
+    if (!fits) {
+        if ((st = check_types(c, d))) {
+            (void)hipStreamSynchronize(c->st);
+            return st;
+        }
+        HIPCHK(hipStreamSynchronize(c->st));
         batch_release(c);
         c->batch = new BatchState();
         c->batch->want_grad = want_grad;
@@ -561,60 +627,76 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
         c->batch->have_weight = have_weight;
         c->batch->any_b = any_b;
         c->batch->fold_mask = fold_mask;
+        // a margin for the metrics of later generations
+        c->batch->rows = std::min(d->ncfact, cfact_rows(top_bin, d->ncfact) + top_bin / 4 + 16);
         if ((st = build_state(c, d, *c->batch))) {
             batch_release(c);
             return st;
         }
     }
     BatchState &b = *c->batch;
+    const bool started = early && fits;
     const size_t P = (size_t)b.g.P, M = (size_t)d->nmembers;
-    HIPCHK(hipEventRecord(c->ev[0], c->st));
-    HIPCHK(hipMemcpyAsync(b.pos.p, d->pos, sizeof(double) * 3 * natoms, in, c->st));
-    HIPCHK(hipMemcpyAsync(b.occ.p, d->occ, sizeof(double) * natoms, in, c->st));
-    if (any_b) HIPCHK(hipMemcpyAsync(b.bdw.p, d->bdw, sizeof(double) * natoms, in, c->st));
-    HIPCHK(hipMemcpyAsync(b.cfact.p, d->cfact, sizeof(double) * 2 * d->ncfact * d->nscat * M, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(b.rten.p, d->rten, sizeof(double) * 9 * M, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(b.sq.p, sq.data(), sizeof(float) * sq.size(), hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(b.target.p, target, sizeof(double) * P * M, in, c->st));
-    if (weight) HIPCHK(hipMemcpyAsync(b.weight.p, weight, sizeof(double) * P * M, in, c->st));
+    if (!dev) {
+        const size_t T = (size_t)std::max<int64_t>(natoms, 1);
+        if ((st = ensure(c, b.pos, sizeof(double) * 3 * T))) return st;
+        if ((st = ensure(c, b.occ, sizeof(double) * T))) return st;
+        if ((st = ensure(c, b.bdw, sizeof(double) * T))) return st;
+        if ((st = ensure(c, b.target, sizeof(double) * P * M))) return st;
+        if (weight && (st = ensure(c, b.weight, sizeof(double) * P * M))) return st;
+        if (want_icalc && (st = ensure(c, b.icalc, sizeof(double) * P * M))) return st;
+        if (want_grad && (st = ensure(c, b.grad, sizeof(double) * 5 * T))) return st;
+    }
+    const StepIO io = dev ? io_dev : own_io(b);
+    if (!started) {
+        HIPCHK(hipEventRecord(c->ev[0], c->st));
+        if (!dev) {
+            HIPCHK(hipMemcpyAsync(b.pos.p, d->pos, sizeof(double) * 3 * natoms, hipMemcpyHostToDevice, c->st));
+            HIPCHK(hipMemcpyAsync(b.occ.p, d->occ, sizeof(double) * natoms, hipMemcpyHostToDevice, c->st));
+            if (any_b) HIPCHK(hipMemcpyAsync(b.bdw.p, d->bdw, sizeof(double) * natoms, hipMemcpyHostToDevice, c->st));
+            HIPCHK(hipMemcpyAsync(b.target.p, target, sizeof(double) * P * M, hipMemcpyHostToDevice, c->st));
+            if (weight) HIPCHK(hipMemcpyAsync(b.weight.p, weight, sizeof(double) * P * M, hipMemcpyHostToDevice, c->st));
+        }
+        if ((st = send_sq(b))) return st;
+    }
+    for (size_t q = 0; q < (size_t)d->nscat * M; ++q)
+        std::memcpy(b.h_cf.p + sizeof(double) * 2 * b.rows * q, d->cfact + 2 * (size_t)d->ncfact * q, sizeof(double) * 2 * b.rows);
+    HIPCHK(hipMemcpyAsync(b.cfact.p, b.h_cf.p, sizeof(double) * 2 * b.rows * d->nscat * M, hipMemcpyHostToDevice, c->st));
+    unsigned char *h_rten = b.h_cf.p + sizeof(double) * 2 * b.rows * d->nscat * M;
+    std::memcpy(h_rten, d->rten, sizeof(double) * 9 * M);
+    HIPCHK(hipMemcpyAsync(b.rten.p, h_rten, sizeof(double) * 9 * M, hipMemcpyHostToDevice, c->st));
 
     if (!b.primed) {
         // records of this call, then the tile / grid-size choice, then the graph
-        if ((st = enqueue(c, b, b.pl.tile, 0, true, 0, false))) return st;
-        if ((st = autotune(c, b))) return st;
+        if ((st = enqueue(c, b, io, b.pl.tile, 0, true, STEP_GEMM, false))) return st;
+        if ((st = autotune(c, b, io))) return st;
         b.primed = true;
-        if (c->graphs) {
-            HIPCHK(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
-            st = enqueue(c, b, b.pl.tile, b.nwg, true, 2, b.queue);
-            hipGraph_t graph = nullptr;
-            hipError_t e = hipStreamEndCapture(c->st, &graph);
-            if (st) {
-                if (graph) (void)hipGraphDestroy(graph);
-                return st;
-            }
-            HIPCHK(e);
-            b.graph = graph;
-            HIPCHK(hipGraphInstantiate(&b.exec, b.graph, nullptr, nullptr, 0));
-        }
     }
-    HIPCHK(hipEventRecord(c->ev[4], c->st));
-    if (b.exec) {
+    if (!dev && c->graphs && !b.exec) {
+        HIPCHK(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
+        st = enqueue(c, b, io, b.pl.tile, b.nwg, true, STEP_GEMM | STEP_REST, b.queue);
+        hipGraph_t graph = nullptr;
+        hipError_t e = hipStreamEndCapture(c->st, &graph);
+        if (st) {
+            if (graph) (void)hipGraphDestroy(graph);
+            return st;
+        }
+        HIPCHK(e);
+        b.graph = graph;
+        HIPCHK(hipGraphInstantiate(&b.exec, b.graph, nullptr, nullptr, 0));
+    }
+    if (!started) HIPCHK(hipEventRecord(c->ev[4], c->st));
+    if (!dev && b.exec) {
         HIPCHK(hipGraphLaunch(b.exec, c->st));
     } else {
-        if ((st = enqueue(c, b, b.pl.tile, b.nwg, true, 2, b.queue))) return st;
+        if ((st = enqueue(c, b, io, b.pl.tile, b.nwg, !started, started ? STEP_REST : STEP_GEMM | STEP_REST, b.queue))) return st;
     }
     HIPCHK(hipEventRecord(c->ev[5], c->st));
-    std::vector<double> part((size_t)b.nblk * M);
-    HIPCHK(hipMemcpyAsync(part.data(), b.chi.p, sizeof(double) * part.size(), hipMemcpyDeviceToHost, c->st));
-    if (icalc) HIPCHK(hipMemcpyAsync(icalc, b.icalc.p, sizeof(double) * P * M, out, c->st));
-    if (grad) HIPCHK(hipMemcpyAsync(grad, b.grad.p, sizeof(double) * 5 * natoms, out, c->st));
+    if (!dev && icalc) HIPCHK(hipMemcpyAsync(icalc, b.icalc.p, sizeof(double) * P * M, hipMemcpyDeviceToHost, c->st));
+    if (!dev && grad) HIPCHK(hipMemcpyAsync(grad, b.grad.p, sizeof(double) * 5 * natoms, hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipEventRecord(c->ev[1], c->st));
     HIPCHK(hipStreamSynchronize(c->st));
-    for (size_t m = 0; m < M; ++m) {
-        double s = 0.0;
-        for (int k = 0; k < b.nblk; ++k) s += part[m * b.nblk + k];
-        chi2[m] = s;
-    }
+    std::memcpy(chi2, b.h_chi.p, sizeof(double) * M);
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, c->ev[4], c->ev[5]));
     c->stats.forward_ms = ms;          // the whole population step (forward + adjoint when requested)

@@ -1,6 +1,8 @@
 // dc_host.h -- host-side state and helpers shared by the C-ABI translation
 // units (dc_api.hip: the Fourier run, dc_refine.hip: the refinement model).
 #pragma once
+#include <algorithm>
+#include <cstring>
 #include <string>
 #include <utility>
 #include <vector>
@@ -14,6 +16,11 @@ struct NufftState;   // dc_nufft.hip
 
 struct DevBuf {
     void *p = nullptr;
+    size_t n = 0;
+};
+// pinned host memory, readable and writable by kernels at the same address
+struct PinBuf {
+    unsigned char *p = nullptr;
     size_t n = 0;
 };
 
@@ -49,7 +56,7 @@ struct dc_ctx {
     DevBuf rec, slice_beg, slice_order, slice_type, lot_slice, partial, cfact, istl, idx, oid, offs, xat, w;
     DevBuf acsf, dsi, csf, wm, wv, lat, out_tcsf, out[5];
     // device buffers of the refinement model
-    DevBuf m_pos, m_w, m_b, m_sq, m_q, m_part, m_grad, m_tiles, m_gi, m_f, m_tgt, m_qt, m_qs, m_bd, m_jw, m_jidx, m_dsl, m_di;
+    DevBuf m_pos, m_w, m_b, m_sq, m_q, m_part, m_grad, m_tiles, m_gi, m_f, m_qt, m_qs, m_jw, m_dsl, m_di;
     // crystal
     bool have_crystal = false;
     DevBuf pos, iscat;
@@ -68,6 +75,15 @@ struct dc_ctx {
     // cells of a lot is one contiguous range
     std::vector<int> tc_start;
     DevBuf runs;
+    // Staging of a call's small host arrays (see stage): packed into h_arena and
+    // copied to arena by one kernel; outputs of host entry points that fit
+    // come back through h_out.  Both belong to the context, whose calls wait
+    // for their stream, and are reused by the next call.
+    PinBuf h_arena, h_out;
+    DevBuf arena;
+    size_t arena_n = 0, arena_done = 0;   // bytes packed / already copied in this call
+    size_t arena_want = 0;                // bytes this call asked for
+    bool arena_busy = false;              // a copy was launched and not waited for
     // this device's dc_scratch array (dc_noalloc.hip), looked up at creation
     void *scratch = nullptr;
     // rec's records carry the rotation hash in AtomRec::pad (PrepArgs::hash_salt):
@@ -78,8 +94,8 @@ struct dc_ctx {
     std::vector<DevBuf *> buffers() {
         return {&rec, &slice_beg, &slice_order, &slice_type, &lot_slice, &partial, &cfact, &istl, &idx, &oid, &offs, &xat, &w,
                 &acsf, &dsi, &csf, &wm, &wv, &lat, &out_tcsf, &out[0], &out[1], &out[2], &out[3], &out[4],
-                &m_pos, &m_w, &m_b, &m_sq, &m_q, &m_part, &m_grad, &m_tiles, &m_gi, &m_f, &m_tgt, &m_qt, &m_qs, &m_bd, &m_jw, &m_jidx, &m_dsl, &m_di,
-                &pos, &iscat, &type_idx, &runs};
+                &m_pos, &m_w, &m_b, &m_sq, &m_q, &m_part, &m_grad, &m_tiles, &m_gi, &m_f, &m_qt, &m_qs, &m_jw, &m_dsl, &m_di,
+                &pos, &iscat, &type_idx, &runs, &arena};
     }
 };
 
@@ -137,6 +153,80 @@ int upload(dc_ctx *c, DevBuf &b, const T *src, size_t count) {
     if (count) HIPCHK(hipMemcpyAsync(b.p, src, sizeof(T) * count, hipMemcpyHostToDevice, c->st));
     return 0;
 }
+
+// Staging.  A call's tables (slice boundaries and types, form-factor rows, lot
+// runs) are a few kilobytes each; copied one by one from pageable memory they
+// cost about 15 us of host time apiece, which is most of a small call.  They
+// are packed into pinned memory instead and one kernel copies them.
+// stage_begin starts a call, stage returns the device address of a packed copy
+// (falling back to upload into b when the arena is full: it grows with the
+// next call, up to ARENA_MAX), stage_flush launches
+// the copy of what has been packed; every launch that reads staged data comes
+// after a flush.
+constexpr size_t ARENA_MIN = 256u << 10, ARENA_MAX = 8u << 20;
+hipError_t launch_stage_copy(const void *src, void *dst, size_t bytes, hipStream_t st);   // dc_lot.hip
+
+inline int pin_ensure(dc_ctx *c, PinBuf &b, size_t bytes) {
+    if (b.n >= bytes) return 0;
+    if (b.p) (void)hipHostFree(b.p);
+    b.p = nullptr;
+    b.n = 0;
+    void *p = nullptr;
+    hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocDefault);
+    if (e != hipSuccess) return hip_err(c, e, "hipHostMalloc");
+    b.p = static_cast<unsigned char *>(p);
+    b.n = bytes;
+    return 0;
+}
+inline int stage_begin(dc_ctx *c) {
+    int st;
+    if (c->arena_busy) HIPCHK(hipStreamSynchronize(c->st));   // an earlier call ended early
+    c->arena_busy = false;
+    size_t n = ARENA_MIN;
+    while (n < c->arena_want && n < ARENA_MAX) n *= 2;
+    n = std::max(n, c->h_arena.n);
+    c->arena_n = c->arena_done = c->arena_want = 0;
+    if ((st = pin_ensure(c, c->h_arena, n))) return st;
+    return ensure(c, c->arena, n);
+}
+template <class T>
+int stage(dc_ctx *c, DevBuf &b, const T *src, size_t count, T *&dev) {
+    const size_t bytes = sizeof(T) * count;
+    const size_t room = (bytes + 255) & ~(size_t)255;
+    c->arena_want += room;
+    if (room > c->h_arena.n - c->arena_n) {
+        int st = upload(c, b, src, count);
+        dev = ptr<T>(b);
+        return st;
+    }
+    if (bytes) std::memcpy(c->h_arena.p + c->arena_n, src, bytes);
+    dev = reinterpret_cast<T *>(static_cast<unsigned char *>(c->arena.p) + c->arena_n);
+    c->arena_n += room;
+    return 0;
+}
+inline int stage_flush(dc_ctx *c) {
+    if (c->arena_n == c->arena_done) return 0;
+    HIPCHK(launch_stage_copy(c->h_arena.p + c->arena_done, static_cast<unsigned char *>(c->arena.p) + c->arena_done,
+                             c->arena_n - c->arena_done, c->st));
+    c->arena_done = c->arena_n;
+    c->arena_busy = true;
+    return 0;
+}
+// Form-factor rows 0 .. rows-1 of the nscat columns of a (ncfact, nscat) table.
+inline int stage_cfact(dc_ctx *c, const double *cfact, int ncfact, int nscat, int rows, double2 *&dev) {
+    if (rows == ncfact) return stage(c, c->cfact, reinterpret_cast<const double2 *>(cfact), (size_t)ncfact * nscat, dev);
+    std::vector<double2> v((size_t)rows * nscat);
+    for (int t = 0; t < nscat; ++t)
+        std::memcpy(v.data() + (size_t)rows * t, cfact + 2 * (size_t)ncfact * t, sizeof(double2) * rows);
+    return stage(c, c->cfact, v.data(), v.size(), dev);
+}
+// Rows of the form-factor table a grid reaches: its largest bin lies at a
+// corner; two rows more cover bins that round up beside it.
+inline int cfact_rows(int corner_bin, int ncfact) { return std::min(ncfact, corner_bin + 3); }
+
+// Outputs of a host entry point up to this size are written by the last
+// kernel into pinned memory and copied to the caller's arrays from there.
+constexpr size_t HOST_OUT_BYTES = 8u << 20;
 
 // Deferred timing: mark() records a pool event on the context stream;
 // span() files (start, end) to be added to a stats field once the host has
@@ -201,6 +291,8 @@ int fold_side(const GemmGeom &gg, int fold_mask, int tile);
 // FOLD_ROWS); a damped launch needs s^2 mirrored about the side's centre.
 Plan plan_gemm(Grid &g, int forced, int only_mapping = -1, int prec = 1, long long natoms = 0,
                int fold_mask = FOLD_COLS | FOLD_ROWS);
+// Geometry of mapping 0, which no tile changes.
+GemmGeom mapping0_geom(const Grid &g);
 // Slice length of a fold tile for a launch's segments, and its predicted time.
 int fold_slices(const GemmGeom &gg, int tile, const std::vector<std::pair<int, int>> &segs, int prec, double &best_us);
 // the sides whose s^2 parts (R row values, then C column values) are mirrored
@@ -208,8 +300,9 @@ int mirrored_sides(const GemmGeom &gg, const float *sq);
 int kchunk_for(const Plan &pl, long long natoms_batch, int prec);
 int kchunk_for(const Plan &pl, const std::vector<std::pair<int, int>> &segs, int prec);
 void add_segments(SliceSet &s, const std::vector<std::pair<int, int>> &segs, int kchunk, int &atom_off);
-// beg: the slices' atom offsets, as uploaded to c->slice_beg (nslice + 1)
-int run_gemm(dc_ctx *c, const Plan &pl, const std::vector<int> &beg, float2 *partial, const float *sq = nullptr);
+// beg: the slices' atom offsets (nslice + 1), d_beg: the same on the device
+int run_gemm(dc_ctx *c, const Plan &pl, const std::vector<int> &beg, const int *d_beg, float2 *partial,
+             const float *sq = nullptr);
 // atoms per slice: the context's forced length (dc_set_slice_atoms) or the planned one
 inline int slice_len(const dc_ctx *c, int planned) { return c->slice_atoms > 0 ? c->slice_atoms : planned; }
 // the plan's geometry with the context's dither salt

@@ -21,6 +21,11 @@ struct PrepArgs {
     const float *bdw;       // per-atom isotropic B in AtomRec::pad (null: 0)
     const double *occ_src;  // caller-order occupancy read through idx (overrides w)
     const double *bdw_src;  // caller-order B read through idx (overrides bdw)
+    // derivative directions: record k is atom idx[k % dn] of direction and
+    // component k / dn = 5 direction + q with the weight docc (q = 0), occ dx,
+    // occ dy, occ dz (1..3) or occ dB (4) of dpar(5, dnat, ndir)
+    const double *dpar;
+    long long dn, dnat;
     uint32_t hash_salt;     // nonzero: AtomRec::pad = dither_hash32(record, salt) instead of B
                             // (records of undamped GEMMs only; the adjoints read pad as B)
     long long n;

@@ -34,6 +34,8 @@ __global__ void prep_records_kernel(PrepArgs a, AtomRec *__restrict__ out) {
             const int4 r = a.runs[lo];
             src = a.idx[r.y + (k - r.x)];
             o = r.z;
+        } else if (a.dpar) {
+            src = a.idx[k % a.dn];
         } else {
             src = a.idx ? (long long)a.idx[k] : k;
             if (a.oid) o = a.oid[k];
@@ -69,6 +71,12 @@ __global__ void prep_records_kernel(PrepArgs a, AtomRec *__restrict__ out) {
     }
     r.w = a.occ_src ? (float)a.occ_src[src] : (a.w ? a.w[k] : 1.0f);
     r.pad = a.bdw_src ? (float)a.bdw_src[src] : (a.bdw ? a.bdw[k] : 0.0f);
+    if (a.dpar) {
+        const long long g5 = k / a.dn;
+        const int q = (int)(g5 % 5);
+        const double *dp = a.dpar + 5 * (a.dnat * (g5 / 5) + src);
+        r.w = (float)(q == 0 ? dp[3] : a.occ_src[src] * dp[q == 4 ? 4 : q - 1]);
+    }
     if (a.hash_salt) r.pad = __builtin_bit_cast(float, dither_hash32((uint32_t)k, a.hash_salt));
     out[k] = r;
 }
@@ -357,8 +365,21 @@ __global__ void istl_kernel(Grid g, int *__restrict__ out) {
     out[q] = istl_raw(g, i, (int)(qq % g.n[1]), (int)(qq / g.n[1]));
 }
 
+// Staged arrays from pinned host memory into the device arena (16-byte words;
+// both ends are 256-byte aligned and padded).
+__global__ void stage_copy_kernel(const uint4 *__restrict__ src, uint4 *__restrict__ dst, long long n) {
+    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) dst[k] = src[k];
+}
+
 static inline unsigned nblk(long long n, int b) { return (unsigned)((n + b - 1) / b); }
 
+hipError_t launch_stage_copy(const void *src, void *dst, size_t bytes, hipStream_t st) {
+    const long long n = (long long)((bytes + 15) / 16);
+    if (n <= 0) return hipSuccess;
+    stage_copy_kernel<<<nblk(n, 256), 256, 0, st>>>(static_cast<const uint4 *>(src), static_cast<uint4 *>(dst), n);
+    return hipGetLastError();
+}
 hipError_t launch_prep(const PrepArgs &a, AtomRec *out, hipStream_t st) {
     if (a.n <= 0) return hipSuccess;
     prep_records_kernel<<<nblk(a.n, 256), 256, 0, st>>>(a, out);

@@ -53,7 +53,7 @@ int strucf_setup(dc_ctx *c, const void *xat, int64_t nxat, int64_t ld_xat, const
 int strucf_core(dc_ctx *c, const Grid &g0, long long ntot, const double *d_xat, int64_t nxat, int64_t ld_xat,
                 const double off_shift[9], const int lmn[6], const double2 *d_cfact, int64_t ncfact,
                 const int *d_istl, int lform, AtomRec *rec, int *slice_beg, float2 *partial, double plane_bytes,
-                double *d_tcsf);
+                double *d_tcsf, int fold_mask);
 
 }  // namespace dc
 
@@ -73,17 +73,26 @@ int dc_strucf_dev_noalloc(dc_ctx *c, const double *d_xat, int64_t nxat, int64_t 
     HIPCHK(hipSetDevice(c->device));
     // scratch layout: records | slice boundaries | slice planes
     Grid gp = g;
-    const Plan pl = plan_gemm(gp, c->tile, -1, c->prec, nxat);
-    const int klen = slice_len(c, kchunk_for(pl, nxat, pl.scheme));
-    const long long nslice = std::max<long long>(1, (nxat + klen - 1) / klen);
     const size_t rec_bytes = align256(sizeof(AtomRec) * (size_t)std::max<int64_t>(nxat, 1));
-    const size_t beg_bytes = align256(sizeof(int) * (size_t)(nslice + 1));
-    const size_t plane = sizeof(float2) * (size_t)pl.gg.P;
-    if (rec_bytes + beg_bytes + plane > kScratchBytes) {
+    size_t beg_bytes = 0, plane = 0;
+    auto layout = [&](int fold_mask) {
+        const Plan pl = plan_gemm(gp, c->tile, -1, c->prec, nxat, fold_mask);
+        const int klen = slice_len(c, kchunk_for(pl, nxat, pl.scheme));
+        const long long nslice = std::max<long long>(1, (nxat + klen - 1) / klen);
+        beg_bytes = align256(sizeof(int) * (size_t)(nslice + 1));
+        plane = sizeof(float2) * (size_t)pl.gg.P;
+        return rec_bytes + beg_bytes + plane;
+    };
+    // the general tiles' layout decides what fits; a problem whose folded plan
+    // (another mapping's padding, more slices) does not fit runs on them
+    const size_t need = layout(0);
+    const int fold_mask = need <= kScratchBytes && layout(FOLD_COLS | FOLD_ROWS) <= kScratchBytes ? FOLD_COLS | FOLD_ROWS : 0;
+    (void)layout(fold_mask);
+    if (need > kScratchBytes) {
         char msg[200];
         std::snprintf(msg, sizeof(msg),
                       "dc_strucf_dev_noalloc: needs %zu bytes of scratch (records and one slice plane), holds %zu",
-                      rec_bytes + beg_bytes + plane, kScratchBytes);
+                      need, kScratchBytes);
         return set_err(c, DC_ERR_ARG, DC_ER_LIB, msg);
     }
     unsigned char *base = static_cast<unsigned char *>(c->scratch);
@@ -93,7 +102,7 @@ int dc_strucf_dev_noalloc(dc_ctx *c, const double *d_xat, int64_t nxat, int64_t 
                      lform ? reinterpret_cast<const double2 *>(d_cfact_col) : nullptr, ncfact, lform ? d_istl : nullptr,
                      lform, reinterpret_cast<AtomRec *>(base), reinterpret_cast<int *>(base + rec_bytes),
                      reinterpret_cast<float2 *>(base + rec_bytes + beg_bytes),
-                     (double)(kScratchBytes - rec_bytes - beg_bytes), d_tcsf);
+                     (double)(kScratchBytes - rec_bytes - beg_bytes), d_tcsf, fold_mask);
     if (st) return st;
     HIPCHK(hipEventRecord(c->ev[1], c->st));
     HIPCHK(hipStreamSynchronize(c->st));

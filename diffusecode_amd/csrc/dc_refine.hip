@@ -28,6 +28,12 @@ struct ModelPlan {
     bool separable = true;
     bool any_b = false;
     int nsorted = 0;
+    int rows = 0;                             // form-factor rows the grid reaches
+    // staged device copies
+    const int *idx = nullptr;
+    const float *d_sq = nullptr;
+    const double2 *cfact = nullptr;
+    const double *pos = nullptr, *occ = nullptr, *bdw = nullptr;   // caller order (staged, or the caller's device arrays)
 };
 
 double dotg(const double *a, const double *g, const double *b) {
@@ -49,7 +55,8 @@ int check_model(dc_ctx *c, const dc_model_desc *m) {
 }
 
 // Grid, GEMM plan (rows = abscissa), type-sorted atom order and the s^2 parts.
-int plan_model(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
+// dev: pos, occ and bdw are device arrays, a non-null bdw counts as per-atom B.
+int plan_model(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, bool dev) {
     Grid &g = mp.g;
     for (int k = 0; k < 3; ++k) {
         g.n[k] = g.f[k] = m->inc[k];
@@ -60,7 +67,7 @@ int plan_model(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
     }
     for (int k = 0; k < 9; ++k) g.rten[k] = m->rten[k];
     g.P = (long long)g.f[0] * g.f[1] * g.f[2];
-    const GemmGeom gg = plan_gemm(g, c->tile, 0, model_scheme(c->prec), m->natoms).gg;
+    const GemmGeom gg = mapping0_geom(g);
 
     // metric orthogonality of the abscissa against the other axes
     const double *v1 = m->vi, *v2 = m->vi + 3, *v3 = m->vi + 6;
@@ -96,8 +103,9 @@ int plan_model(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
     for (int64_t n = 0; n < m->natoms; ++n) {
         const int t = m->type[n];
         if (t > 0) mp.order[fill[t]++] = (int)n;
-        if (t > 0 && m->bdw && m->bdw[n] != 0.0) mp.any_b = true;
+        if (!dev && t > 0 && m->bdw && m->bdw[n] != 0.0) mp.any_b = true;
     }
+    if (dev) mp.any_b = m->bdw != nullptr;
     for (int t = 1; t <= m->nscat; ++t)
         if (cnt[t] > 0) mp.segs.push_back({t - 1, cnt[t]});
     // the planes of mapping 0 are the same for every tile; with per-atom B a
@@ -106,34 +114,49 @@ int plan_model(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
                       mp.any_b ? mirrored_sides(gg, mp.sq.data()) : FOLD_COLS | FOLD_ROWS);
     if (mp.any_b && !mp.separable)
         return set_err(c, DC_ERR_ARG, DC_ER_LIB, "model: per-atom B needs vi(:,1) metric-orthogonal to vi(:,2), vi(:,3)");
-    if (max_corner_bin(g) >= m->ncfact)
+    const int top_bin = max_corner_bin(g);
+    if (top_bin >= m->ncfact)
         return set_err(c, DC_ERR_ISTL, DC_ER_FOUR, "sin(theta)/lambda beyond table");
+    mp.rows = cfact_rows(top_bin, m->ncfact);
     return 0;
 }
 
-// Sorted per-atom inputs on the device and the GEMM records (corner phases).
-int upload_model(dc_ctx *c, const dc_model_desc *m, const ModelPlan &mp) {
+// Per-atom inputs and tables on the device and the GEMM records (corner phases).
+int upload_model(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, bool dev) {
     int st;
     const int ns = mp.nsorted;
-    std::vector<float> w(ns), b(ns);
-    for (int k = 0; k < ns; ++k) {
-        const int n = mp.order[k];
-        w[k] = (float)m->occ[n];
-        b[k] = m->bdw ? (float)m->bdw[n] : 0.0f;
+    const size_t n = (size_t)m->natoms;
+    const double *pos = m->pos, *occ = m->occ, *bdw = m->bdw;
+    if (!dev) {
+        double *d_pos, *d_occ, *d_bdw = nullptr;
+        if ((st = stage(c, c->m_pos, m->pos, 3 * n, d_pos))) return st;
+        if ((st = stage(c, c->m_w, m->occ, n, d_occ))) return st;
+        if (m->bdw && (st = stage(c, c->m_b, m->bdw, n, d_bdw))) return st;
+        pos = d_pos;
+        occ = d_occ;
+        bdw = d_bdw;
     }
-    if ((st = upload(c, c->m_pos, m->pos, 3 * (size_t)m->natoms))) return st;
-    if ((st = upload(c, c->idx, mp.order.data(), mp.order.size()))) return st;
-    if ((st = upload(c, c->m_w, w.data(), w.size()))) return st;
-    if ((st = upload(c, c->m_b, b.data(), b.size()))) return st;
-    if ((st = upload(c, c->m_sq, mp.sq.data(), mp.sq.size()))) return st;
+    int *d_idx;
+    float *d_sq;
+    double2 *d_cf;
+    if ((st = stage(c, c->idx, mp.order.data(), mp.order.size(), d_idx))) return st;
+    if ((st = stage(c, c->m_sq, mp.sq.data(), mp.sq.size(), d_sq))) return st;
+    if ((st = stage_cfact(c, m->cfact, m->ncfact, m->nscat, mp.rows, d_cf))) return st;
+    mp.idx = d_idx;
+    mp.d_sq = d_sq;
+    mp.cfact = d_cf;
+    mp.pos = pos;
+    mp.occ = occ;
+    mp.bdw = bdw;
     if ((st = ensure(c, c->rec, sizeof(AtomRec) * std::max(ns, 1)))) return st;
     PrepArgs pa = base_prep(mp.g, 0);
-    pa.src = ptr<double>(c->m_pos);
+    pa.src = pos;
     pa.src_ld = 0;
-    pa.idx = ptr<int>(c->idx);
-    pa.w = ptr<float>(c->m_w);
-    pa.bdw = ptr<float>(c->m_b);
+    pa.idx = mp.idx;
+    pa.occ_src = occ;
+    pa.bdw_src = bdw;
     pa.n = ns;
+    if ((st = stage_flush(c))) return st;
     HIPCHK(launch_prep(pa, ptr<AtomRec>(c->rec), c->st));
     c->rec_hash = false;
     return 0;
@@ -149,25 +172,27 @@ int model_forward(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
     if (ss.beg.empty()) ss.beg.push_back(0);
     const int nslice = (int)ss.type.size();
     ss.lot = {0, nslice};
-    if ((st = upload(c, c->slice_beg, ss.beg.data(), ss.beg.size()))) return st;
-    if ((st = upload(c, c->lot_slice, ss.lot.data(), ss.lot.size()))) return st;
-    if (nslice > 0 && (st = upload(c, c->slice_type, ss.type.data(), ss.type.size()))) return st;
-    if ((st = upload(c, c->cfact, m->cfact, 2 * (size_t)m->ncfact * m->nscat))) return st;
+    int *d_beg, *d_lot, *d_type;
+    if ((st = stage(c, c->slice_beg, ss.beg.data(), ss.beg.size(), d_beg))) return st;
+    if ((st = stage(c, c->lot_slice, ss.lot.data(), ss.lot.size(), d_lot))) return st;
+    if ((st = stage(c, c->slice_type, ss.type.data(), ss.type.size(), d_type))) return st;
+    if ((st = stage_flush(c))) return st;
     if ((st = ensure(c, c->partial, sizeof(float2) * gg.P * std::max(nslice, 1)))) return st;
     if ((st = ensure(c, c->m_f, sizeof(double) * 2 * mp.g.P))) return st;
     if ((st = ensure(c, c->dsi, sizeof(double) * mp.g.P))) return st;
-    HIPCHK(hipEventRecord(c->ev[4], c->st));
-    if ((st = run_gemm(c, mp.pl, ss.beg, ptr<float2>(c->partial), mp.any_b ? ptr<float>(c->m_sq) : nullptr))) return st;
+    hipEvent_t e0, e1;
+    if ((st = mark(c, e0))) return st;
+    if ((st = run_gemm(c, mp.pl, ss.beg, d_beg, ptr<float2>(c->partial), mp.any_b ? mp.d_sq : nullptr))) return st;
     ReduceArgs ra{};
     ra.g = mp.g;
     ra.partial = ptr<float2>(c->partial);
     ra.slice0 = 0;
-    ra.lot_slice = ptr<int>(c->lot_slice);
-    ra.slice_type = ptr<int>(c->slice_type);
+    ra.lot_slice = d_lot;
+    ra.slice_type = d_type;
     ra.nlots = nslice > 0 ? 1 : 0;
     ra.lform = 1;
-    ra.cfact = ptr<double2>(c->cfact);
-    ra.ncfact = m->ncfact;
+    ra.cfact = mp.cfact;
+    ra.ncfact = mp.rows;
     ra.ntype = m->nscat;
     ra.dsi = ptr<double>(c->dsi);
     ra.csf = ptr<double>(c->m_f);
@@ -178,18 +203,15 @@ int model_forward(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
         HIPCHK(hipMemsetAsync(c->m_f.p, 0, sizeof(double) * 2 * mp.g.P, c->st));
         HIPCHK(hipMemsetAsync(c->dsi.p, 0, sizeof(double) * mp.g.P, c->st));
     }
-    HIPCHK(hipEventRecord(c->ev[5], c->st));
-    HIPCHK(hipEventSynchronize(c->ev[5]));
-    float ms = 0.f;
-    HIPCHK(hipEventElapsedTime(&ms, c->ev[4], c->ev[5]));
-    c->stats.forward_ms += ms;
+    if ((st = mark(c, e1))) return st;
+    span(c, e0, e1, &c->stats.forward_ms);
     c->stats.pairs += (double)mp.nsorted * (double)mp.g.P;
     c->stats.slices += nslice;
     return 0;
 }
 
-// Gradient (5, natoms) on the device (m_grad) from F (m_f) and G (m_gi).
-int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
+// Gradient (5, natoms) on the device (grad) from F (m_f) and G (m_gi).
+int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, double *grad) {
     int st;
     if (!mp.separable)
         return set_err(c, DC_ERR_ARG, DC_ER_LIB, "model gradient: needs vi(:,1) metric-orthogonal to vi(:,2), vi(:,3)");
@@ -211,14 +233,15 @@ int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
     const int ntiles = (int)tiles.size() / 4;
     const int ntc = (gg.C + adjoint_tile_cols() - 1) / adjoint_tile_cols();
 
-    HIPCHK(hipEventRecord(c->ev[4], c->st));
-    if ((st = upload(c, c->m_qt, qtype.data(), qtype.size()))) return st;
-    if (ntiles > 0 && (st = upload(c, c->m_tiles, tiles.data(), tiles.size()))) return st;
-    if ((st = upload(c, c->m_tgt, m->occ, (size_t)m->natoms))) return st;
+    hipEvent_t e0, e1;
+    if ((st = mark(c, e0))) return st;
+    int *d_qt, *d_tiles;
+    if ((st = stage(c, c->m_qt, qtype.data(), qtype.size(), d_qt))) return st;
+    if ((st = stage(c, c->m_tiles, tiles.data(), tiles.size(), d_tiles))) return st;
+    if ((st = stage_flush(c))) return st;
     if ((st = ensure(c, c->m_q, sizeof(float2) * gg.P * std::max(nq, 1)))) return st;
     if ((st = ensure(c, c->m_part, sizeof(float) * 6 * (size_t)ntc * std::max(mp.nsorted, 1)))) return st;
-    if ((st = ensure(c, c->m_grad, sizeof(double) * 5 * std::max<int64_t>(m->natoms, 1)))) return st;
-    HIPCHK(hipMemsetAsync(c->m_grad.p, 0, sizeof(double) * 5 * std::max<int64_t>(m->natoms, 1), c->st));
+    HIPCHK(launch_fill_zero(grad, 5 * m->natoms, c->st));
     if (ntiles > 0) {
         HIPCHK(hipMemsetAsync(c->m_q.p, 0, sizeof(float2) * gg.P * nq, c->st));
         QArgs qa{};
@@ -229,18 +252,18 @@ int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
         qa.plane = gg.P;
         qa.f = ptr<double>(c->m_f);
         qa.gi = ptr<double>(c->m_gi);
-        qa.cfact = ptr<double2>(c->cfact);
-        qa.ncfact = m->ncfact;
-        qa.qtype = ptr<int>(c->m_qt);
+        qa.cfact = mp.cfact;
+        qa.ncfact = mp.rows;
+        qa.qtype = d_qt;
         qa.nq = nq;
         qa.q = ptr<float2>(c->m_q);
         HIPCHK(launch_model_q(qa, c->st));
 
         AdjArgs aa{};
         aa.rec = ptr<AtomRec>(c->rec);
-        aa.tiles = ptr<int4>(c->m_tiles);
+        aa.tiles = reinterpret_cast<const int4 *>(d_tiles);
         aa.q = ptr<float2>(c->m_q);
-        aa.sq = ptr<float>(c->m_sq);
+        aa.sq = mp.d_sq;
         aa.part = ptr<float>(c->m_part);
         aa.R = gg.R;
         aa.C = gg.C;
@@ -266,23 +289,20 @@ int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
         fa.part = ptr<float>(c->m_part);
         fa.ntile_c = nset;
         fa.natoms = mp.nsorted;
-        fa.idx = ptr<int>(c->idx);
-        fa.occ = ptr<double>(c->m_tgt);
+        fa.idx = mp.idx;
+        fa.occ = mp.occ;
         for (int k = 0; k < 3; ++k)
             fa.hc[k] = m->eck[k] + (double)aa.rc * m->vi[k] + (double)aa.jc * m->vi[3 + k] + (double)aa.mc * m->vi[6 + k];
         for (int k = 0; k < 9; ++k) fa.v[k] = m->vi[k];
-        fa.grad = ptr<double>(c->m_grad);
+        fa.grad = grad;
         HIPCHK(launch_adjoint_finish(fa, c->st));
     }
-    HIPCHK(hipEventRecord(c->ev[5], c->st));
-    HIPCHK(hipEventSynchronize(c->ev[5]));
-    float ms = 0.f;
-    HIPCHK(hipEventElapsedTime(&ms, c->ev[4], c->ev[5]));
-    c->stats.adjoint_ms += ms;
+    if ((st = mark(c, e1))) return st;
+    span(c, e0, e1, &c->stats.adjoint_ms);
     return 0;
 }
 
-int model_begin(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
+int model_begin(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, bool dev = false) {
     c->err.clear();
     c->err_typ = DC_ER_NONE;
     int st;
@@ -291,17 +311,19 @@ int model_begin(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp) {
     HIPCHK(hipSetDevice(c->device));
     stats_begin(c);
     HIPCHK(hipEventRecord(c->ev[0], c->st));
-    if ((st = plan_model(c, m, mp))) return st;
-    return upload_model(c, m, mp);
+    if ((st = stage_begin(c))) return st;
+    if ((st = plan_model(c, m, mp, dev))) return st;
+    return upload_model(c, m, mp, dev);
 }
 
 int model_end(dc_ctx *c) {
     HIPCHK(hipEventRecord(c->ev[1], c->st));
     HIPCHK(hipStreamSynchronize(c->st));
+    c->arena_busy = false;
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
     c->stats.total_ms = ms;
-    return DC_OK;
+    return resolve_spans(c);
 }
 
 }  // namespace
@@ -327,8 +349,8 @@ int dc_model_vjp(dc_ctx *c, const dc_model_desc *m, const double *fcalc, const d
     if ((st = model_begin(c, m, mp))) return st;
     if ((st = upload(c, c->m_f, fcalc, 2 * (size_t)mp.g.P))) return st;
     if ((st = upload(c, c->m_gi, gi, (size_t)mp.g.P))) return st;
-    if ((st = upload(c, c->cfact, m->cfact, 2 * (size_t)m->ncfact * m->nscat))) return st;
-    if ((st = model_adjoint(c, m, mp))) return st;
+    if ((st = ensure(c, c->m_grad, sizeof(double) * 5 * std::max<int64_t>(m->natoms, 1)))) return st;
+    if ((st = model_adjoint(c, m, mp, ptr<double>(c->m_grad)))) return st;
     HIPCHK(hipMemcpyAsync(grad, c->m_grad.p, sizeof(double) * 5 * m->natoms, hipMemcpyDeviceToHost, c->st));
     return model_end(c);
 }
@@ -344,9 +366,13 @@ int dc_model_jvp(dc_ctx *c, const dc_model_desc *m, const double *fcalc, int ndi
     const long long P = mp.g.P;
     const int ns = mp.nsorted;
     if ((st = upload(c, c->m_f, fcalc, 2 * (size_t)P))) return st;
-    if ((st = upload(c, c->cfact, m->cfact, 2 * (size_t)m->ncfact * m->nscat))) return st;
-    if (m->bdw && (st = upload(c, c->m_bd, m->bdw, (size_t)m->natoms))) return st;
-    if ((st = ensure(c, c->m_di, sizeof(double) * (size_t)P * std::max(ndir, 1) * (df ? 3 : 1)))) return st;
+    double *d_par;
+    if ((st = stage(c, c->m_jw, dparam, 5 * (size_t)m->natoms * ndir, d_par))) return st;
+    // [ndir][P] dI, then dF: pinned memory that the kernel writes, or device
+    const size_t obytes = sizeof(double) * (size_t)P * std::max(ndir, 1) * (df ? 3 : 1);
+    const bool pinned = obytes <= HOST_OUT_BYTES;
+    if ((st = pinned ? pin_ensure(c, c->h_out, obytes) : ensure(c, c->m_di, obytes))) return st;
+    double *out = pinned ? reinterpret_cast<double *>(c->h_out.p) : ptr<double>(c->m_di);
     // directions per batch so that the slice planes fit the budget
     std::vector<std::pair<int, int>> all;
     for (int k = 0; k < 5 * std::min(ndir, 64); ++k) all.insert(all.end(), mp.segs.begin(), mp.segs.end());
@@ -359,19 +385,6 @@ int dc_model_jvp(dc_ctx *c, const dc_model_desc *m, const double *fcalc, int ndi
     for (int d0 = 0; d0 < ndir; d0 += per) {
         if (cancelled(c)) return set_err(c, DC_ERR_CANCEL, DC_ER_COMM, "cancelled");
         const int nd = std::min(per, ndir - d0);
-        // weights per (direction, component) in sorted order, records, slices
-        std::vector<float> w((size_t)nd * 5 * ns);
-        std::vector<int> idx((size_t)nd * 5 * ns);
-        for (int k = 0; k < nd; ++k)
-            for (int q = 0; q < 5; ++q)
-                for (int t = 0; t < ns; ++t) {
-                    const int n = mp.order[t];
-                    const double *dp = dparam + 5 * ((size_t)(d0 + k) * m->natoms + n);
-                    const double o = m->occ[n];
-                    const double v = q == 0 ? dp[3] : (q < 4 ? o * dp[q - 1] : o * dp[4]);
-                    w[((size_t)k * 5 + q) * ns + t] = (float)v;
-                    idx[((size_t)k * 5 + q) * ns + t] = n;
-                }
         SliceSet ss;
         std::vector<int> dsl;
         int off = 0;
@@ -382,81 +395,110 @@ int dc_model_jvp(dc_ctx *c, const dc_model_desc *m, const double *fcalc, int ndi
         dsl.push_back((int)ss.type.size());
         if (ss.beg.empty()) ss.beg.push_back(0);
         const int nslice = (int)ss.type.size();
-        if ((st = upload(c, c->m_jw, w.data(), w.size()))) return st;
-        if ((st = upload(c, c->m_jidx, idx.data(), idx.size()))) return st;
-        if ((st = upload(c, c->m_dsl, dsl.data(), dsl.size()))) return st;
-        if ((st = upload(c, c->slice_beg, ss.beg.data(), ss.beg.size()))) return st;
-        if (nslice > 0 && (st = upload(c, c->slice_type, ss.type.data(), ss.type.size()))) return st;
-        if ((st = ensure(c, c->rec, sizeof(AtomRec) * std::max<size_t>(w.size(), 1)))) return st;
+        const long long nrec = 5LL * nd * ns;
+        int *d_dsl, *d_beg, *d_type;
+        if ((st = stage(c, c->m_dsl, dsl.data(), dsl.size(), d_dsl))) return st;
+        if ((st = stage(c, c->slice_beg, ss.beg.data(), ss.beg.size(), d_beg))) return st;
+        if ((st = stage(c, c->slice_type, ss.type.data(), ss.type.size(), d_type))) return st;
+        if ((st = stage_flush(c))) return st;
+        if ((st = ensure(c, c->rec, sizeof(AtomRec) * (size_t)std::max<long long>(nrec, 1)))) return st;
         if ((st = ensure(c, c->partial, sizeof(float2) * gg.P * std::max(nslice, 1)))) return st;
         PrepArgs pa = base_prep(mp.g, 0);
-        pa.src = ptr<double>(c->m_pos);
+        pa.src = mp.pos;
         pa.src_ld = 0;
-        pa.idx = ptr<int>(c->m_jidx);
-        pa.w = ptr<float>(c->m_jw);
-        pa.bdw_src = m->bdw ? ptr<double>(c->m_bd) : nullptr;
-        pa.n = (long long)w.size();
+        pa.idx = mp.idx;
+        pa.occ_src = mp.occ;
+        pa.bdw_src = mp.bdw;
+        pa.dpar = d_par + 5 * (size_t)m->natoms * d0;
+        pa.dn = std::max(ns, 1);
+        pa.dnat = m->natoms;
+        pa.n = nrec;
         if (pa.n > 0) HIPCHK(launch_prep(pa, ptr<AtomRec>(c->rec), c->st));
         c->rec_hash = false;
-        if ((st = run_gemm(c, mp.pl, ss.beg, ptr<float2>(c->partial), mp.any_b ? ptr<float>(c->m_sq) : nullptr))) return st;
+        if ((st = run_gemm(c, mp.pl, ss.beg, d_beg, ptr<float2>(c->partial), mp.any_b ? mp.d_sq : nullptr))) return st;
         JvpArgs ja{};
         ja.g = mp.g;
         ja.partial = ptr<float2>(c->partial);
-        ja.dslice = ptr<int>(c->m_dsl);
-        ja.slice_type = ptr<int>(c->slice_type);
-        ja.cfact = ptr<double2>(c->cfact);
-        ja.ncfact = m->ncfact;
+        ja.dslice = d_dsl;
+        ja.slice_type = d_type;
+        ja.cfact = mp.cfact;
+        ja.ncfact = mp.rows;
         ja.f = ptr<double>(c->m_f);
         ja.ndir = nd;
-        ja.di = ptr<double>(c->m_di) + (size_t)d0 * P;
-        ja.df = df ? ptr<double>(c->m_di) + (size_t)ndir * P + 2 * (size_t)d0 * P : nullptr;
+        ja.di = out + (size_t)d0 * P;
+        ja.df = df ? out + (size_t)ndir * P + 2 * (size_t)d0 * P : nullptr;
         HIPCHK(launch_jvp_reduce(ja, c->st));
-        c->stats.pairs += (double)w.size() * (double)P;
+        c->stats.pairs += (double)nrec * (double)P;
         c->stats.slices += nslice;
     }
     HIPCHK(hipEventRecord(c->ev[5], c->st));
-    if (ndir > 0) {
-        HIPCHK(hipMemcpyAsync(di, c->m_di.p, sizeof(double) * (size_t)P * ndir, hipMemcpyDeviceToHost, c->st));
+    if (ndir > 0 && !pinned) {
+        HIPCHK(hipMemcpyAsync(di, out, sizeof(double) * (size_t)P * ndir, hipMemcpyDeviceToHost, c->st));
         if (df)
-            HIPCHK(hipMemcpyAsync(df, ptr<double>(c->m_di) + (size_t)ndir * P, sizeof(double) * 2 * (size_t)P * ndir,
-                                  hipMemcpyDeviceToHost, c->st));
+            HIPCHK(hipMemcpyAsync(df, out + (size_t)ndir * P, sizeof(double) * 2 * (size_t)P * ndir, hipMemcpyDeviceToHost, c->st));
     }
     if ((st = model_end(c))) return st;
+    if (pinned) {
+        std::memcpy(di, out, sizeof(double) * (size_t)P * ndir);
+        if (df) std::memcpy(df, out + (size_t)ndir * P, sizeof(double) * 2 * (size_t)P * ndir);
+    }
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, c->ev[4], c->ev[5]));
     c->stats.forward_ms = ms;
     return DC_OK;
 }
 
-int dc_model_chi2(dc_ctx *c, const dc_model_desc *m, const double *target, const double *weight, double *chi2,
-                  double *icalc, double *grad) {
+// dev: the per-atom arrays of m, target, weight, icalc and grad are device
+// arrays, read and written in place.
+static int model_chi2(dc_ctx *c, const dc_model_desc *m, const double *target, const double *weight, double *chi2,
+                      double *icalc, double *grad, bool dev) {
     if (!c) return DC_ERR_ARG;
     if (!target || !chi2) return set_err(c, DC_ERR_ARG, DC_ER_LIB, "dc_model_chi2: null pointer");
     ModelPlan mp;
     int st;
-    if ((st = model_begin(c, m, mp))) return st;
+    if ((st = model_begin(c, m, mp, dev))) return st;
     if ((st = model_forward(c, m, mp))) return st;
     const long long P = mp.g.P;
-    if ((st = ensure(c, c->m_gi, sizeof(double) * (P + CHI2_BLOCKS)))) return st;
-    if ((st = ensure(c, c->w, sizeof(double) * 2 * P))) return st;
-    double *d_t = ptr<double>(c->w);
-    double *d_w = weight ? d_t + P : nullptr;
-    HIPCHK(hipMemcpyAsync(d_t, target, sizeof(double) * P, hipMemcpyHostToDevice, c->st));
-    if (weight) HIPCHK(hipMemcpyAsync(d_w, weight, sizeof(double) * P, hipMemcpyHostToDevice, c->st));
-    double *d_gi = ptr<double>(c->m_gi);
-    HIPCHK(launch_chi2_resid(ptr<double>(c->dsi), d_t, d_w, P, d_gi, d_gi + P, CHI2_BLOCKS, c->st));
-    std::vector<double> bs(CHI2_BLOCKS);
-    HIPCHK(hipMemcpyAsync(bs.data(), d_gi + P, sizeof(double) * CHI2_BLOCKS, hipMemcpyDeviceToHost, c->st));
-    if (icalc) HIPCHK(hipMemcpyAsync(icalc, c->dsi.p, sizeof(double) * P, hipMemcpyDeviceToHost, c->st));
+    if ((st = ensure(c, c->m_gi, sizeof(double) * P))) return st;
+    const double *d_t = target, *d_w = weight;
+    if (!dev) {
+        if ((st = ensure(c, c->w, sizeof(double) * 2 * P))) return st;
+        double *t = ptr<double>(c->w);
+        HIPCHK(hipMemcpyAsync(t, target, sizeof(double) * P, hipMemcpyHostToDevice, c->st));
+        if (weight) HIPCHK(hipMemcpyAsync(t + P, weight, sizeof(double) * P, hipMemcpyHostToDevice, c->st));
+        d_t = t;
+        d_w = weight ? t + P : nullptr;
+    }
+    // the blocks' sums come back through pinned memory
+    if ((st = pin_ensure(c, c->h_out, sizeof(double) * CHI2_BLOCKS))) return st;
+    double *sums = reinterpret_cast<double *>(c->h_out.p);
+    HIPCHK(launch_chi2_resid(ptr<double>(c->dsi), d_t, d_w, P, ptr<double>(c->m_gi), sums, CHI2_BLOCKS, c->st));
+    if (icalc)
+        HIPCHK(hipMemcpyAsync(icalc, c->dsi.p, sizeof(double) * P, dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, c->st));
     if (grad) {
-        if ((st = model_adjoint(c, m, mp))) return st;
-        HIPCHK(hipMemcpyAsync(grad, c->m_grad.p, sizeof(double) * 5 * m->natoms, hipMemcpyDeviceToHost, c->st));
+        double *d_grad = grad;
+        if (!dev) {
+            if ((st = ensure(c, c->m_grad, sizeof(double) * 5 * std::max<int64_t>(m->natoms, 1)))) return st;
+            d_grad = ptr<double>(c->m_grad);
+        }
+        if ((st = model_adjoint(c, m, mp, d_grad))) return st;
+        if (!dev) HIPCHK(hipMemcpyAsync(grad, d_grad, sizeof(double) * 5 * m->natoms, hipMemcpyDeviceToHost, c->st));
     }
     if ((st = model_end(c))) return st;
     double s = 0.0;
-    for (double v : bs) s += v;
+    for (int k = 0; k < CHI2_BLOCKS; ++k) s += sums[k];
     *chi2 = s;
     return DC_OK;
+}
+
+int dc_model_chi2(dc_ctx *c, const dc_model_desc *m, const double *target, const double *weight, double *chi2,
+                  double *icalc, double *grad) {
+    return model_chi2(c, m, target, weight, chi2, icalc, grad, false);
+}
+
+int dc_model_chi2_dev(dc_ctx *c, const dc_model_desc *m, const double *target, const double *weight, double *chi2,
+                      double *icalc, double *grad) {
+    return model_chi2(c, m, target, weight, chi2, icalc, grad, true);
 }
 
 }  // extern "C"

@@ -71,6 +71,22 @@ class RefineModel:
         d, keep = self.desc(pos, occ, bdw)
         return self.ctx.model_chi2(d, target, weight, want_grad)
 
+    # device face --------------------------------------------------------------
+    def on_device(self, pos, occ, bdw, target, weight):
+        """Whether the tensors of a chi2 call can be used where they lie: all on
+        the context's device, with the model's shapes."""
+        n = len(self.types)
+        every = [pos, occ, bdw, target] + ([] if weight is None else [weight])
+        if not all(isinstance(t, torch.Tensor) and t.is_cuda and t.device.index == self.ctx.device_index() for t in every):
+            return False
+        return (pos.shape == (n, 3) and occ.shape == (n,) and bdw.shape == (n,) and
+                all(tuple(t.shape) == self.shape for t in every[3:]))
+
+    def chi2_dev(self, pos, occ, bdw, target, weight, grad):
+        n = len(self.types)
+        d, keep = self.desc(np.empty((n, 3)), np.empty(n), np.empty(n))   # the per-atom arrays are the device's
+        return self.ctx.model_chi2_dev(d, pos, occ, bdw, target, weight, grad=grad)
+
     # torch face ---------------------------------------------------------------
     def intensity(self, pos, occ, bdw):
         """I over the grid (float64 tensor of shape inc) with autograd."""
@@ -114,11 +130,31 @@ class IntensityFn(torch.autograd.Function):
         return gp, go, gb, None
 
 
+def _dev(t):
+    return t.detach().to(torch.float64).contiguous()
+
+
+def _dev_grid(t):
+    """A map over the grid in the library's order, abscissa fastest."""
+    return t.detach().to(torch.float64).permute(2, 1, 0).contiguous()
+
+
 class Chi2Fn(torch.autograd.Function):
-    """chi^2 and its gradient from one dc_model_chi2 call."""
+    """chi^2 and its gradient from one dc_model_chi2 call; tensors that all
+    live on the context's device stay there (dc_model_chi2_dev)."""
 
     @staticmethod
     def forward(ctx, pos, occ, bdw, model, target, weight):
+        if model.on_device(pos, occ, bdw, target, weight):
+            n = len(model.types)
+            p, o, b, t = _dev(pos), _dev(occ), _dev(bdw), _dev_grid(target)
+            w = None if weight is None else _dev_grid(weight)
+            g = torch.empty((n, 5), dtype=torch.float64, device=pos.device)
+            # the library works on its own stream
+            torch.cuda.current_stream(pos.device).synchronize()
+            chi = model.chi2_dev(p, o, b, t, w, g)
+            ctx.grads = [x.to(v.dtype).contiguous() for x, v in zip((g[:, :3], g[:, 3], g[:, 4]), (pos, occ, bdw))]
+            return torch.tensor(chi, dtype=torch.float64, device=pos.device)
         t = np.asfortranarray(_np(target))
         w = None if weight is None else np.asfortranarray(_np(weight))
         chi, icalc, g = model.chi2_np(_np(pos), _np(occ), _np(bdw), t, w, want_grad=True)

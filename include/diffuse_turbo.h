@@ -315,6 +315,15 @@ int dc_model_jvp(dc_ctx *ctx, const dc_model_desc *model, const double *fcalc, i
 int dc_model_chi2(dc_ctx *ctx, const dc_model_desc *model, const double *target, const double *weight,
                   double *chi2, double *icalc, double *grad);
 
+/* The same with the per-atom arrays on the device: model->pos, ->occ, ->bdw
+ * (non-NULL = per-atom B), target, weight, icalc and grad are device pointers
+ * on the context's device, read and written in place; type, cfact and chi2
+ * stay host arrays.  Work pending on them on other streams must have finished. */
+int dc_model_chi2_dev(dc_ctx *ctx, const dc_model_desc *model, const double *target, const double *weight,
+                      double *chi2, double *icalc, double *grad);
+/* Device ordinal of the context. */
+int dc_device_index(const dc_ctx *ctx);
+
 /*
  * Population scoring (DIFFEV, diffev/prog/diffev_kdo.f90:676 running one
  * macro per member over lib_f90/with_mpi.f90:281-609): nmembers refinement
