@@ -12,22 +12,32 @@
 // parameter (finite differences, refine/prog/refine_run.f90:491-600); here
 // they come from one pass that reuses the forward's phase generation.
 //
-// GEMM form (grid rows r = abscissa, columns c = (ordinate, top) flattened
-// with period C0; the grid must be metric-orthogonal between rows and
+// GEMM form (grid rows r = abscissa, columns c = (ordinate, top) flattened;
+// the grid must be metric-orthogonal between rows and
 // columns so that s^2 = s_r^2 + s_c^2 and E splits as A(r,n) B(c,n)):
 //     Z_w(n, c) = sum_r w(r) A(r, n) Q(r, c),   w in {1, r - rc, s_r^2}
-// on MFMA (FP32, K = grid rows, A generated per stage, Q streamed from HBM),
-// then an epilogue contracts each Z with the generated column factor B(c, n)
+// on MFMA, then an epilogue contracts each Z with the column factor B(c, n)
 // and the column weights (1, j - jc, m - mc, s_c^2).  h_p,a is affine in
 // (r, j, m), so the three row weights and four column weights give every
 // sum above; the weights are centred to keep the FP32 terms small.
 //
-// Split variant (BF16x3, v_mfma_f32_16x16x32_bf16): the weighted A elements
-// are split into BF16 hi + lo in FP32 and stored in LDS in the two forms of
-// the real embedding; Q comes pre-split (q_split_kernel) in a layout whose
-// 16-byte words are exactly one lane's MFMA operand, loaded from L2 into
-// registers one stage ahead.  Products hi.hi + hi.lo + lo.hi, FP32
-// accumulation, the same epilogue.
+// Mirrored rows.  About the centre of the rows A(+-j) = d_j (cos +- i sin),
+// so that with S = wQ(+j) + wQ(-j) and D = wQ(+j) - wQ(-j)
+//     sum over +-j of w A Q = d_j (cos S + i sin D):
+// half the real products of the row-by-row sum, for every weight.  It needs
+// d_j = exp(-B s_j^2) alike on both sides (s_r^2 mirrored, or no B); other
+// grids run the same kernel with each row as its own pair, where the
+// coefficients of cos and sin are Q and iQ.
+//
+// The coefficients (weights applied, S and D formed in FP32) are split once per
+// call into 16-bit parts and stored as the words of the MFMA operand
+// (adj_words_kernel): 3 parts and 6 products (hh, hm, mh, hl, lh, mm) in FP32,
+// which keep 24 bits of both operands -- the dropped terms are below 2^-25 of a
+// product, less than FP32's own rounding of it.  The split precisions take 2
+// FP16 parts and 3 products, the coefficients of a column tile scaled by one
+// power of two to FP16's range (22 bits against the largest; two BF16 parts
+// hold 16, and S and D, being sums, then cost 1.4 times the row-by-row
+// error).  Either unit runs 16 times the FP32 rate.
 #include <algorithm>
 #include <atomic>
 
@@ -35,753 +45,432 @@
 
 namespace dc {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 namespace {
 
-constexpr int WA = 2, WC = 2, NWA = 1, NWC = 8;   // 16x16 tiles per wave, waves per work-group
-constexpr int NA = 16 * WA * NWA;                  // atoms per work-group
-constexpr int NC = 16 * WC * NWC;                  // grid columns per work-group
-constexpr int NT = 64 * NWA * NWC;
-constexpr int KR = 16;                             // grid rows per LDS stage
-static_assert(NT == NA * KR, "one A element per thread and stage");
-static_assert(KR == 16, "row tables hold 16 rows per stage");
-constexpr int MAXST = 64;                          // stages with tabulated row factors (R <= 1024)
-constexpr int KP = 2 * KR;                         // real K per stage (re, im interleaved)
+constexpr int AW = 4;               // waves of a work-group
+constexpr int NT = 64 * AW;
+constexpr int WA = 2;               // 16-atom tiles of a wave
+constexpr int NA = 16 * WA * AW;    // atoms of a work-group
+constexpr int CT = 16;              // grid columns of a tile
+constexpr int KP = 16;              // row pairs of a k-step: one 16x16x32 product
+constexpr int WALK_TILES = 256 / CT;   // tiles of one unit of the column walk
+constexpr int MAX_WALK = 32;
+constexpr int MAX_GROUPS = 64;      // column ranges, each a partial set
+constexpr int RESYNC = 4;           // tiles between exact column phases
 constexpr float LOG2E = 1.4426950408889634f;
+// k-steps a wave keeps its A operands of in registers (24 VGPRs a step with 3
+// parts, 16 with 2); longer grids are cut into row chunks, each a partial set.
+constexpr int max_ksteps(int parts) { return parts == 3 ? 3 : 5; }
 
-// Column factors of the epilogue, exact two-level: column col0 + 16h + l of
-// atom n has phase TH[n][h] + l ca + delta w (delta = 1 past the wrap of the
-// flattened columns, at l >= wpos[h]; w = ca1 - C0 ca).
-struct ColTables {
-    float2 th[NA][NC / 16];
-    float2 tl[NA][2][16];
-    int wpos[NC / 16];
-};
+// (x, y) as NP pairs (x in the low half) whose sums are x and y: three BF16
+// parts, exactly, or two FP16 parts, to 2^-23 (2^-25 where that is larger)
+template <int NP>
+__device__ __forceinline__ void split(float x, float y, uint32_t (&part)[NP]) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        if constexpr (NP == 3) {
+            const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x, y}, bf16x2));
+            part[p] = h;
+            x -= __builtin_bit_cast(float, h << 16);
+            y -= __builtin_bit_cast(float, h & 0xFFFF0000u);
+        } else {
+            const f16x2 h = __builtin_convertvector((f32x2){x, y}, f16x2);
+            part[p] = __builtin_bit_cast(uint32_t, h);
+            x -= (float)h[0];
+            y -= (float)h[1];
+        }
+    }
+}
+template <int NP>
+__device__ __forceinline__ f32x4 mfma(u32x4 x, u32x4 y, f32x4 c) {
+    if constexpr (NP == 3)
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x), __builtin_bit_cast(bf16x8, y), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x), __builtin_bit_cast(f16x8, y), c, 0, 0, 0);
+}
 
-// Row factors, exact two-level: row 16 s + rr of atom n has phase
-// 16 s ra + rr ra, so A = RH[s][n] * RL[n][rr] (grids of up to S stages).
-template <int S>
-struct RowTablesT {
-    float2 rh[S][NA];
-    // row-major with a padded row (8 float2): the stage builders read 4 rows
-    // x 8 atoms per half-wave, which then fall on distinct banks
-    float2 rl[16][NA + 8];
-};
-using RowTables = RowTablesT<MAXST>;
-
-struct AdSmem {
-    float a[2][KP][NA];       // A(k', atom), k' = 2 rr + (0 re, 1 im)
-    float2 q[2][KR][NC];      // Q(rr, column)
-    float sr[2][KR];          // s^2 row parts of the stage rows
-    AtomRec at[NA];
-    float red[NWC][NA][6];    // per column-wave partial sums (fixed-order reduction)
-    ColTables ct;
-    RowTables rt;
-};
+__device__ __forceinline__ float exp2i(int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); }
+// e with 2^e <= x < 2^(e + 1), kept within +-100 (0 of zero)
+__device__ __forceinline__ int exponent(float x) {
+    return x == 0.0f ? 0 : min(100, max(-100, (int)(__builtin_bit_cast(uint32_t, x) >> 23 & 0xFF) - 127));
+}
+// Powers of two that bring the row weights to 1 at most (2 parts; 1 with 3).
+template <int NP>
+__device__ __forceinline__ void weight_scales(const AdjArgs &a, const float *__restrict__ sq, float (&sg)[3]) {
+    sg[0] = sg[1] = sg[2] = 1.0f;
+    if constexpr (NP == 2) {
+        float m = 0.0f;
+        for (int r = threadIdx.x & 63; r < a.R; r += 64) m = fmaxf(m, fabsf(sq[r]));
+#pragma unroll
+        for (int h = 1; h < 64; h *= 2) m = fmaxf(m, __shfl_xor(m, h));
+        sg[1] = exp2i(-1 - exponent(fmaxf(a.rc, 0.5f)));
+        sg[2] = exp2i(-1 - exponent(m));
+    }
+}
 
 __device__ __forceinline__ float2 cis(uint64_t ph) {
     float c, s;
-    sincos_turn((uint32_t)((ph + 0x80000000ull) >> 32), c, s);
+    sincos_turn_fine((uint32_t)((ph + 0x80000000ull) >> 32), c, s);
     return make_float2(c, s);
 }
-
-template <class RT>
-__device__ __forceinline__ void build_row_tables(RT &rt, const AtomRec *at, int nst) {
-    for (int x = threadIdx.x; x < NA * (16 + nst); x += NT) {
-        const int n = x % NA, e = x / NA;
-        if (e < 16)
-            rt.rl[e][n] = cis((uint64_t)e * at[n].ra);
-        else
-            rt.rh[e - 16][n] = cis((uint64_t)(16 * (e - 16)) * at[n].ra);
-    }
+__device__ __forceinline__ float2 cmul(float2 a, float2 b) {
+    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
-// A element of atom n at row r = 16 s + rr (r < R): row phase and exp(-B s_r^2)
-template <class RT>
-__device__ __forceinline__ float2 row_element(const RT &rt, const AtomRec &ar, int n, int s, int rr, int r, bool tab,
-                                              float s2) {
-    float2 v;
-    if (tab) {
-        const float2 h = rt.rh[s][n], l = rt.rl[rr][n];
-        v = make_float2(h.x * l.x - h.y * l.y, h.x * l.y + h.y * l.x);
+// Rows of pair p: r1 and, when folded, its mirror r0 (-1: none); false past the
+// last pair.  a.center: the centre row is no pair, the epilogue adds it.
+__device__ __forceinline__ bool pair_rows(const AdjArgs &a, int p, int &r1, int &r0) {
+    r0 = -1;
+    if (!a.fold) {
+        r1 = p;
+        return p < a.R;
+    }
+    const int h = a.R / 2;
+    p += a.center;
+    r1 = h + p;
+    if (a.R & 1) {
+        if (p > 0) r0 = h - p;
     } else {
-        v = cis((uint64_t)r * ar.ra);
+        r0 = h - 1 - p;
     }
-    const float d = __builtin_amdgcn_exp2f(-ar.pad * LOG2E * s2);
-    return make_float2(v.x * d, v.y * d);
+    return r1 < a.R;
 }
 
-// A of stage rows r0..r0+KR-1 (one element per thread) and the Q rows.
-__device__ __forceinline__ void load_stage(AdSmem &sm, int buf, const AdjArgs &a, const float *__restrict__ sq,
-                                           int st, int col0, int na, long long qbase, bool tab) {
-    const int t = threadIdx.x;
-    const int r0 = st * KR;
-    {
-        const int at = t & (NA - 1), rr = t / NA;      // NT == NA * KR
-        const int r = r0 + rr;
-        float2 v = make_float2(0.f, 0.f);
-        if (r < a.R && at < na) v = row_element(sm.rt, sm.at[at], at, st, rr, r, tab, sq[r]);
-        sm.a[buf][2 * rr][at] = v.x;
-        sm.a[buf][2 * rr + 1][at] = v.y;
-    }
+// Q planes -> operand words of one (plane, column tile, k-step): for weight w,
+// component (re, im) and part, lane l holds column l % 16 of the tile and the
+// (cos, sin) coefficients of pairs 4 (l / 16) .. + 3 of the step.
+// One work-group per (plane, tile), a wave per k-step.  2 parts: the tile's
+// coefficients are scaled to below 2^15, and the scale noted.
+template <int NP>
+__global__ void __launch_bounds__(256) adj_words_kernel(AdjArgs a, int plane0, int nplane, u32x4 *__restrict__ out) {
+    constexpr int NW = 6 * NP;
+    __shared__ float red[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float *scales = reinterpret_cast<float *>(out + (long long)nplane * a.ctiles * a.nkt * (NW * 64));
+    for (long long x = blockIdx.x; x < (long long)nplane * a.ctiles; x += gridDim.x) {
+        const int ct = (int)(x % a.ctiles), pl = (int)(x / a.ctiles);
+        const int c = ct * CT + (lane & 15);
+        const bool in = c < a.C && c % a.C0 < a.f1;
+        const float *sq = a.sq + (long long)((plane0 + pl) / a.planes_per_sq) * a.sq_stride;
+        const float2 *q = a.q + (long long)(plane0 + pl) * a.plane + c;
+        float sg[3], scale = 1.0f;
+        weight_scales<NP>(a, sq, sg);
+        if constexpr (NP == 2) {
+            float m = 0.0f;
+            if (in)
+                for (int r = threadIdx.x >> 4; r < a.R; r += 16) {
+                    const float2 v = q[(long long)a.C * r];
+                    m = fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)));
+                }
 #pragma unroll
-    for (int u = 0; u < (KR * NC) / NT; ++u) {
-        const int e = t + u * NT;
-        const int rr = e / NC, cc = e % NC;
-        const int r = r0 + rr, col = col0 + cc;
-        sm.q[buf][rr][cc] = (r < a.R && col < a.C) ? a.q[qbase + col + (long long)a.C * r] : make_float2(0.f, 0.f);
-    }
-    if (t < KR) sm.sr[buf][t] = r0 + t < a.R ? sq[r0 + t] : 0.0f;
-}
-
-// Epilogue shared by the FP32 and split kernels: lane holds atoms 4 lg + v of
-// column li of every 16x16 tile; contract with the generated column factor
-// and weights, reduce over columns in a fixed order, write the partials.
-// Three steps: column tables of the tile at col0 (epi_tables), contraction
-// into per-lane column sums (epi_contract, adds to acc), reduction over lanes
-// and waves into partial set `set` (epi_reduce).
-__device__ __forceinline__ void epi_tables(const AdjArgs &a, const AtomRec *at, ColTables &ct, int col0) {
-    // two-level column tables of the work-group's atoms (caller synchronised the LDS)
-    constexpr int NH = NC / 16, NE = NH + 32;
-    for (int x = threadIdx.x; x < NA * NE; x += NT) {
-        const int n = x / NE, e = x % NE;
-        const AtomRec &ar = at[n];
-        if (e < NH) {
-            const int c0 = col0 + 16 * e;
-            ct.th[n][e] = cis(ar.p0 + (uint64_t)(c0 % a.C0) * ar.ca + (uint64_t)(c0 / a.C0) * ar.ca1);
-            if (n == 0) ct.wpos[e] = a.C0 - c0 % a.C0;
-        } else {
-            const int d = (e - NH) >> 4, l = (e - NH) & 15;
-            const uint64_t w = ar.ca1 - (uint64_t)a.C0 * ar.ca;
-            ct.tl[n][d][l] = cis((uint64_t)l * ar.ca + (d ? w : 0ull));
+            for (int h = 1; h < 64; h *= 2) m = fmaxf(m, __shfl_xor(m, h));
+            __syncthreads();   // the previous tile's maxima have been read
+            if (lane == 0) red[wave] = m;
+            __syncthreads();
+            m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+            scale = exp2i(13 - exponent(m));
+            if (threadIdx.x == 0) scales[x] = scale;
         }
-    }
-}
-
-__device__ __forceinline__ void epi_contract(const AdjArgs &a, const float *__restrict__ sq, const AtomRec *at,
-                                             const ColTables &ct, const f32x4 (&accR)[3][WA][WC],
-                                             const f32x4 (&accI)[3][WA][WC], int col0, float (&acc)[WA][4][6]) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-    const int wa0 = (wave % NWA) * 16 * WA, wc0 = (wave / NWA) * 16 * WC;
+        for (int k = wave; k < a.nkt; k += 4) {
+            u32x4 w[3][2][NP];
 #pragma unroll
-    for (int j = 0; j < WC; ++j) {
-        const int col = col0 + wc0 + 16 * j + li;
-        const int jj = col % a.C0, mm = col / a.C0;
-        const bool valid = col < a.C && jj < a.f1;
-        const float sc = valid ? sq[a.R + col] : 0.0f;
-        const float wj = (float)jj - a.jc, wm = (float)mm - a.mc;
-        const int h = wc0 / 16 + j;
-        const int dl = li >= ct.wpos[h] ? 1 : 0;
-#pragma unroll
-        for (int i = 0; i < WA; ++i)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int n = wa0 + 16 * i + 4 * lg + v;
-                const float2 th = ct.th[n][h], tl = ct.tl[n][dl][li];
-                float2 b = make_float2(th.x * tl.x - th.y * tl.y, th.x * tl.y + th.y * tl.x);
-                const float d = valid ? __builtin_amdgcn_exp2f(-at[n].pad * LOG2E * sc) : 0.0f;
-                b = make_float2(b.x * d, b.y * d);
-                const float z0r = accR[0][i][j][v], z0i = accI[0][i][j][v];
-                const float tr = z0r * b.x - z0i * b.y;
-                const float ti = z0r * b.y + z0i * b.x;
-                const float u1 = accR[1][i][j][v] * b.y + accI[1][i][j][v] * b.x;
-                const float u2 = accR[2][i][j][v] * b.x - accI[2][i][j][v] * b.y;
-                acc[i][v][0] += tr;
-                acc[i][v][1] += ti;
-                acc[i][v][2] += u1;
-                acc[i][v][3] += wj * ti;
-                acc[i][v][4] += wm * ti;
-                acc[i][v][5] += u2 + sc * tr;
-            }
-    }
-}
-
-// Sum of the per-wave partials (red, synchronised by the caller) in wave
-// order, written as partial set `set`.
-__device__ __forceinline__ void epi_write(const AdjArgs &a, const float (&red)[NWC][NA][6], int set, int atom0,
-                                          int na) {
-    float *out = a.part + ((long long)set * a.natoms + atom0) * 6;
-    for (int x = threadIdx.x; x < na * 6; x += NT) {
-        float v = 0.0f;
-#pragma unroll
-        for (int w = 0; w < NWC; ++w) v += (&red[w][0][0])[x];
-        out[x] = v;
-    }
-}
-
-__device__ __forceinline__ void epi_reduce(const AdjArgs &a, float (&red)[NWC][NA][6], float (&acc)[WA][4][6],
-                                           int set, int atom0, int na) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-    const int wa0 = (wave % NWA) * 16 * WA;
-    // sum over the 16 columns of a lane group, then over the waves of a row of tiles
-#pragma unroll
-    for (int i = 0; i < WA; ++i)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-#pragma unroll
-            for (int k = 0; k < 6; ++k) {
-                float x = acc[i][v][k];
-                x += __shfl_xor(x, 1);
-                x += __shfl_xor(x, 2);
-                x += __shfl_xor(x, 4);
-                x += __shfl_xor(x, 8);
-                if (li == 0) red[wave / NWA][wa0 + 16 * i + 4 * lg + v][k] = x;
-            }
-    __syncthreads();
-    epi_write(a, red, set, atom0, na);
-}
-
-// Row-local lane exchange (data-parallel primitives): lane li of each 16-lane
-// row reads lane src(li) of the same row.
-template <int CTRL>
-__device__ __forceinline__ float dpp(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
-}
-constexpr int DPP_ROW_MIRROR = 0x140;        // src = 15 - li
-constexpr int DPP_ROW_HALF_MIRROR = 0x141;   // src = (li & 8) | (7 - (li & 7))
-constexpr int DPP_QUAD_XOR2 = 0x4E;          // quad_perm [2,3,0,1]: src = li ^ 2
-constexpr int DPP_QUAD_XOR1 = 0xB1;          // quad_perm [1,0,3,2]: src = li ^ 1
-
-// Sums the 48 per-lane column sums of a 16-lane row over its lanes and
-// scatters the totals: four halving exchanges (partners 15 - li, the mirror
-// inside the half-row, li ^ 2, li ^ 1; bit 8, 4, 2, 1 of li picks the half a
-// lane keeps) leave lane li with the row totals of flat entries 3 li, 3 li + 1,
-// 3 li + 2 of acc (flat = (4 i + v) 6 + k).  Fixed order, so deterministic.
-__device__ __forceinline__ void row_reduce_scatter(const float (&acc)[WA][4][6], float (&out)[3], int li) {
-    static_assert(WA * 4 * 6 == 48, "48 column sums per lane");
-    const float *x = &acc[0][0][0];
-    float y[24], z[12], w[6];
-#pragma unroll
-    for (int j = 0; j < 24; ++j) {
-        const bool h = (li & 8) != 0;
-        y[j] = (h ? x[24 + j] : x[j]) + dpp<DPP_ROW_MIRROR>(h ? x[j] : x[24 + j]);
-    }
-#pragma unroll
-    for (int j = 0; j < 12; ++j) {
-        const bool h = (li & 4) != 0;
-        z[j] = (h ? y[12 + j] : y[j]) + dpp<DPP_ROW_HALF_MIRROR>(h ? y[j] : y[12 + j]);
-    }
-#pragma unroll
-    for (int j = 0; j < 6; ++j) {
-        const bool h = (li & 2) != 0;
-        w[j] = (h ? z[6 + j] : z[j]) + dpp<DPP_QUAD_XOR2>(h ? z[j] : z[6 + j]);
-    }
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        const bool h = (li & 1) != 0;
-        out[j] = (h ? w[3 + j] : w[j]) + dpp<DPP_QUAD_XOR1>(h ? w[j] : w[3 + j]);
-    }
-}
-
-__device__ __forceinline__ void adjoint_epilogue(const AdjArgs &a, const float *__restrict__ sq,
-                                                 const AtomRec *at, float (&red)[NWC][NA][6], ColTables &ct,
-                                                 f32x4 (&accR)[3][WA][WC], f32x4 (&accI)[3][WA][WC], int col0,
-                                                 int atom0, int na) {
-    epi_tables(a, at, ct, col0);
-    __syncthreads();
-    float acc[WA][4][6];
-#pragma unroll
-    for (int i = 0; i < WA; ++i)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-#pragma unroll
-            for (int k = 0; k < 6; ++k) acc[i][v][k] = 0.0f;
-    epi_contract(a, sq, at, ct, accR, accI, col0, acc);
-    epi_reduce(a, red, acc, blockIdx.x, atom0, na);
-}
-
-__global__ void __launch_bounds__(NT) adjoint_kernel(AdjArgs a) {
-    __shared__ AdSmem sm;
-    const int4 tile = a.tiles[blockIdx.y];
-    const int atom0 = tile.x, na = tile.y - tile.x;
-    const long long qbase = (long long)tile.z * a.plane;
-    const float *sq = a.sq + (long long)tile.w * a.sq_stride;
-    const int col0 = blockIdx.x * NC;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-    const int wa0 = (wave % NWA) * 16 * WA, wc0 = (wave / NWA) * 16 * WC;
-
-    for (int x = threadIdx.x; x < NA; x += NT) {
-        AtomRec r{};
-        if (x < na) r = a.rec[atom0 + x];
-        sm.at[x] = r;
-    }
-    __syncthreads();
-
-    f32x4 accR[3][WA][WC], accI[3][WA][WC];
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-        for (int i = 0; i < WA; ++i)
-#pragma unroll
-            for (int j = 0; j < WC; ++j) {
-                accR[k][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-                accI[k][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-
-    const int nst = (a.R + KR - 1) / KR;
-    const bool tab = nst <= MAXST;
-    if (tab) build_row_tables(sm.rt, sm.at, nst);
-    __syncthreads();
-    load_stage(sm, 0, a, sq, 0, col0, na, qbase, tab);
-    __syncthreads();
-    for (int s = 0; s < nst; ++s) {
-        const int buf = s & 1;
-        if (s + 1 < nst) load_stage(sm, buf ^ 1, a, sq, s + 1, col0, na, qbase, tab);
-        const bool im = (lg & 1) != 0;
-#pragma unroll
-        for (int ks = 0; ks < KR / 2; ++ks) {
-            const int rr = 2 * ks + (lg >> 1);
-            const float wr = (float)(s * KR + rr) - a.rc;
-            const float ws = sm.sr[buf][rr];
-            float av[WA][3];
-#pragma unroll
-            for (int i = 0; i < WA; ++i) {
-                const float x = sm.a[buf][4 * ks + lg][wa0 + 16 * i + li];
-                av[i][0] = x;
-                av[i][1] = x * wr;
-                av[i][2] = x * ws;
-            }
-#pragma unroll
-            for (int j = 0; j < WC; ++j) {
-                const float2 b = sm.q[buf][rr][wc0 + 16 * j + li];
-                const float bR = im ? -b.y : b.x;
-                const float bI = im ? b.x : b.y;
-#pragma unroll
-                for (int i = 0; i < WA; ++i)
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        accR[k][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][k], bR, accR[k][i][j], 0, 0, 0);
-                        accI[k][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][k], bI, accI[k][i][j], 0, 0, 0);
+            for (int e = 0; e < 4; ++e) {
+                int r1, r0;
+                float2 q1 = make_float2(0.f, 0.f), q0 = q1;
+                float w1[3] = {1.0f, 0.0f, 0.0f}, w0[3] = {1.0f, 0.0f, 0.0f};
+                if (in && pair_rows(a, KP * k + 4 * (lane >> 4) + e, r1, r0)) {
+                    q1 = q[(long long)a.C * r1];
+                    w1[1] = ((float)r1 - a.rc) * sg[1];
+                    w1[2] = sq[r1] * sg[2];
+                    if (r0 >= 0) {
+                        q0 = q[(long long)a.C * r0];
+                        w0[1] = ((float)r0 - a.rc) * sg[1];
+                        w0[2] = sq[r0] * sg[2];
                     }
+                }
+                if constexpr (NP == 2) {
+                    q1 = make_float2(q1.x * scale, q1.y * scale);
+                    q0 = make_float2(q0.x * scale, q0.y * scale);
+                }
+#pragma unroll
+                for (int v = 0; v < 3; ++v) {
+                    const float2 x1 = make_float2(q1.x * w1[v], q1.y * w1[v]), x0 = make_float2(q0.x * w0[v], q0.y * w0[v]);
+                    uint32_t re[NP], im[NP];
+                    split<NP>(x1.x + x0.x, x0.y - x1.y, re);   // S.re, -D.im
+                    split<NP>(x1.y + x0.y, x1.x - x0.x, im);   // S.im, D.re
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) {
+                        w[v][0][p][e] = re[p];
+                        w[v][1][p][e] = im[p];
+                    }
+                }
             }
-        }
-        __syncthreads();
-    }
-
-    adjoint_epilogue(a, sq, sm.at, sm.red, sm.ct, accR, accI, col0, atom0, na);
-}
-
-// ---------------------------------------------------------------------------
-// Split BF16x3 adjoint.
-constexpr int SKR = 16;   // grid rows per stage: one 16x16x32 k-step (K' = 32)
-
-__device__ __forceinline__ uint32_t bpack(float x, float y) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x, y}, bf16x2));
-}
-// (x, y) = hi + lo, both packed BF16 pairs (x in the low half)
-__device__ __forceinline__ void bsplit(float x, float y, uint32_t &hi, uint32_t &lo) {
-    hi = bpack(x, y);
-    lo = bpack(x - __builtin_bit_cast(float, hi << 16), y - __builtin_bit_cast(float, hi & 0xFFFF0000u));
-}
-__device__ __forceinline__ uint32_t rot16(uint32_t w) { return (w >> 16) | (w << 16); }
-
-// One stage of split A in LDS: [form (re,-im) | (im,re)][weight][hi | lo][row group][atom]
-typedef u32x4 StageA[2][3][2][4][NA];
-
-struct AdSmemS {
-    StageA a[2];                  // double-buffered stages
-    AtomRec at[NA];
-    float red[NWC][NA][6];
-    ColTables ct;
-    RowTables rt;
-};
-
-// A of stage st (rows 16 st .. 16 st + 15): thread (atom, row group g, e)
-// makes row 4g + e, all three weights, both forms, hi and lo.
-template <class RT>
-__device__ __forceinline__ void gen_stage_split(StageA &dst, const RT &rt, const AtomRec *ats, const AdjArgs &a,
-                                                const float *__restrict__ sq, int st, int na, bool tab) {
-    const int t = threadIdx.x;
-    // e fastest: a wave's 4-byte stores of one plane cover 64 consecutive words
-    // (with the atom fastest they met on the same banks four at a time;
-    // measured with the padded row tables: population forward + adjoint
-    // 11.73 -> 11.43 ms, identical results)
-    const int e = t & 3, at = (t >> 2) & (NA - 1), g = t / (4 * NA);
-    const int rr = 4 * g + e, r = st * SKR + rr;
-    float2 v = make_float2(0.f, 0.f);
-    float s2 = 0.0f;
-    if (r < a.R && at < na) {
-        s2 = sq[r];
-        v = row_element(rt, ats[at], at, st, rr, r, tab, s2);
-    }
-    const float wt[3] = {1.0f, (float)r - a.rc, s2};
+            u32x4 *o = out + (x * a.nkt + k) * (NW * 64) + lane;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        uint32_t hi, lo;
-        bsplit(v.x * wt[k], v.y * wt[k], hi, lo);
-        reinterpret_cast<uint32_t *>(&dst[0][k][0][g][at])[e] = hi ^ 0x80000000u;
-        reinterpret_cast<uint32_t *>(&dst[1][k][0][g][at])[e] = rot16(hi);
-        reinterpret_cast<uint32_t *>(&dst[0][k][1][g][at])[e] = lo ^ 0x80000000u;
-        reinterpret_cast<uint32_t *>(&dst[1][k][1][g][at])[e] = rot16(lo);
-    }
-}
-
-// B operand words of stage st: lane (column li, row group lg) of each of the
-// wave's 16-column tiles starting at column cw (zero past the padded columns).
-__device__ __forceinline__ void load_bwords(const uint32_t *__restrict__ qh, const uint32_t *__restrict__ ql,
-                                            const AdjArgs &a, int cw, int st, u32x4 (&bh)[WC], u32x4 (&bl)[WC]) {
-    const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+            for (int v = 0; v < 6; ++v)
 #pragma unroll
-    for (int j = 0; j < WC; ++j) {
-        const int col = cw + 16 * j + li;
-        const long long o = ((long long)(st * 4 + lg) * a.C + col) * 4;
-        if (col < a.C) {
-            bh[j] = *reinterpret_cast<const u32x4 *>(qh + o);
-            bl[j] = *reinterpret_cast<const u32x4 *>(ql + o);
-        } else {
-            bh[j] = u32x4{0u, 0u, 0u, 0u};
-            bl[j] = u32x4{0u, 0u, 0u, 0u};
+                for (int p = 0; p < NP; ++p) o[(v * NP + p) * 64] = w[v >> 1][v & 1][p];
         }
     }
 }
 
-// The 72 MFMAs of one stage of one wave: hi.hi + hi.lo + lo.hi for the three
-// row weights, both forms of the real embedding, WA x WC tiles.
-__device__ __forceinline__ void split_mfma_stage(const StageA &sa, const u32x4 (&bh)[WC], const u32x4 (&bl)[WC],
-                                                 f32x4 (&accR)[3][WA][WC], f32x4 (&accI)[3][WA][WC], int wa0) {
-    const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+// What bounds it: the matrix products (36 or 18 of 16x16x32 a k-step, wave and
+// atom tile) with the epilogue's VALU work beside them.  A wave owns 32 atoms:
+// their A operands of every k-step of the row chunk stay in registers, made
+// once; the work-group's waves share the words of one (column tile, k-step)
+// through LDS, double-buffered, the next step's loads in flight in registers
+// while this one's products run (one barrier a step).  The words are the
+// MFMA's rows and the atoms its columns, so a lane's 4 results of a tile
+// belong to one atom: the epilogue sums them in the lane and keeps six FP64
+// totals an atom over the whole column range, with no exchange until the end.
+// (32x32x16 products, the same work, need twice the accumulators and spilled.)
+// An odd row count whose centre row would open a k-step of its own (65 rows:
+// 32 pairs and the centre) has it added by the epilogue instead, in FP32.
+// Measured, 32,768 atoms on 65^3 points in FP32: 2.55 ms of FP32 products row
+// by row -> 0.55 ms (0.25 ms of it matrix products at their peak) + 0.012 ms
+// for the words; 24 members on 129^2 in the split precisions 0.595 -> 0.15 ms.
+// The gradient's error against FP64 (relative to its norm; x, occ, B) went from
+// 1.8e-7, 9e-8, 1.0e-7 to 1.2e-7, 5e-8, 6e-8 in FP32 and from 3.5e-6,
+// 1.1e-6, 1.8e-6 to 1.4e-7, 6e-8, 7e-8 in the split precisions.
+template <int NP, int NK>
+__global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, int plane0, int nplane, const u32x4 *__restrict__ words) {
+    constexpr int NW = 6 * NP, LD = (NW + AW - 1) / AW;
+    __shared__ u32x4 sq_w[2][NW][64];
+    __shared__ float4 col[2][CT];          // s_c^2, j - jc, m - mc, scaled s_c^2 of the tile's columns
+    __shared__ float2 qcen[2][CT];         // Q of the centre row
+    const int4 tile = a.tiles[tile0 + blockIdx.y];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int li = lane & 15, lg = lane >> 4;
+    const float *sq = a.sq + (long long)tile.w * a.sq_stride;
+    const int group = blockIdx.x % a.groups, chunk = blockIdx.x / a.groups;
+    const int ct0 = group * a.tpg, ct1 = min(a.ctiles, ct0 + a.tpg);
+    const int k0 = chunk * NK;
+    const int n0 = tile.x + wave * 16 * WA + li;
+    const bool active = tile.x + wave * 16 * WA < tile.y;      // wave-uniform
+    const bool center = a.center && chunk == 0;
+    float sg[3];
+    weight_scales<NP>(a, sq, sg);
+    const float s2c = sq[a.R / 2], s2cs = s2c * sg[2];
+
+    // per atom: A operands, phase of the row origin, column factors: tl[v] of
+    // the 4 columns a lane holds, rot of one tile, wrap of a step from the end
+    // of one ordinate run to the next (runs are at least a tile long)
+    u32x4 A[NK][WA][NP];
+    uint64_t ph[WA], ca[WA], ca1[WA];
+    float bl2[WA], cen[WA];
+    float2 tl[WA][4], rot[WA], wrap[WA];
+    const bool half = a.fold && !(a.R & 1);    // the centre lies half a step past row (R - 1) / 2
 #pragma unroll
     for (int i = 0; i < WA; ++i) {
-        u32x4 A[2][3][2];
+        AtomRec at{};
+        if (n0 + 16 * i < tile.y) at = a.rec[n0 + 16 * i];
+        const uint64_t hs = half ? at.ra >> 1 : 0;
+        bl2[i] = -at.pad * LOG2E;
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
+        for (int k = 0; k < NK; ++k)
 #pragma unroll
-            for (int k = 0; k < 3; ++k)
-#pragma unroll
-                for (int p = 0; p < 2; ++p) A[f][k][p] = sa[f][k][p][lg][wa0 + 16 * i + li];
-#pragma unroll
-        for (int j = 0; j < WC; ++j)
-#pragma unroll
-            for (int t = 0; t < 3; ++t)          // hi.hi, hi.lo, lo.hi
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const int p = t == 2 ? 1 : 0;
-                    const u32x4 y = t == 1 ? bl[j] : bh[j];
-                    accR[k][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(bf16x8, A[0][k][p]), __builtin_bit_cast(bf16x8, y), accR[k][i][j], 0, 0, 0);
-                    accI[k][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(bf16x8, A[1][k][p]), __builtin_bit_cast(bf16x8, y), accI[k][i][j], 0, 0, 0);
+            for (int e = 0; e < 4; ++e) {
+                const int p = KP * (k0 + k) + 4 * lg + e;
+                int r1, r0;
+                float2 v = make_float2(0.f, 0.f);
+                if (pair_rows(a, p, r1, r0)) {
+                    v = cis((uint64_t)(p + a.center) * at.ra + hs);
+                    const float d = __builtin_amdgcn_exp2f(bl2[i] * sq[r1]);
+                    v = make_float2(v.x * d, v.y * d);
                 }
-    }
-}
-
-__global__ void __launch_bounds__(NT) adjoint_split_kernel(AdjArgs a) {
-    __shared__ AdSmemS sm;
-    const int4 tile = a.tiles[blockIdx.y];
-    const int atom0 = tile.x, na = tile.y - tile.x;
-    const float *sq = a.sq + (long long)tile.w * a.sq_stride;
-    const uint32_t *qh = a.qs + (long long)tile.z * 2 * a.Rg * a.C * 4;
-    const uint32_t *ql = qh + (long long)a.Rg * a.C * 4;
-    const int col0 = blockIdx.x * NC;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-    const int wa0 = (wave % NWA) * 16 * WA, wc0 = (wave / NWA) * 16 * WC;
-
-    for (int x = threadIdx.x; x < NA; x += NT) {
-        AtomRec r{};
-        if (x < na) r = a.rec[atom0 + x];
-        sm.at[x] = r;
-    }
-    __syncthreads();
-
-    f32x4 accR[3][WA][WC], accI[3][WA][WC];
+                uint32_t w[NP];
+                split<NP>(v.x, v.y, w);
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-        for (int i = 0; i < WA; ++i)
-#pragma unroll
-            for (int j = 0; j < WC; ++j) {
-                accR[k][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-                accI[k][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int q = 0; q < NP; ++q) A[k][i][q][e] = w[q];
             }
-
-    const int nst = (a.R + SKR - 1) / SKR;
-    const bool tab = nst <= MAXST;
-    if (tab) build_row_tables(sm.rt, sm.at, nst);
-    __syncthreads();
-    u32x4 bh[WC], bl[WC], nbh[WC], nbl[WC];
-    load_bwords(qh, ql, a, col0 + wc0, 0, bh, bl);
-    gen_stage_split(sm.a[0], sm.rt, sm.at, a, sq, 0, na, tab);
-    __syncthreads();
-    for (int s = 0; s < nst; ++s) {
-        const int buf = s & 1;
-        if (s + 1 < nst) {
-            load_bwords(qh, ql, a, col0 + wc0, s + 1, nbh, nbl);
-            gen_stage_split(sm.a[buf ^ 1], sm.rt, sm.at, a, sq, s + 1, na, tab);
-        }
-        split_mfma_stage(sm.a[buf], bh, bl, accR, accI, wa0);
-        if (s + 1 < nst) {
+        ph[i] = at.p0 + hs + (a.fold ? (uint64_t)((a.R - 1) / 2) * at.ra : 0);
+        ca[i] = at.ca;
+        ca1[i] = at.ca1;
+        cen[i] = __builtin_amdgcn_exp2f(bl2[i] * s2c);
+        rot[i] = cis(CT * at.ca);
+        wrap[i] = cis(at.ca1 - (uint64_t)a.C0 * at.ca);
 #pragma unroll
-            for (int j = 0; j < WC; ++j) {
-                bh[j] = nbh[j];
-                bl[j] = nbl[j];
-            }
-        }
-        __syncthreads();
+        for (int v = 0; v < 4; ++v) tl[i][v] = cis((uint64_t)v * at.ca);
     }
-    adjoint_epilogue(a, sq, sm.at, sm.red, sm.ct, accR, accI, col0, atom0, na);
-}
+    const bool damp = __any(bl2[0] != 0.0f || bl2[1] != 0.0f);
+    static_assert(WA == 2, "damp");
 
-// Split adjoint for short grids (R <= 16 RES_ST rows): the work-group makes
-// A for every stage once, keeps it in LDS, and walks a range of a.ctpg column
-// tiles.  The stages of one column tile run without barriers (A is read-only,
-// B streams into registers one stage ahead, also across column tiles); the
-// epilogue's column sums accumulate per lane over the whole range, so the
-// partial set is the column range (blockIdx.x), not the column tile.
-constexpr int RES_ST = 5;
-constexpr int RES_MAXCT = 32;   // column tiles per work-group at most (bounds the FP32 column sums)
-
-// Epilogue of one column tile of a walk: column tables, contraction, and the
-// row totals added into the lane's running sums tot (entries 3 li .. 3 li + 2).
-__device__ __forceinline__ void walk_tile_epilogue(const AdjArgs &a, const float *__restrict__ sq, const AtomRec *at,
-                                                   ColTables &ct, const f32x4 (&accR)[3][WA][WC],
-                                                   const f32x4 (&accI)[3][WA][WC], int col0, float (&tot)[3]) {
-    const int li = threadIdx.x & 15;
-    __syncthreads();   // the previous tile's contraction has read the column tables
-    epi_tables(a, at, ct, col0);
-    __syncthreads();
-    float acc[WA][4][6];
+    double tot[WA][6];
 #pragma unroll
     for (int i = 0; i < WA; ++i)
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
+        for (int k = 0; k < 6; ++k) tot[i][k] = 0.0;
+    // words of (column tile, k-step): contiguous over the chunk's steps, then a
+    // jump over the other chunks' to the next column tile
+    const u32x4 *src = words + (((long long)(tile.z - plane0) * a.ctiles + ct0) * a.nkt + k0) * (NW * 64);
+    const long long jump = (long long)(a.nkt - NK + 1) * (NW * 64);
+    const float *scales = reinterpret_cast<const float *>(words + (long long)nplane * a.ctiles * a.nkt * (NW * 64)) +
+                          (long long)(tile.z - plane0) * a.ctiles;
+    u32x4 reg[LD];
+    auto fetch = [&]() {
 #pragma unroll
-            for (int k = 0; k < 6; ++k) acc[i][v][k] = 0.0f;
-    epi_contract(a, sq, at, ct, accR, accI, col0, acc);
-    float part[3];
-    row_reduce_scatter(acc, part, li);
+        for (int u = 0; u < LD; ++u)
+            if (AW * (u + 1) <= NW || wave + AW * u < NW) reg[u] = src[(wave + AW * u) * 64 + lane];
+    };
+    auto put = [&](int buf) {
 #pragma unroll
-    for (int q = 0; q < 3; ++q) tot[q] += part[q];
-}
-
-// End of a walk: the lanes' totals into the per-wave slots, summed over the
-// waves in order and written as partial set blockIdx.x.
-__device__ __forceinline__ void walk_finish(const AdjArgs &a, float (&red)[NWC][NA][6], const float (&tot)[3], int atom0,
-                                            int na) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-    const int wa0 = (wave % NWA) * 16 * WA;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        const int f = 3 * li + q, i = f / 24, v = (f / 6) % 4, k = f % 6;
-        red[wave / NWA][wa0 + 16 * i + 4 * lg + v][k] = tot[q];
+        for (int u = 0; u < LD; ++u)
+            if (AW * (u + 1) <= NW || wave + AW * u < NW) sq_w[buf][wave + AW * u][lane] = reg[u];
+    };
+    // the next tile's column values likewise, a tile ahead (threads 0..15)
+    float csq = 0.0f;
+    float2 cq = make_float2(0.f, 0.f);
+    int cj = 0, cm = 0;
+    auto fetch_col = [&](int ct) {
+        const int c = ct * CT + (int)threadIdx.x;
+        cj = c % a.C0;
+        cm = c / a.C0;
+        const bool in = threadIdx.x < CT && c < a.C && cj < a.f1;
+        csq = in ? sq[a.R + c] : 0.0f;
+        cq = in && center ? a.q[tile.z * a.plane + c + (long long)a.C * (a.R / 2)] : make_float2(0.f, 0.f);
+        if constexpr (NP == 2)
+            if (in) {
+                const float scale = scales[ct];
+                cq = make_float2(cq.x * scale, cq.y * scale);
+            }
+    };
+    auto put_col = [&](int ct) {
+        if (threadIdx.x < CT) {
+            col[ct & 1][threadIdx.x] = make_float4(csq, (float)cj - a.jc, (float)cm - a.mc, csq * sg[2]);
+            qcen[ct & 1][threadIdx.x] = cq;
+        }
+    };
+    if (ct0 < ct1) {
+        fetch();
+        fetch_col(ct0);
+        put(0);
+        put_col(ct0);
     }
     __syncthreads();
-    epi_write(a, red, blockIdx.x, atom0, na);
-}
-
-struct AdSmemR {
-    StageA a[RES_ST];
-    AtomRec at[NA];
-    float red[NWC][NA][6];
-    ColTables ct;
-    RowTablesT<RES_ST> rt;
-};
-
-__global__ void __launch_bounds__(NT) adjoint_split_res_kernel(AdjArgs a) {
-    __shared__ AdSmemR sm;
-    const int4 tile = a.tiles[blockIdx.y];
-    const int atom0 = tile.x, na = tile.y - tile.x;
-    const float *sq = a.sq + (long long)tile.w * a.sq_stride;
-    const uint32_t *qh = a.qs + (long long)tile.z * 2 * a.Rg * a.C * 4;
-    const uint32_t *ql = qh + (long long)a.Rg * a.C * 4;
-    const int ntc = (a.C + NC - 1) / NC;
-    const int ct0 = blockIdx.x * a.ctpg, ct1 = min(ntc, ct0 + a.ctpg);
-    const int wave = threadIdx.x >> 6;
-    const int wa0 = (wave % NWA) * 16 * WA, wc0 = (wave / NWA) * 16 * WC;
-
-    for (int x = threadIdx.x; x < NA; x += NT) {
-        if (x < na)
-            sm.at[x] = a.rec[atom0 + x];
-        else
-            sm.at[x] = AtomRec{};
-    }
-    __syncthreads();
-    const int nst = (a.R + SKR - 1) / SKR;   // <= RES_ST, checked by the launcher
-    build_row_tables(sm.rt, sm.at, nst);
-    __syncthreads();
-    for (int s = 0; s < nst; ++s) gen_stage_split(sm.a[s], sm.rt, sm.at, a, sq, s, na, true);
-    u32x4 bh[WC], bl[WC], nbh[WC], nbl[WC];
-    if (ct0 < ct1) load_bwords(qh, ql, a, ct0 * NC + wc0, 0, bh, bl);
-    __syncthreads();
-
-    float tot[3] = {0.0f, 0.0f, 0.0f};   // row totals of flat entries 3 li .. 3 li + 2, over the column range
+    int buf = 0;
+    float2 th[WA];
     for (int ct = ct0; ct < ct1; ++ct) {
-        f32x4 accR[3][WA][WC], accI[3][WA][WC];
+        f32x4 acc[6][WA];
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
+        for (int x = 0; x < 6; ++x)
 #pragma unroll
-            for (int i = 0; i < WA; ++i)
+            for (int i = 0; i < WA; ++i) acc[x][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int j = 0; j < WC; ++j) {
-                    accR[k][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-                    accI[k][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-                }
-        for (int s = 0; s < nst; ++s) {
-            // next (column tile, stage) of the walk
-            const int nct = s + 1 < nst ? ct : ct + 1, ns = s + 1 < nst ? s + 1 : 0;
-            const bool more = nct < ct1;
-            if (more) load_bwords(qh, ql, a, nct * NC + wc0, ns, nbh, nbl);
-            split_mfma_stage(sm.a[s], bh, bl, accR, accI, wa0);
-            if (more) {
+        for (int k = 0; k < NK; ++k) {
+            // (the last step of the range fetches its own words again)
+            src += k + 1 < NK ? NW * 64 : ct + 1 < ct1 ? jump : 0;
+            fetch();
+            if (k == 0) fetch_col(ct + 1);
+            if (active) {
 #pragma unroll
-                for (int j = 0; j < WC; ++j) {
-                    bh[j] = nbh[j];
-                    bl[j] = nbl[j];
+                for (int x = 0; x < 6; ++x) {
+                    u32x4 w[NP];
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) w[p] = sq_w[buf][x * NP + p][lane];
+                    // the small products first
+#pragma unroll
+                    for (int s = NP - 1; s >= 0; --s)
+#pragma unroll
+                        for (int p = s; p >= 0; --p)
+#pragma unroll
+                            for (int i = 0; i < WA; ++i)
+                                acc[x][i] = mfma<NP>(w[p], A[k][i][s - p], acc[x][i]);
                 }
             }
+            put(buf ^ 1);
+            if (k == NK - 1) put_col(ct + 1);
+            buf ^= 1;
+            __syncthreads();
         }
-        walk_tile_epilogue(a, sq, sm.at, sm.ct, accR, accI, ct * NC, tot);
-    }
-    walk_finish(a, sm.red, tot, atom0, na);
-}
-
-// FP32 adjoint for short grids, the same walk: the FP32 A elements of every
-// stage (20 KB for 5 stages) stay in LDS, and each lane loads its Q operands
-// (row 2 ks + lg / 2 of the stage, column li of each 16-column tile) from L2
-// into registers: each k-step's slot is refilled with the next (column tile,
-// stage) as soon as its MFMAs have read it, a stage ahead of use.
-struct AdSmemRF {
-    float a[RES_ST][KP][NA];   // A(k', atom), k' = 2 rr + (0 re, 1 im)
-    float sr[RES_ST][KR];
-    AtomRec at[NA];
-    float red[NWC][NA][6];
-    ColTables ct;
-    RowTablesT<RES_ST> rt;
-};
-
-__device__ __forceinline__ void load_qslot(const AdjArgs &a, long long qbase, int cw, int st, int ks, float2 (&q)[WC]) {
-    const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+        if (!active) continue;
+        // contraction with the column factors: lane holds columns 4 lg + v
+        const int cb = ct * CT + 4 * lg, j0 = cb % a.C0, m0 = cb / a.C0;
+        if ((ct - ct0) % RESYNC == 0) {
 #pragma unroll
-    for (int j = 0; j < WC; ++j) {
-        const int r = st * KR + 2 * ks + (lg >> 1), col = cw + 16 * j + li;
-        q[j] = (r < a.R && col < a.C) ? a.q[qbase + col + (long long)a.C * r] : make_float2(0.f, 0.f);
-    }
-}
-
-__global__ void __launch_bounds__(NT) adjoint_res_kernel(AdjArgs a) {
-    __shared__ AdSmemRF sm;
-    const int4 tile = a.tiles[blockIdx.y];
-    const int atom0 = tile.x, na = tile.y - tile.x;
-    const long long qbase = (long long)tile.z * a.plane;
-    const float *sq = a.sq + (long long)tile.w * a.sq_stride;
-    const int ntc = (a.C + NC - 1) / NC;
-    const int ct0 = blockIdx.x * a.ctpg, ct1 = min(ntc, ct0 + a.ctpg);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-    const int wa0 = (wave % NWA) * 16 * WA, wc0 = (wave / NWA) * 16 * WC;
-    const bool im = (lg & 1) != 0;
-
-    for (int x = threadIdx.x; x < NA; x += NT) {
-        if (x < na)
-            sm.at[x] = a.rec[atom0 + x];
-        else
-            sm.at[x] = AtomRec{};
-    }
-    __syncthreads();
-    const int nst = (a.R + KR - 1) / KR;   // <= RES_ST, checked by the launcher
-    build_row_tables(sm.rt, sm.at, nst);
-    __syncthreads();
-    for (int s = 0; s < nst; ++s) {
-        const int t = threadIdx.x, at = t & (NA - 1), rr = t / NA;   // NT == NA * KR
-        const int r = s * KR + rr;
-        float2 v = make_float2(0.f, 0.f);
-        if (r < a.R && at < na) v = row_element(sm.rt, sm.at[at], at, s, rr, r, true, sq[r]);
-        sm.a[s][2 * rr][at] = v.x;
-        sm.a[s][2 * rr + 1][at] = v.y;
-        if (t < KR) sm.sr[s][t] = s * KR + t < a.R ? sq[s * KR + t] : 0.0f;
-    }
-    float2 qr[KR / 2][WC];
-    if (ct0 < ct1)
+            for (int i = 0; i < WA; ++i) th[i] = cis(ph[i] + (uint64_t)j0 * ca[i] + (uint64_t)m0 * ca1[i]);
+        } else {
 #pragma unroll
-        for (int ks = 0; ks < KR / 2; ++ks) load_qslot(a, qbase, ct0 * NC + wc0, 0, ks, qr[ks]);
-    __syncthreads();
-
-    float tot[3] = {0.0f, 0.0f, 0.0f};
-    for (int ct = ct0; ct < ct1; ++ct) {
-        f32x4 accR[3][WA][WC], accI[3][WA][WC];
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-#pragma unroll
-            for (int i = 0; i < WA; ++i)
-#pragma unroll
-                for (int j = 0; j < WC; ++j) {
-                    accR[k][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-                    accI[k][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-                }
-        for (int s = 0; s < nst; ++s) {
-            const int nct = s + 1 < nst ? ct : ct + 1, ns = s + 1 < nst ? s + 1 : 0;
-            const bool more = nct < ct1;
-#pragma unroll
-            for (int ks = 0; ks < KR / 2; ++ks) {
-                const int rr = 2 * ks + (lg >> 1);
-                const float wr = (float)(s * KR + rr) - a.rc;
-                const float ws = sm.sr[s][rr];
-                float av[WA][3];
-#pragma unroll
-                for (int i = 0; i < WA; ++i) {
-                    const float x = sm.a[s][4 * ks + lg][wa0 + 16 * i + li];
-                    av[i][0] = x;
-                    av[i][1] = x * wr;
-                    av[i][2] = x * ws;
-                }
-#pragma unroll
-                for (int j = 0; j < WC; ++j) {
-                    const float2 b = qr[ks][j];
-                    const float bR = im ? -b.y : b.x;
-                    const float bI = im ? b.x : b.y;
-#pragma unroll
-                    for (int i = 0; i < WA; ++i)
-#pragma unroll
-                        for (int k = 0; k < 3; ++k) {
-                            accR[k][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][k], bR, accR[k][i][j], 0, 0, 0);
-                            accI[k][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][k], bI, accI[k][i][j], 0, 0, 0);
-                        }
-                }
-                if (more) load_qslot(a, qbase, nct * NC + wc0, ns, ks, qr[ks]);
+            for (int i = 0; i < WA; ++i) {
+                th[i] = cmul(th[i], rot[i]);
+                const float2 t = cmul(th[i], wrap[i]);
+                th[i] = j0 < CT ? t : th[i];   // the lane's columns began a new run since the last tile
             }
         }
-        walk_tile_epilogue(a, sq, sm.at, sm.ct, accR, accI, ct * NC, tot);
-    }
-    walk_finish(a, sm.red, tot, atom0, na);
-}
-
-// FP32 complex Q planes -> split words: for plane t, part (hi, lo), row
-// group g (rows 4g..4g+3) and column c one 16-byte word of 4 packed pairs.
-__global__ void q_split_kernel(const float2 *__restrict__ q, int nq, int R, int C, long long plane, int Rg,
-                               uint32_t *__restrict__ qs) {
-    const long long n = (long long)nq * Rg * C;
-    for (long long x = (long long)blockIdx.x * blockDim.x + threadIdx.x; x < n; x += (long long)gridDim.x * blockDim.x) {
-        const int c = (int)(x % C);
-        const long long y = x / C;
-        const int g = (int)(y % Rg);
-        const long long t = y / Rg;
-        u32x4 hi, lo;
+        float inv = 1.0f;
+        if constexpr (NP == 2) inv = 1.0f / scales[ct];   // a power of two: exact
+        float4 w[4];
+        float2 qc[4];
+        float d[WA][4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int r = 4 * g + e;
-            const float2 v = r < R ? q[t * plane + c + (long long)C * r] : make_float2(0.f, 0.f);
-            uint32_t h, l;
-            bsplit(v.x, v.y, h, l);
-            hi[e] = h;
-            lo[e] = l;
+        for (int v = 0; v < 4; ++v) {
+            w[v] = col[ct & 1][4 * lg + v];
+            qc[v] = qcen[ct & 1][4 * lg + v];
+#pragma unroll
+            for (int i = 0; i < WA; ++i) d[i][v] = 1.0f;
         }
-        uint32_t *base = qs + t * 2 * Rg * (long long)C * 4;
-        *reinterpret_cast<u32x4 *>(base + ((long long)g * C + c) * 4) = hi;
-        *reinterpret_cast<u32x4 *>(base + ((long long)(Rg + g) * C + c) * 4) = lo;
+        if (damp)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+                for (int i = 0; i < WA; ++i) d[i][v] = __builtin_amdgcn_exp2f(bl2[i] * w[v].x);
+#pragma unroll
+        for (int i = 0; i < WA; ++i) {
+            const float2 thw = cmul(th[i], wrap[i]);
+            float s[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                float2 b = cmul(j0 + v >= a.C0 ? thw : th[i], tl[i][v]);
+                b = make_float2(b.x * d[i][v], b.y * d[i][v]);
+                const float qr = cen[i] * qc[v].x, qi = cen[i] * qc[v].y;
+                const float z0r = acc[0][i][v] + qr, z0i = acc[1][i][v] + qi;
+                const float z2r = acc[4][i][v] + s2cs * qr, z2i = acc[5][i][v] + s2cs * qi;
+                const float tr = z0r * b.x - z0i * b.y;
+                const float ti = z0r * b.y + z0i * b.x;
+                s[0] += tr;
+                s[1] += ti;
+                s[2] += acc[2][i][v] * b.y + acc[3][i][v] * b.x;
+                s[3] += w[v].y * ti;
+                s[4] += w[v].z * ti;
+                s[5] += (z2r * b.x - z2i * b.y) + w[v].w * tr;
+            }
+#pragma unroll
+            for (int k = 0; k < 6; ++k) tot[i][k] += (double)(NP == 2 ? s[k] * inv : s[k]);
+        }
+    }
+    if (!active) return;
+#pragma unroll
+    for (int i = 0; i < WA; ++i) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            tot[i][k] += __shfl_xor(tot[i][k], 16);
+            tot[i][k] += __shfl_xor(tot[i][k], 32);
+        }
+        tot[i][2] /= (double)sg[1];
+        tot[i][5] /= (double)sg[2];
+        if (lg == 0 && n0 + 16 * i < tile.y) {
+            double *out = a.part + ((long long)blockIdx.x * a.natoms + n0 + 16 * i) * 6;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) out[k] = tot[i][k];
+        }
     }
 }
 
-// Column-tile partials -> gradients in the caller's atom order (FP64).
+// Partial sets -> gradients in the caller's atom order (FP64).
 __global__ void adjoint_finish_kernel(AdjFinishArgs a) {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= a.natoms) return;
     double s[6] = {0, 0, 0, 0, 0, 0};
-    for (int t = 0; t < a.ntile_c; ++t) {
-        const float *p = a.part + ((long long)t * a.natoms + n) * 6;
-        for (int k = 0; k < 6; ++k) s[k] += (double)p[k];
+    for (int t = 0; t < a.nset; ++t) {
+        const double *p = a.part + ((long long)t * a.natoms + n) * 6;
+        for (int k = 0; k < 6; ++k) s[k] += p[k];
     }
     const long long ci = a.idx[n];
     const double o = a.occ[ci];
@@ -991,13 +680,7 @@ hipError_t launch_fill_zero(double *p, long long n, hipStream_t st) {
 }
 
 int adjoint_tile_atoms() { return NA; }
-int adjoint_tile_cols() { return NC; }
-
-// Short grids (R <= 16 RES_ST, every scheme) walk column ranges with A
-// resident in LDS; one such work-group fills a CU, so the walk length is
-// chosen to balance rounds of work-groups over the CUs against the per-group
-// prologue (about half a column tile of work).
-int adjoint_max_walk() { return RES_MAXCT; }
+int adjoint_max_walk() { return MAX_WALK; }
 
 int device_cu_count() {
     static std::atomic<int> cus[64];
@@ -1013,58 +696,73 @@ int device_cu_count() {
     return ncu;
 }
 
-int adjoint_plan(AdjArgs &a, int ntiles, bool split, int force) {
-    const int ntc = std::max(1, (a.C + NC - 1) / NC);
-    a.ctpg = 1;
-    (void)split;
-    if (ntiles <= 0 || a.R <= 0 || (a.R + SKR - 1) / SKR > RES_ST) return ntc;
+void adjoint_plan(AdjArgs &a, int ntiles, bool split, int force) {
+    a.parts = split ? 2 : 3;
+    int pairs = a.fold ? (a.R + 1) / 2 : a.R;
+    a.center = a.fold && (a.R & 1) && pairs > 1 && pairs % KP == 1;
+    pairs -= a.center;
+    const int ks = std::max(1, (pairs + KP - 1) / KP), maxk = max_ksteps(a.parts);
+    a.chunks = (ks + maxk - 1) / maxk;
+    a.nk = (ks + a.chunks - 1) / a.chunks;
+    a.nkt = a.chunks * a.nk;
+    a.ctiles = std::max(1, (a.C + CT - 1) / CT);
+    a.tpg = a.ctiles;
     if (force > 0) {
-        a.ctpg = std::min({force, ntc, RES_MAXCT});
-        return (ntc + a.ctpg - 1) / a.ctpg;
-    }
-    const int ncu = device_cu_count();
-    double best = 0.0;
-    int bestc = 0;
-    for (int ctpg = std::min(ntc, RES_MAXCT); ctpg >= 1; --ctpg) {
-        const long long groups = (ntc + ctpg - 1) / ctpg;
-        const double rounds = (double)((groups * ntiles + ncu - 1) / ncu);
-        const double cost = rounds * (ctpg + 0.5);
-        if (bestc == 0 || cost < best) {
-            best = cost;
-            bestc = ctpg;
+        a.tpg = std::min(a.ctiles, force * WALK_TILES);
+    } else if (ntiles > 0) {
+        // Two work-groups fit a CU; a range costs its tiles and a prologue
+        // (A operands, tables) worth about one tile.
+        const long long slots = 2LL * device_cu_count(), items = (long long)ntiles * a.chunks;
+        double best = 0.0;
+        for (int g = 1; g <= std::min(a.ctiles, MAX_GROUPS); ++g) {
+            const int tpg = (a.ctiles + g - 1) / g;
+            if ((a.ctiles + tpg - 1) / tpg != g) continue;
+            const double cost = (double)((items * g + slots - 1) / slots) * (tpg + 1.0);
+            if (g == 1 || cost < best) {
+                best = cost;
+                a.tpg = tpg;
+            }
         }
     }
-    a.ctpg = bestc;
-    return (ntc + bestc - 1) / bestc;
+    a.groups = (a.ctiles + a.tpg - 1) / a.tpg;
+    a.nset = a.groups * a.chunks;
+    a.walk = (a.tpg + WALK_TILES - 1) / WALK_TILES;
+    a.plane_words = (long long)a.ctiles * a.nkt * 6 * a.parts * 64 + (a.ctiles + 3) / 4;   // and the tiles' scales
 }
 
-hipError_t launch_adjoint(const AdjArgs &a, int ntiles, hipStream_t st, bool split) {
-    if (ntiles <= 0 || a.R <= 0 || a.C <= 0) return hipSuccess;
-    const int ntc = (a.C + NC - 1) / NC;
-    if (a.ctpg < 1 || a.ctpg > RES_MAXCT || (a.ctpg > 1 && (a.R + SKR - 1) / SKR > RES_ST)) return hipErrorInvalidValue;
-    dim3 grid(ntc, ntiles);
-    if (split && (!a.qs || a.Rg * 4 < a.R || a.Rg % 4)) return hipErrorInvalidValue;
-    if (a.ctpg > 1) {
-        grid.x = (ntc + a.ctpg - 1) / a.ctpg;
-        if (split)
-            adjoint_split_res_kernel<<<grid, dim3(NT), 0, st>>>(a);
-        else
-            adjoint_res_kernel<<<grid, dim3(NT), 0, st>>>(a);
-    } else if (split) {
-        adjoint_split_kernel<<<grid, dim3(NT), 0, st>>>(a);
+hipError_t launch_adjoint(const AdjArgs &a, const AdjSpan &s, uint4 *words, hipStream_t st) {
+    if (s.ntiles <= 0 || a.R <= 0 || a.C <= 0) return hipSuccess;
+    if (!words || a.f1 < 1 || a.C0 < a.f1 || (a.C > a.C0 && a.C0 < CT) || a.nk < 1 || a.nk > max_ksteps(a.parts) ||
+        a.nk * a.chunks != a.nkt || a.nkt * KP < (a.fold ? (a.R + 1) / 2 - a.center : a.R) || a.tpg < 1 ||
+        a.groups * a.tpg < a.ctiles || a.planes_per_sq < 1 || s.ntiles > 65535)
+        return hipErrorInvalidValue;
+    u32x4 *w = reinterpret_cast<u32x4 *>(words);
+    const unsigned nb = (unsigned)std::min<long long>((long long)s.nplanes * a.ctiles, 8192);
+    const dim3 grid(a.nset, s.ntiles);
+    auto run = [&](auto kernel) { kernel<<<grid, NT, 0, st>>>(a, s.tile0, s.plane0, s.nplanes, w); };
+    if (a.parts == 2) {
+        adj_words_kernel<2><<<nb, 256, 0, st>>>(a, s.plane0, s.nplanes, w);
+        a.nk == 1 ? run(adjoint_kernel<2, 1>) : a.nk == 2 ? run(adjoint_kernel<2, 2>) : a.nk == 3 ? run(adjoint_kernel<2, 3>)
+            : a.nk == 4 ? run(adjoint_kernel<2, 4>) : run(adjoint_kernel<2, 5>);
     } else {
-        adjoint_kernel<<<grid, dim3(NT), 0, st>>>(a);
+        adj_words_kernel<3><<<nb, 256, 0, st>>>(a, s.plane0, s.nplanes, w);
+        a.nk == 1 ? run(adjoint_kernel<3, 1>) : a.nk == 2 ? run(adjoint_kernel<3, 2>) : run(adjoint_kernel<3, 3>);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_q_split(const float2 *q, int nq, int R, int C, long long plane, int Rg, uint32_t *qs,
-                          hipStream_t st) {
-    const long long n = (long long)nq * Rg * C;
-    if (n <= 0) return hipSuccess;
-    const long long nb = std::min<long long>((n + 255) / 256, 8192);
-    q_split_kernel<<<(unsigned)nb, 256, 0, st>>>(q, nq, R, C, plane, Rg, qs);
-    return hipGetLastError();
+// Runs of planes whose words fit ADJ_WORDS_MAX together (one plane at least), with
+// their tiles, which are in plane order; 65,535 tiles a launch at most.
+std::vector<AdjSpan> adjoint_spans(const AdjArgs &a, const int *tiles, int ntiles) {
+    std::vector<AdjSpan> out;
+    const long long cap = std::max<long long>(1, ADJ_WORDS_MAX / (16 * std::max<long long>(a.plane_words, 1)));
+    for (int t = 0; t < ntiles; ++t) {
+        const int pl = tiles[4 * t + 2];
+        if (out.empty() || pl - out.back().plane0 >= cap || out.back().ntiles == 65535) out.push_back({pl, 1, t, 0});
+        out.back().nplanes = pl - out.back().plane0 + 1;
+        ++out.back().ntiles;
+    }
+    return out;
 }
 
 hipError_t launch_adjoint_finish(const AdjFinishArgs &a, hipStream_t st) {

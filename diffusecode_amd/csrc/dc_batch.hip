@@ -37,8 +37,9 @@ struct BatchState {
     std::vector<std::pair<int, int>> segs;   // (type, atoms) per member and type, member-major
     std::vector<int> seg_member;
     int kchunk = 0;                          // atoms per GEMM slice
-    int nsorted = 0, nslice = 0, ntiles = 0, ntc = 0, nblk = 0;
-    int walk = 1, nset = 0;              // adjoint column tiles per work-group, partial sets
+    int nsorted = 0, nslice = 0, ntiles = 0, nblk = 0;
+    AdjArgs adj{};                       // plan of the reverse pass, and its launches
+    std::vector<AdjSpan> spans;
     int walk_req = 0;                    // the context's adjoint walk setting at planning
     int64_t natoms = 0;
     int rows = 0;                        // form-factor rows on the device (the bins the metrics reach, and a margin)
@@ -262,14 +263,14 @@ int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
         off += segs_all[sg].second;
     }
     b.ntiles = (int)tiles.size() / 4;
-    b.ntc = (gg.C + adjoint_tile_cols() - 1) / adjoint_tile_cols();
-    {
-        AdjArgs pa{};
-        pa.R = gg.R;
-        pa.C = gg.C;
-        b.nset = adjoint_plan(pa, b.ntiles, b.prec != DC_PREC_FP32, c->adj_walk);
-        b.walk = pa.ctpg;
-    }
+    b.adj = AdjArgs{};
+    b.adj.R = gg.R;
+    b.adj.C = gg.C;
+    b.adj.C0 = gg.C0;
+    b.adj.f1 = g.f[1];
+    b.adj.fold = (b.fold_mask & FOLD_ROWS) != 0;
+    adjoint_plan(b.adj, b.ntiles, b.prec != DC_PREC_FP32, c->adj_walk);
+    b.spans = adjoint_spans(b.adj, tiles.data(), b.ntiles);
     b.nblk = (int)std::min<long long>((g.P + 255) / 256, 256);
 
     int st;
@@ -287,13 +288,10 @@ int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
     if ((st = ensure(c, b.chi, sizeof(double) * (size_t)b.nblk * M))) return st;
     if (b.want_grad) {
         if ((st = ensure(c, b.q, sizeof(float2) * gg.P * d->nscat * M))) return st;
-        // padded columns of the Q planes are never written: zero them once
-        HIPCHK(hipMemsetAsync(b.q.p, 0, sizeof(float2) * gg.P * d->nscat * M, c->st));
-        if ((st = ensure(c, b.part, sizeof(float) * 6 * (size_t)b.ntc * std::max(b.nsorted, 1)))) return st;
-        if (c->prec != DC_PREC_FP32) {
-            const size_t rg = (size_t)((gg.R + 15) / 16) * 4;
-            if ((st = ensure(c, b.qs, sizeof(uint32_t) * 8 * rg * gg.C * d->nscat * M))) return st;
-        }
+        if ((st = ensure(c, b.part, sizeof(double) * 6 * (size_t)b.adj.nset * std::max(b.nsorted, 1)))) return st;
+        long long most = 0;
+        for (const AdjSpan &s : b.spans) most = std::max<long long>(most, s.nplanes);
+        if ((st = ensure(c, b.qs, sizeof(uint4) * (size_t)(b.adj.plane_words * most)))) return st;
     }
     return 0;
 }
@@ -391,33 +389,23 @@ int enqueue(dc_ctx *c, BatchState &b, const StepIO &io, int tile, int nwg, bool 
     HIPCHK(hipGetLastError());
     if (b.want_grad) {
         HIPCHK(launch_fill_zero(io.grad, 5 * b.natoms, c->st));
-        AdjArgs aa{};
+        AdjArgs aa = b.adj;
         aa.rec = ptr<AtomRec>(b.rec);
         aa.tiles = ptr<int4>(b.atiles);
         aa.q = ptr<float2>(b.q);
         aa.sq = ptr<float>(b.sq);
         aa.sq_stride = gg.R + gg.C;
-        aa.part = ptr<float>(b.part);
-        aa.R = gg.R;
-        aa.C = gg.C;
-        aa.C0 = gg.C0;
-        aa.f1 = b.g.f[1];
+        aa.planes_per_sq = b.nscat;
+        aa.part = ptr<double>(b.part);
         aa.plane = gg.P;
         aa.natoms = b.nsorted;
         aa.rc = 0.5f * (float)(b.g.f[0] - 1);
         aa.jc = 0.5f * (float)(b.g.f[1] - 1);
         aa.mc = 0.5f * (float)(b.g.f[2] - 1);
-        const bool split = b.prec != DC_PREC_FP32;
-        if (split) {
-            aa.Rg = (gg.R + 15) / 16 * 4;
-            aa.qs = ptr<uint32_t>(b.qs);
-            HIPCHK(launch_q_split(ptr<float2>(b.q), b.nmembers * b.nscat, gg.R, gg.C, gg.P, aa.Rg, ptr<uint32_t>(b.qs), c->st));
-        }
-        aa.ctpg = b.walk;
-        HIPCHK(launch_adjoint(aa, b.ntiles, c->st, split));
+        for (const AdjSpan &s : b.spans) HIPCHK(launch_adjoint(aa, s, ptr<uint4>(b.qs), c->st));
         AdjFinishArgs fa{};
-        fa.part = ptr<float>(b.part);
-        fa.ntile_c = b.nset;
+        fa.part = ptr<double>(b.part);
+        fa.nset = b.adj.nset;
         fa.natoms = b.nsorted;
         fa.idx = ptr<int>(b.idx);
         fa.occ = io.occ;
@@ -707,7 +695,7 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
     c->stats.gemm_launches = 1;
     c->stats.gemm_scheme = b.pl.scheme;
     c->stats.gemm_ms = b.tune_best_ms;
-    c->stats.adjoint_walk = want_grad ? b.walk : 0;
+    c->stats.adjoint_walk = want_grad ? b.adj.walk : 0;
     return DC_OK;
 }
 

@@ -31,7 +31,7 @@ struct dc_ctx {
     int tile = -1;                  // forced GEMM tile configuration, -1 = planned
     int autotune = 1;               // batch: time tile shapes on the first call of a shape
     int graphs = 1;                 // batch: capture the population step as a hipGraph
-    int adj_walk = 0;               // split adjoint column walk: 0 planned, else forced (short grids)
+    int adj_walk = 0;               // adjoint column walk: 0 planned, else forced
     int dither = 1;                 // per-atom phase rotation of the phase GEMM (dither_turn)
     int slice_atoms = 0;            // forced atoms per GEMM slice, 0 = planned
     BatchState *batch = nullptr;    // cached plan / buffers / graph of the last batch shape

@@ -1,6 +1,8 @@
 // dc_internal.h -- kernel argument blocks and launchers shared between the
 // kernel translation units and the C-ABI layer.
 #pragma once
+#include <vector>
+
 #include "dc_common.h"
 
 namespace dc {
@@ -142,22 +144,33 @@ hipError_t launch_istl(const Grid &g, int *out, hipStream_t st);
 // [Re S0, Im S0, Im S_r, Im S_j, Im S_m, Re S_s] to part[tile][atom][6].
 struct AdjArgs {
     const AtomRec *rec;     // type-grouped atoms (mapping 0 records, B_n in pad)
-    const int4 *tiles;      // atom tiles: (first, end, Q plane, member), each inside one type
-    const float2 *q;        // Q planes: q[t * plane + c + C * r] (column fastest)
+    const int4 *tiles;      // atom tiles in plane order: (first, end, Q plane, member), each inside one type
+    const float2 *q;        // Q planes: q[t * plane + c + C * r] (column fastest, c = j + C0 m)
     const float *sq;        // s^2 parts: R rows, then C columns (per member: + tile.w * sq_stride)
     long long sq_stride;
-    float *part;            // [partial set][natoms][6]: one set per column tile or column range
-    const uint32_t *qs;     // split scheme: Q as BF16 hi/lo words, per plane [hi|lo][row group][C][4 rows]
-    int Rg;                 // row groups of 4 rows in qs (R padded to a multiple of 16)
+    int planes_per_sq;      // Q planes of one member
+    double *part;           // [partial set][natoms][6]: one set per column range and row chunk
     int R, C, C0, f1;       // rows, padded columns, column period, valid columns per period
     long long plane;        // R * C
     int natoms;
     float rc, jc, mc;       // centres of the row / column index weights
-    int ctpg;               // column tiles per work-group (set by adjoint_plan; 1 = one tile each)
+    int fold;               // rows taken in mirrored pairs (s_r^2 mirrored, or no B)
+    // set by adjoint_plan
+    int parts;              // 16-bit parts of the operands: 3 (BF16) in FP32, 2 (FP16) in the split precisions
+    int center;             // the centre row of the pairs is added apart
+    int nkt, nk, chunks;    // k-steps of 16 row pairs: in all, per row chunk; chunks
+    int ctiles, tpg, groups;   // column tiles: in all, per range; ranges
+    int nset, walk;         // partial sets; column tiles of 256 per work-group
+    long long plane_words;  // 16-byte words of one plane: operands and scales
 };
+// A run of planes whose operand words are made and used by one launch.
+struct AdjSpan {
+    int plane0, nplanes, tile0, ntiles;
+};
+constexpr long long ADJ_WORDS_MAX = 1LL << 30;   // bytes of words made at a time (or one plane's)
 struct AdjFinishArgs {
-    const float *part;
-    int ntile_c, natoms;
+    const double *part;
+    int nset, natoms;
     const int *idx;         // sorted atom -> caller index
     const double *occ;      // caller-order occupancies
     double hc[3], v[9];     // h at the weight centres; grid increments vi(:,1..3)
@@ -215,20 +228,16 @@ struct JvpArgs {
 };
 hipError_t launch_jvp_reduce(const JvpArgs &a, hipStream_t st);
 int adjoint_tile_atoms();
-int adjoint_tile_cols();
-// Chooses the adjoint kernel's column walk for a.R, a.C and ntiles atom
-// tiles (sets a.ctpg) and returns the number of partial sets it writes
-// (<= ceil(C / adjoint_tile_cols())), which adjoint_finish sums.  force > 0
-// asks for that many column tiles per work-group where the walk applies.
-int adjoint_plan(AdjArgs &a, int ntiles, bool split, int force = 0);
+// Cuts the work of ntiles atom tiles (rows, columns, f1 and fold of a set): the
+// fields of a below "set by adjoint_plan".  force > 0 asks for column ranges of
+// that many 256-column tiles.
+void adjoint_plan(AdjArgs &a, int ntiles, bool split, int force = 0);
+std::vector<AdjSpan> adjoint_spans(const AdjArgs &a, const int *tiles, int ntiles);
 // Compute units of the current device (queried once per device; 256 if unknown).
 int device_cu_count();
 int adjoint_max_walk();
-// split = true: BF16x3 MFMA on qs (made by launch_q_split), else FP32 on q.
-hipError_t launch_adjoint(const AdjArgs &a, int ntiles, hipStream_t st, bool split = false);
-// FP32 complex Q planes (c + C r) -> BF16 hi/lo words for the split adjoint.
-hipError_t launch_q_split(const float2 *q, int nq, int R, int C, long long plane, int Rg, uint32_t *qs,
-                          hipStream_t st);
+// Operand words of the span's planes (room for nplanes * plane_words), then its tiles.
+hipError_t launch_adjoint(const AdjArgs &a, const AdjSpan &s, uint4 *words, hipStream_t st);
 hipError_t launch_adjoint_finish(const AdjFinishArgs &a, hipStream_t st);
 hipError_t launch_model_q(const QArgs &a, hipStream_t st);
 hipError_t launch_chi2_resid(const double *icalc, const double *tgt, const double *wt, long long n, double *gi,

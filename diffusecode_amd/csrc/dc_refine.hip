@@ -231,7 +231,6 @@ int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, double *grad
         a0 += n;
     }
     const int ntiles = (int)tiles.size() / 4;
-    const int ntc = (gg.C + adjoint_tile_cols() - 1) / adjoint_tile_cols();
 
     hipEvent_t e0, e1;
     if ((st = mark(c, e0))) return st;
@@ -240,10 +239,8 @@ int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, double *grad
     if ((st = stage(c, c->m_tiles, tiles.data(), tiles.size(), d_tiles))) return st;
     if ((st = stage_flush(c))) return st;
     if ((st = ensure(c, c->m_q, sizeof(float2) * gg.P * std::max(nq, 1)))) return st;
-    if ((st = ensure(c, c->m_part, sizeof(float) * 6 * (size_t)ntc * std::max(mp.nsorted, 1)))) return st;
     HIPCHK(launch_fill_zero(grad, 5 * m->natoms, c->st));
     if (ntiles > 0) {
-        HIPCHK(hipMemsetAsync(c->m_q.p, 0, sizeof(float2) * gg.P * nq, c->st));
         QArgs qa{};
         qa.g = mp.g;
         qa.R = gg.R;
@@ -264,7 +261,7 @@ int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, double *grad
         aa.tiles = reinterpret_cast<const int4 *>(d_tiles);
         aa.q = ptr<float2>(c->m_q);
         aa.sq = mp.d_sq;
-        aa.part = ptr<float>(c->m_part);
+        aa.planes_per_sq = std::max(nq, 1);
         aa.R = gg.R;
         aa.C = gg.C;
         aa.C0 = gg.C0;
@@ -274,20 +271,20 @@ int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, double *grad
         aa.rc = 0.5f * (float)(mp.g.f[0] - 1);
         aa.jc = 0.5f * (float)(mp.g.f[1] - 1);
         aa.mc = 0.5f * (float)(mp.g.f[2] - 1);
-        const bool split = c->prec != DC_PREC_FP32;
-        if (split) {
-            aa.Rg = (int)((gg.R + 15) / 16) * 4;
-            if ((st = ensure(c, c->m_qs, sizeof(uint32_t) * 8 * (size_t)aa.Rg * gg.C * nq))) return st;
-            aa.qs = ptr<uint32_t>(c->m_qs);
-            HIPCHK(launch_q_split(ptr<float2>(c->m_q), nq, gg.R, gg.C, gg.P, aa.Rg, ptr<uint32_t>(c->m_qs), c->st));
-        }
-        const int nset = adjoint_plan(aa, ntiles, split, c->adj_walk);
-        c->stats.adjoint_walk = aa.ctpg;
-        HIPCHK(launch_adjoint(aa, ntiles, c->st, split));
+        aa.fold = !mp.any_b || (mirrored_sides(gg, mp.sq.data()) & FOLD_ROWS);
+        adjoint_plan(aa, ntiles, c->prec != DC_PREC_FP32, c->adj_walk);
+        c->stats.adjoint_walk = aa.walk;
+        if ((st = ensure(c, c->m_part, sizeof(double) * 6 * (size_t)aa.nset * std::max(mp.nsorted, 1)))) return st;
+        aa.part = ptr<double>(c->m_part);
+        const std::vector<AdjSpan> spans = adjoint_spans(aa, tiles.data(), ntiles);
+        long long most = 0;
+        for (const AdjSpan &s : spans) most = std::max<long long>(most, s.nplanes);
+        if ((st = ensure(c, c->m_qs, sizeof(uint4) * (size_t)(aa.plane_words * most)))) return st;
+        for (const AdjSpan &s : spans) HIPCHK(launch_adjoint(aa, s, ptr<uint4>(c->m_qs), c->st));
 
         AdjFinishArgs fa{};
-        fa.part = ptr<float>(c->m_part);
-        fa.ntile_c = nset;
+        fa.part = ptr<double>(c->m_part);
+        fa.nset = aa.nset;
         fa.natoms = mp.nsorted;
         fa.idx = mp.idx;
         fa.occ = mp.occ;

@@ -378,9 +378,10 @@ int dc_batch_chi2_dev(dc_ctx *ctx, const dc_batch_desc *batch, const double *tar
  * the length, dc_set_autotune(ctx, 0) the whole plan. */
 int dc_set_autotune(dc_ctx *ctx, int on);
 int dc_set_graphs(dc_ctx *ctx, int on);
-/* Column walk of the reverse pass (every precision) on grids of at most 80
- * abscissa points (dc_model_vjp, dc_model_chi2, dc_batch_chi2): 0 (default)
- * plans it from the grid and the CU count; 1..32 forces that many column
+/* Column walk of the reverse pass (dc_model_vjp, dc_model_chi2,
+ * dc_batch_chi2): 0 (default)
+ * plans it from the grid and the CU count (in steps of 16 columns, reported
+ * rounded up); 1..32 forces that many column
  * tiles of 256 per work-group (1 = one work-group per column tile).  A tuning
  * knob with no counterpart in DISCUS; it changes the FP32 summation order of
  * the gradient partials, not the result beyond rounding.  Reported back in
