@@ -608,6 +608,7 @@ void dc_destroy(dc_ctx *c) {
     batch_release(c);
     post_release(c);
     nufft_release(c);
+    fft_release(c);
     for (DevBuf *b : c->buffers())
         if (b->p) (void)hipFree(b->p);
     for (PinBuf *b : {&c->h_arena, &c->h_out})

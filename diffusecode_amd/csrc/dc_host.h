@@ -3,6 +3,7 @@
 #pragma once
 #include <algorithm>
 #include <cstring>
+#include <map>
 #include <string>
 #include <utility>
 #include <vector>
@@ -13,6 +14,9 @@
 struct BatchState;   // dc_batch.hip
 struct PostState;    // dc_post.hip
 struct NufftState;   // dc_nufft.hip
+namespace dc {
+struct FftLen;       // dc_fft.h
+}
 
 struct DevBuf {
     void *p = nullptr;
@@ -37,6 +41,7 @@ struct dc_ctx {
     BatchState *batch = nullptr;    // cached plan / buffers / graph of the last batch shape
     PostState *post = nullptr;      // FFT plans and buffers of the post-processing calls
     NufftState *nufft = nullptr;    // fine grid, plans and buffers of the NUFFT technique
+    std::map<int, DevBuf> fft_tw;   // twiddles of the transform lengths used (dc_fft.h; 600 lengths, 10 KB each at most)
     std::string err;
     int err_typ = DC_ER_NONE;
     const volatile int *cancel = nullptr;
@@ -313,6 +318,8 @@ inline GemmGeom launch_geom(const dc_ctx *c, const GemmGeom &g) {
 }
 void batch_release(dc_ctx *c);   // frees the cached batch plan, buffers and graph
 void post_release(dc_ctx *c);    // frees the FFT plans and buffers of the post-processing calls
+int fft_table(dc_ctx *c, FftLen &f);   // f.tw, made on a length's first use
+void fft_release(dc_ctx *c);
 void nufft_release(dc_ctx *c);   // frees the NUFFT fine grid, plans and buffers
 int noalloc_attach(dc_ctx *c);   // device address of this device's dc_scratch (dc_noalloc.hip)
 PrepArgs base_prep(const Grid &g, int mapping);

@@ -24,10 +24,12 @@
 // thread per sub-field), so results repeat bit for bit.
 #include <hipfft/hipfft.h>
 
+#include <algorithm>
 #include <cmath>
 #include <map>
 #include <tuple>
 
+#include "dc_fft.h"
 #include "dc_host.h"
 
 using namespace dc;
@@ -61,6 +63,14 @@ __device__ inline long long nat_off(const Field &f, int b, int i, int j, int k) 
 }
 
 __device__ inline void unflat(const Field &f, long long e, int &b, int &i, int &j, int &k) {
+    if (f.total() <= 0x7FFFFFFF) {     // 32-bit divisions: a quarter of the work of 64-bit ones
+        const unsigned u = (unsigned)e, m0 = f.m[0], m1 = f.m[1], m2 = f.m[2], q = u / m0, r = q / m1, t = r / m2;
+        i = (int)(u - q * m0);
+        j = (int)(q - r * m1);
+        k = (int)(r - t * m2);
+        b = (int)t;
+        return;
+    }
     const long long sub = f.sub();
     b = (int)(e / sub);
     long long r = e - (long long)b * sub;
@@ -137,26 +147,146 @@ struct ProfArgs {
     double sig[3];
 };
 
+__device__ inline double conv_profile(const ProfArgs &p, int i, int j, int k) {
+    const double zpi = 6.283185307179586476925286766559;
+    const int idx[3] = {i, j, k};
+    double v[3];
+    for (int a = 0; a < 3; ++a) v[a] = (double)(idx[a] > p.m[a] / 2 ? idx[a] - p.m[a] : idx[a]);
+    double val = 1.0;
+    for (int rr = 0; rr < p.nd; ++rr) {
+        const double pos = p.tr[rr] * v[0] + p.tr[rr + 3] * v[1] + p.tr[rr + 6] * v[2];
+        val = val * (1.0 / sqrt(zpi) / p.sig[rr] * exp(-0.5 * pos * pos));
+    }
+    return val;
+}
+
 __global__ void conv_profile_kernel(ProfArgs p, double2 *__restrict__ out) {
     const long long n = (long long)p.m[0] * p.m[1] * p.m[2];
-    const double zpi = 6.283185307179586476925286766559;
     for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
-        int idx[3];
-        long long r = e;
-        idx[0] = (int)(r % p.m[0]);
-        r /= p.m[0];
-        idx[1] = (int)(r % p.m[1]);
-        idx[2] = (int)(r / p.m[1]);
-        double v[3];
-        for (int a = 0; a < 3; ++a) v[a] = (double)(idx[a] > p.m[a] / 2 ? idx[a] - p.m[a] : idx[a]);
-        double val = 1.0;
-        for (int rr = 0; rr < p.nd; ++rr) {
-            const double pos = p.tr[rr] * v[0] + p.tr[rr + 3] * v[1] + p.tr[rr + 6] * v[2];
-            val = val * (1.0 / sqrt(zpi) / p.sig[rr] * exp(-0.5 * pos * pos));
-        }
-        out[e] = make_double2(val, 0.0);
+        const int i = (int)(e % p.m[0]);
+        const long long r = e / p.m[0];
+        out[e] = make_double2(conv_profile(p, i, (int)(r % p.m[1]), (int)(r / p.m[1])), 0.0);
     }
 }
+
+// ---- transforms by dc_fft.h: lines of the abscissa (rows) with the maps of
+// map_fwd_kernel / map_rev_kernel as their loads and stores, lines of the
+// other axes (columns, FFT_LINES neighbouring ones at a time) in place, the
+// last axis with the spectrum between its two transforms.  A complex field of
+// 161^3: 5 passes of 33 to 47 us and 90 for the last axis, where the library's
+// transforms with their maps and products took 11 launches, 800 us.
+template <bool CPLX>
+struct SrcMap {
+    Field f;
+    MapAxes a;
+    const double *x;
+    __device__ int nat(int q, int ax) const {
+        const int i = q - 1 - f.m[ax] / 2 + a.lf[ax];
+        return i < 0 ? i + f.m[ax] : i;
+    }
+    __device__ double2 operator()(int b, int i, int j, int k, long long) const {
+        const long long o = nat_off(f, b, nat(i, 0), nat(j, 1), nat(k, 2));
+        if constexpr (CPLX) return make_double2(x[2 * o], x[2 * o + 1]);
+        return make_double2(x[o], 0.0);
+    }
+};
+struct SrcWork {
+    const double2 *w;
+    int m0;
+    __device__ double2 operator()(int, int i, int, int, long long row) const { return w[row * m0 + i]; }
+};
+struct SrcProfile {
+    ProfArgs p;
+    __device__ double2 operator()(int, int i, int j, int k, long long) const { return make_double2(conv_profile(p, i, j, k), 0.0); }
+};
+struct DstWork {
+    double2 *w;
+    int m0;
+    __device__ void operator()(int, int i, int, int, long long row, double2 v) const { w[row * m0 + i] = v; }
+};
+template <bool CPLX>
+struct DstMap {
+    Field f;
+    MapAxes a;
+    double div;
+    double *x;
+    __device__ int nat(int q, int ax) const {
+        const int m = f.m[ax], i = m - 1 - q - m / 2 + a.lr[ax];
+        return i < 0 ? i + m : i >= m ? i - m : i;
+    }
+    __device__ void operator()(int b, int i, int j, int k, long long, double2 v) const {
+        const long long o = nat_off(f, b, nat(i, 0), nat(j, 1), nat(k, 2));
+        if constexpr (CPLX) {
+            x[2 * o] = v.x / div;
+            x[2 * o + 1] = v.y / div;
+        } else {
+            x[o] = v.x / div;
+        }
+    }
+};
+
+__device__ inline double2 spec_mul(const double2 *spec, long long e, double sscale, double2 w) {
+    const double2 t0 = spec[e];
+    const double tr = t0.x * sscale, ti = t0.y * sscale;
+    return make_double2(tr * w.x - ti * w.y, tr * w.y + ti * w.x);
+}
+
+template <class Src, class Dst, bool TW>
+struct RowsOp {
+    static constexpr bool TWICE = TW;
+    int m0, m1, m2;
+    unsigned rows;
+    Src src;
+    Dst dst;
+    const double2 *spec;
+    double sscale;
+    struct Line {
+        const RowsOp &o;
+        bool in;
+        int b, j, k;
+        long long row, spec0;
+        __device__ double2 load(int i) const { return in ? o.src(b, i, j, k, row) : make_double2(0.0, 0.0); }
+        __device__ double2 mid(int i, double2 v) const { return in ? spec_mul(o.spec, spec0 + i, o.sscale, v) : v; }
+        __device__ void store(int i, double2 v) const {
+            if (in) o.dst(b, i, j, k, row, v);
+        }
+    };
+    __device__ Line line(long long g, int l) const {
+        const unsigned row = (unsigned)g * FFT_LINES + l, t = row / (unsigned)m1;
+        const int b = (int)(t / (unsigned)m2);
+        return {*this, row < rows, b, (int)(row - t * m1), (int)(t - (unsigned)b * m2), (long long)row,
+                ((long long)row - (long long)b * m1 * m2) * m0};
+    }
+};
+
+// Lines at stride `inner` (the axis), `inner` neighbours each, a slab of
+// `inner * length` elements each.
+template <bool TW>
+struct ColsOp {
+    static constexpr bool TWICE = TW;
+    double2 *w;
+    unsigned inner, tiles;             // tiles of FFT_LINES neighbours
+    long long slab;
+    const double2 *spec;
+    long long sub;                     // elements of the spectrum
+    double sscale;
+    struct Line {
+        double2 *p;
+        const double2 *sp;
+        unsigned inner;
+        double sscale;
+        __device__ double2 load(int i) const { return p ? p[(long long)i * inner] : make_double2(0.0, 0.0); }
+        __device__ double2 mid(int i, double2 v) const { return p ? spec_mul(sp, (long long)i * inner, sscale, v) : v; }
+        __device__ void store(int i, double2 v) const {
+            if (p) p[(long long)i * inner] = v;
+        }
+    };
+    __device__ Line line(long long g, int l) const {
+        const unsigned o = (unsigned)g / tiles, c = ((unsigned)g - o * tiles) * FFT_LINES + l;
+        const long long e = o * slab + c;
+        return {c < inner ? w + e : nullptr, TW ? spec + e % sub : nullptr, inner, sscale};
+    }
+};
 
 // Lanczos sinc table of do_lanczos_*_fft (lib_lanczos.f90:258-458), written
 // directly in FFT order: FFT element -> natural index by the forward map,
@@ -216,20 +346,26 @@ struct TapArgs {
     double v[MAXTAP];
 };
 
+// One thread per element.  Bound: reading and writing the field (33 MB each at
+// 161^3, 13 us); the taps' other reads hit L1/L2.  Reducing the taps' indices
+// by comparison instead of a division each, and the element's in 32 bits: 48
+// -> 33 us an axis.
 __global__ void axis_conv_kernel(TapArgs t, const double *__restrict__ src, double *__restrict__ dst) {
     const long long n = t.f.total();
     const int m = t.f.m[t.axis];
+    const long long s = t.f.s[t.axis];
     for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
         int b, c3[3];
         unflat(t.f, e, b, c3[0], c3[1], c3[2]);
-        const int q = c3[t.axis];
+        const int q = t.axis == 0 ? c3[0] : t.axis == 1 ? c3[1] : c3[2];
+        const long long o = nat_off(t.f, b, c3[0], c3[1], c3[2]), line = o - q * s;
         double acc = 0.0;
         for (int u = 0; u < t.ntap; ++u) {
-            int cc[3] = {c3[0], c3[1], c3[2]};
-            cc[t.axis] = pmod(q + t.shift - t.r[u], m);
-            acc += src[nat_off(t.f, b, cc[0], cc[1], cc[2])] * t.v[u];
+            int i = q + t.shift - t.r[u];      // r in [0, m), shift 0 or 1
+            i = i < 0 ? i + m : i >= m ? i - m : i;
+            acc += src[line + i * s] * t.v[u];
         }
-        dst[nat_off(t.f, b, c3[0], c3[1], c3[2])] = acc;
+        dst[o] = acc;
     }
 }
 
@@ -268,19 +404,21 @@ __global__ __launch_bounds__(SUM_THREADS) void sum_part_kernel(Field f, int cont
     if (threadIdx.x == 0) part[(long long)b * SUM_BLOCKS + blockIdx.x] = s[0];
 }
 
-__global__ void sum_finish_kernel(int batch, const double *__restrict__ part, double *__restrict__ out) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= batch) return;
+// One wave per sub-field; lanes and then the tree in a fixed order.
+__global__ void __launch_bounds__(64) sum_finish_kernel(int batch, const double *__restrict__ part, double *__restrict__ out) {
+    const int b = blockIdx.x;
     double acc = 0.0;
-    for (int g = 0; g < SUM_BLOCKS; ++g) acc += part[(long long)b * SUM_BLOCKS + g];
-    out[b] = acc;
+    for (int g = threadIdx.x; g < SUM_BLOCKS; g += 64) acc += part[(long long)b * SUM_BLOCKS + g];
+#pragma unroll
+    for (int h = 32; h > 0; h >>= 1) acc += __shfl_xor(acc, h);
+    if (threadIdx.x == 0) out[b] = acc;
 }
 
 // x[b] = (x[b] * num[b]) / den[b]          (four_conv: csf*weight/weight2)
 // x[b] = x[b] * (num[b] / den[b] * mul)    (do_lanczos: outfield*factor)
 template <bool CPLX, bool LANCZOS>
 __global__ void rescale_kernel(Field f, const double *__restrict__ num, const double *__restrict__ den, double mul,
-                               double *__restrict__ x) {
+                               double *x, const double *src = nullptr) {
     const long long n = f.total();
     for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
         int b, i, j, k;
@@ -288,7 +426,7 @@ __global__ void rescale_kernel(Field f, const double *__restrict__ num, const do
         const long long o = nat_off(f, b, i, j, k);
         if (LANCZOS) {
             const double fac = num[b] / den[b] * mul;
-            x[o] = x[o] * fac;
+            x[o] = (src ? src : x)[o] * fac;
         } else if (CPLX) {
             x[2 * o] = x[2 * o] * num[b] / den[b];
             x[2 * o + 1] = x[2 * o + 1] * num[b] / den[b];
@@ -550,6 +688,32 @@ struct PostState {
 };
 
 namespace dc {
+int fft_table(dc_ctx *c, FftLen &f) {
+    auto it = c->fft_tw.find(f.n);
+    if (it == c->fft_tw.end()) {
+        std::vector<double2> t(f.n);
+        const long double turn = 6.283185307179586476925286766559005768L;
+        for (int k = 0; k < f.n; ++k) {
+            const long double x = turn * k / f.n;
+            t[k] = make_double2((double)cosl(x), (double)-sinl(x));
+        }
+        DevBuf b;
+        const int st = upload(c, b, t.data(), t.size());
+        if (st) return st;
+        HIPCHK(hipStreamSynchronize(c->st));   // t has been read
+        it = c->fft_tw.emplace(f.n, b).first;
+    }
+    f.tw = ptr<double2>(it->second);
+    return 0;
+}
+void fft_release(dc_ctx *c) {
+    for (auto &kv : c->fft_tw)
+        if (kv.second.p) (void)hipFree(kv.second.p);
+    c->fft_tw.clear();
+}
+}  // namespace dc
+
+namespace dc {
 void post_release(dc_ctx *c) {
     if (!c->post) return;
     for (auto &kv : c->post->plans) (void)hipfftDestroy(kv.second);
@@ -607,9 +771,70 @@ int field_sums(dc_ctx *c, const Field &f, const double *x, double *out) {
     if (st) return st;
     const int contiguous = f.s[0] == 1 && f.s[1] == f.m[0] && (f.m[2] == 1 || f.s[2] == (long long)f.m[0] * f.m[1]);
     sum_part_kernel<<<dim3(SUM_BLOCKS, f.batch), SUM_THREADS, 0, c->st>>>(f, contiguous, x, ptr<double>(ps.part));
-    sum_finish_kernel<<<(f.batch + 63) / 64, 64, 0, c->st>>>(f.batch, ptr<double>(ps.part), out);
+    sum_finish_kernel<<<f.batch, 64, 0, c->st>>>(f.batch, ptr<double>(ps.part), out);
     HIPCHK(hipGetLastError());
     return 0;
+}
+
+// Axis lengths, where dc_fft.h transforms every one (else the library does
+// them all), and their tables.  Faster than the library's (a convolution's
+// whole call) at every length measured from 33 to 600: 161^3 2144 -> 715 us, 157^3 2030 ->
+// 1216, 199^2 x 100 1496 -> 1215, 256^2 x 64 766 -> 491, 598^2 437 -> 171; except where
+// the library has the radices and the lines are too long for three
+// work-groups a CU: 600^2 x 20 1452 us against 1493.
+int own_fft(dc_ctx *c, const Field &f, FftLen len[3], int &nd, bool &own) {
+    nd = f.m[2] > 1 ? 3 : f.m[1] > 1 ? 2 : 1;
+    own = f.total() < (1LL << 31);
+    for (int a = 0; a < nd; ++a) own = own && fft_length(f.m[a], len[a]) && (f.m[a] <= FFT_COMMON || len[a].radix[0] > 13);
+    int st;
+    for (int a = 0; a < nd && own; ++a)
+        if ((st = fft_table(c, len[a]))) return st;
+    return 0;
+}
+
+template <class Src, class Dst, bool TW>
+int fft_rows(dc_ctx *c, const Field &f, const FftLen &len, const Src &src, const Dst &dst, const double2 *spec, double sscale) {
+    const long long rows = (long long)f.m[1] * f.m[2] * f.batch;
+    const RowsOp<Src, Dst, TW> op{f.m[0], f.m[1], f.m[2], (unsigned)rows, src, dst, spec, sscale};
+    HIPCHK(fft_launch(len, op, (rows + FFT_LINES - 1) / FFT_LINES, c->st));
+    return 0;
+}
+
+// Lines of axis 1 or 2 of w, in place.
+template <bool TW>
+int fft_cols(dc_ctx *c, const Field &f, const FftLen &len, int axis, double2 *w, const double2 *spec, double sscale) {
+    const long long inner = axis == 1 ? f.m[0] : (long long)f.m[0] * f.m[1];
+    const long long outer = axis == 1 ? (long long)f.m[2] * f.batch : f.batch;
+    const long long tiles = (inner + FFT_LINES - 1) / FFT_LINES;
+    const ColsOp<TW> op{w, (unsigned)inner, (unsigned)tiles, inner * f.m[axis], spec, f.sub(), sscale};
+    HIPCHK(fft_launch(len, op, tiles * outer, c->st));
+    return 0;
+}
+
+// Spectrum of the profile / table that src gives, into spec.
+template <class Src>
+int spectrum(dc_ctx *c, const Field &one, const FftLen len[3], int nd, const Src &src, double2 *spec) {
+    int st;
+    if ((st = fft_rows<Src, DstWork, false>(c, one, len[0], src, DstWork{spec, one.m[0]}, nullptr, 0.0))) return st;
+    for (int a = 1; a < nd; ++a)
+        if ((st = fft_cols<false>(c, one, len[a], a, spec, nullptr, 0.0))) return st;
+    return 0;
+}
+
+// map -> transform -> * spec -> transform -> reverse map; the last axis meets
+// the spectrum between its two transforms, so a 3D field takes 5 passes.
+template <bool CPLX>
+int convolve_lines(dc_ctx *c, const Field &f, const FftLen len[3], int nd, const MapAxes &ax, double *x, const double2 *spec,
+                   double sscale, double div, double2 *w) {
+    const SrcMap<CPLX> src{f, ax, x};
+    const DstMap<CPLX> dst{f, ax, div, x};
+    if (nd == 1) return fft_rows<SrcMap<CPLX>, DstMap<CPLX>, true>(c, f, len[0], src, dst, spec, sscale);
+    int st;
+    if ((st = fft_rows<SrcMap<CPLX>, DstWork, false>(c, f, len[0], src, DstWork{w, f.m[0]}, nullptr, 0.0))) return st;
+    if (nd == 3 && (st = fft_cols<false>(c, f, len[1], 1, w, nullptr, 0.0))) return st;
+    if ((st = fft_cols<true>(c, f, len[nd - 1], nd - 1, w, spec, sscale))) return st;
+    if (nd == 3 && (st = fft_cols<false>(c, f, len[1], 1, w, nullptr, 0.0))) return st;
+    return fft_rows<SrcWork, DstMap<CPLX>, false>(c, f, len[0], SrcWork{w, f.m[0]}, dst, nullptr, 0.0);
 }
 
 // One field through map -> FFT -> * spec -> FFT -> reverse map (in place on x).
@@ -619,6 +844,13 @@ int convolve(dc_ctx *c, const Field &f, const MapAxes &ax, bool cplx, double *x,
     int st = ensure(c, ps.work, sizeof(double2) * (size_t)f.total());
     if (st) return st;
     double2 *w = ptr<double2>(ps.work);
+    FftLen len[3];
+    int nd;
+    bool own;
+    if ((st = own_fft(c, f, len, nd, own))) return st;
+    if (own)
+        return cplx ? convolve_lines<true>(c, f, len, nd, ax, x, spec, sscale, div, w)
+                    : convolve_lines<false>(c, f, len, nd, ax, x, spec, sscale, div, w);
     const int gr = grid_for(f.total());
     if (cplx)
         map_fwd_kernel<true><<<gr, 256, 0, c->st>>>(f, ax, x, w);
@@ -692,9 +924,17 @@ int run_conv(dc_ctx *c, const dc_post_desc *d, double *csf, double *dsi, double 
     pa.nd = isdim;
     for (int q = 0; q < 9; ++q) pa.tr[q] = d->res_tr[q];
     double2 *spec = ptr<double2>(ps.spec);
-    conv_profile_kernel<<<grid_for(f.sub()), 256, 0, c->st>>>(pa, spec);
-    HIPCHK(hipGetLastError());
-    if ((st = fft_fwd(c, f, spec))) return st;
+    FftLen len[3];
+    int nd;
+    bool own;
+    if ((st = own_fft(c, f, len, nd, own))) return st;
+    if (own) {
+        if ((st = spectrum(c, f, len, nd, SrcProfile{pa}, spec))) return st;
+    } else {
+        conv_profile_kernel<<<grid_for(f.sub()), 256, 0, c->st>>>(pa, spec);
+        HIPCHK(hipGetLastError());
+        if ((st = fft_fwd(c, f, spec))) return st;
+    }
     const double ntot = (double)f.sub();
     const double sscale = isdim == 1 ? 1.0 / ntot : 1.0 / std::sqrt(ntot);
     // in_pattern / N: 1D in double, 2D/3D through REAL() (single precision)
@@ -776,9 +1016,8 @@ int lanczos_batch(dc_ctx *c, const Field &f, int nd, double nscale, double rcut,
                 cur = 1 - cur;
             }
             HIPCHK(hipGetLastError());
-            if (cur == 1) HIPCHK(hipMemcpyAsync(x, ps.copy.p, sizeof(double) * (size_t)span, hipMemcpyDeviceToDevice, c->st));
-            if ((st = field_sums(c, f, x, sums + f.batch))) return st;         // sum(outfield)
-            rescale_kernel<false, true><<<gr, 256, 0, c->st>>>(f, sums, sums + f.batch, nscale, x);
+            if ((st = field_sums(c, f, bufs[cur], sums + f.batch))) return st;         // sum(outfield)
+            rescale_kernel<false, true><<<gr, 256, 0, c->st>>>(f, sums, sums + f.batch, nscale, x, bufs[cur]);
             HIPCHK(hipGetLastError());
             return 0;
         }
@@ -806,7 +1045,15 @@ int lanczos_batch(dc_ctx *c, const Field &f, int nd, double nscale, double rcut,
     one.batch = 1;
     lanczos_table_kernel<<<grid_for(f.sub()), 256, 0, c->st>>>(t, spec);
     HIPCHK(hipGetLastError());
-    if ((st = fft_fwd(c, one, spec))) return st;
+    FftLen len[3];
+    int ldim;
+    bool own;
+    if ((st = own_fft(c, one, len, ldim, own))) return st;
+    if (own) {
+        if ((st = spectrum(c, one, len, ldim, SrcWork{spec, one.m[0]}, spec))) return st;
+    } else if ((st = fft_fwd(c, one, spec))) {
+        return st;
+    }
     double *sums = ptr<double>(ps.sums);
     if ((st = field_sums(c, f, x, sums))) return st;                        // sum(infield)
     double div = 1.0;                                                       // lib_conv's weight
