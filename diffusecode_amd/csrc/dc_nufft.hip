@@ -25,6 +25,7 @@
 #include <tuple>
 #include <vector>
 
+#include "dc_fft.h"
 #include "dc_host.h"
 
 using namespace dc;
@@ -246,21 +247,6 @@ __global__ __launch_bounds__(256) void spread3_real_kernel(SpreadArgs a, long lo
     }
 }
 
-void launch_spread_real(int w, hipStream_t st, const SpreadArgs &a, long long M, const double *x, const double *y,
-                        const double *z, double sv, int comp, double *g) {
-    const int tg = grid_for(M * w);   // w threads per point
-    switch (w) {
-    case 2: spread3_real_kernel<2><<<tg, 256, 0, st>>>(a, M, x, y, z, sv, comp, g); return;
-    case 4: spread3_real_kernel<4><<<tg, 256, 0, st>>>(a, M, x, y, z, sv, comp, g); return;
-    case 6: spread3_real_kernel<6><<<tg, 256, 0, st>>>(a, M, x, y, z, sv, comp, g); return;
-    case 8: spread3_real_kernel<8><<<tg, 256, 0, st>>>(a, M, x, y, z, sv, comp, g); return;
-    case 10: spread3_real_kernel<10><<<tg, 256, 0, st>>>(a, M, x, y, z, sv, comp, g); return;
-    case 12: spread3_real_kernel<12><<<tg, 256, 0, st>>>(a, M, x, y, z, sv, comp, g); return;
-    case 14: spread3_real_kernel<14><<<tg, 256, 0, st>>>(a, M, x, y, z, sv, comp, g); return;
-    default: spread3_real_kernel<16><<<tg, 256, 0, st>>>(a, M, x, y, z, sv, comp, g); return;
-    }
-}
-
 template <int DIM>
 void launch_spread(int w, int grid, hipStream_t st, const SpreadArgs &a, long long M, const double *x, const double *y,
                    const double *z, const double2 *c, double *g) {
@@ -401,6 +387,299 @@ __global__ void deconv3_kernel(PruneArgs a, const double2 *__restrict__ Z, doubl
     }
 }
 
+// ---- 3D, real constant strengths (run level): no fine grid in memory ---------
+//
+// A work-group owns FFT_LINES = TY x TZ abscissa lines of the fine grid in LDS: it adds up
+// the points whose kernels reach them, transforms them, separates the two
+// types (a real grid each, in the real and the imaginary part) and writes the
+// k >= 0 columns that the output needs -- the other half of a real grid's
+// modes are conjugates.  The y and z passes (dc_fft.h) keep only the needed
+// rows; the z pass writes each mode and its mirror, deconvolved and, for a
+// run, times the form factor onto the sum over the types.
+//
+// Points are sorted into bins of TY x TZ kernel corners (count, scan,
+// scatter with their kernel values), so that a line group reads the points of
+// 5 x 3 bins and neighbouring lines find each other's in L2.
+//
+// Bound: memory, about 0.5 GB a type at 324^3 (161^3 modes).  The path this
+// replaces there (FP64 atomics on the 544 MB grid, library transforms with transposes)
+// wrote and read it 7 times a pair.  256,000 points of 3 types, a call: 3.75 ms,
+// 2.0 of them in the atomics -> 1.19 ms (sorting 0.07, spreading and abscissa
+// 0.42, y 0.21, z 0.28).
+constexpr int SW = 8;                  // kernel width of the technique's tolerance (1e-7)
+constexpr int TY = 4, TZ = 2;
+static_assert(TY * TZ == FFT_LINES, "a lane per line");
+constexpr int ZBINS = (SW - 1 + TZ - 1) / TZ + 1;
+
+struct SpreadPt {
+    double kx[SW], ky[SW], kz[SW];     // kernel values, the strength in kx
+    int l[3];                          // first fine index per axis, in [0, n)
+    int comp;                          // 0: real part, 1: imaginary part
+};
+
+// Where the points of up to SORT_TYPES types come from and which pair and part
+// each belongs to (types 2k and 2k + 1 form pair k).
+constexpr int SORT_TYPES = 16;
+struct SortArgs {
+    int n[3], nby, nbz;
+    double beta, scale[3];
+    const double *x[3];                // coordinates, or
+    const int *idx;                    // atoms of pos times fac
+    const double *pos;
+    double fac[3];
+    int ntype, type0;                  // type0: number of the first type here (even)
+    long long beg[SORT_TYPES + 1];
+    long long first;                   // the call's first point
+    double s[SORT_TYPES];
+};
+
+__device__ inline int sort_point(const SortArgs &a, long long e, int &type, double (&u)[3], int (&l)[3]) {
+    type = 0;
+    while (type + 1 < a.ntype && e >= a.beg[type + 1]) ++type;
+    for (int d = 0; d < 3; ++d) {
+        const double x = a.idx ? a.pos[3 * (long long)a.idx[e] + d] * a.fac[d] : a.x[d][e];
+        const double n = (double)a.n[d];
+        double v = x * a.scale[d];
+        v -= floor(v / n) * n;         // into [0, n)
+        u[d] = v;
+        const int lo = (int)ceil(v - 0.5 * SW);
+        l[d] = lo < 0 ? lo + a.n[d] : lo >= a.n[d] ? lo - a.n[d] : lo;
+        if (l[d] < 0 || l[d] >= a.n[d]) l[d] = 0;   // no finite coordinate: its kernel values are 0
+    }
+    return (((a.type0 + type) >> 1) * a.nbz + l[2] / TZ) * a.nby + l[1] / TY;
+}
+
+// Bin of every point and its place in the bin.
+__global__ void sort_count_kernel(SortArgs a, int *__restrict__ cnt, int2 *__restrict__ place) {
+    const long long e = a.beg[0] + (long long)blockIdx.x * 256 + threadIdx.x;
+    if (e >= a.beg[a.ntype]) return;
+    int t, l[3];
+    double u[3];
+    const int bin = sort_point(a, e, t, u, l);
+    place[e - a.first] = make_int2(bin, atomicAdd(cnt + bin, 1));
+}
+
+// Exclusive scan of n counts in place; start[n] is the total.  One work-group,
+// four counts a thread and round, the next round's in flight: n is 10^4 to 10^5.
+__global__ void __launch_bounds__(1024) sort_scan_kernel(int n, int *__restrict__ start) {
+    __shared__ int wsum[16];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int carry = 0, v[4], nx[4];
+    auto fetch = [&](int at, int (&x)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = at + u < n ? start[at + u] : 0;
+    };
+    fetch(4 * threadIdx.x, v);
+    for (int b = 0; b < n; b += 4096) {
+        const int at = b + 4 * threadIdx.x;
+        fetch(at + 4096, nx);
+        const int own = v[0] + v[1] + v[2] + v[3];
+        int inc = own;
+#pragma unroll
+        for (int h = 1; h < 64; h *= 2) {
+            const int o = __shfl_up(inc, h);
+            if (lane >= h) inc += o;
+        }
+        if (lane == 63) wsum[wave] = inc;
+        __syncthreads();
+        int before = carry;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) {
+            const int x = wsum[w];
+            if (w < wave) before += x;
+            carry += x;
+        }
+        int run = before + inc - own;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (at + u < n) start[at + u] = run;
+            run += v[u];
+            v[u] = nx[u];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) start[n] = carry;
+}
+
+// SW lanes a point: each evaluates one kernel value per axis.
+__global__ void sort_scatter_kernel(SortArgs a, const int *__restrict__ start, const int2 *__restrict__ place,
+                                    SpreadPt *__restrict__ pts) {
+    const long long e = a.beg[0] + (long long)blockIdx.x * (256 / SW) + threadIdx.x / SW;
+    if (e >= a.beg[a.ntype]) return;
+    const int i = threadIdx.x % SW;
+    int t, l[3];
+    double u[3];
+    (void)sort_point(a, e, t, u, l);
+    const int2 at = place[e - a.first];
+    SpreadPt &p = pts[start[at.x] + at.y];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const double lo = ceil(u[d] - 0.5 * SW);
+        const double z = (lo + (double)i - u[d]) * (2.0 / SW), q = 1.0 - z * z;
+        (d == 0 ? p.kx : d == 1 ? p.ky : p.kz)[i] = q > 0.0 ? (d == 0 ? a.s[t] : 1.0) * exp(a.beta * (sqrt(q) - 1.0)) : 0.0;
+    }
+    if (i < 3) p.l[i] = i == 0 ? l[0] : i == 1 ? l[1] : l[2];
+    if (i == 3) p.comp = (a.type0 + t) & 1;
+}
+
+__device__ __forceinline__ double2 swap_ri(double2 v) { return make_double2(v.y, v.x); }
+
+struct SpreadXArgs {
+    int n[3], nby, nbz;
+    const int *start;                  // bins of this pair
+    const SpreadPt *pts;
+    int c0;
+    const int *k0;                     // kept abscissa modes, k >= 0
+    double2 *a, *b;                    // [z][y][c0] of the two types (b: null for one type)
+};
+
+template <int NT, int KIND>
+__global__ void __launch_bounds__(NT, KIND ? 4 : 6) spread_x_kernel(FftLen f, SpreadXArgs a) {
+    extern __shared__ double2 fft_smem[];
+    __shared__ int seg_beg[2 * ZBINS], seg_end[2 * ZBINS];
+    double2 *buf = fft_smem, *tw = fft_smem + (size_t)f.n * FFT_LINES;
+    const int ty = blockIdx.x % a.nby, tz = blockIdx.x / a.nby;
+    const int l = threadIdx.x % FFT_LINES, team = threadIdx.x / FFT_LINES;
+    const int y = ty * TY + l % TY, z = tz * TZ + l / TY;
+    for (int k = threadIdx.x; k < f.n; k += NT) tw[k] = f.tw[k];
+    for (int k = threadIdx.x; k < f.n * FFT_LINES; k += NT) buf[k] = make_double2(0.0, 0.0);
+    if (threadIdx.x < 2 * ZBINS) {
+        // kernel corners from SW - 1 before the tile to its end, modulo n: bins
+        // tz - ZBINS + 1 .. tz, and in each the bins of the ordinate, in two runs where they wrap
+        int zb = tz - (int)threadIdx.x / 2;
+        if (zb < 0) zb += a.nbz;
+        const int ylo = ty * TY - (SW - 1);
+        int b0 = ylo < 0 ? 0 : ylo / TY, b1 = ty;
+        if (threadIdx.x & 1) {
+            b0 = ylo < 0 ? (ylo + a.n[1]) / TY : 1;
+            b1 = ylo < 0 ? a.nby - 1 : 0;
+        }
+        seg_beg[threadIdx.x] = b0 <= b1 ? a.start[zb * a.nby + b0] : 0;
+        seg_end[threadIdx.x] = b0 <= b1 ? a.start[zb * a.nby + b1 + 1] : 0;
+    }
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int s = 0; s < 2 * ZBINS; ++s) total += seg_end[s] - seg_beg[s];
+    for (int i = team; i < total; i += NT / FFT_LINES) {
+        int at = i, s = 0;
+        while (at >= seg_end[s] - seg_beg[s]) {
+            at -= seg_end[s] - seg_beg[s];
+            ++s;
+        }
+        const SpreadPt &p = a.pts[seg_beg[s] + at];
+        int dy = y - p.l[1], dz = z - p.l[2];
+        if (dy < 0) dy += a.n[1];
+        if (dz < 0) dz += a.n[2];
+        if (dy >= SW || dz >= SW || y >= a.n[1]) continue;
+        const double w = p.ky[dy] * p.kz[dz];
+        // (real and imaginary part swapped: a backward transform)
+        double *g = reinterpret_cast<double *>(buf + l) + (p.comp ? 0 : 1);
+        int x = p.l[0];
+#pragma unroll
+        for (int t = 0; t < SW; ++t) {
+            __hip_atomic_fetch_add(g + 2 * FFT_LINES * x, w * p.kx[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            x = x + 1 == a.n[0] ? 0 : x + 1;
+        }
+    }
+    __syncthreads();
+    fft_lines<NT, KIND>(buf, tw, f);
+    if (y >= a.n[1] || z >= a.n[2]) return;
+    const long long row = ((long long)z * a.n[1] + y) * a.c0;
+    for (int i = team; i < a.c0; i += NT / FFT_LINES) {
+        const int k = a.k0[i];
+        const double2 p = swap_ri(buf[k * FFT_LINES + l]), m = swap_ri(buf[(k ? a.n[0] - k : 0) * FFT_LINES + l]);
+        a.a[row + i] = make_double2(0.5 * (p.x + m.x), 0.5 * (p.y - m.y));
+        if (a.b) a.b[row + i] = make_double2(0.5 * (p.y + m.y), 0.5 * (m.x - p.x));
+    }
+}
+
+// y pass: slabs [n1][c0] -> the kept rows [c1][c0].
+struct RealYOp {
+    static constexpr bool TWICE = false;
+    const double2 *in;
+    double2 *out;
+    int n1, c0, c1;
+    unsigned tiles;
+    const int *keep;                   // fine ordinate index -> kept row, or -1
+    struct Line {
+        const double2 *in;
+        double2 *out;
+        int c0;
+        const int *keep;
+        __device__ double2 load(int i) const { return in ? swap_ri(in[(long long)i * c0]) : make_double2(0.0, 0.0); }
+        __device__ void store(int i, double2 v) const {
+            const int j = keep[i];
+            if (in && j >= 0) out[(long long)j * c0] = swap_ri(v);
+        }
+    };
+    __device__ Line line(long long g, int l) const {
+        const unsigned o = (unsigned)g / tiles, c = ((unsigned)g - o * tiles) * FFT_LINES + l;
+        return {c < (unsigned)c0 ? in + (long long)o * n1 * c0 + c : nullptr, out + (long long)o * c1 * c0 + c, c0, keep};
+    }
+};
+
+// z pass: lines [z][c1 c0] -> output modes.
+struct RealZOp {
+    static constexpr bool TWICE = false;
+    const double2 *in;
+    int c0, cc;                        // cc = c1 c0
+    const int *o1p, *o1m, *o2p, *o2m, *o3p, *o3m;   // output index of k and of -k per kept position, or -1
+    int out0, out1;
+    const double *corr[3];             // by output index
+    long long sub[3];
+    // plain modes into fk, or times the form factor of type t onto the sum
+    int form, first, t, ncfact;
+    Grid g;
+    const double2 *cfact;
+    double2 *fk;
+    struct Line {
+        const RealZOp &o;
+        const double2 *in;
+        int p1, p2, m1, m2;
+        double fp, fm;
+        __device__ double2 load(int i) const { return in ? swap_ri(in[(long long)i * o.cc]) : make_double2(0.0, 0.0); }
+        __device__ void put(int a, int b, int c, double f, double2 v) const {
+            const long long e = a + (long long)o.out0 * (b + (long long)o.out1 * c);
+            f *= o.corr[2][c * o.sub[2]];
+            v = make_double2(v.x * f, v.y * f);
+            if (o.form) {
+                const double2 w = o.cfact[(long long)o.t * o.ncfact + istl_point(o.g, a, b, c)];
+                v = make_double2(v.x * w.x - v.y * w.y, v.x * w.y + v.y * w.x);
+                if (!o.first) {
+                    const double2 s = o.fk[e];
+                    v = make_double2(s.x + v.x, s.y + v.y);
+                }
+            }
+            o.fk[e] = v;
+        }
+        __device__ void store(int i, double2 v) const {
+            if (!in) return;
+            v = swap_ri(v);
+            if (p1 >= 0 && o.o3p[i] >= 0) put(p1, p2, o.o3p[i], fp, v);
+            if (m1 >= 0 && o.o3m[i] >= 0) put(m1, m2, o.o3m[i], fm, make_double2(v.x, -v.y));
+        }
+    };
+    __device__ Line line(long long g, int l) const {
+        const int c = (int)(g * FFT_LINES) + l;
+        Line r{*this, c < cc ? in + c : nullptr, -1, -1, -1, -1, 0.0, 0.0};
+        if (c < cc) {
+            const int i = c % c0, j = c / c0;
+            if (o1p[i] >= 0 && o2p[j] >= 0) {
+                r.p1 = o1p[i];
+                r.p2 = o2p[j];
+                r.fp = corr[0][r.p1 * sub[0]] * corr[1][r.p2 * sub[1]];
+            }
+            if (o1m[i] >= 0 && o2m[j] >= 0) {
+                r.m1 = o1m[i];
+                r.m2 = o2m[j];
+                r.fm = corr[0][r.m1 * sub[0]] * corr[1][r.m2 * sub[1]];
+            }
+        }
+        return r;
+    }
+};
+
 __global__ void zero_kernel(long long n, double *__restrict__ p) {
     for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) p[e] = 0.0;
 }
@@ -490,10 +769,19 @@ struct PruneTables {
     std::vector<std::vector<int>> host;   // sources of the uploads, kept alive
 };
 
+// Index tables of the real-strength transform (see SpreadXArgs, RealYOp, RealZOp).
+struct RealTables {
+    int c0 = 0, c1 = 0;
+    DevBuf b[8];                       // k0, keep1, o1p, o1m, o2p, o2m, o3p, o3m
+    std::vector<std::vector<int>> host;   // sources of the uploads, kept alive
+};
+
 struct NufftState {
     std::map<std::tuple<long long, long long, long long>, hipfftHandle> plans;
     std::map<std::pair<long long, long long>, hipfftHandle> plans1d;   // (length, batch): contiguous lines
     std::map<std::array<long long, 13>, PruneTables> prune;
+    std::map<std::array<long long, 12>, RealTables> real;
+    DevBuf pts_sorted, bins, place, wx, wy;                         // real-strength transform
     DevBuf work;                                                     // the y pass of the pruned transform
     std::map<std::tuple<long long, long long, int>, DevBuf> corr;   // (N, n, w) -> 1 / phihat on the device
     std::vector<std::vector<double>> corr_host;                      // sources of the uploads, kept alive
@@ -512,8 +800,11 @@ void nufft_release(dc_ctx *c) {
         for (DevBuf *b : {&t.L0, &t.L1, &t.P[0], &t.P[1], &t.P[2], &t.M[0], &t.M[1], &t.M[2]})
             if (b->p) (void)hipFree(b->p);
     }
+    for (auto &kv : s->real)
+        for (DevBuf &b : kv.second.b)
+            if (b.p) (void)hipFree(b.p);
     if (s->work.p) (void)hipFree(s->work.p);
-    for (DevBuf *b : {&s->grid, &s->pts[0], &s->pts[1], &s->pts[2], &s->c, &s->fk, &s->one, &s->pts2[0], &s->pts2[1],
+    for (DevBuf *b : {&s->pts_sorted, &s->bins, &s->place, &s->wx, &s->wy, &s->grid, &s->pts[0], &s->pts[1], &s->pts[2], &s->c, &s->fk, &s->one, &s->pts2[0], &s->pts2[1],
                       &s->pts2[2], &s->fk2})
         if (b->p) (void)hipFree(b->p);
     for (auto &kv : s->corr)
@@ -729,6 +1020,165 @@ int nu_transform3(dc_ctx *c, const NuParams &p, const double *const corr[3], dou
     return 0;
 }
 
+int real_tables(dc_ctx *c, const NuParams &p, const long long sub[3], const long long out[3], RealTables *&tp) {
+    NufftState &s = nu_state(c);
+    const std::array<long long, 12> key = {p.n[0], p.n[1], p.n[2], p.N[0], p.N[1], p.N[2],
+                                           sub[0], sub[1], sub[2], out[0], out[1], out[2]};
+    auto it = s.real.find(key);
+    if (it != s.real.end()) {
+        tp = &it->second;
+        return 0;
+    }
+    RealTables t;
+    auto mode = [&](int d, long long o) { return o * sub[d] - p.N[d] / 2; };
+    // output index of every mode, by fine index
+    std::vector<int> at[3];
+    for (int d = 0; d < 3; ++d) {
+        at[d].assign((size_t)p.n[d], -1);
+        for (long long o = 0; o < out[d]; ++o) at[d][(size_t)(((mode(d, o) % p.n[d]) + p.n[d]) % p.n[d])] = (int)o;
+    }
+    auto neg = [&](int d, int k) { return k ? (int)p.n[d] - k : 0; };
+    std::vector<int> v[8];
+    for (int k = 0; k <= (int)(p.n[0] / 2); ++k)
+        if (at[0][k] >= 0 || at[0][neg(0, k)] >= 0) {
+            v[0].push_back(k);
+            v[2].push_back(at[0][k]);
+            v[3].push_back(k == neg(0, k) ? -1 : at[0][neg(0, k)]);   // its own mirror is written once
+        }
+    v[1].assign((size_t)p.n[1], -1);
+    for (int k = 0; k < (int)p.n[1]; ++k)
+        if (at[1][k] >= 0 || at[1][neg(1, k)] >= 0) {
+            v[1][k] = (int)v[4].size();
+            v[4].push_back(at[1][k]);
+            v[5].push_back(at[1][neg(1, k)]);
+        }
+    for (int k = 0; k < (int)p.n[2]; ++k) {
+        v[6].push_back(at[2][k]);
+        v[7].push_back(at[2][neg(2, k)]);
+    }
+    t.c0 = (int)v[0].size();
+    t.c1 = (int)v[4].size();
+    for (int q = 0; q < 8; ++q) t.host.push_back(v[q]);
+    int st;
+    for (int q = 0; q < 8; ++q)
+        if ((st = upload(c, t.b[q], t.host[q].data(), t.host[q].size()))) return st;
+    tp = &s.real.emplace(key, std::move(t)).first->second;
+    return 0;
+}
+
+// Whether the real-strength path takes a transform: its kernel width, fine
+// grids that dc_fft.h transforms and that bins and tiles divide (lengths from
+// the kernel's reach on; the sizes of next_smooth are even), and points that
+// 32-bit counts hold.
+bool real_path(const NuParams &p, long long points) {
+    FftLen f;
+    if (p.dim != 3 || p.w != SW || points > (1LL << 27)) return false;
+    for (int d = 0; d < 3; ++d)
+        if (p.n[d] < 2 * SW || !fft_length(p.n[d], f)) return false;
+    return p.n[2] % TZ == 0;
+}
+
+// Sorts the points of the types into s.pts_sorted; bins of pair q from s.bins + q nby nbz.
+int real_sort(dc_ctx *c, const NuParams &p, const SortArgs &src, const std::vector<long long> &beg, const std::vector<double> &str) {
+    NufftState &s = nu_state(c);
+    const int ntype = (int)str.size();
+    SortArgs a = src;
+    for (int d = 0; d < 3; ++d) {
+        a.n[d] = (int)p.n[d];
+        a.scale[d] = (double)p.n[d] / (2.0 * 3.14159265358979323846);
+    }
+    a.nby = (a.n[1] + TY - 1) / TY;
+    a.nbz = a.n[2] / TZ;
+    a.beta = p.beta;
+    const long long nbin = (long long)((ntype + 1) / 2) * a.nby * a.nbz;
+    if (nbin > (1LL << 30)) return set_err(c, DC_ERR_ARG, DC_ER_LIB, "NUFFT: too many types for this grid");
+    int st;
+    if ((st = ensure(c, s.bins, sizeof(int) * (size_t)(nbin + 1)))) return st;
+    const size_t m = (size_t)std::max(1LL, beg[ntype] - beg[0]);
+    if ((st = ensure(c, s.place, sizeof(int2) * m)) || (st = ensure(c, s.pts_sorted, sizeof(SpreadPt) * m))) return st;
+    a.first = beg[0];
+    int *cnt = ptr<int>(s.bins);
+    zero_kernel<<<grid_for((nbin + 2) / 2), 256, 0, c->st>>>((nbin + 1) / 2, reinterpret_cast<double *>(cnt));
+    for (int pass = 0; pass < 2; ++pass) {
+        for (int t0 = 0; t0 < ntype; t0 += SORT_TYPES) {
+            a.type0 = t0;
+            a.ntype = std::min(SORT_TYPES, ntype - t0);
+            for (int t = 0; t <= a.ntype; ++t) a.beg[t] = beg[t0 + t];
+            for (int t = 0; t < a.ntype; ++t) a.s[t] = str[t0 + t];
+            const long long m = a.beg[a.ntype] - a.beg[0];
+            if (m <= 0) continue;
+            if (pass == 0)
+                sort_count_kernel<<<(unsigned)((m + 255) / 256), 256, 0, c->st>>>(a, cnt, ptr<int2>(s.place));
+            else
+                sort_scatter_kernel<<<(unsigned)((m * SW + 255) / 256), 256, 0, c->st>>>(a, cnt, ptr<int2>(s.place),
+                                                                                         ptr<SpreadPt>(s.pts_sorted));
+        }
+        if (pass == 0) sort_scan_kernel<<<1, 1024, 0, c->st>>>((int)nbin, cnt);
+        HIPCHK(hipGetLastError());
+    }
+    return 0;
+}
+
+// Pair q of the sorted types: spread and the x and y passes; planes of type 0
+// and 1 of the pair then in s.wy.
+int real_pair_xy(dc_ctx *c, const NuParams &p, RealTables &t, int pair, bool two) {
+    NufftState &s = nu_state(c);
+    FftLen f[2];
+    int st;
+    for (int d = 0; d < 2; ++d) {
+        (void)fft_length(p.n[d], f[d]);
+        if ((st = fft_table(c, f[d]))) return st;
+    }
+    const int k = two ? 2 : 1;
+    const size_t nx = (size_t)p.n[1] * p.n[2] * t.c0, ny = (size_t)p.n[2] * t.c1 * t.c0;
+    if ((st = ensure(c, s.wx, sizeof(double2) * nx * k)) || (st = ensure(c, s.wy, sizeof(double2) * ny * k))) return st;
+    SpreadXArgs a{};
+    for (int d = 0; d < 3; ++d) a.n[d] = (int)p.n[d];
+    a.nby = (a.n[1] + TY - 1) / TY;
+    a.nbz = a.n[2] / TZ;
+    a.start = ptr<int>(s.bins) + (long long)pair * a.nby * a.nbz;
+    a.pts = ptr<SpreadPt>(s.pts_sorted);
+    a.c0 = t.c0;
+    a.k0 = ptr<int>(t.b[0]);
+    a.a = ptr<double2>(s.wx);
+    a.b = two ? a.a + nx : nullptr;
+    const unsigned nb = (unsigned)a.nby * a.nbz;
+    if (fft_threads(f[0]) == 256)
+        spread_x_kernel<256, 0><<<nb, 256, fft_lds(f[0]), c->st>>>(f[0], a);   // no radix above 5
+    else if (f[0].kind == 0)
+        spread_x_kernel<512, 0><<<nb, 512, fft_lds(f[0]), c->st>>>(f[0], a);
+    else
+        spread_x_kernel<512, 1><<<nb, 512, fft_lds(f[0]), c->st>>>(f[0], a);
+    HIPCHK(hipGetLastError());
+    const unsigned tiles = (unsigned)(t.c0 + FFT_LINES - 1) / FFT_LINES;
+    const RealYOp y{a.a, ptr<double2>(s.wy), a.n[1], t.c0, t.c1, tiles, ptr<int>(t.b[1])};
+    HIPCHK(fft_launch(f[1], y, (long long)tiles * p.n[2] * k, c->st));
+    return 0;
+}
+
+// z pass of type `which` of the pair; op carries the output.
+int real_z(dc_ctx *c, const NuParams &p, RealTables &t, int which, const double *const corr[3], const long long sub[3],
+           const long long out[3], RealZOp op) {
+    NufftState &s = nu_state(c);
+    FftLen f;
+    (void)fft_length(p.n[2], f);
+    const int st = fft_table(c, f);
+    if (st) return st;
+    op.c0 = t.c0;
+    op.cc = t.c0 * t.c1;
+    op.in = ptr<double2>(s.wy) + (size_t)which * p.n[2] * op.cc;
+    const int **tab[6] = {&op.o1p, &op.o1m, &op.o2p, &op.o2m, &op.o3p, &op.o3m};
+    for (int q = 0; q < 6; ++q) *tab[q] = ptr<int>(t.b[2 + q]);
+    op.out0 = (int)out[0];
+    op.out1 = (int)out[1];
+    for (int d = 0; d < 3; ++d) {
+        op.corr[d] = corr[d];
+        op.sub[d] = sub[d];
+    }
+    HIPCHK(fft_launch(f, op, (op.cc + FFT_LINES - 1) / FFT_LINES, c->st));
+    return 0;
+}
+
 // Spread, transform, deconvolve; points/weights already on the device.
 int nufft_run(dc_ctx *c, const NuParams &p, long long M, const double *dx, const double *dy, const double *dz,
               const double2 *dc, int iflag, const long long sub[3], const long long out[3], double2 *dfk) {
@@ -777,8 +1227,10 @@ int nufft_run_real_pair(dc_ctx *c, const NuParams &p, long long ma, const double
     double *g = ptr<double>(s.grid);
     zero_kernel<<<grid_for(2 * ng), 256, 0, c->st>>>(2 * ng, g);
     const SpreadArgs a = spread_args(p);
-    if (ma > 0) launch_spread_real(p.w, c->st, a, ma, xa[0], xa[1], xa[2], sa, 0, g);
-    if (mb > 0) launch_spread_real(p.w, c->st, a, mb, xb[0], xb[1], xb[2], sb, 1, g);
+    // the run level's tolerance fixes the width
+    if (p.w != SW) return set_err(c, DC_ERR_ARG, DC_ER_LIB, "NUFFT: kernel width");
+    if (ma > 0) spread3_real_kernel<SW><<<grid_for(ma * SW), 256, 0, c->st>>>(a, ma, xa[0], xa[1], xa[2], sa, 0, g);
+    if (mb > 0) spread3_real_kernel<SW><<<grid_for(mb * SW), 256, 0, c->st>>>(a, mb, xb[0], xb[1], xb[2], sb, 1, g);
     HIPCHK(hipGetLastError());
     return nu_transform3(c, p, corr, g, iflag, sub, out, fa, mb > 0 ? fb : nullptr);
 }
@@ -854,6 +1306,20 @@ int dc_four_strucf_nufft_dev(dc_ctx *c, int dim, int64_t nat, const double *xpos
     if ((st = nu_params(c, dim, tol, N, p))) return st;
     HIPCHK(hipSetDevice(c->device));
     NufftState &s = nu_state(c);
+    if (nat > 0 && real_path(p, nat)) {
+        const double *corr[3];
+        hipfftHandle h;
+        RealTables *t = nullptr;
+        if ((st = nu_setup(c, p, corr, h, false)) || (st = real_tables(c, p, sub, out, t))) return st;
+        SortArgs sa{};
+        sa.x[0] = xpos;
+        sa.x[1] = ypos;
+        sa.x[2] = zpos;
+        if ((st = real_sort(c, p, sa, {0, nat}, {occ})) || (st = real_pair_xy(c, p, *t, 0, false))) return st;
+        RealZOp op{};
+        op.fk = reinterpret_cast<double2 *>(tcsf);
+        return real_z(c, p, *t, 0, corr, sub, out, op);
+    }
     if ((st = ensure(c, s.c, sizeof(double2) * (size_t)std::max<int64_t>(nat, 1)))) return st;
     occ_weights_kernel<<<grid_for(nat), 256, 0, c->st>>>(nat, occ, ptr<double2>(s.c));
     HIPCHK(hipGetLastError());
@@ -1045,7 +1511,6 @@ int dc_four_run_nufft_dev(dc_ctx *c, const dc_run_desc *r, const double *type_oc
     NufftState &s = nu_state(c);
     const long long ntot = (long long)g.n[0] * g.n[1] * g.n[2];
     if ((st = upload(c, c->cfact, r->cfact, 2 * (size_t)r->ncfact * c->nscat))) return st;
-    if ((st = ensure(c, s.fk, sizeof(double2) * (size_t)ntot))) return st;
     if ((st = ensure(c, c->csf, sizeof(double2) * (size_t)ntot))) return st;   // the sum over types
     double2 *acc = ptr<double2>(c->csf);
     const double pi = 3.14159265358979323846;
@@ -1062,9 +1527,52 @@ int dc_four_run_nufft_dev(dc_ctx *c, const dc_run_desc *r, const double *type_oc
     // the types with atoms, two per transform (real strengths cr_occ: one in
     // each component of the complex grid)
     std::vector<int> types;
+    long long points = 0;
     for (int t = 0; t < c->nscat; ++t)
-        if (c->type_beg[t + 1] > c->type_beg[t]) types.push_back(t);
-    if ((st = ensure(c, s.fk2, sizeof(double2) * (size_t)ntot))) return st;
+        if (c->type_beg[t + 1] > c->type_beg[t]) {
+            types.push_back(t);
+            points += c->type_beg[t + 1] - c->type_beg[t];
+            pairs += (double)(c->type_beg[t + 1] - c->type_beg[t]) * (double)ntot;
+        }
+    if (!types.empty() && real_path(p, points)) {
+        const double *corr[3];
+        hipfftHandle h;
+        if ((st = nu_setup(c, p, corr, h, false))) return st;
+        RealTables *t = nullptr;
+        if ((st = real_tables(c, p, sub, out, t))) return st;
+        SortArgs sa{};
+        sa.idx = ptr<int>(c->type_idx);
+        sa.pos = ptr<double>(c->pos);
+        std::vector<long long> beg;
+        std::vector<double> str;
+        for (int d = 0; d < 3; ++d) sa.fac[d] = fac[d];
+        for (int q : types) {
+            beg.push_back(c->type_beg[q]);   // types without atoms take no room
+            str.push_back(type_occ ? type_occ[q] : 1.0);
+        }
+        beg.push_back(c->type_beg[types.back() + 1]);
+        if ((st = real_sort(c, p, sa, beg, str))) return st;
+        RealZOp op{};
+        op.form = 1;
+        op.ncfact = r->ncfact;
+        op.g = g;
+        op.cfact = ptr<double2>(c->cfact);
+        op.fk = acc;
+        for (size_t q = 0; q < types.size(); q += 2) {
+            if (cancelled(c)) return set_err(c, DC_ERR_CANCEL, DC_ER_COMM, "cancelled");
+            const bool two = q + 1 < types.size();
+            if ((st = real_pair_xy(c, p, *t, (int)(q / 2), two))) return st;
+            for (int w = 0; w < (two ? 2 : 1); ++w) {
+                op.t = types[q + w];
+                op.first = first ? 1 : 0;
+                first = false;
+                if ((st = real_z(c, p, *t, w, corr, sub, out, op))) return st;
+            }
+        }
+        types.clear();
+    }
+    if (!types.empty() && ((st = ensure(c, s.fk, sizeof(double2) * (size_t)ntot)) || (st = ensure(c, s.fk2, sizeof(double2) * (size_t)ntot))))
+        return st;
     for (size_t q = 0; q < types.size(); q += 2) {
         if (cancelled(c)) return set_err(c, DC_ERR_CANCEL, DC_ER_COMM, "cancelled");
         const int ta = types[q], tb = q + 1 < types.size() ? types[q + 1] : -1;
@@ -1094,11 +1602,9 @@ int dc_four_run_nufft_dev(dc_ctx *c, const dc_run_desc *r, const double *type_oc
         form_acc_kernel<<<grid_for(ntot), 256, 0, c->st>>>(g, ta, r->ncfact, first ? 1 : 0, ptr<double2>(c->cfact),
                                                           ptr<double2>(s.fk), acc);
         first = false;
-        pairs += (double)na * (double)ntot;
         if (nb > 0) {
             form_acc_kernel<<<grid_for(ntot), 256, 0, c->st>>>(g, tb, r->ncfact, 0, ptr<double2>(c->cfact), ptr<double2>(s.fk2),
                                                               acc);
-            pairs += (double)nb * (double)ntot;
         }
         HIPCHK(hipGetLastError());
     }
