@@ -41,12 +41,19 @@
 // stage), so of the two waves of a SIMD one generates while the other
 // multiplies; the tables therefore live for three stages.
 //
+// FP32 operands are split into three BF16 parts, which hold all 24 bits, and
+// multiplied in six products; what is left out (second times third parts and
+// smaller) is below 2^-25 of a product, FP32's own rounding of it.  Six products on the BF16 units
+// take 3/8 of the time of the FP32 ones (v_mfma_f32_16x16x4_f32 before: 0.62 ->
+// 0.41 ms for 62,000 atoms x 33 x 65 x 65, now bound by the VALU work; error of F
+// against FP64 4.2e-8 -> 3.1e-8 on a 4,000-atom line, 5.1e-8 -> 4.0e-8 there).
+//
 // Bound: half matrix cores, half the VALU work of forming operands, which
 // overlaps with them only in part (FP16X3, 256 x 176: 47% of the MFMA peak
 // busy, 2.9 other VALU instructions per MFMA).  Measured against dc_gemm.hip:
-// 256,000 atoms x 81 x 161 x 161, FP16X3 10.06 -> 6.2-6.5 ms with equal
-// slices; 62,000 atoms x 33 x 65 x 65, FP32 1.38 -> 0.62 ms; an 8,000-atom
-// 101^2 layer, FP32 174 -> 19 us (with slices cut to fill the device); a
+// 256,000 atoms x 81 x 161 x 161, FP16X3 10.06 -> 6.1 ms with equal
+// slices; 62,000 atoms x 33 x 65 x 65, FP32 1.38 -> 0.41 ms; an 8,000-atom
+// 101^2 layer, FP32 174 -> 17 us (with slices cut to fill the device); a
 // population of 96 (1.8M atoms, 256^2, damped) 2.66 -> 1.6 ms.
 //
 // Epilogue: an even lane holds X and its neighbour Y of the same pair, so
@@ -102,7 +109,7 @@ struct alignas(16) FoldB {
 };
 template <class T>
 struct alignas(16) FoldB<SCH_FP32, T> {
-    alignas(16) float f[T::CT * FKS];       // fb_off
+    alignas(16) uint32_t p[3][T::CT * 16];  // three BF16 parts, pk_off
 };
 template <int SCHEME, class T>
 struct alignas(16) FoldSmem {
@@ -113,10 +120,6 @@ struct alignas(16) FoldSmem {
     float wmax[T::NW];
     int item;
 };
-
-// FP32 columns: 8 chunks of 4 atoms per column, XOR-swizzled so that 16
-// columns of one chunk fall on distinct banks
-__device__ __forceinline__ int fb_off(int col, int chunk) { return col * 32 + 4 * (chunk ^ ((col >> 1) & 7)); }
 
 // K of the operand scales, and its reciprocal to 1e-12: a range of 64 steps of
 // an FP16 hi half, of 20 of a BF16 one (over 8 steps the lo halves of the two
@@ -166,18 +169,28 @@ __device__ __forceinline__ void fold_tables(FoldTables<T> &tb, const int *__rest
     const int a16 = lane & 15, m = lane >> 4, a = 16 * (wave & 1) + a16;
     const uint64_t psi2 = (uint64_t)hash * 0xD6E8FEB86659FD93ull;
     const uint64_t wrp = s1A - (uint64_t)fg.PA * sA;
-    if (wave < 2) {
+    // Who builds what.  Evaluations of sin/cos a lane, by wave pair: FP32 4 | 4 | 3
+    // | 3 (128 x 96), split schemes 3 and their exchange | 5 | 3 | 3 (256 x 176).
+    // The column operands go to the first waves in FP32 and to the last ones in
+    // the split schemes (fold_b).  Measured, both orders of both: FP32 65^3 0.412 ms, with the split
+    // schemes' order 0.47, with both row tables on the first pair 0.42;
+    // FP16X3 161^3 6.1 ms, with the columns on the first waves 6.5, with
+    // the high groups spread as in FP32 6.5.
+    constexpr bool F32 = SCHEME == SCH_FP32;
+    if (wave == 0 || wave == 1) {
+        if (m == 0) tb.dmp[a] = live ? pad * 1.4426950408889634f : 0.0f;
+    }
+    if (wave < (F32 ? 4 : 2)) {
         float2 *t0 = reinterpret_cast<float2 *>(tb.al[0].v) + (a & 1);
         float2 *t1 = reinterpret_cast<float2 *>(tb.al[1].v) + (a & 1);
         const int q = 17 * (a >> 1);
-        if (m == 0) tb.dmp[a] = live ? pad * 1.4426950408889634f : 0.0f;
-        if constexpr (SCHEME == SCH_FP32) {
+        if constexpr (F32) {
+            const bool wrapped = wave >= 2;
+            if (wrapped && fg.PA >= fg.NA) return;
+            float2 *t = wrapped ? t1 : t0;
+            const uint64_t base = psi2 + (wrapped ? wrp : 0ull);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint64_t ph = (uint64_t)(m + 4 * j) * sA + psi2;
-                t0[2 * (q + m + 4 * j)] = fold_cis<SCHEME>(ph);
-                t1[2 * (q + m + 4 * j)] = fold_cis<SCHEME>(ph + wrp);
-            }
+            for (int j = 0; j < 4; ++j) t[2 * (q + m + 4 * j)] = fold_cis<SCHEME>((uint64_t)(m + 4 * j) * sA + base);
         } else {
             // helper m evaluates fold_cis<SCHEME>(m s + psi2), fold_cis<SCHEME>(4m s) and fold_cis<SCHEME>(4m s + w); the
             // four helpers of an atom exchange the last two (see dc_gemm.hip)
@@ -200,7 +213,8 @@ __device__ __forceinline__ void fold_tables(FoldTables<T> &tb, const int *__rest
         return;
     }
     const uint64_t half = (fg.NB & 1) ? 0ull : sB >> 1;
-    if (wave < 4) {
+    const int first = F32 ? 2 : 1;             // the wave pair with the low table of side B
+    if ((wave >> 1) == first) {
         float2 *t = reinterpret_cast<float2 *>(tb.bl) + (a & 1);
         const int q = 9 * (a >> 1);
         t[2 * (q + m)] = fold_cis<SCHEME>((uint64_t)m * sB + half + psi2);
@@ -210,7 +224,9 @@ __device__ __forceinline__ void fold_tables(FoldTables<T> &tb, const int *__rest
     const float ampA = SCHEME == SCH_FP32 ? 1.0f : fscale_k<SCHEME>() / r;
     const float ampB = live ? w * r : 0.0f;
     const uint64_t pa = p0 + (uint64_t)(fg.NB / 2) * sB - half + (uint64_t)a0 * sA + (uint64_t)hi0 * s1A - psi2 + frame;
-    for (int q = ((wave >> 1) - 1) * 4 + m; q < T::RH + T::CH; q += 12) {
+    // FP32: that pair takes one high group a lane, the last one the rest
+    const int step = !F32 ? 12 : (wave >> 1) == first ? T::RH + T::CH : 4;
+    for (int q = ((wave >> 1) - first) * 4 + m; q < T::RH + T::CH; q += step) {
         const bool isb = q >= T::RH;
         const int h = isb ? q - T::RH : q;
         const uint64_t ph = isb ? (uint64_t)(pair0 + 8 * h) * sB - psi2
@@ -232,6 +248,21 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 &hi, u32x4 &lo
         } else {
             const f32x2 h = unpack2<SCHEME>(hi[q]);
             lo[q] = pack2<SCHEME>(x[2 * q] - h.x, x[2 * q + 1] - h.y);
+        }
+    }
+}
+
+// FP32 values as three BF16 parts whose sum they are, exactly.
+__device__ __forceinline__ void split8_3(const float (&x)[8], u32x4 (&p)[3]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        float a = x[2 * q], b = x[2 * q + 1];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            p[k][q] = pack2<SCH_BF16X3>(a, b);
+            const f32x2 h = unpack2<SCH_BF16X3>(p[k][q]);
+            a -= h.x;
+            b -= h.y;
         }
     }
 }
@@ -268,7 +299,7 @@ struct FoldA {
 };
 template <int WR>
 struct FoldA<SCH_FP32, WR> {
-    float re[WR][8], im[WR][8];
+    u32x4 re[WR][3], im[WR][3];
 };
 
 template <int SCHEME, class T, bool DAMP>
@@ -278,11 +309,12 @@ __device__ __forceinline__ void fold_a(FoldA<SCHEME, T::WR> &A, const FoldTables
     for (int i = 0; i < T::WR; ++i) {
         const float4 *tl = tb.al[0].v + dsel[i] + 17 * 4 * lg + li;
         const float4 *th = reinterpret_cast<const float4 *>(tb.ah + (wave * T::WR + i) * FKS + 8 * lg);
+        float re[8], im[8];
+        elems8<DAMP>(tl, 17, th, tb.dmp + 8 * lg, sv[i], re, im);
         if constexpr (SCHEME == SCH_FP32) {
-            elems8<DAMP>(tl, 17, th, tb.dmp + 8 * lg, sv[i], A.re[i], A.im[i]);
+            split8_3(re, A.re[i]);
+            split8_3(im, A.im[i]);
         } else {
-            float re[8], im[8];
-            elems8<DAMP>(tl, 17, th, tb.dmp + 8 * lg, sv[i], re, im);
             split8<SCHEME>(re, A.rh[i], A.rl[i]);
             split8<SCHEME>(im, A.ih[i], A.il[i]);
         }
@@ -296,7 +328,7 @@ template <int SCHEME, class T, bool DAMP>
 __device__ __forceinline__ void fold_b(FoldB<SCHEME, T> &bb, const FoldTables<T> &tb, const float *__restrict__ s_b,
                                        int wave, int lane) {
     const int l = lane & 7, g = (lane >> 3) & 3, hs = lane >> 5;
-    for (int jp = wave; jp < (T::CH + 1) / 2; jp += T::NW) {
+    for (int jp = SCHEME == SCH_FP32 ? wave : T::NW - 1 - wave; jp < (T::CH + 1) / 2; jp += T::NW) {
         const int h = 2 * jp + hs;
         if (h < T::CH) {
             float re[8], im[8];
@@ -312,8 +344,10 @@ __device__ __forceinline__ void fold_b(FoldB<SCHEME, T> &bb, const FoldTables<T>
                 for (int k = 0; k < 8; ++k) x[k] = sn ? im[k] : re[k];
                 const int col = c0 + (sn ? 1 : 0);
                 if constexpr (SCHEME == SCH_FP32) {
-                    *reinterpret_cast<f32x4 *>(&bb.f[fb_off(col, 2 * g)]) = f32x4{x[0], x[1], x[2], x[3]};
-                    *reinterpret_cast<f32x4 *>(&bb.f[fb_off(col, 2 * g + 1)]) = f32x4{x[4], x[5], x[6], x[7]};
+                    u32x4 p[3];
+                    split8_3(x, p);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4 *>(&bb.p[q][pk_off(col, g)]) = p[q];
                 } else {
                     u32x4 hi, lo;
                     split8<SCHEME>(x, hi, lo);
@@ -338,25 +372,27 @@ template <int SCHEME, class T>
 __device__ __forceinline__ void fold_mfma(const FoldB<SCHEME, T> &bb, const FoldA<SCHEME, T::WR> &A,
                                           f32x4 (&accR)[T::WR][T::WC], f32x4 (&accI)[T::WR][T::WC], int li, int lg) {
     if constexpr (SCHEME == SCH_FP32) {
-        f32x4 y0 = *reinterpret_cast<const f32x4 *>(&bb.f[fb_off(li, 2 * lg)]);
-        f32x4 y1 = *reinterpret_cast<const f32x4 *>(&bb.f[fb_off(li, 2 * lg + 1)]);
+        u32x4 y[3], n[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) y[q] = *reinterpret_cast<const u32x4 *>(&bb.p[q][pk_off(li, lg)]);
 #pragma unroll
         for (int j = 0; j < T::WC; ++j) {
-            const int cn = 16 * (j + 1 < T::WC ? j + 1 : j) + li;
-            const f32x4 n0 = *reinterpret_cast<const f32x4 *>(&bb.f[fb_off(cn, 2 * lg)]);
-            const f32x4 n1 = *reinterpret_cast<const f32x4 *>(&bb.f[fb_off(cn, 2 * lg + 1)]);
+            if (j + 1 < T::WC)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) n[q] = *reinterpret_cast<const u32x4 *>(&bb.p[q][pk_off(16 * (j + 1) + li, lg)]);
             __builtin_amdgcn_sched_barrier(0);
+            // the small products first: those of the second and third parts are below FP32's rounding
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const float y = k < 4 ? y0[k & 3] : y1[k & 3];
+            for (int s = 2; s >= 0; --s)
 #pragma unroll
-                for (int i = 0; i < T::WR; ++i) {
-                    accR[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(A.re[i][k], y, accR[i][j], 0, 0, 0);
-                    accI[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(A.im[i][k], y, accI[i][j], 0, 0, 0);
-                }
-            }
-            y0 = n0;
-            y1 = n1;
+                for (int q = s; q >= 0; --q)
+#pragma unroll
+                    for (int i = 0; i < T::WR; ++i) {
+                        accR[i][j] = mfma_k32<SCH_BF16X3>(A.re[i][s - q], y[q], accR[i][j]);
+                        accI[i][j] = mfma_k32<SCH_BF16X3>(A.im[i][s - q], y[q], accI[i][j]);
+                    }
+#pragma unroll
+            for (int q = 0; q < 3; ++q) y[q] = n[q];
         }
     } else {
         u32x4 yh = *reinterpret_cast<const u32x4 *>(&bb.hi[pk_off(li, lg)]);
