@@ -50,8 +50,10 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 METRIC = "atom·hkl pairs/s, split-BF16 MFMA vs plain FP32 HIP, at ≤1e-5 rel err vs FP64"
-PEAK = {"bf16x3": 2500.0, "fp16x3": 2500.0, "fp16x2": 2500.0, "fp32": 157.3}   # TFLOP/s dense
-KSPLIT = {"bf16x3": 3, "fp16x3": 3, "fp16x2": 2, "fp32": 1}
+# TFLOP/s dense of the units each scheme's products run on (FP32: BF16, three parts, six products)
+PEAK = {"bf16x3": 2500.0, "fp16x3": 2500.0, "fp16x2": 2500.0, "fp32": 2500.0}
+# matrix flops per computed pair: 4 (mirrored points share theirs) or, in fp16x2, 8, times the products of the split
+MFMA_FLOPS = {"bf16x3": 12.0, "fp16x3": 12.0, "fp16x2": 16.0, "fp32": 24.0}
 HBM_PEAK = 8000.0   # GB/s
 SHIFT = np.array([0.37, -0.21, 0.113])   # general origin shift of the coherent-sum check
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "phase_gemm_fcc40_161cube_traffic.md")
@@ -205,8 +207,8 @@ def bench_nufft(_lib, torch, c, steps=3):
             "tol": 1e-7, "max_rel_err_sampled": None,
             "_samples": {0.0: dsi[::4, ::4, 80].copy(), 1.0: dsi[::4, ::4, 100].copy()},
             "note": "four_run_nufft on the headline workload: types in pairs, real spread of each type "
-                    "(exponential-of-semicircle, w=8) into one component of a 324^3 complex grid, pruned 3D transform "
-                    "(hipFFT 1D passes, gather-transposes of the needed modes), Hermitian separation and deconvolution, "
+                    "(exponential-of-semicircle, w=8) on lines of a 324^3 grid in LDS, transformed there, Hermitian "
+                    "separation, pruned y and z passes with deconvolution and "
                     "form factor; sum over types and |F|^2; FP64"}
 
 
@@ -280,7 +282,7 @@ def bench_batch(_lib, X, FR, prec, torch):
         out[key] = {"step_ms": ms, "pairs_per_s": pairs / (ms * 1e-3), "call_ms": tot,
                     "info": pop.ctx.batch_info()}
         if not want_grad:
-            fl = 8.0 * KSPLIT[prec] * pairs
+            fl = MFMA_FLOPS[prec] * pairs
             out[key]["mfma_frac_of_peak"] = round(fl / (ms * 1e-3) / 1e12 / PEAK[prec], 4)
             out[key]["gemm_ms_tuned"] = rows[0]["gemm_ms"]
     pop.ctx.close()
@@ -382,21 +384,21 @@ def main():
         dm = d_dsi.view(inc[2], inc[1], inc[0]).cpu().numpy()
         coherent_samples[prec] = {0.0: dm[80, ::4, ::4].T.copy(), 1.0: dm[100, ::4, ::4].T.copy()}
 
-    # dominant kernel: the phase GEMM; algorithmic MFMA flops = 8 x k_split per
+    # dominant kernel: the phase GEMM; algorithmic MFMA flops (MFMA_FLOPS) per
     # computed atom.hkl pair (the GEMM computes the Friedel-reduced region)
     fnum0 = (inc[0] + 1) // 2
     pairs_computed_per_launch = natoms * fnum0 * inc[1] * inc[2] / launches_per_step
-    achieved = 8.0 * KSPLIT[args.prec] * pairs_computed_per_launch / (gemm_launch_ms * 1e-3) / 1e12
+    achieved = MFMA_FLOPS[args.prec] * pairs_computed_per_launch / (gemm_launch_ms * 1e-3) / 1e12
     roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK[args.prec], "unit": "TFLOP/s",
                 "frac": round(achieved / PEAK[args.prec], 4), "traffic": traffic_from_profile(args.prec),
-                "kernel": f"phase_gemm_kernel<{args.prec}>", "avg_launch_ms": round(gemm_launch_ms, 3),
-                "flops_per_launch": 8.0 * KSPLIT[args.prec] * pairs_computed_per_launch,
+                "kernel": f"{'phase_gemm' if args.prec == 'fp16x2' else 'fold_gemm'}_kernel<{args.prec}>", "avg_launch_ms": round(gemm_launch_ms, 3),
+                "flops_per_launch": MFMA_FLOPS[args.prec] * pairs_computed_per_launch,
                 "fp32_kernel": {"avg_launch_ms": round(g32, 3),
-                                "achieved": round(8.0 * pairs_computed_per_launch / (g32 * 1e-3) / 1e12, 2),
+                                "achieved": round(MFMA_FLOPS["fp32"] * pairs_computed_per_launch / (g32 * 1e-3) / 1e12, 2),
                                 "peak": PEAK["fp32"]}}
     for prec, o in others.items():
         roofline[f"{prec}_kernel"] = {"avg_launch_ms": round(o["gemm_ms"], 3),
-                                      "achieved": round(8.0 * KSPLIT[prec] * pairs_computed_per_launch
+                                      "achieved": round(MFMA_FLOPS[prec] * pairs_computed_per_launch
                                                         / (o["gemm_ms"] * 1e-3) / 1e12, 2),
                                       "peak": PEAK[prec]}
 
@@ -441,7 +443,7 @@ def main():
         finally:
             pctx.close()
         mkey = {"bf16x3": "mfma_bf16_tflops", "fp16x3": "mfma_f16_tflops", "fp16x2": "mfma_f16_tflops",
-                "fp32": "mfma_f32_tflops"}[args.prec]
+                "fp32": "mfma_bf16_tflops"}[args.prec]
         roofline["measured_ceilings"] = {k: round(v, 2) if isinstance(v, float) else v for k, v in pk.items()}
         roofline["frac_of_measured_ceiling"] = round(roofline["achieved"] / pk[mkey], 4)
         log(f"peaks: {json.dumps(roofline['measured_ceilings'])}")
