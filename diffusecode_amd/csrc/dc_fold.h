@@ -76,10 +76,11 @@ struct FoldCfg {
 
 // Fold tiles (WR, WC), in the order of their tile indices.  Grids of 2^k + 1
 // points have 17, 33, 65 pairs: WC 3, 5 and 9 hold them with one group to spare
-// where 2, 6 and 11 take another tile or leave 31 and 26% of it empty.
+// where 2, 6 and 11 take another tile or leave 31 and 26% of it empty; 101 and
+// 201 points (51 and 101 pairs) fill 90% of one and two tiles of WC 7, 79% of 8.
 #define DC_FOLD_TILES(X) \
     X(0, 2, 11) X(1, 1, 11) X(2, 2, 8) X(3, 1, 8) X(4, 2, 6) X(5, 1, 6) X(6, 2, 4) X(7, 1, 4) X(8, 1, 2) X(9, 2, 9) X(10, 1, 9) \
-    X(11, 1, 5) X(12, 1, 3)
+    X(11, 1, 5) X(12, 1, 3) X(13, 2, 7)
 // FP32 holds FP64 sums beside its accumulators: 24 WR WC registers
 constexpr bool fold_built(int scheme, int wr, int wc) {
     return split3(scheme) || (scheme == SCH_FP32 && wr == 1 && wc <= 6);

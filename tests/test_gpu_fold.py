@@ -27,7 +27,7 @@ def ctx():
 
 
 def fold_tiles():
-    return range(TILE0, TILE0 + 13)
+    return range(TILE0, TILE0 + 14)
 
 
 @pytest.mark.parametrize("prec", ["fp32", "bf16x3", "fp16x3"])
