@@ -244,8 +244,16 @@ template <int NP, int NK>
 __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, int plane0, int nplane, const u32x4 *__restrict__ words) {
     constexpr int NW = 6 * NP, LD = (NW + AW - 1) / AW;
     __shared__ u32x4 sq_w[2][NW][64];
-    __shared__ float4 col[2][CT];          // s_c^2, j - jc, m - mc, scaled s_c^2 of the tile's columns
-    __shared__ float2 qcen[2][CT];         // Q of the centre row
+    // Values of a tile's columns: those of tile t + 1 are stored in the last
+    // k-step of tile t, before that step's barrier.  With two k-steps or more the
+    // barrier of the first one has let every wave out of the epilogue of tile t - 1,
+    // whose slot they may take.  With one k-step a slower wave may still be in it:
+    // three slots, of which tile t + 1 takes that of t - 2, whose epilogue every
+    // wave left before the barrier that ended tile t - 1.
+    constexpr int SLOTS = NK == 1 ? 3 : 2;
+    __shared__ float4 col[SLOTS][CT];      // s_c^2, j - jc, m - mc, scaled s_c^2 of the tile's columns
+    __shared__ float2 qcen[SLOTS][CT];     // Q of the centre row
+    auto slot_of = [](int ct) { return SLOTS == 2 ? ct & 1 : (int)((unsigned)ct % SLOTS); };
     const int4 tile = a.tiles[tile0 + blockIdx.y];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int li = lane & 15, lg = lane >> 4;
@@ -344,8 +352,8 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
     };
     auto put_col = [&](int ct) {
         if (threadIdx.x < CT) {
-            col[ct & 1][threadIdx.x] = make_float4(csq, (float)cj - a.jc, (float)cm - a.mc, csq * sg[2]);
-            qcen[ct & 1][threadIdx.x] = cq;
+            col[slot_of(ct)][threadIdx.x] = make_float4(csq, (float)cj - a.jc, (float)cm - a.mc, csq * sg[2]);
+            qcen[slot_of(ct)][threadIdx.x] = cq;
         }
     };
     if (ct0 < ct1) {
@@ -411,8 +419,8 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
         float d[WA][4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            w[v] = col[ct & 1][4 * lg + v];
-            qc[v] = qcen[ct & 1][4 * lg + v];
+            w[v] = col[slot_of(ct)][4 * lg + v];
+            qc[v] = qcen[slot_of(ct)][4 * lg + v];
 #pragma unroll
             for (int i = 0; i < WA; ++i) d[i][v] = 1.0f;
         }
