@@ -549,11 +549,37 @@ int dc_batch_info(const dc_ctx *c, int *tile, int *nwg, int *graph, double *tune
 
 namespace {
 
+// Whether the kernels of a step may work on the caller's arrays (pointer and
+// bytes of each; the first nin are inputs): memory of the context's device, and no output
+// that shares bytes with another array -- the reduction writes I before it
+// reads the target, several times over when the autotuner runs.
+struct Span {
+    const void *p;
+    size_t bytes;
+};
+bool in_place(const dc_ctx *c, const Span *s, int n, int nin) {
+    for (int x = 0; x < n; ++x) {
+        if (!s[x].p || !s[x].bytes) continue;
+        hipPointerAttribute_t at{};
+        if (hipPointerGetAttributes(&at, s[x].p) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (at.type != hipMemoryTypeDevice || at.device != c->device) return false;
+        const uintptr_t b = (uintptr_t)s[x].p, e = b + s[x].bytes;
+        for (int y = std::max(x + 1, nin); y < n; ++y)
+            if (s[y].p && b < (uintptr_t)s[y].p + s[y].bytes && (uintptr_t)s[y].p < e) return false;
+    }
+    return true;
+}
+
 // One population step.  dev = false: pos/occ/bdw of d, target, weight, icalc
 // and grad are host arrays, copied to and from the buffers that the replayed
-// graph works on; dev = true: they are device arrays, which the kernels of the
-// step, launched one by one, read and write in place (96 members, 1.8M atoms:
-// the copies moved 400 MB), and a non-null bdw counts as per-atom B.
+// graph works on.  dev = true: they are device arrays, and a non-null bdw counts
+// as per-atom B; the kernels of the step, launched one by one, read and write
+// them in place (96 members, 1.8M atoms: the copies moved 400 MB) where in_place
+// allows it, else they go through the state's buffers as host arrays do, all inputs
+// copied before the first kernel and the outputs after the last.
 int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const double *weight, double *chi2,
                double *icalc, double *grad, bool dev) {
     if (!c) return DC_ERR_ARG;
@@ -587,7 +613,11 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
     // plan's (1.8M atoms: 0.5 ms) and packs the form factors; other types
     // discard what was started.  Everything that was started stays inside the
     // state's buffers, whose sizes the shape fixes.
-    const bool early = dev && shape && c->batch->primed;
+    const size_t nd = sizeof(double), grid_bytes = nd * (size_t)d->nmembers * d->inc[0] * d->inc[1] * d->inc[2];
+    const Span spans[] = {{d->pos, 3 * nd * natoms}, {d->occ, nd * natoms}, {any_b ? d->bdw : nullptr, nd * natoms},
+                          {target, grid_bytes}, {weight, grid_bytes}, {icalc, grid_bytes}, {grad, 5 * nd * natoms}};
+    const bool direct = dev && in_place(c, spans, 7, 5);
+    const bool early = direct && shape && c->batch->primed;
     const StepIO io_dev{d->pos, d->occ, any_b ? d->bdw : nullptr, target, weight, icalc, grad};
     auto send_sq = [&](BatchState &b) -> int {
         std::memcpy(b.h_sq.p, sq.data(), sizeof(float) * sq.size());
@@ -625,7 +655,7 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
     BatchState &b = *c->batch;
     const bool started = early && fits;
     const size_t P = (size_t)b.g.P, M = (size_t)d->nmembers;
-    if (!dev) {
+    if (!direct) {
         const size_t T = (size_t)std::max<int64_t>(natoms, 1);
         if ((st = ensure(c, b.pos, sizeof(double) * 3 * T))) return st;
         if ((st = ensure(c, b.occ, sizeof(double) * T))) return st;
@@ -635,15 +665,17 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
         if (want_icalc && (st = ensure(c, b.icalc, sizeof(double) * P * M))) return st;
         if (want_grad && (st = ensure(c, b.grad, sizeof(double) * 5 * T))) return st;
     }
-    const StepIO io = dev ? io_dev : own_io(b);
+    const StepIO io = direct ? io_dev : own_io(b);
+    const hipMemcpyKind in = dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+    const hipMemcpyKind out = dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     if (!started) {
         HIPCHK(hipEventRecord(c->ev[0], c->st));
-        if (!dev) {
-            HIPCHK(hipMemcpyAsync(b.pos.p, d->pos, sizeof(double) * 3 * natoms, hipMemcpyHostToDevice, c->st));
-            HIPCHK(hipMemcpyAsync(b.occ.p, d->occ, sizeof(double) * natoms, hipMemcpyHostToDevice, c->st));
-            if (any_b) HIPCHK(hipMemcpyAsync(b.bdw.p, d->bdw, sizeof(double) * natoms, hipMemcpyHostToDevice, c->st));
-            HIPCHK(hipMemcpyAsync(b.target.p, target, sizeof(double) * P * M, hipMemcpyHostToDevice, c->st));
-            if (weight) HIPCHK(hipMemcpyAsync(b.weight.p, weight, sizeof(double) * P * M, hipMemcpyHostToDevice, c->st));
+        if (!direct) {
+            HIPCHK(hipMemcpyAsync(b.pos.p, d->pos, sizeof(double) * 3 * natoms, in, c->st));
+            HIPCHK(hipMemcpyAsync(b.occ.p, d->occ, sizeof(double) * natoms, in, c->st));
+            if (any_b) HIPCHK(hipMemcpyAsync(b.bdw.p, d->bdw, sizeof(double) * natoms, in, c->st));
+            HIPCHK(hipMemcpyAsync(b.target.p, target, sizeof(double) * P * M, in, c->st));
+            if (weight) HIPCHK(hipMemcpyAsync(b.weight.p, weight, sizeof(double) * P * M, in, c->st));
         }
         if ((st = send_sq(b))) return st;
     }
@@ -660,7 +692,7 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
         if ((st = autotune(c, b, io))) return st;
         b.primed = true;
     }
-    if (!dev && c->graphs && !b.exec) {
+    if (!direct && c->graphs && !b.exec) {
         HIPCHK(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
         st = enqueue(c, b, io, b.pl.tile, b.nwg, true, STEP_GEMM | STEP_REST, b.queue);
         hipGraph_t graph = nullptr;
@@ -674,14 +706,14 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
         HIPCHK(hipGraphInstantiate(&b.exec, b.graph, nullptr, nullptr, 0));
     }
     if (!started) HIPCHK(hipEventRecord(c->ev[4], c->st));
-    if (!dev && b.exec) {
+    if (!direct && b.exec) {
         HIPCHK(hipGraphLaunch(b.exec, c->st));
     } else {
         if ((st = enqueue(c, b, io, b.pl.tile, b.nwg, !started, started ? STEP_REST : STEP_GEMM | STEP_REST, b.queue))) return st;
     }
     HIPCHK(hipEventRecord(c->ev[5], c->st));
-    if (!dev && icalc) HIPCHK(hipMemcpyAsync(icalc, b.icalc.p, sizeof(double) * P * M, hipMemcpyDeviceToHost, c->st));
-    if (!dev && grad) HIPCHK(hipMemcpyAsync(grad, b.grad.p, sizeof(double) * 5 * natoms, hipMemcpyDeviceToHost, c->st));
+    if (!direct && icalc) HIPCHK(hipMemcpyAsync(icalc, b.icalc.p, sizeof(double) * P * M, out, c->st));
+    if (!direct && grad) HIPCHK(hipMemcpyAsync(grad, b.grad.p, sizeof(double) * 5 * natoms, out, c->st));
     HIPCHK(hipEventRecord(c->ev[1], c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     std::memcpy(chi2, b.h_chi.p, sizeof(double) * M);

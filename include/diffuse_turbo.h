@@ -366,7 +366,12 @@ int dc_batch_chi2(dc_ctx *ctx, const dc_batch_desc *batch, const double *target,
  * device pointers; atom_beg, type, cfact, rten and chi2 stay host arrays.
  * For a host loop that keeps a generation on the GPU (DIFFEV's trial
  * vectors built on the device); replaces the same per-member macro runs as
- * dc_batch_chi2.  Returns when chi2 is written. */
+ * dc_batch_chi2.  Work pending on the arrays on other streams must have
+ * finished.  Arrays on the context's device are read and written in place, by
+ * launches rather than a replayed graph, where icalc and grad share no memory
+ * with another array; otherwise every input is copied before the first kernel
+ * and the outputs after the last, icalc before grad, so an output may take an
+ * input's place.  Returns when chi2, icalc and grad are written. */
 int dc_batch_chi2_dev(dc_ctx *ctx, const dc_batch_desc *batch, const double *target, const double *weight,
                       double *chi2, double *icalc, double *grad);
 /* Autotuner and hipGraph capture of batch calls (both on by default).  The
