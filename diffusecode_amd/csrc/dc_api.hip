@@ -323,11 +323,9 @@ Plan plan_gemm(Grid &g, int forced, int only_mapping, int prec, long long natoms
     const int nt = gemm_num_tiles();
     const int ncu = device_cu_count();
     const bool acc64 = prec == SCHEME_FP32_ACC64;
-    // The folded side needs a mapping that leaves it unwrapped.  FP16X2, whose
-    // results are only good to their rounding, and the FP64-sum scheme keep the
-    // general tiles.
-    const bool can_fold = !acc64 && prec != DC_PREC_FP16X2 && (((fold_mask & FOLD_COLS) && (g.f[2] <= 1 || only_mapping != 0)) ||
-                                     ((fold_mask & FOLD_ROWS) && only_mapping != 1));
+    // The folded side needs a mapping that leaves it unwrapped.
+    const bool can_fold = scheme_folds(prec) && (((fold_mask & FOLD_COLS) && (g.f[2] <= 1 || only_mapping != 0)) ||
+                                                 ((fold_mask & FOLD_ROWS) && only_mapping != 1));
     if (forced >= 0) {
         const TileInfo ti = gemm_tile_info(forced);
         if ((ti.fold && !can_fold) || (acc64 && !ti.acc64) || (prec == DC_PREC_FP32 && ti.no_fp32)) forced = -1;

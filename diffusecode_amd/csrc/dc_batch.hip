@@ -435,7 +435,7 @@ int autotune(dc_ctx *c, BatchState &b, const StepIO &io) {
     const bool fp32_only = b.prec == DC_PREC_FP32;    // tiles built without an FP32 variant are skipped
     auto built = [&](int t) {
         const TileInfo ti = gemm_tile_info(t);
-        return !(fp32_only && ti.no_fp32) && !(ti.fold && !fold_side(b.pl.gg, b.fold_mask, t));
+        return !(fp32_only && ti.no_fp32) && !(ti.fold && !(scheme_folds(b.pl.scheme) && fold_side(b.pl.gg, b.fold_mask, t)));
     };
     // predicted cost: microseconds of the planner's model where a side can be
     // folded (the fold tiles alone are candidates then), else padded work

@@ -89,6 +89,10 @@ struct TileInfo {
 // with FP64 partial sums, which writes two planes (hi, lo) per slice.
 constexpr int SCHEME_FP32_ACC64 = 4;
 inline int planes_per_slice(int scheme) { return scheme == SCHEME_FP32_ACC64 ? 2 : 1; }
+// Schemes that have mirrored-pair tiles.  FP16X2, whose results are only good to
+// their rounding, and the FP64-sum scheme keep the general tiles; a forced tile
+// without a kernel for the call's scheme is ignored.
+inline bool scheme_folds(int scheme) { return scheme != 2 && scheme != SCHEME_FP32_ACC64; }
 
 struct ReduceArgs {
     Grid g;
