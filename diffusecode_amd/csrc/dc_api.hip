@@ -374,6 +374,28 @@ Plan plan_gemm(Grid &g, int forced, int only_mapping, int prec, long long natoms
     return best;
 }
 
+void split_sq(const double *rten, const double *eck, const double *vi, const GemmGeom &gg, int f1, float *out) {
+    auto dot = [&](const double *a, const double *b) {
+        double s = 0.0;
+        for (int r = 0; r < 3; ++r)
+            for (int k = 0; k < 3; ++k) s += a[r] * (rten[r + 3 * k] + rten[k + 3 * r]) * b[k];
+        return 0.125 * s;
+    };
+    // quadratic forms of the indices
+    const double *v1 = vi, *v2 = vi + 3, *v3 = vi + 6;
+    const double c0 = dot(eck, eck), c1 = 2.0 * dot(v1, eck), c11 = dot(v1, v1);
+    const double c2 = 2.0 * dot(v2, eck), c22 = dot(v2, v2), c3 = 2.0 * dot(v3, eck), c33 = dot(v3, v3), c23 = 2.0 * dot(v2, v3);
+    auto row = [&](int i) { return c0 + i * (c1 + i * c11); };
+    double least = row(0);
+    for (int i = 1; i < gg.R; ++i) least = std::min(least, row(i));
+    for (int i = 0; i < gg.R; ++i) out[i] = (float)(row(i) - least);
+    for (int l = 0; l * gg.C0 < gg.C; ++l) {
+        const double top = least + l * (c3 + l * c33), lin = c2 + l * c23;
+        float *o = out + gg.R + l * gg.C0;
+        for (int j = 0; j < gg.C0; ++j) o[j] = j < f1 ? (float)(top + j * (lin + j * c22)) : 0.0f;
+    }
+}
+
 int mirrored_sides(const GemmGeom &gg, const float *sq) {
     auto mirrored = [](const float *v, int n) {
         float top = 0.0f;

@@ -129,7 +129,7 @@ int member_sq(dc_ctx *c, const Grid &g, const GemmGeom &gg, const dc_batch_desc 
     top_bin = 0;
     const int stride = gg.R + gg.C;
     sq.assign((size_t)stride * d->nmembers, 0.0f);
-    const double *v1 = d->vi, *v2 = d->vi + 3, *v3 = d->vi + 6;
+    const double *v1 = d->vi;
     for (int m = 0; m < d->nmembers; ++m) {
         const double *G = d->rten + 9 * m;
         if (need_sep) {
@@ -142,19 +142,7 @@ int member_sq(dc_ctx *c, const Grid &g, const GemmGeom &gg, const dc_batch_desc 
                     return set_err(c, DC_ERR_ARG, DC_ER_LIB, "batch: vi(:,1) not metric-orthogonal to vi(:,2), vi(:,3)");
             }
         }
-        float *s = sq.data() + (size_t)stride * m;
-        for (int i = 0; i < gg.R; ++i) {
-            double h[3];
-            for (int k = 0; k < 3; ++k) h[k] = d->eck[k] + i * v1[k];
-            s[i] = (float)(dotg(h, G, h) / 4.0);
-        }
-        for (int col = 0; col < gg.C; ++col) {
-            const int j = col % gg.C0, l = col / gg.C0;
-            if (j >= g.f[1]) continue;
-            double v[3];
-            for (int k = 0; k < 3; ++k) v[k] = j * v2[k] + l * v3[k];
-            s[gg.R + col] = (float)((dotg(v, G, v) + 2.0 * dotg(v, G, d->eck)) / 4.0);
-        }
+        split_sq(G, d->eck, d->vi, gg, g.f[1], sq.data() + (size_t)stride * m);
         Grid gm = g;
         for (int k = 0; k < 9; ++k) gm.rten[k] = G[k];
         top_bin = std::max(top_bin, max_corner_bin(gm));

@@ -105,7 +105,7 @@ struct alignas(16) FoldTables {
     alignas(16) float2 ah[T::RH * FKS];
     alignas(16) float4 bl[16 * 9];          // side B, 8 pairs
     alignas(16) float2 bh[T::CH * FKS];
-    alignas(16) float dmp[FKS];             // B_n log2(e) (damped variant)
+    alignas(16) float dmp[FKS];             // (B_n - the slice's reference) log2(e) (damped variant)
 };
 template <int SCHEME, class T>
 struct alignas(16) FoldB {
@@ -123,6 +123,9 @@ struct alignas(16) FoldSmem {
     int k16[T::RH], wpos[T::RH];
     float s_b[T::JT];
     float wmax[T::NW];
+    float bmin[T::NW];                      // damped FP16: least B by wave, factors put back
+    alignas(16) float back_a[T::RT];
+    float back_b[T::JT];
     int item;
 };
 
@@ -170,7 +173,7 @@ template <int SCHEME, class T>
 __device__ __forceinline__ void fold_tables(FoldTables<T> &tb, const int *__restrict__ k16s, uint64_t p0, uint64_t sA,
                                             uint64_t s1A, uint64_t sB, float w, float pad, bool live, int a0, int hi0,
                                             const FoldGeom &fg, int pair0, int wave, int lane, uint32_t hash,
-                                            uint64_t frame) {
+                                            uint64_t frame, float bref) {
     const int a16 = lane & 15, m = lane >> 4, a = 16 * (wave & 1) + a16;
     const uint64_t psi2 = (uint64_t)hash * 0xD6E8FEB86659FD93ull;
     const uint64_t wrp = s1A - (uint64_t)fg.PA * sA;
@@ -183,7 +186,7 @@ __device__ __forceinline__ void fold_tables(FoldTables<T> &tb, const int *__rest
     // the high groups spread as in FP32 6.5.
     constexpr bool F32 = SCHEME == SCH_FP32;
     if (wave == 0 || wave == 1) {
-        if (m == 0) tb.dmp[a] = live ? pad * 1.4426950408889634f : 0.0f;
+        if (m == 0) tb.dmp[a] = live && w != 0.0f ? pad * 1.4426950408889634f - bref : 0.0f;
     }
     if (wave < (F32 ? 4 : 2)) {
         float2 *t0 = reinterpret_cast<float2 *>(tb.al[0].v) + (a & 1);
@@ -480,6 +483,8 @@ fold_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice_
         float sv[WR];
 #pragma unroll
         for (int i = 0; i < WR; ++i) sv[i] = 0.0f;
+        constexpr bool SCALED = DAMP && f16ops(SCHEME);   // damp_back
+        float bref = 0.0f;
         if constexpr (DAMP) {
             const float *sqs = sq + (slice_sq ? slice_sq[slice] : 0);
             const float *sa = sqs + (fg.swap ? g.R : 0), *sb = sqs + (fg.swap ? 0 : g.R);
@@ -528,22 +533,37 @@ fold_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice_
             const uint64_t frame = TWO ? fold_frame(slice, st >> 1, g.dither) : 0;
             fold_tables<SCHEME, T>(sm.t[st % 3], sm.k16, r.p0, fg.swap ? r.ca : r.ra, fg.swap ? r.ca1 : r.ra1,
                                    fg.swap ? r.ra : r.ca, r.w * sm.wmax[0], r.pad, k < kend, a0, hi0, fg, pair0, wave, lane,
-                                   hash, frame);
+                                   hash, frame, bref);
         };
         const AtomRec r0 = fetch(0), r1 = fetch(nst > 1 ? 1 : 0);
         AtomRec rn = fetch(nst > 2 ? 2 : 0);
         // FP16 schemes: amplitudes scaled by a power of two, undone in the epilogue
         float wscale = 1.0f, wunscale = 1.0f;
         if constexpr (f16ops(SCHEME)) {
-            float m = 0.0f;
-            for (int k = kbeg + (int)threadIdx.x; k < kend; k += T::NT) m = fmaxf(m, fabsf(rec[k].w));
+            float m = 0.0f, b = NO_B;
+            for (int k = kbeg + (int)threadIdx.x; k < kend; k += T::NT) {
+                const float wk = rec[k].w;
+                m = fmaxf(m, fabsf(wk));
+                if constexpr (SCALED) b = wk != 0.0f ? fminf(b, rec[k].pad) : b;
+            }
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-            if (lane == 0) sm.wmax[wave] = m;
+            for (int o = 32; o > 0; o >>= 1) {
+                m = fmaxf(m, __shfl_xor(m, o));
+                if constexpr (SCALED) b = fminf(b, __shfl_xor(b, o));
+            }
+            if (lane == 0) {
+                sm.wmax[wave] = m;
+                if constexpr (SCALED) sm.bmin[wave] = b;
+            }
             __syncthreads();
             m = 0.0f;
 #pragma unroll
             for (int w = 0; w < T::NW; ++w) m = fmaxf(m, sm.wmax[w]);
+            if constexpr (SCALED) {
+#pragma unroll
+                for (int w = 0; w < T::NW; ++w) b = fminf(b, sm.bmin[w]);
+                bref = damp_ref(b);
+            }
             if (m > 0.0f && m <= 3.0e38f) {
                 int e = 0;
                 (void)frexpf(m, &e);
@@ -560,6 +580,12 @@ fold_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice_
             dsel[i] = fg.PA < fg.NA && li >= sm.wpos[wave * WR + i] ? (int)(sizeof(FoldLow) / sizeof(float4)) : 0;
         FoldA<SCHEME, WR> A{};
         const bool mfma_first = ((wave >> 2) & 1) != 0;
+        if constexpr (SCALED) {
+#pragma unroll
+            for (int i = 0; i < WR; ++i)
+                if (lg == 0) sm.back_a[16 * (wave * WR + i) + li] = damp_back(bref, sv[i]);
+            for (int x = threadIdx.x; x < T::JT; x += T::NT) sm.back_b[x] = damp_back(bref, sm.s_b[x]);
+        }
         tables(0, r0);
         __syncthreads();
         if (nst > 1) tables(1, r1);
@@ -623,11 +649,18 @@ fold_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice_
         const bool wide = fg.sr == 1 && (fg.sc & 1) == 0;
         if (active) {
 #pragma unroll
-            for (int i = 0; i < WR; ++i)
+            for (int i = 0; i < WR; ++i) {
+                f32x4 backa{};
+                if constexpr (SCALED) {
+                    backa = *reinterpret_cast<const f32x4 *>(&sm.back_a[16 * (wave * WR + i) + 4 * lg]);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) backa[v] *= undo * frow_m_undo(v) * last;
+                }
 #pragma unroll
                 for (int j = 0; j < WC; ++j) {
                     const int pr = pair0 + 8 * j + (li >> 1);
                     float2 f[4];
+                    const float backb = SCALED ? sm.back_b[8 * j + (li >> 1)] : 1.0f;
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
                         const float xr = accR[i][j][v], xi = accI[i][j][v];
@@ -635,6 +668,8 @@ fold_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice_
                         const float re = odd ? yr + xi : xr - yi, im = odd ? yi - xr : xi + yr;
                         if constexpr (SCHEME == SCH_FP32) {
                             f[v] = make_float2(re, im);
+                        } else if constexpr (SCALED) {
+                            f[v] = make_float2(re * backa[v] * backb, im * backa[v] * backb);
                         } else {
                             const float um = frow_m_undo(v);
                             f[v] = make_float2(re * undo * um * last, im * undo * um * last);
@@ -654,6 +689,7 @@ fold_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice_
                             if (r4 + v < fg.NA) p[(long long)v * fg.sr] = f[v];
                     }
                 }
+            }
         }
     }
 }

@@ -116,7 +116,7 @@ struct alignas(16) Tables {
     alignas(16) float2 ah[T::RH * KS];
     alignas(16) float2 bl[2][16 * KS];
     alignas(16) float2 bh[T::CH * KS];
-    float dmp[KS];                      // B_n log2(e) of the stage's atoms (damped variant)
+    float dmp[KS];                      // (B_n - the slice's reference) log2(e) of the stage's atoms (damped variant)
 };
 
 template <int SCHEME, class T>
@@ -127,6 +127,7 @@ struct alignas(16) Smem {
     int b_k16[T::CH], b_wpos[T::CH];
     float s_a[T::RT], s_b[T::CT];      // s^2 row / column parts of the tile (damped variant)
     float wmax[T::NW];                 // per-wave max |w| of the slice (FP16 schemes)
+    float bmin[T::NW];                 // and least B (damped)
 };
 
 // Side geometry of the tile: start index, offset along the fast axis, period.
@@ -167,7 +168,7 @@ template <class T, bool SPLIT>
 __device__ __forceinline__ void build_tables(Tables<T> &tb, const int *__restrict__ a_k16,
                                              const int *__restrict__ b_k16, const AtomRec &ar, bool live,
                                              const Side &sa, const Side &sb, int pt, float wscale, uint32_t katom,
-                                             uint32_t salt, bool padh) {
+                                             uint32_t salt, bool padh, float bref) {
     const int a = pt & (KS - 1), r = pt >> 4;
     constexpr int NR = T::NPT / KS;           // helper threads per atom
     static_assert(NR > 8, "the low tables take waves 0 and 1, the high rows need more threads");
@@ -184,7 +185,7 @@ __device__ __forceinline__ void build_tables(Tables<T> &tb, const int *__restric
         psi = dither_turn(katom, salt);
     }
     const uint64_t psi2 = psi * 0xD6E8FEB86659FD93ull;
-    if (r == 0) tb.dmp[a] = live ? ar.pad * 1.4426950408889634f : 0.0f;
+    if (r == 0) tb.dmp[a] = live && ar.w != 0.0f ? ar.pad * 1.4426950408889634f - bref : 0.0f;
     if (r < 8) {
         const bool sideb = r >= 4;
         const int m = r & 3;
@@ -631,13 +632,24 @@ phase_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice
         AtomRec rn = fetch(nst > 2 ? 2 : 0);
         // FP16 schemes: B amplitudes of the slice scaled by 2^-e, max |w| = f 2^e
         // with f in [0.5, 1); the epilogue multiplies by 2^e (both exact)
-        float wscale = 1.0f, wunscale = 1.0f;
+        float wscale = 1.0f, wunscale = 1.0f, bref = 0.0f;
+        constexpr bool SCALED = DAMP && f16ops(SCHEME);   // damp_back
         if constexpr (f16ops(SCHEME)) {
-            float m = 0.0f;
-            for (int k = kbeg + pt; k < kend; k += T::NT) m = fmaxf(m, fabsf(rec[k].w));
+            float m = 0.0f, b = NO_B;
+            for (int k = kbeg + pt; k < kend; k += T::NT) {
+                const float wk = rec[k].w;
+                m = fmaxf(m, fabsf(wk));
+                if constexpr (SCALED) b = wk != 0.0f ? fminf(b, rec[k].pad) : b;
+            }
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-            if ((pt & 63) == 0) sm.wmax[wave] = m;
+            for (int o = 32; o > 0; o >>= 1) {
+                m = fmaxf(m, __shfl_xor(m, o));
+                if constexpr (SCALED) b = fminf(b, __shfl_xor(b, o));
+            }
+            if ((pt & 63) == 0) {
+                sm.wmax[wave] = m;
+                if constexpr (SCALED) sm.bmin[wave] = b;
+            }
         }
         __syncthreads();
         if constexpr (f16ops(SCHEME)) {
@@ -650,12 +662,18 @@ phase_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice
                 wscale = ldexpf(1.0f, -e);
                 wunscale = ldexpf(1.0f, e);
             }
+            if constexpr (SCALED) {
+                float b = NO_B;
+#pragma unroll
+                for (int w = 0; w < T::NW; ++w) b = fminf(b, sm.bmin[w]);
+                bref = damp_ref(b);
+            }
         }
-        build_tables<T, !fp32ops(SCHEME)>(sm.t[0], sm.a_k16, sm.b_k16, r0, kbeg + at < kend, sa, sb, pt, wscale, kbeg + at, g.dither, padh);
+        build_tables<T, !fp32ops(SCHEME)>(sm.t[0], sm.a_k16, sm.b_k16, r0, kbeg + at < kend, sa, sb, pt, wscale, kbeg + at, g.dither, padh, bref);
         __syncthreads();
         const bool awrap = g.R0 < g.R, bwrap = g.C0 < g.C;
         build_elems<SCHEME, T, DAMP>(sm.e[0], sm.t[0], sm.a_wpos, sm.b_wpos, sm.s_a, sm.s_b, wave, awrap, bwrap);
-        if (nst > 1) build_tables<T, !fp32ops(SCHEME)>(sm.t[1], sm.a_k16, sm.b_k16, r1, kbeg + KS + at < kend, sa, sb, pt, wscale, kbeg + KS + at, g.dither, padh);
+        if (nst > 1) build_tables<T, !fp32ops(SCHEME)>(sm.t[1], sm.a_k16, sm.b_k16, r1, kbeg + KS + at < kend, sa, sb, pt, wscale, kbeg + KS + at, g.dither, padh, bref);
         __syncthreads();
         for (int s = 0; s < nst; ++s) {
             const int cur = s & 1, nxt = cur ^ 1;
@@ -691,7 +709,7 @@ phase_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice
                 if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
             }
             if (s + 2 < nst) build_tables<T, !fp32ops(SCHEME)>(sm.t[cur], sm.a_k16, sm.b_k16, rt, kbeg + (s + 2) * KS + at < kend, sa, sb, pt, wscale,
-                                              kbeg + (s + 2) * KS + at, g.dither, padh);
+                                              kbeg + (s + 2) * KS + at, g.dither, padh, bref);
             if (s + 1 < nst) build_elems<SCHEME, T, DAMP>(sm.e[nxt], sm.t[nxt], sm.a_wpos, sm.b_wpos, sm.s_a, sm.s_b, wave, awrap, bwrap);
             if (!mfma_first && live) {
                 if constexpr (D64) {
@@ -739,11 +757,22 @@ phase_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice
         float2 *out = partial + (long long)(slice - slice0) * g.P * (D64 ? 2 : 1);
         const bool wide = !D64 && (g.Rs & 1) == 0;
 #pragma unroll
-        for (int i = 0; i < T::WR; ++i)
+        for (int i = 0; i < T::WR; ++i) {
+            float backa[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) backa[v] = SCALED ? damp_back(bref, sm.s_a[wr0 + 16 * i + 4 * lg + v]) : 1.0f;
 #pragma unroll
             for (int j = 0; j < T::WC; ++j) {
                 const int c = col0 + wc0 + 16 * j + li;
                 if (c >= g.C) continue;
+                if constexpr (SCALED) {
+                    const float backb = damp_back(bref, sm.s_b[wc0 + 16 * j + li]);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        accR[i][j][v] = accR[i][j][v] * backa[v] * backb;
+                        accI[i][j][v] = accI[i][j][v] * backa[v] * backb;
+                    }
+                }
                 if constexpr (!D64) {
                     const int r4 = row0 + wr0 + 16 * i + 4 * lg;
                     if (wide && r4 + 3 < g.R) {
@@ -772,6 +801,8 @@ phase_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice
                     }
                 }
             }
+        }
+        if constexpr (SCALED) __syncthreads();   // s_a and s_b have been read: the next item may write its own
     }
 }
 

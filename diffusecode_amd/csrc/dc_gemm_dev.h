@@ -66,6 +66,23 @@ __device__ __forceinline__ float2 cis(uint64_t ph) {
     return make_float2(c, s);
 }
 
+// Damped FP16 operands.  exp(-B s^2) of a row or column leaves FP16's range (22
+// bits above 2^-2, 65,504 at most) where B s^2 is large either way, so the
+// operands carry exp(-(B - Bref) s^2) and the epilogue multiplies by exp(-Bref s^2).
+// Bref is the least B of the slice's occupied atoms: the factors are at most
+// 1 (s^2 >= 0, split_sq), and those that are small are so beside the term of that
+// atom in the same sum.  (B log2(e) is what the kernels hold.)
+constexpr float NO_B = 3.0e38f;            // least B of no atoms
+__device__ __forceinline__ float damp_ref(float bmin) {
+    const float b = bmin < NO_B ? bmin * 1.4426950408889634f : 0.0f;
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, b)));   // uniform
+}
+// 2^-(bref sv), to FP32's rounding
+__device__ __forceinline__ float damp_back(float bref, float sv) {
+    const float p = bref * sv, lo = __builtin_fmaf(bref, sv, -p);
+    return __builtin_amdgcn_exp2f(-p) * __builtin_fmaf(lo, -0.6931471805599453f, 1.0f);
+}
+
 // Packed planes hold one u32 (re | im << 16) per (row, atom): 16 words per
 // row, the four 16-byte atom quads of a row XOR-swizzled by bits 2..3 of the
 // row so that 16-byte accesses of the element builders (4 atom quads x 4 rows) and

@@ -327,5 +327,11 @@ PrepArgs base_prep(const Grid &g, int mapping);
 // gradient amplifies the error of F, so BF16X3 runs the FP16X3 products there
 // (the same MFMA rate), as the Bragg-subtracted runs do.
 inline int model_scheme(int prec) { return prec == DC_PREC_BF16X3 ? DC_PREC_FP16X3 : prec; }
+// s^2 of a grid (metric rten, corner eck, increments vi) as the sum of a part of
+// the R rows and one of the C columns (f1 valid of each period of C0, the others
+// 0), R + C floats.  The least row part is moved to the columns: on a grid whose rows
+// and columns are orthogonal both parts are then >= 0, and neither factor of
+// exp(-B s^2) exceeds 1 for B >= 0.
+void split_sq(const double *rten, const double *eck, const double *vi, const GemmGeom &gg, int f1, float *out);
 
 }  // namespace dc

@@ -70,7 +70,7 @@ int plan_model(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, bool dev) {
     const GemmGeom gg = mapping0_geom(g);
 
     // metric orthogonality of the abscissa against the other axes
-    const double *v1 = m->vi, *v2 = m->vi + 3, *v3 = m->vi + 6;
+    const double *v1 = m->vi;
     const double n1 = std::sqrt(std::fabs(dotg(v1, m->rten, v1)));
     for (int ax = 1; ax < 3; ++ax) {
         if (m->inc[ax] <= 1) continue;
@@ -79,18 +79,7 @@ int plan_model(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, bool dev) {
         if (std::fabs(dotg(v1, m->rten, v)) > 1e-12 * std::max(1.0, n1 * nv)) mp.separable = false;
     }
     mp.sq.assign((size_t)gg.R + gg.C, 0.0f);
-    for (int i = 0; i < gg.R; ++i) {
-        double h[3];
-        for (int k = 0; k < 3; ++k) h[k] = m->eck[k] + i * v1[k];
-        mp.sq[i] = (float)(dotg(h, m->rten, h) / 4.0);
-    }
-    for (int col = 0; col < gg.C; ++col) {
-        const int j = col % gg.C0, l = col / gg.C0;
-        if (j >= g.f[1]) continue;
-        double d[3];
-        for (int k = 0; k < 3; ++k) d[k] = j * v2[k] + l * v3[k];
-        mp.sq[gg.R + col] = (float)((dotg(d, m->rten, d) + 2.0 * dotg(d, m->rten, m->eck)) / 4.0);
-    }
+    split_sq(m->rten, m->eck, m->vi, gg, g.f[1], mp.sq.data());
 
     // counting sort by type, vacancies dropped
     std::vector<int> cnt(m->nscat + 1, 0);
