@@ -34,14 +34,16 @@
 // (adj_words_kernel): 3 parts and 6 products (hh, hm, mh, hl, lh, mm) in FP32,
 // which keep 24 bits of both operands -- the dropped terms are below 2^-25 of a
 // product, less than FP32's own rounding of it.  The split precisions take 2
-// FP16 parts and 3 products, the coefficients of a column tile scaled by one
-// power of two to FP16's range (22 bits against the largest; two BF16 parts
+// FP16 parts and 3 products, the coefficients of a column scaled by a power of
+// two to FP16's range (22 bits against the largest; two BF16 parts
 // hold 16, and S and D, being sums, then cost 1.4 times the row-by-row
-// error).  Either unit runs 16 times the FP32 rate.
+// error).  FP16's range also has to hold the row factor exp(-B s_r^2): the atoms
+// of a plane carry exp(-(B - Bref) s_r^2) and its coefficients exp(-Bref s_r^2)
+// (adj_ref_kernel).  Either unit runs 16 times the FP32 rate.
 #include <algorithm>
 #include <atomic>
 
-#include "dc_internal.h"
+#include "dc_gemm_dev.h"
 
 namespace dc {
 
@@ -98,9 +100,10 @@ __device__ __forceinline__ f32x4 mfma(u32x4 x, u32x4 y, f32x4 c) {
 }
 
 __device__ __forceinline__ float exp2i(int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); }
-// e with 2^e <= x < 2^(e + 1), kept within +-100 (0 of zero)
+// e with 2^e <= x < 2^(e + 1), kept at -113 at least, so that 2^(13 - e) and its
+// reciprocal are normal numbers (0 of zero)
 __device__ __forceinline__ int exponent(float x) {
-    return x == 0.0f ? 0 : min(100, max(-100, (int)(__builtin_bit_cast(uint32_t, x) >> 23 & 0xFF) - 127));
+    return x == 0.0f ? 0 : min(127, max(-113, (int)(__builtin_bit_cast(uint32_t, x) >> 23 & 0xFF) - 127));
 }
 // Powers of two that bring the row weights to 1 at most (2 parts; 1 with 3).
 template <int NP>
@@ -144,40 +147,101 @@ __device__ __forceinline__ bool pair_rows(const AdjArgs &a, int p, int &r1, int 
     return r1 < a.R;
 }
 
+// Bref (times log2(e)) of the span's planes: the least B of a plane's atoms, whose row factors
+// exp(-(B - Bref) s_r^2) are then at most 1 and hold 17 bits or more down to
+// 2^-7; where B spreads further over the rows, Bref moves up, to factors of
+// 2^14 at most (B may spread over 21 / s_r^2 in all).  Unlike in the forward sum a
+// small factor is not small beside others: it is alone in its atom's gradient.  One work-group a plane;
+// tiles are in plane order, a plane's atoms contiguous.
+__global__ void __launch_bounds__(1024) adj_ref_kernel(AdjArgs a, int tile0, int ntiles, int plane0, float *__restrict__ ref) {
+    __shared__ float red[3][16];
+    const int plane = plane0 + blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    auto first = [&](int p) {              // first tile of a plane >= p
+        int lo = 0, hi = ntiles;
+        while (lo < hi) {
+            const int m = (lo + hi) / 2;
+            if (a.tiles[tile0 + m].z < p) lo = m + 1;
+            else hi = m;
+        }
+        return lo;
+    };
+    const int t0 = first(plane), t1 = first(plane + 1);
+    float b0 = NO_B, b1 = -NO_B, s = 0.0f;
+    if (t0 < t1) {
+        for (int k = a.tiles[tile0 + t0].x + (int)threadIdx.x; k < a.tiles[tile0 + t1 - 1].y; k += 1024) {
+            const float b = a.rec[k].pad;
+            b0 = fminf(b0, b);
+            b1 = fmaxf(b1, b);
+        }
+        const float *sq = a.sq + (long long)(plane / a.planes_per_sq) * a.sq_stride;
+        for (int r = threadIdx.x; r < a.R; r += 1024) s = fmaxf(s, fabsf(sq[r]));
+    }
+#pragma unroll
+    for (int h = 1; h < 64; h *= 2) {
+        b0 = fminf(b0, __shfl_xor(b0, h));
+        b1 = fmaxf(b1, __shfl_xor(b1, h));
+        s = fmaxf(s, __shfl_xor(s, h));
+    }
+    if (lane == 0) {
+        red[0][wave] = b0;
+        red[1][wave] = b1;
+        red[2][wave] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; ++w) {
+            b0 = fminf(b0, red[0][w]);
+            b1 = fmaxf(b1, red[1][w]);
+            s = fmaxf(s, red[2][w]);
+        }
+        ref[blockIdx.x] = b0 > b1 || !(s > 0.0f) ? 0.0f
+                          : LOG2E * b0 + fminf(fmaxf(LOG2E * (b1 - b0) - 7.0f / s, 0.0f), 14.0f / s);
+    }
+}
+
 // Q planes -> operand words of one (plane, column tile, k-step): for weight w,
 // component (re, im) and part, lane l holds column l % 16 of the tile and the
 // (cos, sin) coefficients of pairs 4 (l / 16) .. + 3 of the step.
-// One work-group per (plane, tile), a wave per k-step.  2 parts: the tile's
-// coefficients are scaled to below 2^15, and the scale noted.
+// One work-group per (plane, tile), a wave per k-step.  2 parts: the coefficients
+// of each column, times the rows' exp(-Bref s_r^2), are scaled to below 2^15 (by
+// column, since what the columns' own exp(-B s_c^2) leaves of them differs), and the
+// scales noted: scales[plane][tile][column], then the tiles' least ones, then Bref.
 template <int NP>
 __global__ void __launch_bounds__(256) adj_words_kernel(AdjArgs a, int plane0, int nplane, u32x4 *__restrict__ out) {
     constexpr int NW = 6 * NP;
-    __shared__ float red[4];
+    __shared__ float red[4][CT];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float *scales = reinterpret_cast<float *>(out + (long long)nplane * a.ctiles * a.nkt * (NW * 64));
+    float *tscales = scales + (long long)nplane * a.ctiles * CT;
+    const float *ref = tscales + (long long)nplane * a.ctiles;
     for (long long x = blockIdx.x; x < (long long)nplane * a.ctiles; x += gridDim.x) {
         const int ct = (int)(x % a.ctiles), pl = (int)(x / a.ctiles);
         const int c = ct * CT + (lane & 15);
         const bool in = c < a.C && c % a.C0 < a.f1;
         const float *sq = a.sq + (long long)((plane0 + pl) / a.planes_per_sq) * a.sq_stride;
         const float2 *q = a.q + (long long)(plane0 + pl) * a.plane + c;
-        float sg[3], scale = 1.0f;
+        float sg[3], scale = 1.0f, bref = 0.0f;
         weight_scales<NP>(a, sq, sg);
         if constexpr (NP == 2) {
+            if (a.damped) bref = ref[pl];
             float m = 0.0f;
             if (in)
                 for (int r = threadIdx.x >> 4; r < a.R; r += 16) {
                     const float2 v = q[(long long)a.C * r];
-                    m = fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)));
+                    m = fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)) * damp_back(bref, sq[r]));
                 }
-#pragma unroll
-            for (int h = 1; h < 64; h *= 2) m = fmaxf(m, __shfl_xor(m, h));
+            m = fmaxf(m, __shfl_xor(m, 16));
+            m = fmaxf(m, __shfl_xor(m, 32));
             __syncthreads();   // the previous tile's maxima have been read
-            if (lane == 0) red[wave] = m;
+            if (lane < CT) red[wave][lane] = m;
             __syncthreads();
-            m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+            const int col = lane & 15;
+            m = fmaxf(fmaxf(red[0][col], red[1][col]), fmaxf(red[2][col], red[3][col]));
             scale = exp2i(13 - exponent(m));
-            if (threadIdx.x == 0) scales[x] = scale;
+#pragma unroll
+            for (int h = 1; h < CT; h *= 2) m = fmaxf(m, __shfl_xor(m, h));
+            if (threadIdx.x < CT) scales[x * CT + col] = scale;
+            if (threadIdx.x == 0) tscales[x] = exp2i(13 - exponent(m));
         }
         for (int k = wave; k < a.nkt; k += 4) {
             u32x4 w[3][2][NP];
@@ -186,7 +250,8 @@ __global__ void __launch_bounds__(256) adj_words_kernel(AdjArgs a, int plane0, i
                 int r1, r0;
                 float2 q1 = make_float2(0.f, 0.f), q0 = q1;
                 float w1[3] = {1.0f, 0.0f, 0.0f}, w0[3] = {1.0f, 0.0f, 0.0f};
-                if (in && pair_rows(a, KP * k + 4 * (lane >> 4) + e, r1, r0)) {
+                const bool pair = pair_rows(a, KP * k + 4 * (lane >> 4) + e, r1, r0);
+                if (in && pair) {
                     q1 = q[(long long)a.C * r1];
                     w1[1] = ((float)r1 - a.rc) * sg[1];
                     w1[2] = sq[r1] * sg[2];
@@ -197,8 +262,10 @@ __global__ void __launch_bounds__(256) adj_words_kernel(AdjArgs a, int plane0, i
                     }
                 }
                 if constexpr (NP == 2) {
-                    q1 = make_float2(q1.x * scale, q1.y * scale);
-                    q0 = make_float2(q0.x * scale, q0.y * scale);
+                    // (one factor for both rows of a pair, as their s_r^2 is one)
+                    const float f = in && pair ? damp_back(bref, sq[r1]) * scale : 0.0f;
+                    q1 = make_float2(q1.x * f, q1.y * f);
+                    q0 = make_float2(q0.x * f, q0.y * f);
                 }
 #pragma unroll
                 for (int v = 0; v < 3; ++v) {
@@ -253,6 +320,7 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
     constexpr int SLOTS = NK == 1 ? 3 : 2;
     __shared__ float4 col[SLOTS][CT];      // s_c^2, j - jc, m - mc, scaled s_c^2 of the tile's columns
     __shared__ float2 qcen[SLOTS][CT];     // Q of the centre row
+    __shared__ float crel[SLOTS][CT];      // scale of the tile over that of the column (2 parts)
     auto slot_of = [](int ct) { return SLOTS == 2 ? ct & 1 : (int)((unsigned)ct % SLOTS); };
     const int4 tile = a.tiles[tile0 + blockIdx.y];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -266,6 +334,14 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
     const bool center = a.center && chunk == 0;
     float sg[3];
     weight_scales<NP>(a, sq, sg);
+    // scales of the columns and of the tiles, and Bref (adj_words_kernel)
+    const float *scales = reinterpret_cast<const float *>(words + (long long)nplane * a.ctiles * a.nkt * (NW * 64));
+    const float *tscales = scales + (long long)nplane * a.ctiles * CT;
+    float bref = 0.0f;
+    if constexpr (NP == 2)
+        if (a.damped) bref = (tscales + (long long)nplane * a.ctiles)[tile.z - plane0];
+    scales += (long long)(tile.z - plane0) * a.ctiles * CT;
+    tscales += (long long)(tile.z - plane0) * a.ctiles;
     const float s2c = sq[a.R / 2], s2cs = s2c * sg[2];
 
     // per atom: A operands, phase of the row origin, column factors: tl[v] of
@@ -291,7 +367,7 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
                 float2 v = make_float2(0.f, 0.f);
                 if (pair_rows(a, p, r1, r0)) {
                     v = cis((uint64_t)(p + a.center) * at.ra + hs);
-                    const float d = __builtin_amdgcn_exp2f(bl2[i] * sq[r1]);
+                    const float d = __builtin_amdgcn_exp2f((bl2[i] + bref) * sq[r1]);
                     v = make_float2(v.x * d, v.y * d);
                 }
                 uint32_t w[NP];
@@ -320,8 +396,6 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
     // jump over the other chunks' to the next column tile
     const u32x4 *src = words + (((long long)(tile.z - plane0) * a.ctiles + ct0) * a.nkt + k0) * (NW * 64);
     const long long jump = (long long)(a.nkt - NK + 1) * (NW * 64);
-    const float *scales = reinterpret_cast<const float *>(words + (long long)nplane * a.ctiles * a.nkt * (NW * 64)) +
-                          (long long)(tile.z - plane0) * a.ctiles;
     u32x4 reg[LD];
     auto fetch = [&]() {
 #pragma unroll
@@ -334,7 +408,7 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
             if (AW * (u + 1) <= NW || wave + AW * u < NW) sq_w[buf][wave + AW * u][lane] = reg[u];
     };
     // the next tile's column values likewise, a tile ahead (threads 0..15)
-    float csq = 0.0f;
+    float csq = 0.0f, cr = 1.0f;
     float2 cq = make_float2(0.f, 0.f);
     int cj = 0, cm = 0;
     auto fetch_col = [&](int ct) {
@@ -346,14 +420,16 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
         cq = in && center ? a.q[tile.z * a.plane + c + (long long)a.C * (a.R / 2)] : make_float2(0.f, 0.f);
         if constexpr (NP == 2)
             if (in) {
-                const float scale = scales[ct];
+                const float scale = scales[ct * CT + (int)threadIdx.x];
                 cq = make_float2(cq.x * scale, cq.y * scale);
+                cr = tscales[ct] / scale;      // powers of two
             }
     };
     auto put_col = [&](int ct) {
         if (threadIdx.x < CT) {
             col[slot_of(ct)][threadIdx.x] = make_float4(csq, (float)cj - a.jc, (float)cm - a.mc, csq * sg[2]);
             qcen[slot_of(ct)][threadIdx.x] = cq;
+            if constexpr (NP == 2) crel[slot_of(ct)][threadIdx.x] = cr;
         }
     };
     if (ct0 < ct1) {
@@ -412,8 +488,8 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
                 th[i] = j0 < CT ? t : th[i];   // the lane's columns began a new run since the last tile
             }
         }
-        float inv = 1.0f;
-        if constexpr (NP == 2) inv = 1.0f / scales[ct];   // a power of two: exact
+        double inv = 1.0;
+        if constexpr (NP == 2) inv = (double)(1.0f / tscales[ct]);   // a power of two: exact
         float4 w[4];
         float2 qc[4];
         float d[WA][4];
@@ -422,13 +498,13 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
             w[v] = col[slot_of(ct)][4 * lg + v];
             qc[v] = qcen[slot_of(ct)][4 * lg + v];
 #pragma unroll
-            for (int i = 0; i < WA; ++i) d[i][v] = 1.0f;
+            for (int i = 0; i < WA; ++i) d[i][v] = NP == 2 ? crel[slot_of(ct)][4 * lg + v] : 1.0f;
         }
         if (damp)
 #pragma unroll
             for (int v = 0; v < 4; ++v)
 #pragma unroll
-                for (int i = 0; i < WA; ++i) d[i][v] = __builtin_amdgcn_exp2f(bl2[i] * w[v].x);
+                for (int i = 0; i < WA; ++i) d[i][v] *= __builtin_amdgcn_exp2f(bl2[i] * w[v].x);
 #pragma unroll
         for (int i = 0; i < WA; ++i) {
             const float2 thw = cmul(th[i], wrap[i]);
@@ -450,7 +526,7 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
                 s[5] += (z2r * b.x - z2i * b.y) + w[v].w * tr;
             }
 #pragma unroll
-            for (int k = 0; k < 6; ++k) tot[i][k] += (double)(NP == 2 ? s[k] * inv : s[k]);
+            for (int k = 0; k < 6; ++k) tot[i][k] = NP == 2 ? __builtin_fma((double)s[k], inv, tot[i][k]) : tot[i][k] + (double)s[k];
         }
     }
     if (!active) return;
@@ -735,7 +811,7 @@ void adjoint_plan(AdjArgs &a, int ntiles, bool split, int force) {
     a.groups = (a.ctiles + a.tpg - 1) / a.tpg;
     a.nset = a.groups * a.chunks;
     a.walk = (a.tpg + WALK_TILES - 1) / WALK_TILES;
-    a.plane_words = (long long)a.ctiles * a.nkt * 6 * a.parts * 64 + (a.ctiles + 3) / 4;   // and the tiles' scales
+    a.plane_words = (long long)a.ctiles * a.nkt * 6 * a.parts * 64 + (a.ctiles * (CT + 1) + 4) / 4;   // and the scales, Bref
 }
 
 hipError_t launch_adjoint(const AdjArgs &a, const AdjSpan &s, uint4 *words, hipStream_t st) {
@@ -749,6 +825,8 @@ hipError_t launch_adjoint(const AdjArgs &a, const AdjSpan &s, uint4 *words, hipS
     const dim3 grid(a.nset, s.ntiles);
     auto run = [&](auto kernel) { kernel<<<grid, NT, 0, st>>>(a, s.tile0, s.plane0, s.nplanes, w); };
     if (a.parts == 2) {
+        float *ref = reinterpret_cast<float *>(w + (long long)s.nplanes * a.ctiles * a.nkt * (12 * 64)) + (long long)s.nplanes * a.ctiles * (CT + 1);
+        if (a.damped) adj_ref_kernel<<<s.nplanes, 1024, 0, st>>>(a, s.tile0, s.ntiles, s.plane0, ref);
         adj_words_kernel<2><<<nb, 256, 0, st>>>(a, s.plane0, s.nplanes, w);
         a.nk == 1 ? run(adjoint_kernel<2, 1>) : a.nk == 2 ? run(adjoint_kernel<2, 2>) : a.nk == 3 ? run(adjoint_kernel<2, 3>)
             : a.nk == 4 ? run(adjoint_kernel<2, 4>) : run(adjoint_kernel<2, 5>);

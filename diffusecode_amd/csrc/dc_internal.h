@@ -159,6 +159,7 @@ struct AdjArgs {
     int natoms;
     float rc, jc, mc;       // centres of the row / column index weights
     int fold;               // rows taken in mirrored pairs (s_r^2 mirrored, or no B)
+    int damped;             // records hold B other than 0
     // set by adjoint_plan
     int parts;              // 16-bit parts of the operands: 3 (BF16) in FP32, 2 (FP16) in the split precisions
     int center;             // the centre row of the pairs is added apart

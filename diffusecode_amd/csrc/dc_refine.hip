@@ -261,6 +261,7 @@ int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, double *grad
         aa.jc = 0.5f * (float)(mp.g.f[1] - 1);
         aa.mc = 0.5f * (float)(mp.g.f[2] - 1);
         aa.fold = !mp.any_b || (mirrored_sides(gg, mp.sq.data()) & FOLD_ROWS);
+        aa.damped = mp.any_b;
         adjoint_plan(aa, ntiles, c->prec != DC_PREC_FP32, c->adj_walk);
         c->stats.adjoint_walk = aa.walk;
         if ((st = ensure(c, c->m_part, sizeof(double) * 6 * (size_t)aa.nset * std::max(mp.nsorted, 1)))) return st;
