@@ -188,14 +188,17 @@ static double reduce_us(double planes, double plane_elems) {
 // 1.2e-6 for 17,067 atoms in dc_gemm.hip; 8,704 costs 1% more planes and items
 // than twice that).  Launches that fill the device with shorter slices cap
 // them at the length that gives 1,024 items of 256 x 176 outputs, as
-// kchunk_atoms does (lots of 4,000 atoms: error of the cross-lot variance
-// 3.2e-7 with slices of 700 atoms in dc_gemm.hip, 7.3e-7 with 2,000 here).
+// kchunk_atoms does, or at 704 atoms: lots of 860 atoms a type on 151 x 87 x 2
+// points, errors of F, <F> and the cross-lot variance (means of 8 crystals) 1.2e-7,
+// 3.9e-8 and 3.7e-7, with one slice of up to 1,024 a type 2.1e-7, 5.2e-8 and
+// 7.0e-7, in dc_gemm.hip 1.7e-7, 6.1e-8 and 7.0e-7; 32 lots of 4,000 atoms on 201 x 201
+// x 4 cost 4% more than with 1,024 (586 -> 611 us).
 // FP32 sums are FP64: its slices are bounded by the one rounding of a plane.
-constexpr int KCHUNK_FOLD_MIN = 64, KCHUNK_FOLD_MAX = 8704, KCHUNK_FOLD_FP32 = 2048;
+constexpr int KCHUNK_FOLD_MIN = 64, KCHUNK_FOLD_SMALL = 704, KCHUNK_FOLD_MAX = 8704, KCHUNK_FOLD_FP32 = 2048;
 static int fold_cap(const GemmGeom &gg, long long natoms, int prec) {
     if (prec == DC_PREC_FP32) return KCHUNK_FOLD_FP32;
     const long long k = (long long)((double)natoms * gg.R * gg.C / (256.0 * 176.0 * 1024.0));
-    return (int)std::min<long long>(std::max<long long>(k, 1024), KCHUNK_FOLD_MAX);
+    return (int)std::min<long long>(std::max<long long>(k, KCHUNK_FOLD_SMALL), KCHUNK_FOLD_MAX);
 }
 
 // Makespan of n counted groups of equal items, (microseconds, count), the
