@@ -198,7 +198,10 @@ constexpr int KCHUNK_FOLD_MIN = 64, KCHUNK_FOLD_SMALL = 704, KCHUNK_FOLD_MAX = 8
 static int fold_cap(const GemmGeom &gg, long long natoms, int prec) {
     if (prec == DC_PREC_FP32) return KCHUNK_FOLD_FP32;
     const long long k = (long long)((double)natoms * gg.R * gg.C / (256.0 * 176.0 * 1024.0));
-    return (int)std::min<long long>(std::max<long long>(k, KCHUNK_FOLD_SMALL), KCHUNK_FOLD_MAX);
+    // planes that would not fit the budget: slices as long as dc_gemm.hip's
+    const double fit = (double)natoms * (double)gg.P * sizeof(float2) / PARTIAL_BUDGET;
+    const int most = (int)std::min<double>(std::max<double>(KCHUNK_FOLD_MAX, std::ceil(fit)), KCHUNK_SEARCH_MAX);
+    return (int)std::min<long long>(std::max<long long>(k, KCHUNK_FOLD_SMALL), most);
 }
 
 // Makespan of n counted groups of equal items, (microseconds, count), the
@@ -276,6 +279,7 @@ int fold_slices(const GemmGeom &gg, int tile, const std::vector<std::pair<int, i
             groups[q] = {(double)((len + 31) / 32) * stage_us + FOLD_ITEM_US, sl * sizes[q].second * wgs};
             planes += sl * sizes[q].second;
         }
+        if (ns > n0 && (double)planes * (double)gg.P * sizeof(float2) > PARTIAL_BUDGET) break;   // shorter slices: more planes yet
         const double us = makespan(groups.data(), (int)groups.size(), ncu) + reduce_us((double)planes, (double)gg.P);
         if (us < best_us * (1.0 - 1e-9)) {
             best_us = us;
