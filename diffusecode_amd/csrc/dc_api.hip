@@ -188,20 +188,20 @@ static double reduce_us(double planes, double plane_elems) {
 // 1.2e-6 for 17,067 atoms in dc_gemm.hip; 8,704 costs 1% more planes and items
 // than twice that).  Launches that fill the device with shorter slices cap
 // them at the length that gives 1,024 items of 256 x 176 outputs, as
-// kchunk_atoms does, or at 704 atoms: lots of 860 atoms a type on 151 x 87 x 2
+// kchunk_atoms does, or at 1,024 atoms, in lots at 704: lots of 860 atoms a type on 151 x 87 x 2
 // points, errors of F, <F> and the cross-lot variance (means of 8 crystals) 1.2e-7,
 // 3.9e-8 and 3.7e-7, with one slice of up to 1,024 a type 2.1e-7, 5.2e-8 and
 // 7.0e-7, in dc_gemm.hip 1.7e-7, 6.1e-8 and 7.0e-7; 32 lots of 4,000 atoms on 201 x 201
 // x 4 cost 4% more than with 1,024 (586 -> 611 us).
 // FP32 sums are FP64: its slices are bounded by the one rounding of a plane.
-constexpr int KCHUNK_FOLD_MIN = 64, KCHUNK_FOLD_SMALL = 704, KCHUNK_FOLD_MAX = 8704, KCHUNK_FOLD_FP32 = 2048;
-static int fold_cap(const GemmGeom &gg, long long natoms, int prec) {
+constexpr int KCHUNK_FOLD_MIN = 64, KCHUNK_FOLD_SMALL = 1024, KCHUNK_FOLD_LOTS = 704, KCHUNK_FOLD_MAX = 8704, KCHUNK_FOLD_FP32 = 2048;
+static int fold_cap(const GemmGeom &gg, long long natoms, int prec, bool lots) {
     if (prec == DC_PREC_FP32) return KCHUNK_FOLD_FP32;
     const long long k = (long long)((double)natoms * gg.R * gg.C / (256.0 * 176.0 * 1024.0));
     // planes that would not fit the budget: slices as long as dc_gemm.hip's
     const double fit = (double)natoms * (double)gg.P * sizeof(float2) / PARTIAL_BUDGET;
     const int most = (int)std::min<double>(std::max<double>(KCHUNK_FOLD_MAX, std::ceil(fit)), KCHUNK_SEARCH_MAX);
-    return (int)std::min<long long>(std::max<long long>(k, KCHUNK_FOLD_SMALL), most);
+    return (int)std::min<long long>(std::max<long long>(k, lots ? KCHUNK_FOLD_LOTS : KCHUNK_FOLD_SMALL), most);
 }
 
 // Makespan of n counted groups of equal items, (microseconds, count), the
@@ -242,7 +242,7 @@ static double makespan(ItemGroup *gr, int n, int ncu) {
 // near-equal slices (add_segments), one item per (slice, tile).  The lengths
 // tried are those of 1, 2, 3, ... slices of the longest segment, thinned to
 // steps of about 1/8 once there are many.
-int fold_slices(const GemmGeom &gg, int tile, const std::vector<std::pair<int, int>> &segs, int prec, double &best_us) {
+int fold_slices(const GemmGeom &gg, int tile, const std::vector<std::pair<int, int>> &segs, int prec, double &best_us, bool lots) {
     const TileInfo ti = gemm_tile_info(tile);
     const long long wgs = gemm_items(gg, tile);
     const int ncu = device_cu_count();
@@ -255,7 +255,7 @@ int fold_slices(const GemmGeom &gg, int tile, const std::vector<std::pair<int, i
             sizes.push_back({sg.second, 1});
             natoms += sg.second;
         }
-    const int cap = fold_cap(gg, natoms, prec);
+    const int cap = fold_cap(gg, natoms, prec, lots);
     best_us = 1e300;
     if (sizes.empty()) return cap;
     std::sort(sizes.begin(), sizes.end(), std::greater<std::pair<int, long long>>());
@@ -436,10 +436,10 @@ int kchunk_for(const Plan &pl, long long natoms_batch, int prec) {
 // reduce).  FP32 searches between half its fixed slice cap and the cap.
 // Launches that already have 16 rounds of items or more, and
 // populations (many segments), keep the rule of kchunk_atoms.
-int kchunk_for(const Plan &pl, const std::vector<std::pair<int, int>> &segs, int prec) {
+int kchunk_for(const Plan &pl, const std::vector<std::pair<int, int>> &segs, int prec, bool lots) {
     if (gemm_tile_info(pl.tile).fold) {
         double us;
-        return fold_slices(pl.gg, pl.tile, segs, prec, us);
+        return fold_slices(pl.gg, pl.tile, segs, prec, us, lots);
     }
     long long natoms = 0;
     for (auto &sg : segs) natoms += std::max(sg.second, 0);
@@ -1104,7 +1104,7 @@ long long lot_type_runs(const dc_ctx *c, const std::vector<CellRun> &cruns, int 
 // types to slice_type, staged with the slice tables before the launch.
 int gemm_segments(dc_ctx *c, const Grid &g, const Plan &pl, GatherList &gl,
                   const double *explicit_pos, SliceSet &ss, int &nslice, bool use_type_lists,
-                  const std::vector<int> &group_seg, const int *&lot_slice, const int *&slice_type) {
+                  const std::vector<int> &group_seg, const int *&lot_slice, const int *&slice_type, bool lots = false) {
     const GemmGeom &gg = pl.gg;
     const int mapping = pl.mapping;
     int st = 0;
@@ -1147,7 +1147,7 @@ int gemm_segments(dc_ctx *c, const Grid &g, const Plan &pl, GatherList &gl,
     pa.hash_salt = launch_geom(c, gg).dither;   // run_gemm below launches undamped
     int off = 0;
     ss = SliceSet();
-    add_segments(ss, gl.segs, slice_len(c, kchunk_for(pl, gl.segs, pl.scheme)), off);
+    add_segments(ss, gl.segs, slice_len(c, kchunk_for(pl, gl.segs, pl.scheme, lots)), off);
     if (ss.beg.empty()) ss.beg.push_back(0);
     const int ngemm = (int)ss.type.size();
     // schemes with two planes per slice (hi, lo): the reductions see each
@@ -1413,7 +1413,7 @@ static int four_run(dc_ctx *c, const dc_run_desc *r, double *d_csf, double *d_ac
         lot_first_seg.push_back((int)gl.segs.size());
         SliceSet ss;
         int nslice = 0;
-        if ((st = gemm_segments(c, g, pl, gl, nullptr, ss, nslice, !lots, lot_first_seg, lot_slice, slice_type))) return st;
+        if ((st = gemm_segments(c, g, pl, gl, nullptr, ss, nslice, !lots, lot_first_seg, lot_slice, slice_type, lots))) return st;
         pairs += (double)n_batch * (double)ntot;
         nslices_total += nslice;
         ReduceArgs ra{};

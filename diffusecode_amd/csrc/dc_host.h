@@ -299,11 +299,12 @@ Plan plan_gemm(Grid &g, int forced, int only_mapping = -1, int prec = 1, long lo
 // Geometry of mapping 0, which no tile changes.
 GemmGeom mapping0_geom(const Grid &g);
 // Slice length of a fold tile for a launch's segments, and its predicted time.
-int fold_slices(const GemmGeom &gg, int tile, const std::vector<std::pair<int, int>> &segs, int prec, double &best_us);
+int fold_slices(const GemmGeom &gg, int tile, const std::vector<std::pair<int, int>> &segs, int prec, double &best_us,
+                bool lots = false);
 // the sides whose s^2 parts (R row values, then C column values) are mirrored
 int mirrored_sides(const GemmGeom &gg, const float *sq);
 int kchunk_for(const Plan &pl, long long natoms_batch, int prec);
-int kchunk_for(const Plan &pl, const std::vector<std::pair<int, int>> &segs, int prec);
+int kchunk_for(const Plan &pl, const std::vector<std::pair<int, int>> &segs, int prec, bool lots = false);
 void add_segments(SliceSet &s, const std::vector<std::pair<int, int>> &segs, int kchunk, int &atom_off);
 // beg: the slices' atom offsets (nslice + 1), d_beg: the same on the device
 int run_gemm(dc_ctx *c, const Plan &pl, const std::vector<int> &beg, const int *d_beg, float2 *partial,
