@@ -152,7 +152,8 @@ __device__ __forceinline__ bool pair_rows(const AdjArgs &a, int p, int &r1, int 
 // 2^-7; where B spreads further over the rows, Bref moves up, to factors of
 // 2^14 at most (B may spread over 21 / s_r^2 in all).  Unlike in the forward sum a
 // small factor is not small beside others: it is alone in its atom's gradient.  One work-group a plane;
-// tiles are in plane order, a plane's atoms contiguous.
+// tiles are in plane order, a plane's atoms contiguous.  Bound by latency: 9 us for 48
+// planes of 4,000 atoms, and no less with the search, the reads or the reduction wider.
 __global__ void __launch_bounds__(1024) adj_ref_kernel(AdjArgs a, int tile0, int ntiles, int plane0, float *__restrict__ ref) {
     __shared__ float red[3][16];
     const int plane = plane0 + blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -308,7 +309,7 @@ __global__ void __launch_bounds__(256) adj_words_kernel(AdjArgs a, int plane0, i
 // 1.8e-7, 9e-8, 1.0e-7 to 1.2e-7, 5e-8, 6e-8 in FP32 and from 3.5e-6,
 // 1.1e-6, 1.8e-6 to 1.4e-7, 6e-8, 7e-8 in the split precisions.
 template <int NP, int NK>
-__global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, int plane0, int nplane, const u32x4 *__restrict__ words) {
+__global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, int plane0, int nplane, int chunk0, const u32x4 *__restrict__ words) {
     constexpr int NW = 6 * NP, LD = (NW + AW - 1) / AW;
     __shared__ u32x4 sq_w[2][NW][64];
     // Values of a tile's columns: those of tile t + 1 are stored in the last
@@ -326,7 +327,7 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int li = lane & 15, lg = lane >> 4;
     const float *sq = a.sq + (long long)tile.w * a.sq_stride;
-    const int group = blockIdx.x % a.groups, chunk = blockIdx.x / a.groups;
+    const int group = blockIdx.x % a.groups, chunk = chunk0 + blockIdx.x / a.groups;
     const int ct0 = group * a.tpg, ct1 = min(a.ctiles, ct0 + a.tpg);
     const int k0 = chunk * NK;
     const int n0 = tile.x + wave * 16 * WA + li;
@@ -542,7 +543,7 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
         if (lg == 0 && n0 + 16 * i < tile.y) {
             double *out = a.part + ((long long)blockIdx.x * a.natoms + n0 + 16 * i) * 6;
 #pragma unroll
-            for (int k = 0; k < 6; ++k) out[k] = tot[i][k];
+            for (int k = 0; k < 6; ++k) out[k] = chunk0 > 0 ? out[k] + tot[i][k] : tot[i][k];
         }
     }
 }
@@ -809,7 +810,9 @@ void adjoint_plan(AdjArgs &a, int ntiles, bool split, int force) {
         }
     }
     a.groups = (a.ctiles + a.tpg - 1) / a.tpg;
-    a.nset = a.groups * a.chunks;
+    // row chunks of later launches add to the sets of the first
+    a.nchunk = (int)std::min<long long>(a.chunks, std::max<long long>(1, ADJ_PART_MAX / (48LL * a.groups * std::max(a.natoms, 1))));
+    a.nset = a.groups * a.nchunk;
     a.walk = (a.tpg + WALK_TILES - 1) / WALK_TILES;
     a.plane_words = (long long)a.ctiles * a.nkt * 6 * a.parts * 64 + (a.ctiles * (CT + 1) + 4) / 4;   // and the scales, Bref
 }
@@ -817,13 +820,17 @@ void adjoint_plan(AdjArgs &a, int ntiles, bool split, int force) {
 hipError_t launch_adjoint(const AdjArgs &a, const AdjSpan &s, uint4 *words, hipStream_t st) {
     if (s.ntiles <= 0 || a.R <= 0 || a.C <= 0) return hipSuccess;
     if (!words || a.f1 < 1 || a.C0 < a.f1 || (a.C > a.C0 && a.C0 < CT) || a.nk < 1 || a.nk > max_ksteps(a.parts) ||
-        a.nk * a.chunks != a.nkt || a.nkt * KP < (a.fold ? (a.R + 1) / 2 - a.center : a.R) || a.tpg < 1 ||
+        a.nk * a.chunks != a.nkt || a.nchunk < 1 || a.nset != a.groups * a.nchunk || a.nkt * KP < (a.fold ? (a.R + 1) / 2 - a.center : a.R) || a.tpg < 1 ||
         a.groups * a.tpg < a.ctiles || a.planes_per_sq < 1 || s.ntiles > 65535)
         return hipErrorInvalidValue;
     u32x4 *w = reinterpret_cast<u32x4 *>(words);
     const unsigned nb = (unsigned)std::min<long long>((long long)s.nplanes * a.ctiles, 8192);
-    const dim3 grid(a.nset, s.ntiles);
-    auto run = [&](auto kernel) { kernel<<<grid, NT, 0, st>>>(a, s.tile0, s.plane0, s.nplanes, w); };
+    auto run = [&](auto kernel) {
+        for (int c = 0; c < a.chunks; c += a.nchunk) {
+            const dim3 grid(a.groups * std::min(a.nchunk, a.chunks - c), s.ntiles);
+            kernel<<<grid, NT, 0, st>>>(a, s.tile0, s.plane0, s.nplanes, c, w);
+        }
+    };
     if (a.parts == 2) {
         float *ref = reinterpret_cast<float *>(w + (long long)s.nplanes * a.ctiles * a.nkt * (12 * 64)) + (long long)s.nplanes * a.ctiles * (CT + 1);
         if (a.damped) adj_ref_kernel<<<s.nplanes, 1024, 0, st>>>(a, s.tile0, s.ntiles, s.plane0, ref);

@@ -258,6 +258,7 @@ int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
     b.adj.f1 = g.f[1];
     b.adj.fold = (b.fold_mask & FOLD_ROWS) != 0;
     b.adj.damped = b.any_b;
+    b.adj.natoms = b.nsorted;
     adjoint_plan(b.adj, b.ntiles, b.prec != DC_PREC_FP32, c->adj_walk);
     b.spans = adjoint_spans(b.adj, tiles.data(), b.ntiles);
     b.nblk = (int)std::min<long long>((g.P + 255) / 256, 256);

@@ -165,7 +165,8 @@ struct AdjArgs {
     int center;             // the centre row of the pairs is added apart
     int nkt, nk, chunks;    // k-steps of 16 row pairs: in all, per row chunk; chunks
     int ctiles, tpg, groups;   // column tiles: in all, per range; ranges
-    int nset, walk;         // partial sets; column tiles of 256 per work-group
+    int nchunk;             // row chunks a launch
+    int nset, walk;         // partial sets (groups x nchunk); column tiles of 256 per work-group
     long long plane_words;  // 16-byte words of one plane: operands and scales
 };
 // A run of planes whose operand words are made and used by one launch.
@@ -173,6 +174,7 @@ struct AdjSpan {
     int plane0, nplanes, tile0, ntiles;
 };
 constexpr long long ADJ_WORDS_MAX = 1LL << 30;   // bytes of words made at a time (or one plane's)
+constexpr long long ADJ_PART_MAX = 2LL << 30;    // bytes of partial sets (or those of one row chunk)
 struct AdjFinishArgs {
     const double *part;
     int nset, natoms;
@@ -233,7 +235,7 @@ struct JvpArgs {
 };
 hipError_t launch_jvp_reduce(const JvpArgs &a, hipStream_t st);
 int adjoint_tile_atoms();
-// Cuts the work of ntiles atom tiles (rows, columns, f1 and fold of a set): the
+// Cuts the work of ntiles atom tiles (rows, columns, f1, fold and natoms of a set): the
 // fields of a below "set by adjoint_plan".  force > 0 asks for column ranges of
 // that many 256-column tiles.
 void adjoint_plan(AdjArgs &a, int ntiles, bool split, int force = 0);
