@@ -353,8 +353,6 @@ int dc_model_jvp(dc_ctx *c, const dc_model_desc *m, const double *fcalc, int ndi
     const long long P = mp.g.P;
     const int ns = mp.nsorted;
     if ((st = upload(c, c->m_f, fcalc, 2 * (size_t)P))) return st;
-    double *d_par;
-    if ((st = stage(c, c->m_jw, dparam, 5 * (size_t)m->natoms * ndir, d_par))) return st;
     // [ndir][P] dI, then dF: pinned memory that the kernel writes, or device
     const size_t obytes = sizeof(double) * (size_t)P * std::max(ndir, 1) * (df ? 3 : 1);
     const bool pinned = obytes <= HOST_OUT_BYTES;
@@ -383,7 +381,9 @@ int dc_model_jvp(dc_ctx *c, const dc_model_desc *m, const double *fcalc, int ndi
         if (ss.beg.empty()) ss.beg.push_back(0);
         const int nslice = (int)ss.type.size();
         const long long nrec = 5LL * nd * ns;
+        double *d_par;
         int *d_dsl, *d_beg, *d_type;
+        if ((st = stage(c, c->m_jw, dparam + 5 * (size_t)m->natoms * d0, 5 * (size_t)m->natoms * nd, d_par))) return st;
         if ((st = stage(c, c->m_dsl, dsl.data(), dsl.size(), d_dsl))) return st;
         if ((st = stage(c, c->slice_beg, ss.beg.data(), ss.beg.size(), d_beg))) return st;
         if ((st = stage(c, c->slice_type, ss.type.data(), ss.type.size(), d_type))) return st;
@@ -396,7 +396,7 @@ int dc_model_jvp(dc_ctx *c, const dc_model_desc *m, const double *fcalc, int ndi
         pa.idx = mp.idx;
         pa.occ_src = mp.occ;
         pa.bdw_src = mp.bdw;
-        pa.dpar = d_par + 5 * (size_t)m->natoms * d0;
+        pa.dpar = d_par;
         pa.dn = std::max(ns, 1);
         pa.dnat = m->natoms;
         pa.n = nrec;
