@@ -381,7 +381,7 @@ Plan plan_gemm(Grid &g, int forced, int only_mapping, int prec, long long natoms
     return best;
 }
 
-void split_sq(const double *rten, const double *eck, const double *vi, const GemmGeom &gg, int f1, float *out) {
+void split_sq(const double *rten, const double *eck, const double *vi, const GemmGeom &gg, int f1, bool f16, float *out) {
     auto dot = [&](const double *a, const double *b) {
         double s = 0.0;
         for (int r = 0; r < 3; ++r)
@@ -393,13 +393,17 @@ void split_sq(const double *rten, const double *eck, const double *vi, const Gem
     const double c0 = dot(eck, eck), c1 = 2.0 * dot(v1, eck), c11 = dot(v1, v1);
     const double c2 = 2.0 * dot(v2, eck), c22 = dot(v2, v2), c3 = 2.0 * dot(v3, eck), c33 = dot(v3, v3), c23 = 2.0 * dot(v2, v3);
     auto row = [&](int i) { return c0 + i * (c1 + i * c11); };
-    double least = row(0);
-    for (int i = 1; i < gg.R; ++i) least = std::min(least, row(i));
-    for (int i = 0; i < gg.R; ++i) out[i] = (float)(row(i) - least);
+    double least = f16 ? row(0) : 0.0;
+    for (int i = 1; i < gg.R && f16; ++i) least = std::min(least, row(i));
+    float *lo = out + gg.R + gg.C;
+    auto put = [&](int k, double v) {
+        out[k] = (float)v;
+        if (f16) lo[k] = (float)(v - (double)out[k]);
+    };
+    for (int i = 0; i < gg.R; ++i) put(i, row(i) - least);
     for (int l = 0; l * gg.C0 < gg.C; ++l) {
         const double top = least + l * (c3 + l * c33), lin = c2 + l * c23;
-        float *o = out + gg.R + l * gg.C0;
-        for (int j = 0; j < gg.C0; ++j) o[j] = j < f1 ? (float)(top + j * (lin + j * c22)) : 0.0f;
+        for (int j = 0; j < gg.C0; ++j) put(gg.R + l * gg.C0 + j, j < f1 ? top + j * (lin + j * c22) : 0.0);
     }
 }
 

@@ -37,6 +37,7 @@ struct BatchState {
     std::vector<std::pair<int, int>> segs;   // (type, atoms) per member and type, member-major
     std::vector<int> seg_member;
     int kchunk = 0;                          // atoms per GEMM slice
+    int sq_stride = 0;                       // floats of a member's s^2 parts
     int nsorted = 0, nslice = 0, ntiles = 0, nblk = 0;
     AdjArgs adj{};                       // plan of the reverse pass, and its launches
     std::vector<AdjSpan> spans;
@@ -127,8 +128,9 @@ int check_types(dc_ctx *c, const dc_batch_desc *d) {
 int member_sq(dc_ctx *c, const Grid &g, const GemmGeom &gg, const dc_batch_desc *d, std::vector<float> &sq, bool need_sep,
               int &top_bin) {
     top_bin = 0;
-    const int stride = gg.R + gg.C;
-    sq.assign((size_t)stride * d->nmembers, 0.0f);
+    const bool f16 = f16_scheme(model_scheme(c->prec));
+    const int stride = sq_floats(gg, f16);
+    sq.resize((size_t)stride * d->nmembers);
     const double *v1 = d->vi;
     for (int m = 0; m < d->nmembers; ++m) {
         const double *G = d->rten + 9 * m;
@@ -142,7 +144,7 @@ int member_sq(dc_ctx *c, const Grid &g, const GemmGeom &gg, const dc_batch_desc 
                     return set_err(c, DC_ERR_ARG, DC_ER_LIB, "batch: vi(:,1) not metric-orthogonal to vi(:,2), vi(:,3)");
             }
         }
-        split_sq(G, d->eck, d->vi, gg, g.f[1], sq.data() + (size_t)stride * m);
+        split_sq(G, d->eck, d->vi, gg, g.f[1], f16, sq.data() + (size_t)stride * m);
         Grid gm = g;
         for (int k = 0; k < 9; ++k) gm.rten[k] = G[k];
         top_bin = std::max(top_bin, max_corner_bin(gm));
@@ -164,7 +166,7 @@ int make_slices(dc_ctx *c, BatchState &b, int kchunk) {
         mslice.push_back((int)ss.type.size());
         for (; sg < b.segs.size() && b.seg_member[sg] == m; ++sg) {
             add_segments(ss, {b.segs[sg]}, kchunk, off);
-            while ((int)slice_sq.size() < (int)ss.type.size()) slice_sq.push_back(m * (gg.R + gg.C));
+            while ((int)slice_sq.size() < (int)ss.type.size()) slice_sq.push_back(m * b.sq_stride);
         }
     }
     mslice.push_back((int)ss.type.size());
@@ -221,6 +223,7 @@ int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
     g = batch_grid(d);
     b.pl = plan_gemm(g, c->tile, 0, model_scheme(c->prec), d->atom_beg[d->nmembers], b.fold_mask);
     const GemmGeom &gg = b.pl.gg;
+    b.sq_stride = sq_floats(gg, f16_scheme(b.pl.scheme));
 
     // member-major, type-sorted atom order; adjoint tiles; slices
     std::vector<int> tiles;
@@ -271,10 +274,10 @@ int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
     if ((st = ensure(c, b.rec, sizeof(AtomRec) * std::max(b.nsorted, 1)))) return st;
     if ((st = ensure(c, b.cfact, sizeof(double) * 2 * (size_t)b.rows * d->nscat * M))) return st;
     if ((st = pin_ensure(c, b.h_cf, sizeof(double) * (2 * (size_t)b.rows * d->nscat + 9) * M))) return st;
-    if ((st = pin_ensure(c, b.h_sq, sizeof(float) * (size_t)(gg.R + gg.C) * M))) return st;
+    if ((st = pin_ensure(c, b.h_sq, sizeof(float) * (size_t)b.sq_stride * M))) return st;
     if ((st = pin_ensure(c, b.h_chi, sizeof(double) * M))) return st;
     if ((st = ensure(c, b.rten, sizeof(double) * 9 * M))) return st;
-    if ((st = ensure(c, b.sq, sizeof(float) * (size_t)(gg.R + gg.C) * M))) return st;
+    if ((st = ensure(c, b.sq, sizeof(float) * (size_t)b.sq_stride * M))) return st;
     if ((st = ensure(c, b.chi, sizeof(double) * (size_t)b.nblk * M))) return st;
     if (b.want_grad) {
         if ((st = ensure(c, b.q, sizeof(float2) * gg.P * d->nscat * M))) return st;
@@ -384,7 +387,7 @@ int enqueue(dc_ctx *c, BatchState &b, const StepIO &io, int tile, int nwg, bool 
         aa.tiles = ptr<int4>(b.atiles);
         aa.q = ptr<float2>(b.q);
         aa.sq = ptr<float>(b.sq);
-        aa.sq_stride = gg.R + gg.C;
+        aa.sq_stride = b.sq_stride;
         aa.planes_per_sq = b.nscat;
         aa.part = ptr<double>(b.part);
         aa.plane = gg.P;
@@ -594,7 +597,7 @@ int batch_chi2(dc_ctx *c, const dc_batch_desc *d, const double *target, const do
         const Grid g = batch_grid(d);
         const GemmGeom gg = mapping0_geom(g);
         if ((st = member_sq(c, g, gg, d, sq, any_b || want_grad, top_bin))) return st;
-        for (int m = 0; m < d->nmembers && any_b; ++m) fold_mask &= mirrored_sides(gg, sq.data() + (size_t)m * (gg.R + gg.C));
+        for (int m = 0; m < d->nmembers && any_b; ++m) fold_mask &= mirrored_sides(gg, sq.data() + sq.size() / d->nmembers * m);
     }
     const bool shape = same_shape(c->batch, c, d, want_grad, want_icalc, have_weight, any_b) &&
                        c->batch->fold_mask == fold_mask && cfact_rows(top_bin, d->ncfact) <= c->batch->rows;

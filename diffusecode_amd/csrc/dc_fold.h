@@ -123,9 +123,9 @@ struct alignas(16) FoldSmem {
     int k16[T::RH], wpos[T::RH];
     float s_b[T::JT];
     float wmax[T::NW];
-    float bmin[T::NW];                      // damped FP16: least B by wave, factors put back
-    alignas(16) float back_a[T::RT];
-    float back_b[T::JT];
+    float bmin[T::NW];                      // damped FP16: least B by wave, factors put back (damp_back2)
+    alignas(16) float2 back_a[T::RT];       // and the scales of the row and the slice
+    float2 back_b[T::JT];
     int item;
 };
 
@@ -186,7 +186,7 @@ __device__ __forceinline__ void fold_tables(FoldTables<T> &tb, const int *__rest
     // the high groups spread as in FP32 6.5.
     constexpr bool F32 = SCHEME == SCH_FP32;
     if (wave == 0 || wave == 1) {
-        if (m == 0) tb.dmp[a] = live && w != 0.0f ? pad * 1.4426950408889634f - bref : 0.0f;
+        if (m == 0) tb.dmp[a] = live && w != 0.0f ? (pad - bref) * 1.4426950408889634f : 0.0f;
     }
     if (wave < (F32 ? 4 : 2)) {
         float2 *t0 = reinterpret_cast<float2 *>(tb.al[0].v) + (a & 1);
@@ -581,10 +581,19 @@ fold_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice_
         FoldA<SCHEME, WR> A{};
         const bool mfma_first = ((wave >> 2) & 1) != 0;
         if constexpr (SCALED) {
+            // what the floats of sq leave of s^2 lies behind them
+            const float *lo = sq + (slice_sq ? slice_sq[slice] : 0) + g.R + g.C;
+            const float *la = lo + (fg.swap ? g.R : 0), *lb = lo + (fg.swap ? 0 : g.R) + fg.NB / 2 + pair0;
 #pragma unroll
-            for (int i = 0; i < WR; ++i)
-                if (lg == 0) sm.back_a[16 * (wave * WR + i) + li] = damp_back(bref, sv[i]);
-            for (int x = threadIdx.x; x < T::JT; x += T::NT) sm.back_b[x] = damp_back(bref, sm.s_b[x]);
+            for (int i = 0; i < WR; ++i) {
+                const int r = wr0 + 16 * i + li;
+                if (lg == 0)
+                    sm.back_a[16 * (wave * WR + i) + li] =
+                        damp_back2(bref, sv[i], r < fg.NA ? la[r] : 0.0f,
+                                   (double)frow_j_undo(li >> 2) * frow_m_undo(li & 3) * fscale_undo<SCHEME>() * wunscale);
+            }
+            for (int x = threadIdx.x; x < T::JT; x += T::NT)
+                sm.back_b[x] = damp_back2(bref, sm.s_b[x], pair0 + x < J ? lb[x] : 0.0f, 1.0);
         }
         tables(0, r0);
         __syncthreads();
@@ -650,17 +659,15 @@ fold_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice_
         if (active) {
 #pragma unroll
             for (int i = 0; i < WR; ++i) {
-                f32x4 backa{};
-                if constexpr (SCALED) {
-                    backa = *reinterpret_cast<const f32x4 *>(&sm.back_a[16 * (wave * WR + i) + 4 * lg]);
+                float2 backa[4];
+                if constexpr (SCALED)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) backa[v] *= undo * frow_m_undo(v) * last;
-                }
+                    for (int v = 0; v < 4; ++v) backa[v] = sm.back_a[16 * (wave * WR + i) + 4 * lg + v];
 #pragma unroll
                 for (int j = 0; j < WC; ++j) {
                     const int pr = pair0 + 8 * j + (li >> 1);
                     float2 f[4];
-                    const float backb = SCALED ? sm.back_b[8 * j + (li >> 1)] : 1.0f;
+                    const float2 backb = SCALED ? sm.back_b[8 * j + (li >> 1)] : make_float2(1.0f, 0.0f);
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
                         const float xr = accR[i][j][v], xi = accI[i][j][v];
@@ -669,7 +676,8 @@ fold_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice_
                         if constexpr (SCHEME == SCH_FP32) {
                             f[v] = make_float2(re, im);
                         } else if constexpr (SCALED) {
-                            f[v] = make_float2(re * backa[v] * backb, im * backa[v] * backb);
+                            const float2 b = mul2(backa[v], backb);
+                            f[v] = make_float2(__builtin_fmaf(re, b.x, re * b.y), __builtin_fmaf(im, b.x, im * b.y));
                         } else {
                             const float um = frow_m_undo(v);
                             f[v] = make_float2(re * undo * um * last, im * undo * um * last);

@@ -185,7 +185,7 @@ __device__ __forceinline__ void build_tables(Tables<T> &tb, const int *__restric
         psi = dither_turn(katom, salt);
     }
     const uint64_t psi2 = psi * 0xD6E8FEB86659FD93ull;
-    if (r == 0) tb.dmp[a] = live && ar.w != 0.0f ? ar.pad * 1.4426950408889634f - bref : 0.0f;
+    if (r == 0) tb.dmp[a] = live && ar.w != 0.0f ? (ar.pad - bref) * 1.4426950408889634f : 0.0f;
     if (r < 8) {
         const bool sideb = r >= 4;
         const int m = r & 3;
@@ -758,19 +758,27 @@ phase_gemm_kernel(const AtomRec *__restrict__ rec, const int *__restrict__ slice
         const bool wide = !D64 && (g.Rs & 1) == 0;
 #pragma unroll
         for (int i = 0; i < T::WR; ++i) {
-            float backa[4];
+            float2 backa[4];
+            const float *sqlo = nullptr;      // what the floats of sq leave of s^2
+            if constexpr (SCALED) {
+                sqlo = sq + (slice_sq ? slice_sq[slice] : 0) + g.R + g.C;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) backa[v] = SCALED ? damp_back(bref, sm.s_a[wr0 + 16 * i + 4 * lg + v]) : 1.0f;
+                for (int v = 0; v < 4; ++v) {
+                    const int x = wr0 + 16 * i + 4 * lg + v;
+                    backa[v] = damp_back2(bref, sm.s_a[x], row0 + x < g.R ? sqlo[row0 + x] : 0.0f, 1.0);
+                }
+            }
 #pragma unroll
             for (int j = 0; j < T::WC; ++j) {
                 const int c = col0 + wc0 + 16 * j + li;
                 if (c >= g.C) continue;
                 if constexpr (SCALED) {
-                    const float backb = damp_back(bref, sm.s_b[wc0 + 16 * j + li]);
+                    const float2 backb = damp_back2(bref, sm.s_b[wc0 + 16 * j + li], sqlo[g.R + c], 1.0);
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
-                        accR[i][j][v] = accR[i][j][v] * backa[v] * backb;
-                        accI[i][j][v] = accI[i][j][v] * backa[v] * backb;
+                        const float2 b = mul2(backa[v], backb);
+                        accR[i][j][v] = __builtin_fmaf(accR[i][j][v], b.x, accR[i][j][v] * b.y);
+                        accI[i][j][v] = __builtin_fmaf(accI[i][j][v], b.x, accI[i][j][v] * b.y);
                     }
                 }
                 if constexpr (!D64) {

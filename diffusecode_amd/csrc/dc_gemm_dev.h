@@ -71,11 +71,38 @@ __device__ __forceinline__ float2 cis(uint64_t ph) {
 // operands carry exp(-(B - Bref) s^2) and the epilogue multiplies by exp(-Bref s^2).
 // Bref is the least B of the slice's occupied atoms: the factors are at most
 // 1 (s^2 >= 0, split_sq), and those that are small are so beside the term of that
-// atom in the same sum.  (B log2(e) is what the kernels hold.)
+// atom in the same sum.
 constexpr float NO_B = 3.0e38f;            // least B of no atoms
 __device__ __forceinline__ float damp_ref(float bmin) {
-    const float b = bmin < NO_B ? bmin * 1.4426950408889634f : 0.0f;
+    const float b = bmin < NO_B ? bmin : 0.0f;
     return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, b)));   // uniform
+}
+// c exp(-bref (s + lo)) as a float and what is left of it (to 1e-11); lo: what a
+// float leaves of s^2.  The factor is one for a whole row or column, and s^2 is for all
+// atoms, so their rounding does not average out as that of the operands does.
+// (24 members on 93 x 215 points, chi^2, which amplifies a common error of F by
+// I / (I - T): 2.9e-6 with the factor in one float.)
+__device__ __forceinline__ float2 damp_back2(float bref, float s, float lo, double c) {
+    const double p = -1.44269504088896340736 * (double)bref * ((double)s + (double)lo), n = rint(fmax(-1000.0, fmin(1000.0, p)));
+    const double x = (p - n) * 0.69314718055994530942;
+    double e = 1.0 / 362880.0;             // exp(x), |x| <= 0.35: Taylor to x^9, 1e-11
+    e = __builtin_fma(e, x, 1.0 / 40320.0);
+    e = __builtin_fma(e, x, 1.0 / 5040.0);
+    e = __builtin_fma(e, x, 1.0 / 720.0);
+    e = __builtin_fma(e, x, 1.0 / 120.0);
+    e = __builtin_fma(e, x, 1.0 / 24.0);
+    e = __builtin_fma(e, x, 1.0 / 6.0);
+    e = __builtin_fma(e, x, 0.5);
+    e = __builtin_fma(e, x, 1.0);
+    e = __builtin_fma(e, x, 1.0);
+    const double d = ldexp(e * c, (int)n);
+    const float h = (float)d;
+    return make_float2(h, (float)(d - (double)h));
+}
+// the product of two such factors
+__device__ __forceinline__ float2 mul2(float2 a, float2 b) {
+    const float h = a.x * b.x;
+    return make_float2(h, __builtin_fmaf(a.x, b.x, -h) + __builtin_fmaf(a.x, b.y, a.y * b.x));
 }
 // 2^-(bref sv), to FP32's rounding
 __device__ __forceinline__ float damp_back(float bref, float sv) {

@@ -330,9 +330,12 @@ PrepArgs base_prep(const Grid &g, int mapping);
 inline int model_scheme(int prec) { return prec == DC_PREC_BF16X3 ? DC_PREC_FP16X3 : prec; }
 // s^2 of a grid (metric rten, corner eck, increments vi) as the sum of a part of
 // the R rows and one of the C columns (f1 valid of each period of C0, the others
-// 0), R + C floats.  The least row part is moved to the columns: on a grid whose rows
-// and columns are orthogonal both parts are then >= 0, and neither factor of
-// exp(-B s^2) exceeds 1 for B >= 0.
-void split_sq(const double *rten, const double *eck, const double *vi, const GemmGeom &gg, int f1, float *out);
+// 0), R + C floats.  For the schemes with FP16 operands (sq_floats: twice as many)
+// the least row part is moved to the columns -- on a grid whose rows and columns are
+// orthogonal both parts are then >= 0, and neither factor of exp(-B s^2) exceeds 1
+// for B >= 0 -- and behind the floats lie what they leave of the parts (damp_back2).
+inline bool f16_scheme(int scheme) { return scheme == DC_PREC_FP16X2 || scheme == DC_PREC_FP16X3; }
+inline int sq_floats(const GemmGeom &gg, bool f16) { return (gg.R + gg.C) * (f16 ? 2 : 1); }
+void split_sq(const double *rten, const double *eck, const double *vi, const GemmGeom &gg, int f1, bool f16, float *out);
 
 }  // namespace dc

@@ -78,8 +78,9 @@ int plan_model(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, bool dev) {
         const double nv = std::sqrt(std::fabs(dotg(v, m->rten, v)));
         if (std::fabs(dotg(v1, m->rten, v)) > 1e-12 * std::max(1.0, n1 * nv)) mp.separable = false;
     }
-    mp.sq.assign((size_t)gg.R + gg.C, 0.0f);
-    split_sq(m->rten, m->eck, m->vi, gg, g.f[1], mp.sq.data());
+    const bool f16 = f16_scheme(model_scheme(c->prec));
+    mp.sq.resize((size_t)sq_floats(gg, f16));
+    split_sq(m->rten, m->eck, m->vi, gg, g.f[1], f16, mp.sq.data());
 
     // counting sort by type, vacancies dropped
     std::vector<int> cnt(m->nscat + 1, 0);
