@@ -39,7 +39,7 @@
 // hold 16, and S and D, being sums, then cost 1.4 times the row-by-row
 // error).  FP16's range also has to hold the row factor exp(-B s_r^2): the atoms
 // of a plane carry exp(-(B - Bref) s_r^2) and its coefficients exp(-Bref s_r^2)
-// (adj_ref_kernel).  Either unit runs 16 times the FP32 rate.
+// (adj_begin_kernel).  Either unit runs 16 times the FP32 rate.
 #include <algorithm>
 #include <atomic>
 
@@ -147,36 +147,39 @@ __device__ __forceinline__ bool pair_rows(const AdjArgs &a, int p, int &r1, int 
     return r1 < a.R;
 }
 
-// Bref (times log2(e)) of the span's planes: the least B of a plane's atoms, whose row factors
+// What a reverse pass starts with: the gradient array cleared (vacancies keep 0)
+// and, for damped passes in 2 parts, Bref (times log2(e)) of every plane, a
+// work-group each: the least B of the plane's atoms, whose row factors
 // exp(-(B - Bref) s_r^2) are then at most 1 and hold 17 bits or more down to
 // 2^-7; where B spreads further over the rows, Bref moves up, to factors of
-// 2^14 at most (B may spread over 21 / s_r^2 in all).  Unlike in the forward sum a
-// small factor is not small beside others: it is alone in its atom's gradient.  One work-group a plane;
-// tiles are in plane order, a plane's atoms contiguous.  Bound by latency: 9 us for 48
-// planes of 4,000 atoms, and no less with the search, the reads or the reduction wider.
-__global__ void __launch_bounds__(1024) adj_ref_kernel(AdjArgs a, int tile0, int ntiles, int plane0, float *__restrict__ ref) {
-    __shared__ float red[3][16];
-    const int plane = plane0 + blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    auto first = [&](int p) {              // first tile of a plane >= p
-        int lo = 0, hi = ntiles;
-        while (lo < hi) {
-            const int m = (lo + hi) / 2;
-            if (a.tiles[tile0 + m].z < p) lo = m + 1;
-            else hi = m;
-        }
-        return lo;
-    };
-    const int t0 = first(plane), t1 = first(plane + 1);
-    float b0 = NO_B, b1 = -NO_B, s = 0.0f;
-    if (t0 < t1) {
-        for (int k = a.tiles[tile0 + t0].x + (int)threadIdx.x; k < a.tiles[tile0 + t1 - 1].y; k += 1024) {
-            const float b = a.rec[k].pad;
-            b0 = fminf(b0, b);
-            b1 = fmaxf(b1, b);
-        }
-        const float *sq = a.sq + (long long)(plane / a.planes_per_sq) * a.sq_stride;
-        for (int r = threadIdx.x; r < a.R; r += 1024) s = fmaxf(s, fabsf(sq[r]));
+// 2^14 at most (B may spread over 21 / s_r^2 in all).  Unlike in the forward sum
+// a small factor is not small beside others: it is alone in its atom's gradient.
+// Bound by latency: two dependent reads beside the clearing, which alone took a
+// launch of its own before.
+constexpr int BEGIN_THREADS = 1024;
+__global__ void __launch_bounds__(BEGIN_THREADS) adj_begin_kernel(AdjArgs a, int nref, double *__restrict__ grad, long long ngrad) {
+    __shared__ float red[3][BEGIN_THREADS / 64];
+    if ((int)blockIdx.x >= nref) {
+        for (long long k = (long long)(blockIdx.x - nref) * BEGIN_THREADS + threadIdx.x; k < ngrad;
+             k += (long long)(gridDim.x - nref) * BEGIN_THREADS)
+            grad[k] = 0.0;
+        return;
     }
+    const int plane = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int2 range = a.ranges[plane];
+    float b0 = NO_B, b1 = -NO_B, s = 0.0f;
+    for (long long k = range.x + (int)threadIdx.x; k < range.y; k += 8 * BEGIN_THREADS) {
+        float b[8];                        // eight reads in flight
+#pragma unroll
+        for (int u = 0; u < 8; ++u) b[u] = a.rec[min(k + u * BEGIN_THREADS, (long long)range.y - 1)].pad;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            b0 = fminf(b0, b[u]);
+            b1 = fmaxf(b1, b[u]);
+        }
+    }
+    const float *sq = a.sq + (long long)(plane / a.planes_per_sq) * a.sq_stride;
+    for (int r = threadIdx.x; r < a.R; r += BEGIN_THREADS) s = fmaxf(s, fabsf(sq[r]));
 #pragma unroll
     for (int h = 1; h < 64; h *= 2) {
         b0 = fminf(b0, __shfl_xor(b0, h));
@@ -190,13 +193,14 @@ __global__ void __launch_bounds__(1024) adj_ref_kernel(AdjArgs a, int tile0, int
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < 16; ++w) {
+#pragma unroll
+        for (int w = 1; w < BEGIN_THREADS / 64; ++w) {
             b0 = fminf(b0, red[0][w]);
             b1 = fmaxf(b1, red[1][w]);
             s = fmaxf(s, red[2][w]);
         }
-        ref[blockIdx.x] = b0 > b1 || !(s > 0.0f) ? 0.0f
-                          : LOG2E * b0 + fminf(fmaxf(LOG2E * (b1 - b0) - 7.0f / s, 0.0f), 14.0f / s);
+        a.ref[plane] = b0 > b1 || !(s > 0.0f) ? 0.0f
+                       : LOG2E * b0 + fminf(fmaxf(LOG2E * (b1 - b0) - 7.0f / s, 0.0f), 14.0f / s);
     }
 }
 
@@ -206,7 +210,7 @@ __global__ void __launch_bounds__(1024) adj_ref_kernel(AdjArgs a, int tile0, int
 // One work-group per (plane, tile), a wave per k-step.  2 parts: the coefficients
 // of each column, times the rows' exp(-Bref s_r^2), are scaled to below 2^15 (by
 // column, since what the columns' own exp(-B s_c^2) leaves of them differs), and the
-// scales noted: scales[plane][tile][column], then the tiles' least ones, then Bref.
+// scales noted: scales[plane][tile][column], then the tiles' least ones.
 template <int NP>
 __global__ void __launch_bounds__(256) adj_words_kernel(AdjArgs a, int plane0, int nplane, u32x4 *__restrict__ out) {
     constexpr int NW = 6 * NP;
@@ -214,7 +218,6 @@ __global__ void __launch_bounds__(256) adj_words_kernel(AdjArgs a, int plane0, i
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float *scales = reinterpret_cast<float *>(out + (long long)nplane * a.ctiles * a.nkt * (NW * 64));
     float *tscales = scales + (long long)nplane * a.ctiles * CT;
-    const float *ref = tscales + (long long)nplane * a.ctiles;
     for (long long x = blockIdx.x; x < (long long)nplane * a.ctiles; x += gridDim.x) {
         const int ct = (int)(x % a.ctiles), pl = (int)(x / a.ctiles);
         const int c = ct * CT + (lane & 15);
@@ -224,7 +227,7 @@ __global__ void __launch_bounds__(256) adj_words_kernel(AdjArgs a, int plane0, i
         float sg[3], scale = 1.0f, bref = 0.0f;
         weight_scales<NP>(a, sq, sg);
         if constexpr (NP == 2) {
-            if (a.damped) bref = ref[pl];
+            if (a.damped) bref = a.ref[plane0 + pl];
             float m = 0.0f;
             if (in)
                 for (int r = threadIdx.x >> 4; r < a.R; r += 16) {
@@ -335,12 +338,12 @@ __global__ void __launch_bounds__(NT, 2) adjoint_kernel(AdjArgs a, int tile0, in
     const bool center = a.center && chunk == 0;
     float sg[3];
     weight_scales<NP>(a, sq, sg);
-    // scales of the columns and of the tiles, and Bref (adj_words_kernel)
+    // scales of the columns and of the tiles (adj_words_kernel)
     const float *scales = reinterpret_cast<const float *>(words + (long long)nplane * a.ctiles * a.nkt * (NW * 64));
     const float *tscales = scales + (long long)nplane * a.ctiles * CT;
     float bref = 0.0f;
     if constexpr (NP == 2)
-        if (a.damped) bref = (tscales + (long long)nplane * a.ctiles)[tile.z - plane0];
+        if (a.damped) bref = a.ref[tile.z];
     scales += (long long)(tile.z - plane0) * a.ctiles * CT;
     tscales += (long long)(tile.z - plane0) * a.ctiles;
     const float s2c = sq[a.R / 2], s2cs = s2c * sg[2];
@@ -734,11 +737,6 @@ __global__ void jvp_reduce_kernel(JvpArgs a) {
     }
 }
 
-__global__ void fill_zero_kernel(double *p, long long n) {
-    for (long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long long)gridDim.x * blockDim.x)
-        p[k] = 0.0;
-}
-
 }  // namespace
 
 hipError_t launch_batch_reduce(const BatchReduceArgs &a, int nblocks, hipStream_t st) {
@@ -754,13 +752,6 @@ hipError_t launch_batch_reduce(const BatchReduceArgs &a, int nblocks, hipStream_
 hipError_t launch_jvp_reduce(const JvpArgs &a, hipStream_t st) {
     if (a.g.P <= 0 || a.ndir <= 0) return hipSuccess;
     jvp_reduce_kernel<<<(unsigned)((a.g.P + 255) / 256), 256, 0, st>>>(a);
-    return hipGetLastError();
-}
-
-hipError_t launch_fill_zero(double *p, long long n, hipStream_t st) {
-    if (n <= 0) return hipSuccess;
-    const long long nb = std::min<long long>((n + 255) / 256, 4096);
-    fill_zero_kernel<<<(unsigned)nb, 256, 0, st>>>(p, n);
     return hipGetLastError();
 }
 
@@ -814,7 +805,16 @@ void adjoint_plan(AdjArgs &a, int ntiles, bool split, int force) {
     a.nchunk = (int)std::min<long long>(a.chunks, std::max<long long>(1, ADJ_PART_MAX / (48LL * a.groups * std::max(a.natoms, 1))));
     a.nset = a.groups * a.nchunk;
     a.walk = (a.tpg + WALK_TILES - 1) / WALK_TILES;
-    a.plane_words = (long long)a.ctiles * a.nkt * 6 * a.parts * 64 + (a.ctiles * (CT + 1) + 4) / 4;   // and the scales, Bref
+    a.plane_words = (long long)a.ctiles * a.nkt * 6 * a.parts * 64 + (a.ctiles * (CT + 1) + 3) / 4;   // and the scales
+}
+
+hipError_t launch_adj_begin(const AdjArgs &a, int nplanes, double *grad, long long ngrad, hipStream_t st) {
+    const int nref = a.parts == 2 && a.damped ? nplanes : 0;
+    if (nref > 0 && (!a.ranges || !a.ref || a.planes_per_sq < 1)) return hipErrorInvalidValue;
+    const long long nz = std::min<long long>((std::max<long long>(ngrad, 0) + BEGIN_THREADS - 1) / BEGIN_THREADS, 1024);
+    if (nref + nz <= 0) return hipSuccess;
+    adj_begin_kernel<<<(unsigned)(nref + nz), BEGIN_THREADS, 0, st>>>(a, nref, grad, ngrad);
+    return hipGetLastError();
 }
 
 hipError_t launch_adjoint(const AdjArgs &a, const AdjSpan &s, uint4 *words, hipStream_t st) {
@@ -832,8 +832,6 @@ hipError_t launch_adjoint(const AdjArgs &a, const AdjSpan &s, uint4 *words, hipS
         }
     };
     if (a.parts == 2) {
-        float *ref = reinterpret_cast<float *>(w + (long long)s.nplanes * a.ctiles * a.nkt * (12 * 64)) + (long long)s.nplanes * a.ctiles * (CT + 1);
-        if (a.damped) adj_ref_kernel<<<s.nplanes, 1024, 0, st>>>(a, s.tile0, s.ntiles, s.plane0, ref);
         adj_words_kernel<2><<<nb, 256, 0, st>>>(a, s.plane0, s.nplanes, w);
         a.nk == 1 ? run(adjoint_kernel<2, 1>) : a.nk == 2 ? run(adjoint_kernel<2, 2>) : a.nk == 3 ? run(adjoint_kernel<2, 3>)
             : a.nk == 4 ? run(adjoint_kernel<2, 4>) : run(adjoint_kernel<2, 5>);

@@ -46,7 +46,7 @@ struct BatchState {
     int rows = 0;                        // form-factor rows on the device (the bins the metrics reach, and a margin)
     PinBuf h_cf, h_sq, h_chi;            // pinned: form-factor rows, s^2 parts, chi^2 of the members
     DevBuf pos, occ, bdw, idx, rec, sbeg, stype, ssq, msl, sorder, partial, cfact, rten, sq, target, weight, icalc,
-        chi, q, qs, atiles, part, grad, wq;
+        chi, q, qs, atiles, aranges, aref, part, grad, wq;
     bool queue = false;                  // GEMM items from a device counter (autotuner's choice)
     bool primed = false;                 // records built and autotuned once
     hipGraph_t graph = nullptr;
@@ -55,7 +55,7 @@ struct BatchState {
 
     std::vector<DevBuf *> buffers() {
         return {&pos, &occ, &bdw, &idx, &rec, &sbeg, &stype, &ssq, &msl, &sorder, &partial, &cfact, &rten, &sq,
-                &target, &weight, &icalc, &chi, &q, &qs, &atiles, &part, &grad, &wq};
+                &target, &weight, &icalc, &chi, &q, &qs, &atiles, &aranges, &aref, &part, &grad, &wq};
     }
 };
 
@@ -246,8 +246,10 @@ int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
     b.nsorted = (int)b.order.size();
     int off = 0;
     const int na = adjoint_tile_atoms();
+    std::vector<int2> ranges((size_t)d->nmembers * d->nscat, make_int2(0, 0));
     for (size_t sg = 0; sg < segs_all.size(); ++sg) {
         const int m = seg_member[sg];
+        ranges[(size_t)m * d->nscat + segs_all[sg].first] = make_int2(off, off + segs_all[sg].second);
         for (int k = 0; k < segs_all[sg].second; k += na)
             tiles.insert(tiles.end(), {off + k, off + std::min(segs_all[sg].second, k + na),
                                        m * d->nscat + segs_all[sg].first, m});
@@ -271,6 +273,8 @@ int build_state(dc_ctx *c, const dc_batch_desc *d, BatchState &b) {
     if ((st = upload(c, b.idx, b.order.data(), b.order.size()))) return st;
     if ((st = make_slices(c, b, slice_len(c, kchunk_for(b.pl, b.segs, b.pl.scheme))))) return st;
     if ((st = upload(c, b.atiles, tiles.data(), tiles.size()))) return st;
+    if ((st = upload(c, b.aranges, ranges.data(), ranges.size()))) return st;
+    if ((st = ensure(c, b.aref, sizeof(float) * ranges.size()))) return st;
     if ((st = ensure(c, b.rec, sizeof(AtomRec) * std::max(b.nsorted, 1)))) return st;
     if ((st = ensure(c, b.cfact, sizeof(double) * 2 * (size_t)b.rows * d->nscat * M))) return st;
     if ((st = pin_ensure(c, b.h_cf, sizeof(double) * (2 * (size_t)b.rows * d->nscat + 9) * M))) return st;
@@ -381,7 +385,6 @@ int enqueue(dc_ctx *c, BatchState &b, const StepIO &io, int tile, int nwg, bool 
     chi_finish_kernel<<<b.nmembers, 256, 0, c->st>>>(ptr<double>(b.chi), b.nblk, reinterpret_cast<double *>(b.h_chi.p));
     HIPCHK(hipGetLastError());
     if (b.want_grad) {
-        HIPCHK(launch_fill_zero(io.grad, 5 * b.natoms, c->st));
         AdjArgs aa = b.adj;
         aa.rec = ptr<AtomRec>(b.rec);
         aa.tiles = ptr<int4>(b.atiles);
@@ -395,6 +398,9 @@ int enqueue(dc_ctx *c, BatchState &b, const StepIO &io, int tile, int nwg, bool 
         aa.rc = 0.5f * (float)(b.g.f[0] - 1);
         aa.jc = 0.5f * (float)(b.g.f[1] - 1);
         aa.mc = 0.5f * (float)(b.g.f[2] - 1);
+        aa.ranges = ptr<int2>(b.aranges);
+        aa.ref = ptr<float>(b.aref);
+        HIPCHK(launch_adj_begin(aa, b.nmembers * b.nscat, io.grad, 5 * b.natoms, c->st));
         for (const AdjSpan &s : b.spans) HIPCHK(launch_adjoint(aa, s, ptr<uint4>(b.qs), c->st));
         AdjFinishArgs fa{};
         fa.part = ptr<double>(b.part);

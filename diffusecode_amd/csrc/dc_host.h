@@ -61,7 +61,7 @@ struct dc_ctx {
     DevBuf rec, slice_beg, slice_order, slice_type, lot_slice, partial, cfact, istl, idx, oid, offs, xat, w;
     DevBuf acsf, dsi, csf, wm, wv, lat, out_tcsf, out[5];
     // device buffers of the refinement model
-    DevBuf m_pos, m_w, m_b, m_sq, m_q, m_part, m_grad, m_tiles, m_gi, m_f, m_qt, m_qs, m_jw, m_dsl, m_di;
+    DevBuf m_pos, m_w, m_b, m_sq, m_q, m_part, m_grad, m_tiles, m_gi, m_f, m_qt, m_qs, m_jw, m_dsl, m_di, m_rng, m_ref;
     // crystal
     bool have_crystal = false;
     DevBuf pos, iscat;
@@ -99,7 +99,7 @@ struct dc_ctx {
     std::vector<DevBuf *> buffers() {
         return {&rec, &slice_beg, &slice_order, &slice_type, &lot_slice, &partial, &cfact, &istl, &idx, &oid, &offs, &xat, &w,
                 &acsf, &dsi, &csf, &wm, &wv, &lat, &out_tcsf, &out[0], &out[1], &out[2], &out[3], &out[4],
-                &m_pos, &m_w, &m_b, &m_sq, &m_q, &m_part, &m_grad, &m_tiles, &m_gi, &m_f, &m_qt, &m_qs, &m_jw, &m_dsl, &m_di,
+                &m_pos, &m_w, &m_b, &m_sq, &m_q, &m_part, &m_grad, &m_tiles, &m_gi, &m_f, &m_qt, &m_qs, &m_jw, &m_dsl, &m_di, &m_rng, &m_ref,
                 &pos, &iscat, &type_idx, &runs, &arena};
     }
 };

@@ -160,6 +160,8 @@ struct AdjArgs {
     float rc, jc, mc;       // centres of the row / column index weights
     int fold;               // rows taken in mirrored pairs (s_r^2 mirrored, or no B)
     int damped;             // records hold B other than 0
+    const int2 *ranges;     // first atom and end of every plane's atoms (damped, 2 parts)
+    float *ref;             // and what launch_adj_begin makes of them, a float a plane
     // set by adjoint_plan
     int parts;              // 16-bit parts of the operands: 3 (BF16) in FP32, 2 (FP16) in the split precisions
     int center;             // the centre row of the pairs is added apart
@@ -216,7 +218,6 @@ struct BatchReduceArgs {
     float2 *q;              // (plane, nscat, nmembers) or null
 };
 hipError_t launch_batch_reduce(const BatchReduceArgs &a, int nblocks, hipStream_t st);
-hipError_t launch_fill_zero(double *p, long long n, hipStream_t st);
 // Forward-mode derivative (JVP) of I along ndir parameter directions: slice
 // group 5k + q of the GEMM holds direction k weighted by q = (docc,
 // occ dx, occ dy, occ dz, occ dB); per pixel
@@ -243,6 +244,8 @@ std::vector<AdjSpan> adjoint_spans(const AdjArgs &a, const int *tiles, int ntile
 // Compute units of the current device (queried once per device; 256 if unknown).
 int device_cu_count();
 int adjoint_max_walk();
+// Clears the ngrad gradients and, where the pass needs it, sets a.ref of all planes.
+hipError_t launch_adj_begin(const AdjArgs &a, int nplanes, double *grad, long long ngrad, hipStream_t st);
 // Operand words of the span's planes (room for nplanes * plane_words), then its tiles.
 hipError_t launch_adjoint(const AdjArgs &a, const AdjSpan &s, uint4 *words, hipStream_t st);
 hipError_t launch_adjoint_finish(const AdjFinishArgs &a, hipStream_t st);

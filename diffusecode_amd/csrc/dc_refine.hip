@@ -212,9 +212,11 @@ int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, double *grad
     // atom tiles inside one type
     const int na = adjoint_tile_atoms();
     std::vector<int> tiles;
+    std::vector<int2> ranges(std::max(nq, 1), make_int2(0, 0));
     int a0 = 0;
     for (int t = 0; t < nq; ++t) {
         const int n = mp.segs[t].second;
+        ranges[t] = make_int2(a0, a0 + n);
         for (int b = 0; b < n; b += na) {
             tiles.insert(tiles.end(), {a0 + b, a0 + std::min(n, b + na), t, 0});
         }
@@ -225,11 +227,14 @@ int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, double *grad
     hipEvent_t e0, e1;
     if ((st = mark(c, e0))) return st;
     int *d_qt, *d_tiles;
+    int2 *d_ranges;
     if ((st = stage(c, c->m_qt, qtype.data(), qtype.size(), d_qt))) return st;
     if ((st = stage(c, c->m_tiles, tiles.data(), tiles.size(), d_tiles))) return st;
+    if ((st = stage(c, c->m_rng, ranges.data(), ranges.size(), d_ranges))) return st;
     if ((st = stage_flush(c))) return st;
     if ((st = ensure(c, c->m_q, sizeof(float2) * gg.P * std::max(nq, 1)))) return st;
-    HIPCHK(launch_fill_zero(grad, 5 * m->natoms, c->st));
+    if ((st = ensure(c, c->m_ref, sizeof(float) * ranges.size()))) return st;
+    if (ntiles == 0) HIPCHK(launch_adj_begin(AdjArgs{}, 0, grad, 5 * m->natoms, c->st));
     if (ntiles > 0) {
         QArgs qa{};
         qa.g = mp.g;
@@ -267,6 +272,9 @@ int model_adjoint(dc_ctx *c, const dc_model_desc *m, ModelPlan &mp, double *grad
         c->stats.adjoint_walk = aa.walk;
         if ((st = ensure(c, c->m_part, sizeof(double) * 6 * (size_t)aa.nset * std::max(mp.nsorted, 1)))) return st;
         aa.part = ptr<double>(c->m_part);
+        aa.ranges = d_ranges;
+        aa.ref = ptr<float>(c->m_ref);
+        HIPCHK(launch_adj_begin(aa, nq, grad, 5 * m->natoms, c->st));
         const std::vector<AdjSpan> spans = adjoint_spans(aa, tiles.data(), ntiles);
         long long most = 0;
         for (const AdjSpan &s : spans) most = std::max<long long>(most, s.nplanes);
