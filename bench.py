@@ -244,14 +244,14 @@ def bench_post(_lib, FR, torch, steps=5):
     ctx.close()
     ms = t / steps * 1e3
     return {"ms": round(ms, 3), "grid": list(inc), "pixels_per_s": n / (ms * 1e-3),
-            "steps": "four_weight + Lanczos(dsi) + four_conv(csf, dsi, dsi3d) + Lanczos(dsi3d), FP64, hipFFT Z2Z"}
+            "steps": "four_weight + Lanczos(dsi) + four_conv(csf, dsi, dsi3d) + Lanczos(dsi3d), FP64 line transforms"}
 
 
 def bench_batch(_lib, X, FR, prec, torch):
     """Population step (chi^2 of 96 members against their own layers): the
     generation's arrays (positions, occupancies, B, targets) resident in HBM,
     steps issued back to back as a DIFFEV loop on the device would; the first
-    call plans, autotunes and captures the graph."""
+    call plans and autotunes."""
     from diffusecode_amd.population import Population
     crs = X.population()
     eck, vi, inc = FR.grid_block((-4.0, -4.0, 0.0), (4.0, 4.0, 0.0), (256, 256, 1))
@@ -270,7 +270,7 @@ def bench_batch(_lib, X, FR, prec, torch):
            "inputs": "device-resident generation arrays, steps back to back"}
     for want_grad in (False, True):
         g = d_grad if want_grad else None
-        pop.ctx.batch_chi2_dev(desc, d_pos, d_occ, d_bdw, d_t, grad=g)      # plan, tune, capture
+        pop.ctx.batch_chi2_dev(desc, d_pos, d_occ, d_bdw, d_t, grad=g)      # plan, tune
         rows = []
         for it in range(6):
             pop.ctx.batch_chi2_dev(desc, d_pos, d_occ, d_bdw, d_t, grad=g)

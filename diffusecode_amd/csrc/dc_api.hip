@@ -165,10 +165,13 @@ int fold_side(const GemmGeom &gg, int fold_mask, int tile) {
 
 // Time model of a launch with a fold tile, in microseconds on one MI355X: a
 // stage of 32 atoms costs its MFMAs on a SIMD's two waves (measured at the
-// sustained clock: 0.091 per 16 x 16 block for the three products; FP32's six fit
-// 0.34 tile by tile, but 0.49 ranks slice counts as measured: 62,000 atoms x 33 x
-// 65 x 65 in 60 slices and 4 full rounds 0.41 ms, in 44 and 3 rounds 0.43) plus the operand generation that does not overlap with
-// them, and an item its set-up and epilogue.
+// sustained clock: 0.091 per 16 x 16 block for the three products) plus the
+// operand generation that does not overlap with them, and an item its set-up and
+// epilogue.  FP32's six products fit 0.34 tile by tile; 0.49, with what the longer
+// generation leaves exposed, ranks the slice counts: over ten grids from 1,001
+// points x 4,000 atoms to 250 x 250 x 3 x 176,000 the planned call took 0.93
+// to 1.04 of the best of 15 forced lengths (FP16X3, within its limits on the
+// length: 0.95 to 1.21, the limits being the price of its accuracy).
 static double fold_stage_us(const TileInfo &ti, int prec) {
     const double wr = ti.rt / 128.0, wc = ti.ct / 16.0;
     const double m = prec == DC_PREC_FP32 ? 0.49 : 0.091;

@@ -64,9 +64,10 @@ __host__ __device__ inline uint64_t dither_turn(uint32_t k, uint32_t salt) {
 // The same rotation from a 32-bit avalanche hash (the murmur3 finaliser) in
 // the top 32 bits of the turn: about a third of the VALU work of the 64-bit
 // one, which every thread of a GEMM stage evaluates for its atom (split
-// schemes: headline GEMM -1.9%).  The FP32 schemes keep the 64-bit hash:
-// their results stay as they were, one of their 1e-6 tests sitting within
-// 10% of the bar.
+// schemes: headline GEMM -1.9%).  The FP32 schemes of the general tiles keep
+// the 64-bit hash: their results stay as they were, one of their 1e-6 tests
+// sitting within 10% of the bar.  The mirrored-pair tiles take this one in
+// every scheme (FP32 for its tables' turns, dc_fold.h).
 __host__ __device__ inline uint32_t dither_hash32(uint32_t k, uint32_t salt) {
     uint32_t h = k * 0x9E3779B1u + salt;
     h ^= h >> 16;

@@ -49,12 +49,13 @@
 // against FP64 4.2e-8 -> 3.1e-8 on a 4,000-atom line, 5.1e-8 -> 4.0e-8 there).
 //
 // Bound: half matrix cores, half the VALU work of forming operands, which
-// overlaps with them only in part (FP16X3, 256 x 176: 47% of the MFMA peak
-// busy, 2.9 other VALU instructions per MFMA).  Measured against dc_gemm.hip:
-// 256,000 atoms x 81 x 161 x 161, FP16X3 10.06 -> 6.1 ms with equal
-// slices; 62,000 atoms x 33 x 65 x 65, FP32 1.38 -> 0.41 ms; an 8,000-atom
-// 101^2 layer, FP32 174 -> 17 us (with slices cut to fill the device); a
-// population of 96 (1.8M atoms, 256^2, damped) 2.66 -> 1.6 ms.
+// overlaps with them only in part (256 x 176: matrix cores busy 42% of the time in
+// FP16X3, 47% in BF16X3, 3.0 and 3.3 other VALU instructions per MFMA; FP32
+// 128 x 96 37% and 7.3).  Measured against dc_gemm.hip:
+// 256,000 atoms x 81 x 161 x 161, FP16X3 10.06 -> 6.75 ms (6.7 to 7.2 from box to
+// box); 62,000 atoms x 33 x 65 x 65, FP32 1.38 -> 0.39 ms; an 8,000-atom
+// 101^2 layer, FP32 174 -> 15 us (with slices cut to fill the device); a
+// population of 96 (1.8M atoms, 256^2, damped) 2.66 -> 1.5 ms.
 //
 // Epilogue: an even lane holds X and its neighbour Y of the same pair, so
 // one quad permute gives each lane one finished column.
@@ -74,10 +75,14 @@ struct FoldCfg {
     static constexpr int RH = RT / 16, CH = WC;    // 16-row groups, 8-pair groups
 };
 
-// Fold tiles (WR, WC), in the order of their tile indices.  Grids of 2^k + 1
-// points have 17, 33, 65 pairs: WC 3, 5 and 9 hold them with one group to spare
-// where 2, 6 and 11 take another tile or leave 31 and 26% of it empty; 101 and
-// 201 points (51 and 101 pairs) fill 90% of one and two tiles of WC 7, 79% of 8.
+// Fold tiles (WR, WC), in the order of their tile indices.  The WC of one row
+// block are close enough together that 25 pairs or more fill 77% of their
+// tiles at least and 92% on the average (9 to 24 pairs: 82%); those of two row
+// blocks start at 4, since few columns leave their row operands, formed anew
+// for every tile of columns, too little to multiply with (49 pairs or more: 83%
+// at least).  What a half-empty tile costs: 33 pairs in 48 instead of 40, 0.456
+// -> 0.426 ms a call (62,000 atoms x 33 x 65 x 65, FP32); 101 in 128
+// instead of 112, 0.474 -> 0.444 ms (GEMM of 32 lots, 804 rows, FP16X3).
 #define DC_FOLD_TILES(X) \
     X(0, 2, 11) X(1, 1, 11) X(2, 2, 8) X(3, 1, 8) X(4, 2, 6) X(5, 1, 6) X(6, 2, 4) X(7, 1, 4) X(8, 1, 2) X(9, 2, 9) X(10, 1, 9) \
     X(11, 1, 5) X(12, 1, 3) X(13, 2, 7)
@@ -182,7 +187,7 @@ __device__ __forceinline__ void fold_tables(FoldTables<T> &tb, const int *__rest
     // The column operands go to the first waves in FP32 and to the last ones in
     // the split schemes (fold_b).  Measured, both orders of both: FP32 65^3 0.412 ms, with the split
     // schemes' order 0.47, with both row tables on the first pair 0.42;
-    // FP16X3 161^3 6.1 ms, with the columns on the first waves 6.5, with
+    // FP16X3 161^3 (on the fastest box) 6.1 ms, with the columns on the first waves 6.5, with
     // the high groups spread as in FP32 6.5.
     constexpr bool F32 = SCHEME == SCH_FP32;
     if (wave == 0 || wave == 1) {

@@ -5,7 +5,9 @@ metric, scored by chi^2 against its own target grid in one pass.
 DIFFEV runs one DISCUS macro per member over an MPI farm
 (diffev/prog/diffev_kdo.f90:676, lib_f90/with_mpi.f90:281-609); here the
 whole generation is one persistent GEMM launch plus one fused reduction and
-one adjoint launch, replayed as a hipGraph from the second generation on.
+one adjoint launch, replayed as a hipGraph from the second generation on where
+its arrays come from the host (score) and launched one by one, on the arrays where
+they lie, where they are the device's (Context.batch_chi2_dev).
 """
 from __future__ import annotations
 

@@ -51,7 +51,9 @@ extern "C" {
 #define DC_ER_LIB 99            /* library-side errors (no DISCUS equivalent) */
 
 /* ---- arithmetic of the phase GEMM --------------------------------------- */
-#define DC_PREC_FP32 0          /* plain FP32 MFMA (the drop-in)            */
+#define DC_PREC_FP32 0          /* FP32 operands and results (the drop-in):
+                                   all 24 bits, in three BF16 parts and six
+                                   MFMA products, or FP32 MFMA              */
 #define DC_PREC_BF16X3 1        /* split BF16 hi/lo, 3 MFMA products; runs with
                                    the <F> subtraction or the cross-lot variance
                                    (dc_four_run*) and the forward sums of
@@ -333,9 +335,10 @@ int dc_device_index(const dc_ctx *ctx);
  * in one pass: one persistent phase-GEMM launch over all members' atoms, one
  * fused reduction, and (grad != NULL) one adjoint launch.  The first call of
  * a batch shape (member sizes, types, grid, precision, outputs requested)
- * plans, autotunes the GEMM tile and grid size, and captures the step as a
- * hipGraph; later calls of the same shape (new positions, occupancies, B,
- * form factors, metrics, targets) upload and replay it.
+ * plans and autotunes the GEMM tile and grid size, and on host arrays captures
+ * the step as a hipGraph; later calls of the same shape (new positions,
+ * occupancies, B, form factors, metrics, targets) upload and replay it.
+ * (dc_batch_chi2_dev on device arrays launches the kernels one by one.)
  * Arrays: pos (3, total), type/occ/bdw (total) member after member
  * (atom_beg[m] .. atom_beg[m+1]-1); cfact (ncfact, nscat, nmembers);
  * rten (9, nmembers); target/weight/icalc (P, nmembers) with P =
@@ -394,8 +397,9 @@ int dc_set_graphs(dc_ctx *ctx, int on);
 int dc_set_adjoint_walk(dc_ctx *ctx, int walk);
 /* Choice of the last batch shape: tile configuration, persistent work-groups
  * (0 = one per work item; negative = that many work-groups taking the work
- * items, longest first, from a device counter), whether a graph replays it,
- * autotuned GEMM ms. */
+ * items, longest first, from a device counter), whether a graph replays it
+ * (calls on host arrays, and device calls that go through copies), autotuned
+ * GEMM ms. */
 int dc_batch_info(const dc_ctx *ctx, int *tile, int *nwg, int *graph, double *tune_ms);
 
 /* ------------------------------------------------------------------------
